@@ -374,18 +374,38 @@ __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-__device__ __forceinline__ long wave_sum(long v) {
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
-}
-
 // v of lane l (l the same in every lane)
 __device__ __forceinline__ long read_lane(long v, int l) {
   const unsigned long long u = (unsigned long long)v;
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, l);
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
   return (long)(((unsigned long long)hi << 32) | lo);
+}
+
+// v moved across lanes by one DPP step (a register move: no LDS round trip as
+// a shuffle makes); lanes of rows outside kRows, or with no source, get 0.
+template <int kCtrl, int kRows = 0xf>
+__device__ __forceinline__ long dpp_move(long v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(unsigned long)v, kCtrl, kRows, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), kCtrl, kRows, 0xf, true);
+  return (long)(((unsigned long)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+
+constexpr int kDppShr1 = 0x111, kDppShr2 = 0x112, kDppShr4 = 0x114, kDppShr8 = 0x118;
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E;                // quad_perm [1,0,3,2], [2,3,0,1]
+constexpr int kDppHalfMirror = 0x141, kDppMirror = 0x140;      // within 8, within 16 lanes
+constexpr int kDppBcast15 = 0x142, kDppBcast31 = 0x143;        // last lane of the row(s) below
+
+// Sum over the wavefront's 64 lanes, all of them active (the callers' flow is
+// uniform): row sums by mirrors, then row to row; lane 63 holds the total.
+__device__ __forceinline__ long wave_sum(long v) {
+  v += dpp_move<kDppXor1>(v);
+  v += dpp_move<kDppXor2>(v);
+  v += dpp_move<kDppHalfMirror>(v);
+  v += dpp_move<kDppMirror>(v);
+  v += dpp_move<kDppBcast15, 0xa>(v);
+  v += dpp_move<kDppBcast31, 0xc>(v);
+  return read_lane(v, kWave - 1);
 }
 
 __device__ __forceinline__ i128 wave_sum128(i128 v) {
@@ -402,43 +422,72 @@ __device__ __forceinline__ i128 wave_sum128(i128 v) {
   return (i128)(((u128)(unsigned long)hi << 64) | (u128)lo);
 }
 
+// Inclusive scan over the wavefront's 64 lanes, all of them active.
 __device__ __forceinline__ long wave_incl_scan(long v) {
-  const int lane = lane_id();
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const long t = __shfl_up(v, off);
-    if (lane >= off) v += t;
-  }
+  v += dpp_move<kDppShr1>(v);
+  v += dpp_move<kDppShr2>(v);
+  v += dpp_move<kDppShr4>(v);
+  v += dpp_move<kDppShr8>(v);
+  v += dpp_move<kDppBcast15, 0xa>(v);
+  v += dpp_move<kDppBcast31, 0xc>(v);
   return v;
+}
+
+// A sum of terms m * lambda, |m| < 2^31 (a count, degree or sum of them),
+// |lambda| < 2^54: each lambda is split at bit 24 and the two products are
+// summed apart, value = h * 2^24 + l, so a term is two 32-bit multiply-adds
+// (an int128 product of 64-bit operands is about ten, at a quarter of the
+// ALU's rate).  Exact: the terms of one dS or MDL change or hold disjoint
+// edges' counts, so the |m| of each kind of term sum to at most the total
+// weight (< 2^31), at most four kinds of term do so, and |lambda| <= ln(2^31)
+// * 2^48 < 2^52.5 puts |h| below 2^62 and |l| below 2^58.  With the wavefront
+// sums by DPP and a dS's 16 uniform terms spread over 16 lanes it took
+// k_nodal from 126 to 90 VGPRs, a resumed chain at N = 50000 from 2.60 to
+// 2.19 ms and the N = 20000 partition from 25.5 to 22.5 ms.
+constexpr int kAccSplit = 24;
+struct Acc {
+  long h, l;
+};
+
+__device__ __forceinline__ void acc_add(Acc& a, int32_t m, int64_t L) {
+  a.h += (long)m * (long)(int32_t)(L >> kAccSplit);
+  a.l += (long)m * (long)((int32_t)L & ((1 << kAccSplit) - 1));
+}
+
+__device__ __forceinline__ i128 acc_value(const Acc& a) {
+  return (i128)(((u128)(i128)a.h << kAccSplit) + (u128)(i128)a.l);
 }
 
 // The terms read the lambda table unconditionally (lambda of m <= 0 reads
 // lam[0] = 0) and select the result, so the table loads of a whole dS are
 // issued together: a load under `if (m > 0)` would sit in its own branch and
 // wait for every earlier term's loads first.
-__device__ __forceinline__ int64_t lam_of(const int64_t* lam, int64_t m) {
-  return lam[m > 0 ? m : 0];
+__device__ __forceinline__ int64_t lam_of(const int64_t* lam, int32_t m) {
+  return lam[max(m, 0)];
 }
 
-// m * lambda(m): one L term
-__device__ __forceinline__ i128 Lterm(const int64_t* lam, int64_t m) {
-  const int64_t L = lam_of(lam, m);
-  return m > 0 ? (i128)m * (i128)L : (i128)0;
+// + or - m * lambda(m): one L term (0 for m <= 0)
+__device__ __forceinline__ void add_L(Acc& a, const int64_t* lam, int32_t m) {
+  acc_add(a, max(m, 0), lam_of(lam, m));
+}
+__device__ __forceinline__ void sub_L(Acc& a, const int64_t* lam, int32_t m) {
+  acc_add(a, -max(m, 0), lam_of(lam, m));
 }
 
-// m * lambda(d): one degree-factor term; inf when m > 0 and d == 0
-__device__ __forceinline__ i128 Pterm(const int64_t* lam, int64_t m, int64_t d, bool& inf) {
-  const int64_t L = lam_of(lam, d);
-  inf = inf || (m > 0 && d <= 0);
-  return (m > 0 && d > 0) ? (i128)m * (i128)L : (i128)0;
-}
-
-// T(m, x, y) = m*(lambda(m)-lambda(x)-lambda(y)); inf when m > 0 and x*y == 0
-__device__ __forceinline__ i128 Tterm(const int64_t* lam, int64_t m, int64_t x, int64_t y,
+// sign * m * lambda(d): one degree-factor term; inf when m > 0 and d == 0
+__device__ __forceinline__ void add_P(Acc& a, const int64_t* lam, int sign, int32_t m, int32_t d,
                                       bool& inf) {
+  inf = inf || (m > 0 && d <= 0);
+  acc_add(a, sign * max(m, 0), lam_of(lam, d));
+}
+
+// sign * T(m, x, y) = m*(lambda(m)-lambda(x)-lambda(y)); inf when m > 0 and x*y == 0
+__device__ __forceinline__ void add_T(Acc& a, const int64_t* lam, int sign, int32_t m, int32_t x,
+                                      int32_t y, bool& inf) {
   const int64_t Lm = lam_of(lam, m), Lx = lam_of(lam, x), Ly = lam_of(lam, y);
-  inf = inf || (m > 0 && (x <= 0 || y <= 0));
-  return (m > 0 && x > 0 && y > 0) ? (i128)m * (i128)(Lm - Lx - Ly) : (i128)0;
+  const bool bad = x <= 0 || y <= 0;
+  inf = inf || (m > 0 && bad);
+  acc_add(a, bad ? 0 : sign * max(m, 0), Lm - Lx - Ly);
 }
 
 // per-lane part of sum_{lo <= key <= x, key != excl} M[a][key] + M[key][a]
@@ -1170,22 +1219,25 @@ __global__ void k_iota(int64_t n, int32_t* v) {
 // data_S = -(sum_ab L(M_ab) - sum_a L(d_out[a]) - sum_b L(d_in[b]))
 // ---------------------------------------------------------------------------
 
-__device__ void block_store128(i128 v, long* out) {
-  __shared__ long s_hi[16];
-  __shared__ unsigned long s_lo[16];
-  v = wave_sum128(v);
+__device__ void block_store(Acc v, long* out) {
+  __shared__ long s_h[16], s_l[16];
+  v.h = wave_sum(v.h);
+  v.l = wave_sum(v.l);
   const int w = threadIdx.x / kWave;
   if (lane_id() == 0) {
-    s_hi[w] = (long)(v >> 64);
-    s_lo[w] = (unsigned long)(u128)v;
+    s_h[w] = v.h;
+    s_l[w] = v.l;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    i128 t = 0;
-    for (int i = 0; i < (int)(blockDim.x / kWave); ++i)
-      t += (i128)(((u128)(unsigned long)s_hi[i] << 64) | (u128)s_lo[i]);
-    out[0] = (long)(t >> 64);
-    out[1] = (long)(unsigned long)(u128)t;
+    Acc t{0, 0};
+    for (int i = 0; i < (int)(blockDim.x / kWave); ++i) {
+      t.h += s_h[i];
+      t.l += s_l[i];
+    }
+    const i128 x = acc_value(t);
+    out[0] = (long)(x >> 64);
+    out[1] = (long)(unsigned long)(u128)x;
   }
 }
 
@@ -1197,15 +1249,17 @@ __global__ __launch_bounds__(256) void k_entropy(const Slot* __restrict__ kv,
                                                  long* part) {
   const int64_t used = (int64_t)gst->used;  // every live slab lies below
   const int64_t nslots = used < P ? used : P;
-  i128 acc = 0;
+  Acc acc{0, 0};
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nslots; i += stride) {
     const int32_t v = kv[i].o;  // each M[a][b] once, as o of row a
-    if (v > 0) acc += (i128)v * (i128)lam[v];
+    if (v > 0) acc_add(acc, v, lam[v]);
   }
-  for (int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; b < B; b += stride)
-    acc -= Lterm(lam, d_out[b]) + Lterm(lam, d_in[b]);
-  block_store128(acc, part + 2 * blockIdx.x);
+  for (int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; b < B; b += stride) {
+    sub_L(acc, lam, d_out[b]);
+    sub_L(acc, lam, d_in[b]);
+  }
+  block_store(acc, part + 2 * blockIdx.x);
 }
 
 // Carry-out order (graph_parallel.hpp:1230) on the device: blocks sorted by
@@ -1244,29 +1298,36 @@ struct MergeArgs {
   unsigned long* best_lo;
 };
 
-// L(m1) + L(m2) - L(m1+m2) when both counts are non-zero, else 0.
-__device__ __forceinline__ i128 overlap_pair(const int64_t* lam, int32_t m1, int32_t m2) {
-  return (m1 > 0 && m2 > 0) ? Lterm(lam, m1) + Lterm(lam, m2) - Lterm(lam, (int64_t)m1 + m2)
-                            : (i128)0;
+// + L(m1) + L(m2) - L(m1+m2) when both counts are non-zero (no branch: a
+// wavefront's pairs are rarely all zero, and the loads of two pairs overlap).
+__device__ __forceinline__ void overlap_pair(Acc& acc, const int64_t* lam, int32_t m1,
+                                             int32_t m2) {
+  const bool both = m1 > 0 && m2 > 0;
+  const int32_t a = both ? m1 : 0, b = both ? m2 : 0;
+  const int64_t La = lam[a], Lb = lam[b], Lab = lam[a + b];
+  acc_add(acc, a, La);
+  acc_add(acc, b, Lb);
+  acc_add(acc, -(a + b), Lab);
 }
 
 // per-lane part of sum_{i not in {r,s}} [L(m1) + L(m2) - L(m1+m2)] over the
 // keys where rows r and s of M are both non-zero, and the same over the
 // columns (the only terms that survive the factorised merge dS): one pass
 // over the shorter block row, probing the other for each of its keys.
-__device__ i128 merge_overlap_lane(const MView& m, const int64_t* lam, int32_t r, int32_t s) {
+__device__ Acc merge_overlap_lane(const MView& m, const int64_t* lam, int32_t r, int32_t s) {
   const int lane = lane_id();
   const bool r_short = m.cap[r] <= m.cap[s];
   const int32_t a1 = r_short ? r : s, a2 = r_short ? s : r;
   const Row R1 = m_row(m, a1), R2 = m_row(m, a2);
   const bool direct = R1.c == m.B;
-  i128 acc = 0;
+  Acc acc{0, 0};
   if (direct) {  // then so is the longer row: key j sits at slot j of both
     for (int32_t j = lane; j < R1.c; j += kWave) {
       const int2 c1 = *reinterpret_cast<const int2*>(&m.kv[R1.o + j].o);
       const int2 c2 = *reinterpret_cast<const int2*>(&m.kv[R2.o + j].o);
       if (j == r || j == s) continue;
-      acc += overlap_pair(lam, c1.x, c2.x) + overlap_pair(lam, c1.y, c2.y);
+      overlap_pair(acc, lam, c1.x, c2.x);
+      overlap_pair(acc, lam, c1.y, c2.y);
     }
     return acc;
   }
@@ -1289,7 +1350,8 @@ __device__ i128 merge_overlap_lane(const MView& m, const int64_t* lam, int32_t r
     for (int u = 0; u < kOvl; ++u) {
       if (q[u].k < 0) continue;
       const Cnt c2 = m_value(m, R2, q[u].k, p[u]);
-      acc += overlap_pair(lam, q[u].o, c2.o) + overlap_pair(lam, q[u].i, c2.i);
+      overlap_pair(acc, lam, q[u].o, c2.o);
+      overlap_pair(acc, lam, q[u].i, c2.i);
     }
   }
   return acc;
@@ -1337,11 +1399,11 @@ __device__ __forceinline__ int32_t rowlds_find(const RowLds& L, int32_t b) {
 // merge_overlap_lane with row r from LDS: r's entries probe row s, or, when
 // s's slab is at most four times r's key count, s's slab is scanned and its
 // keys are looked up in r.
-__device__ i128 merge_overlap_lds(const MView& m, const int64_t* lam, int32_t r, int32_t s,
+__device__ Acc merge_overlap_lds(const MView& m, const int64_t* lam, int32_t r, int32_t s,
                                   const RowLds& L) {
   const int lane = lane_id();
   const Row RS = m_row(m, s);
-  i128 acc = 0;
+  Acc acc{0, 0};
   if (RS.c <= 4 * L.n) {
     const bool direct = RS.c == m.B;
     for (int32_t j = lane; j < RS.c; j += kWave) {
@@ -1350,18 +1412,16 @@ __device__ i128 merge_overlap_lds(const MView& m, const int64_t* lam, int32_t r,
       if (i < 0 || (q.o <= 0 && q.i <= 0) || i == r || i == s) continue;
       const int32_t p = rowlds_find(L, i);
       if (p < 0) continue;
-      const int32_t o1 = L.o[p], i1 = L.i[p];
-      if (o1 > 0 && q.o > 0) acc += Lterm(lam, o1) + Lterm(lam, q.o) - Lterm(lam, (int64_t)o1 + q.o);
-      if (i1 > 0 && q.i > 0) acc += Lterm(lam, i1) + Lterm(lam, q.i) - Lterm(lam, (int64_t)i1 + q.i);
+      overlap_pair(acc, lam, L.o[p], q.o);
+      overlap_pair(acc, lam, L.i[p], q.i);
     }
   } else {
     for (int32_t e = lane; e < L.n; e += kWave) {
       const int32_t i = L.k[e];
       if (i == r || i == s) continue;
       const Cnt c2 = m_value(m, RS, i, m_probe(m, RS, i));
-      const int32_t o1 = L.o[e], i1 = L.i[e];
-      if (o1 > 0 && c2.o > 0) acc += Lterm(lam, o1) + Lterm(lam, c2.o) - Lterm(lam, (int64_t)o1 + c2.o);
-      if (i1 > 0 && c2.i > 0) acc += Lterm(lam, i1) + Lterm(lam, c2.i) - Lterm(lam, (int64_t)i1 + c2.i);
+      overlap_pair(acc, lam, L.o[e], c2.o);
+      overlap_pair(acc, lam, L.i[e], c2.i);
     }
   }
   return acc;
@@ -1370,8 +1430,8 @@ __device__ i128 merge_overlap_lds(const MView& m, const int64_t* lam, int32_t r,
 __device__ void merge_one(const MergeArgs& a, int32_t r, int32_t idx, int32_t* scr,
                           const RowLds& L, int32_t& s_out, i128& dS_out) {
   const int32_t B = a.B;
-  const int64_t dor = a.d_out[r], dir = a.d_in[r];
-  const int64_t k = dor + dir;
+  const int32_t dor = a.d_out[r], dir = a.d_in[r];
+  const int64_t k = (int64_t)dor + dir;
   uint64_t x[4];
   if (a.uni)
     predrawn(a.uni, a.stream + (uint64_t)r * (uint64_t)a.K + (uint64_t)idx, x);
@@ -1401,22 +1461,27 @@ __device__ void merge_one(const MergeArgs& a, int32_t r, int32_t idx, int32_t* s
   }
   const int64_t* lam = a.lam;
   const Cnt crs = m_get(a.M, r, s);  // M[r][s], M[s][r]
-  const int64_t Mrr = m_get(a.M, r, r).o, Mrs = crs.o;
-  const int64_t Msr = crs.i, Mss = m_get(a.M, s, s).o;
-  const int64_t dos = a.d_out[s], dis = a.d_in[s];
-  const int64_t dos2 = dos + dor, dis2 = dis + dir;
-  i128 acc = L.n >= 0 ? merge_overlap_lds(a.M, lam, r, s, L) : merge_overlap_lane(a.M, lam, r, s);
-  acc = wave_sum128(acc);
+  const int32_t Mrr = m_get(a.M, r, r).o, Mrs = crs.o;
+  const int32_t Msr = crs.i, Mss = m_get(a.M, s, s).o;
+  const int32_t dos = a.d_out[s], dis = a.d_in[s];
+  const int32_t dos2 = dos + dor, dis2 = dis + dir;
+  const Acc ov = L.n >= 0 ? merge_overlap_lds(a.M, lam, r, s, L) : merge_overlap_lane(a.M, lam, r, s);
+  Acc acc{wave_sum(ov.h), wave_sum(ov.l)};
   bool inf = false;
-  const i128 old_c = Tterm(lam, Mrr, dir, dor, inf) + Tterm(lam, Mrs, dis, dor, inf) +
-                     Tterm(lam, Msr, dir, dos, inf) + Tterm(lam, Mss, dis, dos, inf);
-  const i128 new_c = Tterm(lam, Mrr + Mrs + Msr + Mss, dis2, dos2, inf);
-  const int64_t Xr = dor - Mrr - Mrs, Xs = dos - Msr - Mss;
-  const int64_t Yr = dir - Mrr - Msr, Ys = dis - Mrs - Mss;
-  const i128 deg = -Pterm(lam, Xr, dor, inf) - Pterm(lam, Xs, dos, inf) +
-                   Pterm(lam, Xr + Xs, dos2, inf) - Pterm(lam, Yr, dir, inf) -
-                   Pterm(lam, Ys, dis, inf) + Pterm(lam, Yr + Ys, dis2, inf);
-  dS_out = old_c - new_c + acc + deg;
+  add_T(acc, lam, 1, Mrr, dir, dor, inf);
+  add_T(acc, lam, 1, Mrs, dis, dor, inf);
+  add_T(acc, lam, 1, Msr, dir, dos, inf);
+  add_T(acc, lam, 1, Mss, dis, dos, inf);
+  add_T(acc, lam, -1, Mrr + Mrs + Msr + Mss, dis2, dos2, inf);
+  const int32_t Xr = dor - Mrr - Mrs, Xs = dos - Msr - Mss;
+  const int32_t Yr = dir - Mrr - Msr, Ys = dis - Mrs - Mss;
+  add_P(acc, lam, -1, Xr, dor, inf);
+  add_P(acc, lam, -1, Xs, dos, inf);
+  add_P(acc, lam, 1, Xr + Xs, dos2, inf);
+  add_P(acc, lam, -1, Yr, dir, inf);
+  add_P(acc, lam, -1, Ys, dis, inf);
+  add_P(acc, lam, 1, Yr + Ys, dis2, inf);
+  dS_out = acc_value(acc);
 }
 
 __global__ __launch_bounds__(kWave* kMergeWaves, 5) void k_merge(MergeArgs a) {
@@ -1702,25 +1767,25 @@ __device__ __forceinline__ void list_entry(const GraphView& g, int64_t o0, int64
 // neighbour-block table.  All lookups of a pass are issued before any is
 // resolved.
 __device__ __forceinline__ i128 nodal_delta(const NodalArgs& a, const Table& T, int32_t r,
-                                            int32_t s, Row rM, int64_t dor, int64_t dir,
-                                            int64_t kc, int64_t k_out, int64_t k_in, long wself,
+                                            int32_t s, Row rM, int32_t dor, int32_t dir,
+                                            int64_t kc, int32_t k_out, int32_t k_in, long wself_sum,
                                             bool& inf, long& bytes, int32_t s_pre, Row sM_pre,
-                                            int64_t dos_pre, int64_t dis_pre) {
+                                            int32_t dos_pre, int32_t dis_pre) {
   const int lane = lane_id();
   const int64_t* lam = a.lam;
   // s's row and degrees (loaded ahead when s is the uniform draw); the table
   // is compacted while they load
   const bool pre = s == s_pre;
   const Row sM = pre ? sM_pre : m_row(a.M, s);
-  const int64_t dos = pre ? dos_pre : a.d_out[s], dis = pre ? dis_pre : a.d_in[s];
-  long wor = 0, wir = 0, wos = 0, wis = 0;
-  const int32_t nent = tab_compact(T, r, s, wor, wir, wos, wis);
+  const int32_t dos = pre ? dos_pre : a.d_out[s], dis = pre ? dis_pre : a.d_in[s];
+  long wor_l = 0, wir_l = 0, wos_l = 0, wis_l = 0;
+  const int32_t nent = tab_compact(T, r, s, wor_l, wir_l, wos_l, wis_l);
   // corner: (r, r), (r, s) with (s, r) beside it, (s, s)
   const Probe pRR = m_probe(a.M, rM, r), pRS = m_probe(a.M, rM, s);
   const Probe pSS = m_probe(a.M, sM, s);
   // changed entries of rows r, s (out-edges, o) and columns r, s (in-edges,
   // i): one probe of block row r and one of s per neighbour block
-  i128 acc = 0;
+  Acc acc{0, 0};
   long lookups = 0;
   bool neg = false;
   for (int32_t j = lane; j < nent; j += kWave) {
@@ -1729,63 +1794,84 @@ __device__ __forceinline__ i128 nodal_delta(const NodalArgs& a, const Table& T, 
     const Cnt cr = m_value(a.M, rM, b, p0), cs = m_value(a.M, sM, b, p1);
     lookups += 2;
     if (wo > 0) {
-      const int64_t Rr = cr.o, Rs = cs.o;
-      neg |= Rr - wo < 0;
-      acc += Lterm(lam, Rr) + Lterm(lam, Rs) - Lterm(lam, Rr - wo) - Lterm(lam, Rs + wo);
+      neg |= cr.o - wo < 0;
+      add_L(acc, lam, cr.o);
+      add_L(acc, lam, cs.o);
+      sub_L(acc, lam, cr.o - wo);
+      sub_L(acc, lam, cs.o + wo);
     }
     if (wi > 0) {
-      const int64_t Cr = cr.i, Cs = cs.i;
-      neg |= Cr - wi < 0;
-      acc += Lterm(lam, Cr) + Lterm(lam, Cs) - Lterm(lam, Cr - wi) - Lterm(lam, Cs + wi);
+      neg |= cr.i - wi < 0;
+      add_L(acc, lam, cr.i);
+      add_L(acc, lam, cs.i);
+      sub_L(acc, lam, cr.i - wi);
+      sub_L(acc, lam, cs.i + wi);
     }
   }
   if (neg) atomicOr(&a.status->flags, kFlagNegative);
-  acc = wave_sum128(acc);
   // blocks r and s own one table slot each, so one lane at most holds their
   // weights; the other entries' weights are the rest of k_out / k_in
-  const unsigned long long hr = __ballot(wor != 0 || wir != 0);
-  const unsigned long long hs = __ballot(wos != 0 || wis != 0);
-  wor = hr ? read_lane(wor, __ffsll(hr) - 1) : 0;
-  wir = hr ? read_lane(wir, __ffsll(hr) - 1) : 0;
-  wos = hs ? read_lane(wos, __ffsll(hs) - 1) : 0;
-  wis = hs ? read_lane(wis, __ffsll(hs) - 1) : 0;
-  const long Wo = k_out - wor - wos, Wi = k_in - wir - wis;
-  if (__ballot(wself != 0)) wself = wave_sum(wself);  // self-loops are rare
+  const unsigned long long hr = __ballot(wor_l != 0 || wir_l != 0);
+  const unsigned long long hs = __ballot(wos_l != 0 || wis_l != 0);
+  const int lr = hr ? __ffsll(hr) - 1 : 0, ls = hs ? __ffsll(hs) - 1 : 0;
+  const int32_t wor = __builtin_amdgcn_readlane((int32_t)wor_l, lr);
+  const int32_t wir = __builtin_amdgcn_readlane((int32_t)wir_l, lr);
+  const int32_t wos = __builtin_amdgcn_readlane((int32_t)wos_l, ls);
+  const int32_t wis = __builtin_amdgcn_readlane((int32_t)wis_l, ls);
+  const int32_t Wo = k_out - wor - wos, Wi = k_in - wir - wis;
+  int32_t wself = 0;
+  if (__ballot(wself_sum != 0)) wself = (int32_t)wave_sum(wself_sum);  // self-loops are rare
   // neighbour ids + labels (+ weights); rows (offset + capacity) and degrees
   // of r and s; 2 block-row lookups (key + two counts) per changed entry and
   // 3 corner lookups
   bytes += (a.g.out_w ? 12 : 8) * kc + 24 + 16 + 12 * (wave_sum(lookups) + 3);
   const Cnt crs = m_value(a.M, rM, s, pRS);
-  const int64_t Mrr = m_value(a.M, rM, r, pRR).o, Mrs = crs.o;
-  const int64_t Msr = crs.i, Mss = m_value(a.M, sM, s, pSS).o;
-  const int64_t dor2 = dor - k_out, dos2 = dos + k_out, dir2 = dir - k_in, dis2 = dis + k_in;
-  int64_t rr2, rs2, sr2, ss2;
+  const int32_t Mrr = m_value(a.M, rM, r, pRR).o, Mrs = crs.o;
+  const int32_t Msr = crs.i, Mss = m_value(a.M, sM, s, pSS).o;
+  int32_t rr2, rs2, sr2, ss2;
   if (!a.exact) {  // graph_parallel.hpp:1117-1145: only out-edges update the rows
     rr2 = Mrr - wor;
     rs2 = Mrs - wos;
     sr2 = Msr + wor;
     ss2 = Mss + wos;
   } else {  // graph.cu:1414-1426, with a self-loop moving (r,r) -> (s,s)
-    const int64_t wor_ = wor - wself, wir_ = wir - wself;
+    const int32_t wor_ = wor - wself, wir_ = wir - wself;
     rr2 = Mrr - wor_ - wself - wir_;
     rs2 = Mrs - wos + wir_;
     sr2 = Msr + wor_ - wis;
     ss2 = Mss + wos + wis + wself;
   }
-  bool old_inf = false;
-  const i128 old_c = Tterm(lam, Mrr, dir, dor, old_inf) + Tterm(lam, Mrs, dis, dor, old_inf) +
-                     Tterm(lam, Msr, dir, dos, old_inf) + Tterm(lam, Mss, dis, dos, old_inf);
-  const i128 new_c = Tterm(lam, rr2, dir2, dor2, inf) + Tterm(lam, rs2, dis2, dor2, inf) +
-                     Tterm(lam, sr2, dir2, dos2, inf) + Tterm(lam, ss2, dis2, dos2, inf);
-  const int64_t Xr = dor - Mrr - Mrs, Xs = dos - Msr - Mss;
-  const int64_t Yr = dir - Mrr - Msr, Ys = dis - Mrs - Mss;
-  const i128 deg_old = Pterm(lam, Xr, dor, old_inf) + Pterm(lam, Xs, dos, old_inf) +
-                       Pterm(lam, Yr, dir, old_inf) + Pterm(lam, Ys, dis, old_inf);
-  const i128 deg_new = Pterm(lam, Xr - Wo, dor2, inf) + Pterm(lam, Xs + Wo, dos2, inf) +
-                       Pterm(lam, Yr - Wi, dir2, inf) + Pterm(lam, Ys + Wi, dis2, inf);
+  const int32_t Xr = dor - Mrr - Mrs, Xs = dos - Msr - Mss;
+  const int32_t Yr = dir - Mrr - Msr, Ys = dis - Mrs - Mss;
   if (rr2 < 0 || rs2 < 0 || sr2 < 0 || ss2 < 0 || Xr - Wo < 0 || Yr - Wi < 0)
     atomicOr(&a.status->flags, kFlagNegative);
-  return old_c - new_c + acc - deg_old + deg_new;
+  // The 16 corner and degree terms, one per lane (in every lane they were a
+  // quarter of the kernel's arithmetic).  Lane bits: col (0: column r, 1: s),
+  // row (0: row r, 1: s), new (0: before the move, 1: after), deg.
+  //   deg = 0: T(M[row][col], d_in[col], d_out[row])
+  //   deg = 1: the row's other out-edges X (col = 0) or the column's other
+  //            in-edges Y (col = 1) of block `row`, m * lambda(degree)
+  // each + before and - after, the degree terms the other way round.
+  const bool col = lane & 1, row = lane & 2, now = lane & 4, deg = lane & 8;
+  const bool in2 = deg ? row : col;  // whose d_in
+  const int32_t dout = (row ? dos : dor) + (now ? (row ? k_out : -k_out) : 0);
+  const int32_t din = (in2 ? dis : dir) + (now ? (in2 ? k_in : -k_in) : 0);
+  const int32_t mt = now ? (row ? (col ? ss2 : sr2) : (col ? rs2 : rr2))
+                         : (row ? (col ? Mss : Msr) : (col ? Mrs : Mrr));
+  const int32_t dW = now ? (col ? Wi : Wo) : 0;
+  const int32_t mp = (col ? (row ? Ys : Yr) : (row ? Xs : Xr)) + (row ? dW : -dW);
+  const int32_t m = deg ? mp : mt;
+  const int32_t d1 = deg && !col ? dout : din, d2 = deg ? 1 : dout;  // lambda(1) = 0
+  const bool bad = d1 <= 0 || d2 <= 0;
+  const int64_t c = lam_of(lam, deg ? 0 : m) - lam_of(lam, d1) - lam_of(lam, d2);
+  if (lane < 16) {
+    const int32_t mm = bad ? 0 : max(m, 0);
+    acc_add(acc, now ? -mm : mm, c);
+  }
+  inf = __ballot(lane < 16 && now && bad && m > 0) != 0;
+  acc.h = wave_sum(acc.h);
+  acc.l = wave_sum(acc.l);
+  return acc_value(acc);
 }
 
 // One nodal proposal (graph_parallel.hpp:990-1222) for node n, batch item
@@ -1809,12 +1895,12 @@ __device__ __forceinline__ long nodal_one(const NodalArgs& a, int64_t item, int3
   else
     usap::philox4x64((uint64_t)n, 0, stream0 + (uint64_t)a.bidx, usap::kTagNodal, a.seed, 0, x);
   const Row rM = m_row(a.M, r);
-  const int64_t dor = a.d_out[r], dir = a.d_in[r];
+  const int32_t dor = a.d_out[r], dir = a.d_in[r];
   // the uniform draw's block, the proposal in most cases: its row and
   // degrees load with r's
   const int32_t s_pre = (int32_t)usap::idx_of(x[2], B);
   const Row sM_pre = m_row(a.M, s_pre);
-  const int64_t dos_pre = a.d_out[s_pre], dis_pre = a.d_in[s_pre];
+  const int32_t dos_pre = a.d_out[s_pre], dis_pre = a.d_in[s_pre];
   int64_t k_out = kco, k_in = kci;
   if (g.out_w) {
     long so = 0, si = 0;
@@ -1884,8 +1970,8 @@ __device__ __forceinline__ long nodal_one(const NodalArgs& a, int64_t item, int3
   int32_t acc = 0;
   if (s != r) {
     wave_fence();  // the table is complete
-    dS = nodal_delta(a, T, r, s, rM, dor, dir, kc, k_out, k_in, wself, inf, bytes, s_pre, sM_pre,
-                     dos_pre, dis_pre);
+    dS = nodal_delta(a, T, r, s, rM, dor, dir, kc, (int32_t)k_out, (int32_t)k_in, wself, inf,
+                     bytes, s_pre, sM_pre, dos_pre, dis_pre);
     acc = (inf || dS < 0) ? 1 : 0;
   }
   if (lane == 0) {
