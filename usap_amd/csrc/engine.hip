@@ -129,16 +129,9 @@ struct GraphView {
   const int32_t* in_w;
 };
 
-// One slot of a block row slab: key (-1 empty; unused in a direct row) and
-// the pair's two counts, o = M[a][key] and i = M[key][a].  (o, i) is 8-byte
-// aligned: one 64-bit atomic adds to both.
-struct __align__(16) Slot {
-  int32_t k, pad;
-  int32_t o, i;
-};
-
-// The two counts of a block pair (a, b): o = M[a][b], i = M[b][a].
-struct Cnt {
+// The two counts of a block pair (a, b): o = M[a][b], i = M[b][a]; 8-byte
+// aligned, one 64-bit atomic adds to both.
+struct __align__(8) Cnt {
   int32_t o, i;
 };
 
@@ -147,7 +140,8 @@ struct MView {
   const int64_t* off;
   const int32_t* cap;
   int32_t* nkeys;
-  Slot* kv;        // row slabs
+  int32_t* key;    // row slabs: keys (-1 empty; unused in a direct row) ...
+  Cnt* cnt;        // ... and the counts of each slot
   int32_t* bs;     // [B][kNBK]: sum of the row's o + i per key bucket
   int32_t* gpend;  // [B]: increments of the row waiting in the overflow buffer
   int32_t* ovf;    // [4][ovf_cap]: (row, key, do, di) increments that found no free slot
@@ -193,43 +187,44 @@ __device__ __forceinline__ int64_t m_slot(const MView& m, Row R, int32_t b) {
   return R.c == m.B ? R.o + b : R.o + (int64_t)(hash32(b) & (uint32_t)(R.c - 1));
 }
 
-// A lookup's first probe: the slot with the key and count found there.  The
+// A lookup's first probe: the slot with the key and counts found there.  The
 // callers issue several probes before resolving any, so a wavefront has all
 // of its lookups in flight at once instead of one memory latency per lookup.
 struct Probe {
   uint32_t h;  // slot within the row
-  int32_t k, o, i;
+  int32_t k;
+  Cnt c;
 };
+
+__device__ __forceinline__ uint32_t m_home(const MView& m, Row R, int32_t b) {
+  return R.c == m.B ? (uint32_t)b : hash32(b) & (uint32_t)(R.c - 1);
+}
 
 __device__ __forceinline__ Probe m_probe(const MView& m, Row R, int32_t b) {
   Probe p;
-  p.h = R.c == m.B ? (uint32_t)b : hash32(b) & (uint32_t)(R.c - 1);
-  const Slot q = m.kv[R.o + p.h];
-  p.k = q.k;
-  p.o = q.o;
-  p.i = q.i;
+  p.h = m_home(m, R, b);
+  p.k = R.c == m.B ? b : m.key[R.o + p.h];
+  p.c = m.cnt[R.o + p.h];
   return p;
 }
 
 // Linear probing on from slot `slot` of a hashed row after a collision there.
-__device__ __forceinline__ Cnt m_value_more(const Slot* kv, int64_t o, int32_t c, int32_t b,
-                                            int64_t slot) {
-  const uint32_t mask = (uint32_t)c - 1;
-  uint32_t h = (uint32_t)(slot - o);
-  for (int32_t probe = 1; probe < c; ++probe) {
+__device__ __forceinline__ Cnt m_value_more(const MView& m, Row R, int32_t b, uint32_t h) {
+  const uint32_t mask = (uint32_t)R.c - 1;
+  for (int32_t probe = 1; probe < R.c; ++probe) {
     h = (h + 1) & mask;
-    const Slot q = kv[o + h];
-    if (q.k == b) return Cnt{q.o, q.i};
-    if (q.k < 0) return Cnt{0, 0};
+    const int32_t k = m.key[R.o + h];
+    if (k == b) return m.cnt[R.o + h];
+    if (k < 0) return Cnt{0, 0};
   }
   return Cnt{0, 0};
 }
 
 // (M[a][b], M[b][a]) from the first probe p of key b in row R of a.
 __device__ __forceinline__ Cnt m_value(const MView& m, Row R, int32_t b, const Probe& p) {
-  if (R.c == m.B || p.k == b) return Cnt{p.o, p.i};
+  if (p.k == b) return p.c;
   if (p.k < 0) return Cnt{0, 0};
-  return m_value_more(m.kv, R.o, R.c, b, R.o + p.h);
+  return m_value_more(m, R, b, p.h);
 }
 
 // (M[a][b], M[b][a])
@@ -241,9 +236,9 @@ __device__ __forceinline__ Cnt m_get(const MView& m, int32_t a, int32_t b) {
 // o += dout, i += din with one 64-bit atomic.  Exact as long as neither count
 // leaves [0, 2^31) at any point, which holds for every caller: a decrement
 // only removes edges the count held when the kernel started.
-__device__ __forceinline__ void cnt_add(Slot* q, int32_t dout, int32_t din) {
+__device__ __forceinline__ void cnt_add(Cnt* q, int32_t dout, int32_t din) {
   const long long d = (long long)din * 4294967296LL + (long long)dout;
-  atomicAdd(reinterpret_cast<unsigned long long*>(&q->o), (unsigned long long)d);
+  atomicAdd(reinterpret_cast<unsigned long long*>(q), (unsigned long long)d);
 }
 
 constexpr int32_t kMaxWalk = 16;  // probes before a nodal-batch increment is parked
@@ -261,7 +256,7 @@ __device__ __forceinline__ void m_add_at(const MView& m, int32_t a, Row R, int32
   if (kBuckets && dout + din != 0)
     atomicAdd(&m.bs[(int64_t)a * kNBK + (b >> m.bshift)], dout + din);
   if (R.c == m.B || k == b) {
-    cnt_add(&m.kv[slot], dout, din);
+    cnt_add(&m.cnt[slot], dout, din);
     return;
   }
   const bool dec = dout < 0 || din < 0;
@@ -273,19 +268,19 @@ __device__ __forceinline__ void m_add_at(const MView& m, int32_t a, Row R, int32
     // an increment whose key is still absent after kMaxWalk slots is parked
     // (k_grow grows the row) rather than walking a crowded row
     if (kBuckets && !dec && probe >= kMaxWalk) break;
-    if (probe > 0) k = ld_relaxed(&m.kv[o + h].k);
+    if (probe > 0) k = ld_relaxed(&m.key[o + h]);
     if (k < 0) {
       if (dec) {
         atomicOr(flags, kFlagMissing);
         return;
       }
-      k = atomicCAS(&m.kv[o + h].k, -1, b);
+      k = atomicCAS(&m.key[o + h], -1, b);
       if (k == -1) {
         if (kBuckets) {
           // the counts and the key count without waiting for either: k_grow
           // finds the rows past 1/slack load (short probe chains for the
           // lookups, most of which miss) from the key counts themselves
-          cnt_add(&m.kv[o + h], dout, din);
+          cnt_add(&m.cnt[o + h], dout, din);
           atomicAdd(&m.nkeys[a], 1);
           return;
         }
@@ -295,7 +290,7 @@ __device__ __forceinline__ void m_add_at(const MView& m, int32_t a, Row R, int32
       }
     }
     if (k == b) {
-      cnt_add(&m.kv[o + h], dout, din);
+      cnt_add(&m.cnt[o + h], dout, din);
       return;
     }
     h = (h + 1) & mask;
@@ -316,29 +311,30 @@ __device__ __forceinline__ void m_add_at(const MView& m, int32_t a, Row R, int32
 }
 
 // Where m_add_at starts for key b in row R: the keys of kWin slots from b's
-// home slot are read at once (one memory latency for most probe chains) and
-// the first that holds b or is empty is returned with its slot; if none does,
-// the window's last slot, from which m_add_at walks on.
+// home slot are read at once (two 16-byte loads; one memory latency for most
+// probe chains) and the first that holds b or is empty is returned with its
+// slot; if none does, the window's last slot, from which m_add_at walks on.
+// The window ends at the slab's end at the latest.  Keys only go from empty
+// to set, so a plain load is as good as a relaxed atomic one.
 constexpr int kWin = 8;
+typedef int32_t Key4 __attribute__((ext_vector_type(4), aligned(4)));  // 4-byte aligned
 __device__ __forceinline__ int32_t m_first_key(const MView& m, Row R, int32_t b, int64_t& slot) {
   if (R.c == m.B) {
     slot = R.o + b;
     return b;
   }
-  const uint32_t mask = (uint32_t)R.c - 1;  // hashed rows hold >= 32 slots
-  const uint32_t h = hash32(b) & mask;
-  int32_t k[kWin];
-#pragma unroll
-  for (int q = 0; q < kWin; ++q) k[q] = ld_relaxed(&m.kv[R.o + ((h + q) & mask)].k);
+  const uint32_t h = hash32(b) & ((uint32_t)R.c - 1);  // hashed rows hold >= 32 slots
+  const uint32_t w0 = min(h, (uint32_t)R.c - kWin);
+  const Key4* w = reinterpret_cast<const Key4*>(m.key + R.o + w0);
+  const Key4 lo = w[0], hi = w[1];
+  const int32_t k[kWin] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
   int32_t kk = k[kWin - 1];
-  uint32_t pos = (h + kWin - 1) & mask;
-  bool found = false;
+  uint32_t pos = w0 + kWin - 1;
 #pragma unroll
-  for (int q = 0; q < kWin; ++q) {
-    if (!found && (k[q] == b || k[q] < 0)) {
-      found = true;
+  for (int q = kWin - 2; q >= 0; --q) {  // the first slot from h on that ends the chain
+    if (w0 + q >= h && (k[q] == b || k[q] < 0)) {
       kk = k[q];
-      pos = (h + q) & mask;
+      pos = w0 + q;
     }
   }
   slot = R.o + pos;
@@ -498,11 +494,12 @@ __device__ __forceinline__ long count_range_lane(const MView& m, int64_t o, int3
   long acc = 0;
   if (c == m.B) {
     for (int32_t i = lo + lane; i <= x; i += kWave)
-      if (i != excl) acc += (long)m.kv[o + i].o + m.kv[o + i].i;
+      if (i != excl) acc += (long)m.cnt[o + i].o + m.cnt[o + i].i;
   } else {
     for (int32_t j = lane; j < c; j += kWave) {
-      const Slot q = m.kv[o + j];
-      if (q.k >= lo && q.k <= x && q.k != excl) acc += (long)q.o + q.i;
+      const int32_t k = m.key[o + j];
+      const Cnt q = m.cnt[o + j];
+      if (k >= lo && k <= x && k != excl) acc += (long)q.o + q.i;
     }
   }
   return acc;
@@ -516,7 +513,7 @@ __device__ __forceinline__ void gather_row(const MView& m, Row R, int32_t lo, in
   const int lane = lane_id();
   if (R.c == m.B) {
     for (int32_t i = lane; i < hi - lo; i += kWave) {
-      const Slot q = m.kv[R.o + lo + i];
+      const Cnt q = m.cnt[R.o + lo + i];
       atomicAdd(&scr[i], q.o + q.i);
     }
     bytes += 8 * (long)(hi - lo);
@@ -530,8 +527,8 @@ __device__ __forceinline__ void gather_row(const MView& m, Row R, int32_t lo, in
       k[q] = -1;
       v[q] = 0;
       if (j < R.c) {
-        const Slot x = m.kv[R.o + j];
-        k[q] = x.k;
+        const Cnt x = m.cnt[R.o + j];
+        k[q] = m.key[R.o + j];
         v[q] = x.o + x.i;
       }
     }
@@ -564,19 +561,23 @@ __device__ __forceinline__ void lookup_bucket(const MView& m, Row R, int32_t lo,
       if (key < hi) pend |= 1u << q;
     }
     for (int32_t step = 0; step < R.c && __ballot(pend != 0); ++step) {
-      Slot x[4];
+      int32_t k[4];
+      Cnt x[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        if ((pend >> q) & 1) x[q] = m.kv[R.o + h[q]];
+        if ((pend >> q) & 1) {
+          k[q] = m.key[R.o + h[q]];
+          x[q] = m.cnt[R.o + h[q]];
+        }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         bytes += 16 * (long)__popcll(__ballot((pend >> q) & 1));
         if (!((pend >> q) & 1)) continue;
         const int32_t key = base + q * kWave + lane;
-        if (x[q].k == key) {
+        if (k[q] == key) {
           wv[q] = x[q].o + x[q].i;
           pend &= ~(1u << q);
-        } else if (x[q].k < 0) {
+        } else if (k[q] < 0) {
           pend &= ~(1u << q);
         } else {
           h[q] = (h[q] + 1) & mask;
@@ -684,7 +685,7 @@ __device__ __forceinline__ int32_t select_combined(const MView& M, int32_t u, in
     long w = 0;
     const int32_t i = lo + lane;
     if (lane < width && i != excl) {
-      const Slot q = M.kv[RM.o + i];
+      const Cnt q = M.cnt[RM.o + i];
       w = (long)q.o + q.i;
     }
     bytes += 8 * (long)width;
@@ -701,7 +702,7 @@ __device__ __forceinline__ int32_t select_combined(const MView& M, int32_t u, in
           const int32_t i = base + q * kWave + lane;
           v[q] = 0;
           if (i < width) {
-            const Slot x = M.kv[RM.o + lo + i];
+            const Cnt x = M.cnt[RM.o + lo + i];
             v[q] = x.o + x.i;
           }
         }
@@ -837,10 +838,12 @@ __global__ void k_caps(int32_t B, int32_t slack, const int32_t* ecnt_out, const 
   tmp[a] = c;
 }
 
-__global__ void k_fill(Slot* kv, int64_t n) {
+// key null: every row is direct, no key is read.
+__global__ void k_fill(int32_t* key, Cnt* cnt, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
-    kv[i] = Slot{-1, 0, 0, 0};
+    if (key) key[i] = -1;
+    cnt[i] = Cnt{0, 0};
   }
 }
 
@@ -979,7 +982,10 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_build_rows(
     }
   }
   wave_fence();
-  for (int32_t j = lane; j < c; j += kWave) M.kv[o + j] = Slot{tk[j], 0, to[j], ti[j]};
+  for (int32_t j = lane; j < c; j += kWave) {
+    M.key[o + j] = tk[j];
+    M.cnt[o + j] = Cnt{to[j], ti[j]};
+  }
   nk = wave_sum(nk);
   if (lane == 0) M.nkeys[a] = (int32_t)nk;
   if (__ballot(full)) {
@@ -1006,8 +1012,8 @@ __global__ __launch_bounds__(256) void k_insert_small(int64_t E, const int32_t* 
     const int32_t v = s_h[i];
     if (!v) continue;
     const int32_t a = i / B, b = i - a * B;
-    atomicAdd(&M.kv[M.off[a] + b].o, v);
-    atomicAdd(&M.kv[M.off[b] + a].i, v);
+    atomicAdd(&M.cnt[M.off[a] + b].o, v);
+    atomicAdd(&M.cnt[M.off[b] + a].i, v);
   }
 }
 
@@ -1065,8 +1071,8 @@ __global__ __launch_bounds__(256) void k_bucket_sums(MView m) {
   const int32_t c = m.cap[a];
   const bool direct = c == m.B;
   for (int32_t j = lane; j < c; j += kWave) {
-    const Slot q = m.kv[o + j];
-    const int32_t k = direct ? j : q.k;
+    const Cnt q = m.cnt[o + j];
+    const int32_t k = direct ? j : m.key[o + j];
     const int32_t v = q.o + q.i;
     if (k >= 0 && v != 0) atomicAdd(&bk[k >> m.bshift], v);
   }
@@ -1241,7 +1247,7 @@ __device__ void block_store(Acc v, long* out) {
   }
 }
 
-__global__ __launch_bounds__(256) void k_entropy(const Slot* __restrict__ kv,
+__global__ __launch_bounds__(256) void k_entropy(const Cnt* __restrict__ cnt,
                                                  const GrowState* gst,
                                                  const int32_t* __restrict__ d_out,
                                                  const int32_t* __restrict__ d_in, int32_t B,
@@ -1252,7 +1258,7 @@ __global__ __launch_bounds__(256) void k_entropy(const Slot* __restrict__ kv,
   Acc acc{0, 0};
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nslots; i += stride) {
-    const int32_t v = kv[i].o;  // each M[a][b] once, as o of row a
+    const int32_t v = cnt[i].o;  // each M[a][b] once, as o of row a
     if (v > 0) acc_add(acc, v, lam[v]);
   }
   for (int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; b < B; b += stride) {
@@ -1323,11 +1329,10 @@ __device__ Acc merge_overlap_lane(const MView& m, const int64_t* lam, int32_t r,
   Acc acc{0, 0};
   if (direct) {  // then so is the longer row: key j sits at slot j of both
     for (int32_t j = lane; j < R1.c; j += kWave) {
-      const int2 c1 = *reinterpret_cast<const int2*>(&m.kv[R1.o + j].o);
-      const int2 c2 = *reinterpret_cast<const int2*>(&m.kv[R2.o + j].o);
+      const Cnt c1 = m.cnt[R1.o + j], c2 = m.cnt[R2.o + j];
       if (j == r || j == s) continue;
-      overlap_pair(acc, lam, c1.x, c2.x);
-      overlap_pair(acc, lam, c1.y, c2.y);
+      overlap_pair(acc, lam, c1.o, c2.o);
+      overlap_pair(acc, lam, c1.i, c2.i);
     }
     return acc;
   }
@@ -1335,21 +1340,24 @@ __device__ Acc merge_overlap_lane(const MView& m, const int64_t* lam, int32_t r,
   // the other row issued before any is resolved
   constexpr int kOvl = 4;
   for (int32_t base = 0; base < R1.c; base += kOvl * kWave) {
-    Slot q[kOvl];
+    int32_t k[kOvl];
+    Cnt q[kOvl];
 #pragma unroll
     for (int u = 0; u < kOvl; ++u) {
       const int32_t j = base + u * kWave + lane;
-      q[u] = j < R1.c ? m.kv[R1.o + j] : Slot{-1, 0, 0, 0};
-      if (q[u].k < 0 || (q[u].o <= 0 && q[u].i <= 0) || q[u].k == r || q[u].k == s) q[u].k = -1;
+      k[u] = j < R1.c ? m.key[R1.o + j] : -1;
+      q[u] = j < R1.c ? m.cnt[R1.o + j] : Cnt{0, 0};
     }
     Probe p[kOvl];
 #pragma unroll
-    for (int u = 0; u < kOvl; ++u)
-      if (q[u].k >= 0) p[u] = m_probe(m, R2, q[u].k);
+    for (int u = 0; u < kOvl; ++u) {
+      if ((q[u].o <= 0 && q[u].i <= 0) || k[u] == r || k[u] == s) k[u] = -1;
+      if (k[u] >= 0) p[u] = m_probe(m, R2, k[u]);
+    }
 #pragma unroll
     for (int u = 0; u < kOvl; ++u) {
-      if (q[u].k < 0) continue;
-      const Cnt c2 = m_value(m, R2, q[u].k, p[u]);
+      if (k[u] < 0) continue;
+      const Cnt c2 = m_value(m, R2, k[u], p[u]);
       overlap_pair(acc, lam, q[u].o, c2.o);
       overlap_pair(acc, lam, q[u].i, c2.i);
     }
@@ -1407,8 +1415,8 @@ __device__ Acc merge_overlap_lds(const MView& m, const int64_t* lam, int32_t r, 
   if (RS.c <= 4 * L.n) {
     const bool direct = RS.c == m.B;
     for (int32_t j = lane; j < RS.c; j += kWave) {
-      const Slot q = m.kv[RS.o + j];
-      const int32_t i = direct ? j : q.k;
+      const Cnt q = m.cnt[RS.o + j];
+      const int32_t i = direct ? j : m.key[RS.o + j];
       if (i < 0 || (q.o <= 0 && q.i <= 0) || i == r || i == s) continue;
       const int32_t p = rowlds_find(L, i);
       if (p < 0) continue;
@@ -1505,8 +1513,8 @@ __global__ __launch_bounds__(kWave* kMergeWaves, 5) void k_merge(MergeArgs a) {
   if (fits) {
     const bool direct = R.c == a.B;
     for (int32_t j = threadIdx.x; j < R.c; j += blockDim.x) {
-      const Slot q = a.M.kv[R.o + j];
-      const int32_t key = direct ? j : q.k;
+      const Cnt q = a.M.cnt[R.o + j];
+      const int32_t key = direct ? j : a.M.key[R.o + j];
       if (key >= 0 && (q.o > 0 || q.i > 0)) {
         const int32_t p = atomicAdd(&s_rn, 1);
         if (p < kRowLds) {
@@ -1790,7 +1798,13 @@ __device__ __forceinline__ i128 nodal_delta(const NodalArgs& a, const Table& T, 
   bool neg = false;
   for (int32_t j = lane; j < nent; j += kWave) {
     const int32_t b = T.tk[j], wo = T.two[j], wi = T.twi[j];
-    const Probe p0 = m_probe(a.M, rM, b), p1 = m_probe(a.M, sM, b);
+    // n's edges into b put b among row r's keys; row s, when hashed, is most
+    // often a uniform draw without b (B >= 8 slabs is >= 16 row degrees), so
+    // its keys alone are read first
+    const Probe p0 = m_probe(a.M, rM, b);
+    Probe p1{m_home(a.M, sM, b), b, {0, 0}};
+    if (sM.c != a.M.B) p1.k = a.M.key[sM.o + p1.h];
+    if (p1.k == b) p1.c = a.M.cnt[sM.o + p1.h];
     const Cnt cr = m_value(a.M, rM, b, p0), cs = m_value(a.M, sM, b, p1);
     lookups += 2;
     if (wo > 0) {
@@ -2109,7 +2123,7 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_aq(AqArgs a) {
     const int32_t c = a.M.cap[bb];
     long nz = 0;
     for (int32_t j = lane; j < c; j += kWave) {
-      const Slot q = a.M.kv[o + j];
+      const Cnt q = a.M.cnt[o + j];
       nz += (q.o > 0 ? 1 : 0) + (q.i > 0 ? 1 : 0);
     }
     blk += 16 + 8 * (unsigned long long)wave_sum(nz) + 12;
@@ -2142,12 +2156,12 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_aq(AqArgs a) {
 // Profiling only: 16 bytes per non-zero of M (its entry read from the row
 // and from the column structure of graph_parallel.hpp:761-988), spread over
 // acc[0 .. kAqSlots).
-__global__ __launch_bounds__(256) void k_nnz_bytes(const Slot* __restrict__ kv, int64_t P,
+__global__ __launch_bounds__(256) void k_nnz_bytes(const Cnt* __restrict__ cnt, int64_t P,
                                                    unsigned long long* acc) {
   long c = 0;
   for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < P;
        j += (int64_t)gridDim.x * blockDim.x)
-    c += kv[j].o > 0 ? 1 : 0;
+    c += cnt[j].o > 0 ? 1 : 0;
   c = wave_sum(c);
   if (lane_id() == 0 && c)
     atomicAdd(&acc[(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave) % kAqSlots],
@@ -2531,7 +2545,8 @@ struct GrowSide {
   int64_t* off;
   int32_t* cap;
   int32_t* nkeys;
-  Slot* kv;
+  int32_t* key;
+  Cnt* cnt;
   int32_t* gpend;
   const int32_t* ovf;
   int32_t ovf_cap;
@@ -2560,23 +2575,23 @@ __device__ void replay_row(const GrowSide& g, int32_t a, int64_t o, int32_t c, i
     const int32_t b = g.ovf[g.ovf_cap + i];
     const int32_t dout = g.ovf[2 * g.ovf_cap + i], din = g.ovf[3 * g.ovf_cap + i];
     if (c == B) {
-      cnt_add(&g.kv[o + b], dout, din);
+      cnt_add(&g.cnt[o + b], dout, din);
       continue;
     }
     const uint32_t mask = (uint32_t)c - 1;
     uint32_t h = hash32(b) & mask;
     bool done = false;
     for (int32_t probe = 0; probe < c && !done; ++probe) {
-      int32_t k = __hip_atomic_load(&g.kv[o + h].k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      int32_t k = ld_relaxed(&g.key[o + h]);
       if (k < 0) {
-        k = atomicCAS(&g.kv[o + h].k, -1, b);
+        k = atomicCAS(&g.key[o + h], -1, b);
         if (k == -1) {
           atomicAdd(&g.nkeys[a], 1);
           k = b;
         }
       }
       if (k == b) {
-        cnt_add(&g.kv[o + h], dout, din);
+        cnt_add(&g.cnt[o + h], dout, din);
         done = true;
       }
       h = (h + 1) & mask;
@@ -2680,8 +2695,8 @@ __global__ __launch_bounds__(256) void k_grow(GrowArgs ga) {
     if (threadIdx.x == 0) s_live = 0;
     __syncthreads();
     for (int32_t j = threadIdx.x; j < c; j += blockDim.x) {
-      const Slot x = g.kv[o + j];
-      const int32_t k = dold ? j : x.k;
+      const Cnt x = g.cnt[o + j];
+      const int32_t k = dold ? j : g.key[o + j];
       if (k >= 0 && (x.o != 0 || x.i != 0)) {
         const int32_t i = atomicAdd(&s_live, 1);
         if (gather) {
@@ -2699,18 +2714,22 @@ __global__ __launch_bounds__(256) void k_grow(GrowArgs ga) {
       // in place: the slab rewritten with the live entries only
       if (c <= kGrowLds) {
         lds_slab(s_k, s_o, s_i, live, t_k, t_o, t_i, c, false);
-        for (int32_t j = threadIdx.x; j < c; j += blockDim.x)
-          g.kv[o + j] = Slot{t_k[j], 0, t_o[j], t_i[j]};
+        for (int32_t j = threadIdx.x; j < c; j += blockDim.x) {
+          g.key[o + j] = t_k[j];
+          g.cnt[o + j] = Cnt{t_o[j], t_i[j]};
+        }
       } else {
-        for (int32_t j = threadIdx.x; j < c; j += blockDim.x) g.kv[o + j] = Slot{-1, 0, 0, 0};
+        for (int32_t j = threadIdx.x; j < c; j += blockDim.x) {
+          g.key[o + j] = -1;
+          g.cnt[o + j] = Cnt{0, 0};
+        }
         __threadfence_block();
         __syncthreads();
         const uint32_t mask = (uint32_t)c - 1;
         for (int32_t i = threadIdx.x; i < live; i += blockDim.x) {
           uint32_t h = hash32(s_k[i]) & mask;
-          while (atomicCAS(&g.kv[o + h].k, -1, s_k[i]) != -1) h = (h + 1) & mask;
-          g.kv[o + h].o = s_o[i];
-          g.kv[o + h].i = s_i[i];
+          while (atomicCAS(&g.key[o + h], -1, s_k[i]) != -1) h = (h + 1) & mask;
+          g.cnt[o + h] = Cnt{s_o[i], s_i[i]};
         }
       }
       __threadfence_block();
@@ -2751,30 +2770,33 @@ __global__ __launch_bounds__(256) void k_grow(GrowArgs ga) {
       if (ncap > 0) {
         const int64_t nb = s_base;
         if (inlds) {
-          for (int32_t j = threadIdx.x; j < ncap; j += blockDim.x)
-            g.kv[nb + j] = Slot{t_k[j], 0, t_o[j], t_i[j]};
-          // the old slab stays in the pool as zeros until a rebuild
-          for (int32_t j = threadIdx.x; j < c; j += blockDim.x) g.kv[o + j] = Slot{-1, 0, 0, 0};
+          for (int32_t j = threadIdx.x; j < ncap; j += blockDim.x) {
+            g.key[nb + j] = t_k[j];
+            g.cnt[nb + j] = Cnt{t_o[j], t_i[j]};
+          }
+          // the old slab's counts stay in the pool as zeros until a rebuild
+          for (int32_t j = threadIdx.x; j < c; j += blockDim.x) g.cnt[o + j] = Cnt{0, 0};
         } else {
-          for (int32_t i = threadIdx.x; i < ncap; i += blockDim.x) g.kv[nb + i] = Slot{-1, 0, 0, 0};
+          for (int32_t i = threadIdx.x; i < ncap; i += blockDim.x) {
+            g.key[nb + i] = -1;
+            g.cnt[nb + i] = Cnt{0, 0};
+          }
           __threadfence_block();
           __syncthreads();
           const bool dnew = ncap == B;
           const uint32_t mask = (uint32_t)ncap - 1;
           for (int32_t j = threadIdx.x; j < c; j += blockDim.x) {
-            const Slot x = g.kv[o + j];
-            if (x.k < 0 || (x.o == 0 && x.i == 0)) continue;
-            g.kv[o + j].o = 0;
-            g.kv[o + j].i = 0;
+            const int32_t k = g.key[o + j];
+            const Cnt x = g.cnt[o + j];
+            if (k < 0 || (x.o == 0 && x.i == 0)) continue;
+            g.cnt[o + j] = Cnt{0, 0};
             if (dnew) {
-              g.kv[nb + x.k].o = x.o;
-              g.kv[nb + x.k].i = x.i;
+              g.cnt[nb + k] = x;
               continue;
             }
-            uint32_t h = hash32(x.k) & mask;
-            while (atomicCAS(&g.kv[nb + h].k, -1, x.k) != -1) h = (h + 1) & mask;
-            g.kv[nb + h].o = x.o;
-            g.kv[nb + h].i = x.i;
+            uint32_t h = hash32(k) & mask;
+            while (atomicCAS(&g.key[nb + h], -1, k) != -1) h = (h + 1) & mask;
+            g.cnt[nb + h] = x;
           }
         }
         __threadfence_block();
@@ -2811,7 +2833,8 @@ struct DevSpM {
   int64_t* off = nullptr;
   int32_t* cap = nullptr;
   int32_t* nkeys = nullptr;
-  Slot* kv = nullptr;     // row slabs [P]
+  int32_t* key = nullptr;  // row slabs [P]: keys
+  Cnt* cnt = nullptr;      // and counts
   int32_t* bs = nullptr;  // [bs_rows][kNBK]
   int32_t bs_rows = 0;
   int32_t* gpend = nullptr;  // [N]
@@ -3043,7 +3066,8 @@ MView view(const DevSpM& m, int32_t B) {
   v.off = m.off;
   v.cap = m.cap;
   v.nkeys = m.nkeys;
-  v.kv = m.kv;
+  v.key = m.key;
+  v.cnt = m.cnt;
   v.bs = m.bs;
   v.gpend = m.gpend;
   v.ovf = m.ovf;
@@ -3220,13 +3244,16 @@ int rebuild_M(usap_engine* e) {
   // the next rebuild, and k_grow only has the batch's error flags to fold
   e->all_direct = tot == (int64_t)B * B;
   if (3 * m.total > m.P) {  // two thirds of the pool is headroom for rows that grow
-    dfree(e, m.kv);
+    dfree(e, m.key);
+    dfree(e, m.cnt);
     const int64_t P = 3 * m.total + (int64_t)4 * B + 4096;
-    if (int rc = dalloc(e, &m.kv, (size_t)P)) return rc;
+    m.P = 0;
+    if (int rc = dalloc(e, &m.key, (size_t)P)) return rc;
+    if (int rc = dalloc(e, &m.cnt, (size_t)P)) return rc;
     m.P = P;
   }
   if (m.total > 0) k_fill<<<std::min<int64_t>(blocks_for(m.total, 256), 8192), 256, 0, st>>>(
-      m.kv, m.total);
+      e->all_direct ? nullptr : m.key, m.cnt, m.total);
   k_reset_grow<<<1, 1, 0, st>>>(m.gst, (unsigned long long)m.total);
   if (m.bs_rows < B) {
     dfree(e, m.bs);
@@ -3384,7 +3411,8 @@ int usap_destroy(usap_engine* e) {
     dfree(e, m->off);
     dfree(e, m->cap);
     dfree(e, m->nkeys);
-    dfree(e, m->kv);
+    dfree(e, m->key);
+    dfree(e, m->cnt);
     dfree(e, m->bs);
     dfree(e, m->gpend);
     dfree(e, m->ovf);
@@ -4076,11 +4104,13 @@ int usap_get_M_coo(usap_engine* e, int64_t cap, int32_t* rows, int32_t* cols, in
   const int64_t used = std::min<int64_t>((int64_t)gs.used, e->M.P);
   std::vector<int64_t> off((size_t)B + 1);
   std::vector<int32_t> capv((size_t)B);
-  std::vector<Slot> kv((size_t)used);
+  std::vector<int32_t> key((size_t)used);
+  std::vector<Cnt> cnt((size_t)used);
   HIPCHK(hipMemcpyAsync(off.data(), e->M.off, sizeof(int64_t) * (B + 1), hipMemcpyDeviceToHost, st));
   HIPCHK(hipMemcpyAsync(capv.data(), e->M.cap, sizeof(int32_t) * B, hipMemcpyDeviceToHost, st));
   if (used > 0) {
-    HIPCHK(hipMemcpyAsync(kv.data(), e->M.kv, sizeof(Slot) * used, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync(key.data(), e->M.key, sizeof(int32_t) * used, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync(cnt.data(), e->M.cnt, sizeof(Cnt) * used, hipMemcpyDeviceToHost, st));
   }
   HIPCHK(hipStreamSynchronize(st));
   std::vector<std::pair<int32_t, int32_t>> row;
@@ -4088,8 +4118,8 @@ int usap_get_M_coo(usap_engine* e, int64_t cap, int32_t* rows, int32_t* cols, in
   for (int32_t a = 0; a < B; ++a) {
     row.clear();
     for (int64_t j = 0; j < capv[a]; ++j) {
-      const int32_t c = capv[a] == B ? (int32_t)j : kv[off[a] + j].k;
-      const int32_t v = kv[off[a] + j].o;  // M[a][c]
+      const int32_t c = capv[a] == B ? (int32_t)j : key[off[a] + j];
+      const int32_t v = cnt[off[a] + j].o;  // M[a][c]
       if (c >= 0 && v != 0) row.emplace_back(c, v);
     }
     std::sort(row.begin(), row.end());
@@ -4115,7 +4145,7 @@ namespace {
 int launch_entropy(usap_engine* e, long* part = nullptr) {
   const int64_t work = std::max<int64_t>(e->M.P, e->B);
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(kEntropyBlocks, blocks_for(work, 1024)));
-  k_entropy<<<grid, 256, 0, e->stream>>>(e->M.kv, e->M.gst, e->d_out, e->d_in, e->B, e->lam,
+  k_entropy<<<grid, 256, 0, e->stream>>>(e->M.cnt, e->M.gst, e->d_out, e->d_in, e->B, e->lam,
                                          e->M.P, part ? part : e->ent_part);
   return grid;
 }
@@ -4258,7 +4288,7 @@ int usap_merge_propose(usap_engine* e, int32_t K, uint64_t stream, int32_t* best
   ev_rec(e, 1);
   if (e->prof) {  // the reference algorithm's bytes: 2 (4 (B+1) + 8 nnz(M)) + 24 B
     k_nnz_bytes<<<(unsigned)std::min<int64_t>(4096, std::max<int64_t>(1, blocks_for(e->M.P, 256))),
-                  256, 0, e->stream>>>(e->M.kv, e->M.P, e->aq_acc + 2 * kAqSlots);
+                  256, 0, e->stream>>>(e->M.cnt, e->M.P, e->aq_acc + 2 * kAqSlots);
     HIPCHK(hipGetLastError());
     e->kp[USAP_K_MERGE].model_bytes += 8.0 * ((double)B + 1.0) + 24.0 * (double)B;
   }
@@ -4489,7 +4519,8 @@ int launch_batch(usap_engine* e, int32_t beg, int32_t end, int32_t bidx, size_t 
     gs.off = m.off;
     gs.cap = m.cap;
     gs.nkeys = m.nkeys;
-    gs.kv = m.kv;
+    gs.key = m.key;
+    gs.cnt = m.cnt;
     gs.gpend = m.gpend;
     gs.ovf = m.ovf;
     gs.ovf_cap = m.ovf_cap;
