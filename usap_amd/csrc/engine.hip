@@ -180,7 +180,13 @@ struct Row {
   int32_t c;
 };
 
-__device__ __forceinline__ Row m_row(const MView& m, int32_t a) { return Row{m.off[a], m.cap[a]}; }
+// kD: every row of M is direct (the host knows it from the rebuild), so row a
+// is the a-th B slots of the pool: no row header to load before a lookup, no
+// key, no probing.
+template <bool kD = false>
+__device__ __forceinline__ Row m_row(const MView& m, int32_t a) {
+  return kD ? Row{(int64_t)a * m.B, m.B} : Row{m.off[a], m.cap[a]};
+}
 
 // First slot of key b in row R (the column itself in a direct row).
 __device__ __forceinline__ int64_t m_slot(const MView& m, Row R, int32_t b) {
@@ -196,14 +202,16 @@ struct Probe {
   Cnt c;
 };
 
+template <bool kD = false>
 __device__ __forceinline__ uint32_t m_home(const MView& m, Row R, int32_t b) {
-  return R.c == m.B ? (uint32_t)b : hash32(b) & (uint32_t)(R.c - 1);
+  return kD || R.c == m.B ? (uint32_t)b : hash32(b) & (uint32_t)(R.c - 1);
 }
 
+template <bool kD = false>
 __device__ __forceinline__ Probe m_probe(const MView& m, Row R, int32_t b) {
   Probe p;
-  p.h = m_home(m, R, b);
-  p.k = R.c == m.B ? b : m.key[R.o + p.h];
+  p.h = m_home<kD>(m, R, b);
+  p.k = kD || R.c == m.B ? b : m.key[R.o + p.h];
   p.c = m.cnt[R.o + p.h];
   return p;
 }
@@ -221,8 +229,9 @@ __device__ __forceinline__ Cnt m_value_more(const MView& m, Row R, int32_t b, ui
 }
 
 // (M[a][b], M[b][a]) from the first probe p of key b in row R of a.
+template <bool kD = false>
 __device__ __forceinline__ Cnt m_value(const MView& m, Row R, int32_t b, const Probe& p) {
-  if (p.k == b) return p.c;
+  if (kD || p.k == b) return p.c;
   if (p.k < 0) return Cnt{0, 0};
   return m_value_more(m, R, b, p.h);
 }
@@ -429,6 +438,35 @@ __device__ __forceinline__ long wave_incl_scan(long v) {
   return v;
 }
 
+template <int kCtrl, int kRows = 0xf>
+__device__ __forceinline__ uint32_t dpp_move32(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, kRows, 0xf, true);
+}
+
+__device__ __forceinline__ uint32_t wave_incl_scan32(uint32_t v) {
+  v += dpp_move32<kDppShr1>(v);
+  v += dpp_move32<kDppShr2>(v);
+  v += dpp_move32<kDppShr4>(v);
+  v += dpp_move32<kDppShr8>(v);
+  v += dpp_move32<kDppBcast15, 0xa>(v);
+  v += dpp_move32<kDppBcast31, 0xc>(v);
+  return v;
+}
+
+__device__ __forceinline__ uint32_t read_lane32(uint32_t v, int l) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+}
+
+__device__ __forceinline__ uint32_t wave_sum32(uint32_t v) {
+  return read_lane32(wave_incl_scan32(v), kWave - 1);
+}
+
+// floor(x * W / 2^64) for W < 2^32, as usap::idx_of
+__device__ __forceinline__ uint32_t idx32(uint64_t x, uint32_t W) {
+  const uint64_t hi = (x >> 32) * W, lo = (x & 0xffffffffull) * W;
+  return (uint32_t)((hi + (lo >> 32)) >> 32);
+}
+
 // A sum of terms m * lambda, |m| < 2^31 (a count, degree or sum of them),
 // |lambda| < 2^54: each lambda is split at bit 24 and the two products are
 // summed apart, value = h * 2^24 + l, so a term is two 32-bit multiply-adds
@@ -592,87 +630,71 @@ __device__ __forceinline__ void lookup_bucket(const MView& m, Row R, int32_t lo,
   }
 }
 
-// Index of the t-th unit in the LDS weights scr[0, width) (t < their sum):
-// each lane sums a contiguous run of entries, one wavefront scan finds the
-// run, and the lane owning it walks it.
-__device__ __forceinline__ int32_t scan_scratch(const int32_t* scr, int32_t width, int64_t t) {
-  const int lane = lane_id();
-  const int32_t per = (width + kWave - 1) / kWave;
-  const int32_t b0 = lane * per;
-  long sum = 0;
-  for (int32_t k = 0; k < per; ++k)
-    if (b0 + k < width) sum += scr[b0 + k];
-  const long inc = wave_incl_scan(sum);
-  const int f = __ffsll((unsigned long long)__ballot(inc > t)) - 1;
-  if (f < 0) return width - 1;
-  long tl = t - (__shfl(inc, f) - __shfl(sum, f));
-  int32_t res = width - 1;
-  if (lane == f) {
-    for (int32_t k = 0; k < per && b0 + k < width; ++k) {
-      const long w = scr[b0 + k];
-      if (tl < w) {
-        res = b0 + k;
-        break;
-      }
-      tl -= w;
-    }
-  }
-  return __shfl(res, f);
+// A row's kNBK bucket sums, kNBK / 64 consecutive ones per lane (buckets past
+// the last key are 0).
+constexpr int kBkLane = kNBK / kWave;
+struct Sums {
+  uint32_t w[kBkLane];
+};
+
+__device__ __forceinline__ Sums load_sums(const MView& M, int32_t u) {
+  static_assert(kBkLane == 8, "two 16-byte loads per lane");
+  const uint4* p = reinterpret_cast<const uint4*>(M.bs + (int64_t)u * kNBK) + 2 * lane_id();
+  const uint4 a = p[0], b = p[1];
+  return Sums{{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}};
 }
 
 // Inverse-CDF pick over the combined weights M[u][i] + M[i][u] (block row
 // u: o + i), ascending i, skipping i == excl: the first i whose running sum
 // exceeds t (graph_parallel.hpp:849-850 / :1061-1062 with exact integer
-// weights).  The caller guarantees t < total weight.  Two levels: the row's
-// bucket sums (all loaded at once) locate the key bucket [lo, hi); the
-// bucket's weights then come from one load per key when the row is direct and
-// the bucket is at most a wavefront wide, else they are gathered into the
+// weights; a row's weights sum to less than 2^32).  The caller guarantees t <
+// total weight and has loaded the row's bucket sums.  Two levels: the bucket
+// sums locate the key bucket [lo, hi); the bucket's weights then come from
+// one load per key when the row is direct, else they are gathered into the
 // wavefront's LDS scratch `scr` (scr_cap ints) -- a hashed row by scanning its
 // slab, which costs a few loads per lane where looking up each absent key
 // would walk a probe chain, or, when the slab holds kLookupRatio times the
 // bucket's keys or more, by looking each key up (a whole-slab scan of a
-// 16384-slot row took one wavefront ~120 us) -- and searched with one scan.
-__device__ __forceinline__ int32_t select_combined(const MView& M, int32_t u, int64_t t,
-                                                   int32_t excl, int32_t* scr, int32_t scr_cap,
-                                                   long& bytes) {
+// 16384-slot row took one wavefront ~120 us) -- and searched 512 keys at a
+// time.
+template <bool kD>
+__device__ __forceinline__ int32_t select_combined(const MView& M, int32_t u, uint32_t t,
+                                                   int32_t excl, Sums S, int32_t* scr,
+                                                   int32_t scr_cap, long& bytes) {
   const int lane = lane_id();
   const int32_t B = M.B;
   const int sh = M.bshift;
-  const Row RM = m_row(M, u);
   const int32_t nbk = ((B - 1) >> sh) + 1;
-  const int32_t* bM = M.bs + (int64_t)u * kNBK;
-  constexpr int kQ = kNBK / kWave;
-  long wq[kQ];
-#pragma unroll
-  for (int q = 0; q < kQ; ++q) {
-    const int32_t j = q * kWave + lane;
-    wq[q] = j < nbk ? (long)bM[j] : 0;
-  }
+  const Row RM = m_row<kD>(M, u);
   bytes += 12 + 4 * (long)nbk;
   if (excl >= 0) {
-    const Probe p = m_probe(M, RM, excl);
-    const Cnt x = m_value(M, RM, excl, p);
-    const long wx = (long)x.o + x.i;
+    const Cnt x = m_value<kD>(M, RM, excl, m_probe<kD>(M, RM, excl));
     bytes += 12;
     const int32_t xb = excl >> sh;
 #pragma unroll
-    for (int q = 0; q < kQ; ++q)
-      if (q * kWave + lane == xb) wq[q] -= wx;
+    for (int q = 0; q < kBkLane; ++q)
+      if (lane * kBkLane + q == xb) S.w[q] -= (uint32_t)x.o + (uint32_t)x.i;
   }
   // level 1: bucket jb holding the t-th unit
-  int32_t jb = nbk - 1;
+  uint32_t own = 0;
 #pragma unroll
-  for (int q = 0; q < kQ; ++q) {
-    const long inc = wave_incl_scan(wq[q]);
-    const long tot = __shfl(inc, kWave - 1);
-    if (t < tot) {
-      const int f = __ffsll((unsigned long long)__ballot(inc > t)) - 1;
-      jb = q * kWave + f;
-      t -= __shfl(inc, f) - __shfl(wq[q], f);
-      break;
-    }
-    t -= tot;
+  for (int q = 0; q < kBkLane; ++q) own += S.w[q];
+  const uint32_t inc = wave_incl_scan32(own);
+  const unsigned long long past = __ballot(inc > t);
+  const int f = past ? __ffsll(past) - 1 : kWave - 1;
+  int j = 0;
+  uint32_t rest = t - (inc - own), before = 0;  // in lane f: the units before t in its buckets
+#pragma unroll
+  for (int q = 0; q < kBkLane - 1; ++q) {
+    before += S.w[q];
+    if (rest >= before) j = q + 1;
   }
+  before = 0;
+#pragma unroll
+  for (int q = 0; q < kBkLane - 1; ++q)
+    if (q < j) before += S.w[q];
+  const int32_t jb = min((int32_t)read_lane32((uint32_t)(lane * kBkLane + j), f), nbk - 1);
+  t = read_lane32(rest - before, f);
   // level 2: keys [lo, hi) of that bucket in ascending order
   const int32_t lo = jb << sh;
   const int32_t hi = min(B, lo + (1 << sh));
@@ -681,39 +703,21 @@ __device__ __forceinline__ int32_t select_combined(const MView& M, int32_t u, in
   // that key's weight, so the bucket is the pick (the scans below would
   // return lo too, also for the excluded key's emptied bucket)
   if (width == 1) return lo;
-  if (width <= kWave && RM.c == B) {  // direct row: one load per key
-    long w = 0;
-    const int32_t i = lo + lane;
-    if (lane < width && i != excl) {
-      const Cnt q = M.cnt[RM.o + i];
-      w = (long)q.o + q.i;
+  const bool direct = kD || RM.c == B;
+  if (!direct && width > scr_cap) {  // wider than the scratch: bisection inside the bucket
+    int32_t a = lo, b = hi - 1;
+    while (a < b) {
+      const int32_t mid = a + (b - a) / 2;
+      const long c = wave_sum(count_range_lane(M, RM.o, RM.c, lo, mid, excl));
+      if (c > (long)t)
+        b = mid;
+      else
+        a = mid + 1;
     }
-    bytes += 8 * (long)width;
-    const long inc = wave_incl_scan(w);
-    const int f = __ffsll((unsigned long long)__ballot(inc > t)) - 1;
-    return f < 0 ? hi - 1 : lo + f;
+    return a;
   }
-  if (width <= scr_cap) {
-    if (RM.c == B) {
-      for (int32_t base = 0; base < width; base += 4 * kWave) {
-        int32_t v[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int32_t i = base + q * kWave + lane;
-          v[q] = 0;
-          if (i < width) {
-            const Cnt x = M.cnt[RM.o + lo + i];
-            v[q] = x.o + x.i;
-          }
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int32_t i = base + q * kWave + lane;
-          if (i < width) scr[i] = v[q];
-        }
-      }
-      bytes += 8 * (long)width;
-    } else if (RM.c >= kLookupRatio * width) {
+  if (!direct) {
+    if (RM.c >= kLookupRatio * width) {
       lookup_bucket(M, RM, lo, hi, scr, bytes);
     } else {
       for (int32_t i = lane; i < width; i += kWave) scr[i] = 0;
@@ -721,21 +725,34 @@ __device__ __forceinline__ int32_t select_combined(const MView& M, int32_t u, in
       gather_row(M, RM, lo, hi, scr, bytes);
     }
     wave_fence();
-    if (lane == 0 && excl >= lo && excl < hi) scr[excl - lo] = 0;
-    wave_fence();
-    return lo + scan_scratch(scr, width, t);
+  } else {
+    bytes += 8 * (long)width;
   }
-  // buckets wider than the scratch: bisection inside the bucket
-  int32_t a = lo, b = hi - 1;
-  while (a < b) {
-    const int32_t mid = a + (b - a) / 2;
-    const long c = wave_sum(count_range_lane(M, RM.o, RM.c, lo, mid, excl));
-    if (c > t)
-      b = mid;
-    else
-      a = mid + 1;
+  for (int32_t base = 0; base < width; base += 8 * kWave) {
+    uint32_t v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int32_t i = base + q * kWave + lane;
+      v[q] = 0;
+      if (i < width && lo + i != excl) {
+        if (direct) {
+          const Cnt x = M.cnt[RM.o + lo + i];
+          v[q] = (uint32_t)x.o + (uint32_t)x.i;
+        } else {
+          v[q] = (uint32_t)scr[i];
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      if (base + q * kWave >= width) break;
+      const uint32_t c = wave_incl_scan32(v[q]);
+      const unsigned long long hit = __ballot(c > t);
+      if (hit) return lo + base + q * kWave + __ffsll(hit) - 1;
+      t -= read_lane32(c, kWave - 1);
+    }
   }
-  return a;
+  return hi - 1;
 }
 
 // t-th unit of the node's neighbour list (out-neighbours then in-neighbours,
@@ -1451,7 +1468,7 @@ __device__ void merge_one(const MergeArgs& a, int32_t r, int32_t idx, int32_t* s
   } else {
     long bytes = 0;
     const int64_t t0 = (int64_t)usap::idx_of(x[0], k);
-    const int32_t u = L.n >= 0 ? rowlds_pick(L, t0) : select_combined(a.M, r, t0, -1, scr, kScr, bytes);
+    const int32_t u = L.n >= 0 ? rowlds_pick(L, t0) : select_combined<false>(a.M, r, (uint32_t)t0, -1, load_sums(a.M, r), scr, kScr, bytes);
     const int64_t da = (int64_t)a.d_out[u] + a.d_in[u];
     if (usap::uniform_branch(x[1], da, B)) {
       s = usap::uniform_not_r(x[2], r, B);
@@ -1459,7 +1476,7 @@ __device__ void merge_one(const MergeArgs& a, int32_t r, int32_t idx, int32_t* s
       const Cnt ur = m_get(a.M, u, r);  // M[u][r], M[r][u]
       const int64_t W2 = da - ur.o - ur.i;
       s = W2 == 0 ? usap::uniform_not_r(x[2], r, B)
-                  : select_combined(a.M, u, usap::idx_of(x[3], W2), r, scr, kScr, bytes);
+                  : select_combined<false>(a.M, u, idx32(x[3], (uint32_t)W2), r, load_sums(a.M, u), scr, kScr, bytes);
     }
   }
   s_out = s;
@@ -1602,7 +1619,6 @@ __global__ __launch_bounds__(kWave* kMergeWaves, 5) void k_merge(MergeArgs a) {
 // ---------------------------------------------------------------------------
 
 constexpr int kEdgeRegs = 4;     // list entries per lane per pass (256 per wavefront)
-constexpr int kScrNodal = 1024;  // k_nodal's LDS scratch per wavefront (one key bucket)
 
 // Workgroups are dispatched to the GPU's 8 XCDs (each with its own L2) in
 // turn: workgroup b runs on XCD b % 8.  Block b of a batch kernel takes item
@@ -1633,6 +1649,18 @@ struct BlockPart {
 // and degrees of r and s, the label.
 __device__ __forceinline__ long apply_tally(int64_t kc) { return 52 + 60 * kc + 32 + 32 + 4; }
 
+// One proposal as k_apply and the callers read it.
+struct __align__(16) Prop {
+  int32_t s, r;      // proposed block, old block
+  int32_t acc, inf;  // accepted; -1: dS is -inf
+};
+
+// Its exact dS.
+struct __align__(16) PropDs {
+  long hi;
+  unsigned long lo;
+};
+
 struct NodalArgs {
   GraphView g;
   MView M;
@@ -1643,17 +1671,12 @@ struct NodalArgs {
   int32_t B;
   int32_t beg, end;
   int32_t exact;
-  int32_t bidx;  // batch index in the sweep: random stream sweep->stream0 + bidx
-  uint64_t seed;
-  const uint64_t* uni;  // pre-drawn stream: node n takes draw sweep->stream0 + n; else null
+  const uint64_t* draws;  // four words per draw: node n's at n, or, predrawn,
+  int32_t predrawn;       // at sweep->stream0 + n
   const int64_t* big_off;
   int32_t* big_tab;
-  int32_t* prop_s;
-  long* prop_hi;
-  unsigned long* prop_lo;
-  int32_t* prop_inf;
-  int32_t* prop_acc;
-  int32_t* prop_r;
+  Prop* prop;
+  PropDs* prop_ds;
   int32_t* prop_u;  // profiling: block of the drawn neighbour (-1: none), else null
   BlockPart* part;
   Status* status;
@@ -1771,241 +1794,590 @@ __device__ __forceinline__ void list_entry(const GraphView& g, int64_t o0, int64
   }
 }
 
-// dS of moving node n from r to s (r != s), factorised, from its complete
-// neighbour-block table.  All lookups of a pass are issued before any is
-// resolved.
-__device__ __forceinline__ i128 nodal_delta(const NodalArgs& a, const Table& T, int32_t r,
-                                            int32_t s, Row rM, int32_t dor, int32_t dir,
-                                            int64_t kc, int32_t k_out, int32_t k_in, long wself_sum,
-                                            bool& inf, long& bytes, int32_t s_pre, Row sM_pre,
-                                            int32_t dos_pre, int32_t dis_pre) {
+// Orders this wavefront's LDS writes and atomics before its later LDS reads:
+// the LDS runs one wavefront's operations in order, so only the compiler has
+// to keep it (no wait for loads in flight).
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The Philox words of nodes [beg, end), 4 per node, batch i = [beg + i * batch,
+// ...) from stream sweep->stream0 + i: one thread per node, where every lane of
+// a node's k_nodal wavefront would compute the same 80 multiplies.
+__global__ void k_draw(int32_t beg, int32_t end, int32_t batch, uint64_t seed, const Sweep* sweep,
+                       uint64_t* __restrict__ draws) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (beg + i >= end) return;
+  const int64_t n = beg + i;
+  uint64_t x[4];
+  usap::philox4x64((uint64_t)n, 0, sweep->stream0 + (uint64_t)(i / batch), usap::kTagNodal, seed, 0,
+                   x);
+  ulonglong2* q = reinterpret_cast<ulonglong2*>(draws + 4 * n);
+  q[0] = make_ulonglong2(x[0], x[1]);
+  q[1] = make_ulonglong2(x[2], x[3]);
+}
+
+// What moving node n from r to s changes outside the neighbour blocks: the
+// counts of the corner, the degrees of r and s, n's weights into r and s.
+struct Corner {
+  int32_t rr, rs, sr, ss;      // M[r][r], M[r][s], M[s][r], M[s][s]
+  int32_t dor, dir, dos, dis;  // degrees of r and s
+  int32_t k_out, k_in;         // n's out- and in-weight
+  int32_t wor, wir, wos, wis;  // n's weights into (out) and from (in) r and s
+  int32_t wself;               // n's self-loops
+};
+
+// Adds the move's 16 corner and degree terms to acc, one per lane (in every
+// lane they were a quarter of the kernel's arithmetic); inf: the moved state
+// has an infinite term.  Lane bits: col (0: column r, 1: s), row (0: row r, 1:
+// s), now (0: before the move, 1: after), deg.
+//   deg = 0: T(M[row][col], d_in[col], d_out[row])
+//   deg = 1: the row's other out-edges X (col = 0) or the column's other
+//            in-edges Y (col = 1) of block `row`, m * lambda(degree)
+// each + before and - after, the degree terms the other way round.
+__device__ __forceinline__ void corner_terms(const NodalArgs& a, const Corner& c, Acc& acc,
+                                             bool& inf) {
   const int lane = lane_id();
-  const int64_t* lam = a.lam;
-  // s's row and degrees (loaded ahead when s is the uniform draw); the table
-  // is compacted while they load
-  const bool pre = s == s_pre;
-  const Row sM = pre ? sM_pre : m_row(a.M, s);
-  const int32_t dos = pre ? dos_pre : a.d_out[s], dis = pre ? dis_pre : a.d_in[s];
-  long wor_l = 0, wir_l = 0, wos_l = 0, wis_l = 0;
-  const int32_t nent = tab_compact(T, r, s, wor_l, wir_l, wos_l, wis_l);
-  // corner: (r, r), (r, s) with (s, r) beside it, (s, s)
-  const Probe pRR = m_probe(a.M, rM, r), pRS = m_probe(a.M, rM, s);
-  const Probe pSS = m_probe(a.M, sM, s);
-  // changed entries of rows r, s (out-edges, o) and columns r, s (in-edges,
-  // i): one probe of block row r and one of s per neighbour block
-  Acc acc{0, 0};
-  long lookups = 0;
-  bool neg = false;
-  for (int32_t j = lane; j < nent; j += kWave) {
-    const int32_t b = T.tk[j], wo = T.two[j], wi = T.twi[j];
-    // n's edges into b put b among row r's keys; row s, when hashed, is most
-    // often a uniform draw without b (B >= 8 slabs is >= 16 row degrees), so
-    // its keys alone are read first
-    const Probe p0 = m_probe(a.M, rM, b);
-    Probe p1{m_home(a.M, sM, b), b, {0, 0}};
-    if (sM.c != a.M.B) p1.k = a.M.key[sM.o + p1.h];
-    if (p1.k == b) p1.c = a.M.cnt[sM.o + p1.h];
-    const Cnt cr = m_value(a.M, rM, b, p0), cs = m_value(a.M, sM, b, p1);
-    lookups += 2;
-    if (wo > 0) {
-      neg |= cr.o - wo < 0;
-      add_L(acc, lam, cr.o);
-      add_L(acc, lam, cs.o);
-      sub_L(acc, lam, cr.o - wo);
-      sub_L(acc, lam, cs.o + wo);
-    }
-    if (wi > 0) {
-      neg |= cr.i - wi < 0;
-      add_L(acc, lam, cr.i);
-      add_L(acc, lam, cs.i);
-      sub_L(acc, lam, cr.i - wi);
-      sub_L(acc, lam, cs.i + wi);
-    }
-  }
-  if (neg) atomicOr(&a.status->flags, kFlagNegative);
-  // blocks r and s own one table slot each, so one lane at most holds their
-  // weights; the other entries' weights are the rest of k_out / k_in
-  const unsigned long long hr = __ballot(wor_l != 0 || wir_l != 0);
-  const unsigned long long hs = __ballot(wos_l != 0 || wis_l != 0);
-  const int lr = hr ? __ffsll(hr) - 1 : 0, ls = hs ? __ffsll(hs) - 1 : 0;
-  const int32_t wor = __builtin_amdgcn_readlane((int32_t)wor_l, lr);
-  const int32_t wir = __builtin_amdgcn_readlane((int32_t)wir_l, lr);
-  const int32_t wos = __builtin_amdgcn_readlane((int32_t)wos_l, ls);
-  const int32_t wis = __builtin_amdgcn_readlane((int32_t)wis_l, ls);
-  const int32_t Wo = k_out - wor - wos, Wi = k_in - wir - wis;
-  int32_t wself = 0;
-  if (__ballot(wself_sum != 0)) wself = (int32_t)wave_sum(wself_sum);  // self-loops are rare
-  // neighbour ids + labels (+ weights); rows (offset + capacity) and degrees
-  // of r and s; 2 block-row lookups (key + two counts) per changed entry and
-  // 3 corner lookups
-  bytes += (a.g.out_w ? 12 : 8) * kc + 24 + 16 + 12 * (wave_sum(lookups) + 3);
-  const Cnt crs = m_value(a.M, rM, s, pRS);
-  const int32_t Mrr = m_value(a.M, rM, r, pRR).o, Mrs = crs.o;
-  const int32_t Msr = crs.i, Mss = m_value(a.M, sM, s, pSS).o;
   int32_t rr2, rs2, sr2, ss2;
   if (!a.exact) {  // graph_parallel.hpp:1117-1145: only out-edges update the rows
-    rr2 = Mrr - wor;
-    rs2 = Mrs - wos;
-    sr2 = Msr + wor;
-    ss2 = Mss + wos;
+    rr2 = c.rr - c.wor;
+    rs2 = c.rs - c.wos;
+    sr2 = c.sr + c.wor;
+    ss2 = c.ss + c.wos;
   } else {  // graph.cu:1414-1426, with a self-loop moving (r,r) -> (s,s)
-    const int32_t wor_ = wor - wself, wir_ = wir - wself;
-    rr2 = Mrr - wor_ - wself - wir_;
-    rs2 = Mrs - wos + wir_;
-    sr2 = Msr + wor_ - wis;
-    ss2 = Mss + wos + wis + wself;
+    const int32_t wor_ = c.wor - c.wself, wir_ = c.wir - c.wself;
+    rr2 = c.rr - wor_ - c.wself - wir_;
+    rs2 = c.rs - c.wos + wir_;
+    sr2 = c.sr + wor_ - c.wis;
+    ss2 = c.ss + c.wos + c.wis + c.wself;
   }
-  const int32_t Xr = dor - Mrr - Mrs, Xs = dos - Msr - Mss;
-  const int32_t Yr = dir - Mrr - Msr, Ys = dis - Mrs - Mss;
+  const int32_t Wo = c.k_out - c.wor - c.wos, Wi = c.k_in - c.wir - c.wis;
+  const int32_t Xr = c.dor - c.rr - c.rs, Xs = c.dos - c.sr - c.ss;
+  const int32_t Yr = c.dir - c.rr - c.sr, Ys = c.dis - c.rs - c.ss;
   if (rr2 < 0 || rs2 < 0 || sr2 < 0 || ss2 < 0 || Xr - Wo < 0 || Yr - Wi < 0)
     atomicOr(&a.status->flags, kFlagNegative);
-  // The 16 corner and degree terms, one per lane (in every lane they were a
-  // quarter of the kernel's arithmetic).  Lane bits: col (0: column r, 1: s),
-  // row (0: row r, 1: s), new (0: before the move, 1: after), deg.
-  //   deg = 0: T(M[row][col], d_in[col], d_out[row])
-  //   deg = 1: the row's other out-edges X (col = 0) or the column's other
-  //            in-edges Y (col = 1) of block `row`, m * lambda(degree)
-  // each + before and - after, the degree terms the other way round.
   const bool col = lane & 1, row = lane & 2, now = lane & 4, deg = lane & 8;
   const bool in2 = deg ? row : col;  // whose d_in
-  const int32_t dout = (row ? dos : dor) + (now ? (row ? k_out : -k_out) : 0);
-  const int32_t din = (in2 ? dis : dir) + (now ? (in2 ? k_in : -k_in) : 0);
+  const int32_t dout = (row ? c.dos : c.dor) + (now ? (row ? c.k_out : -c.k_out) : 0);
+  const int32_t din = (in2 ? c.dis : c.dir) + (now ? (in2 ? c.k_in : -c.k_in) : 0);
   const int32_t mt = now ? (row ? (col ? ss2 : sr2) : (col ? rs2 : rr2))
-                         : (row ? (col ? Mss : Msr) : (col ? Mrs : Mrr));
+                         : (row ? (col ? c.ss : c.sr) : (col ? c.rs : c.rr));
   const int32_t dW = now ? (col ? Wi : Wo) : 0;
   const int32_t mp = (col ? (row ? Ys : Yr) : (row ? Xs : Xr)) + (row ? dW : -dW);
   const int32_t m = deg ? mp : mt;
   const int32_t d1 = deg && !col ? dout : din, d2 = deg ? 1 : dout;  // lambda(1) = 0
   const bool bad = d1 <= 0 || d2 <= 0;
-  const int64_t c = lam_of(lam, deg ? 0 : m) - lam_of(lam, d1) - lam_of(lam, d2);
+  const int64_t L = lam_of(a.lam, deg ? 0 : m) - lam_of(a.lam, d1) - lam_of(a.lam, d2);
   if (lane < 16) {
     const int32_t mm = bad ? 0 : max(m, 0);
-    acc_add(acc, now ? -mm : mm, c);
+    acc_add(acc, now ? -mm : mm, L);
   }
   inf = __ballot(lane < 16 && now && bad && m > 0) != 0;
-  acc.h = wave_sum(acc.h);
-  acc.l = wave_sum(acc.l);
-  return acc_value(acc);
 }
 
-// One nodal proposal (graph_parallel.hpp:990-1222) for node n, batch item
-// `item`; returns its algorithmic bytes.  The loads form a short chain: own
-// label and list bounds; the list (ids) with r's rows and degrees; the
-// neighbours' labels with the drawn neighbour's; its block's degrees (and, when
-// the proposal follows M, its rows' bucket sums and one bucket); s's rows and
-// degrees; then every lookup of the dS at once.
-template <bool kBig>
-__device__ __forceinline__ long nodal_one(const NodalArgs& a, int64_t item, int32_t n, int32_t r,
-                                          int64_t o0, int64_t kco, int64_t i0, int64_t kci,
-                                          uint64_t stream0, int32_t* tab, int32_t* scr,
-                                          int32_t& acc_out, int32_t& inf_out, i128& dS_out) {
+// The result of one proposal.
+struct Nodal {
+  int32_t s, u, acc;
+  bool inf;
+  i128 dS;
+  long bytes;  // algorithmic bytes (profiling)
+};
+
+// Adds unit (b, w, in) of a node moving r -> s to acc: its edges to (in: from)
+// block b, given block row r's and row s's counts of b.  Branch-free: w = 0
+// with zero counts adds nothing.
+__device__ __forceinline__ void unit_terms(Acc& acc, const int64_t L[4], int32_t mr, int32_t ms,
+                                           int32_t w) {
+  acc_add(acc, max(mr, 0), L[0]);
+  acc_add(acc, max(ms, 0), L[1]);
+  acc_add(acc, -max(mr - w, 0), L[2]);
+  acc_add(acc, -max(ms + w, 0), L[3]);
+}
+
+constexpr int kLdsWave = 1024;     // LDS ints per wavefront: a unit table, or one key bucket
+constexpr int kRegUnits = 4;       // list entries per lane of a node one wavefront handles
+constexpr uint32_t kNoUnit = ~0u;  // empty unit-table slot
+
+__device__ __forceinline__ uint32_t unit_key(int32_t b, bool in) {
+  return 2u * (uint32_t)b + (in ? 1u : 0u);
+}
+
+// One nodal proposal (graph_parallel.hpp:990-1222) by one wavefront, for a
+// node of at most 64 U list entries.  A lane holds U entries; those that share
+// a block and a direction are summed into one of them, the unit's owner, by
+// a hash table in LDS that only decides ownership and sums weights: the unit
+// itself, its lookups and its terms stay in the owner's registers.
+//
+// The kernel is bound by its chain of dependent loads, so each step's are in
+// flight together: the list, with r's row header and degrees and those of the
+// uniform draw's block; the entries' labels (the drawn neighbour's among
+// them); then row r's counts of every entry's block, the drawn block's
+// degrees and, M hashed (B is then at least 16 times a row's degree, so the
+// uniform draw is nearly always the proposal), the uniform block's keys, or, M
+// dense (the drawn block's row decides most often), that row's bucket sums;
+// then s's counts unless they are there; then the lambda table.
+// Launch averages against one path through an LDS table with row headers
+// always read (90 VGPRs, 40 KB of LDS a workgroup, Philox in every lane): N =
+// 1000 12.1 -> 5.8 us, N = 20000 (5000-node batches) 28.8 -> 9.8, N = 50000
+// (12500-node batches) 42.5 -> 15.8, 4096-node batches at B = 100000 28.8 ->
+// 20.1.
+template <bool kD, bool kW, int U>
+__device__ __forceinline__ void nodal_regs(const NodalArgs& a, int32_t n, int32_t r, int64_t o0,
+                                           int64_t i0, int32_t kco, int32_t kc,
+                                           const uint64_t x[4], int32_t* lds, Nodal& out) {
   const int lane = lane_id();
   const GraphView& g = a.g;
+  const MView& M = a.M;
   const int32_t B = a.B;
-  const int64_t kc = kco + kci;
-  uint64_t x[4];
-  if (a.uni)
-    predrawn(a.uni, stream0 + (uint64_t)n, x);
-  else
-    usap::philox4x64((uint64_t)n, 0, stream0 + (uint64_t)a.bidx, usap::kTagNodal, a.seed, 0, x);
-  const Row rM = m_row(a.M, r);
+  const Row rM = m_row<kD>(M, r);
   const int32_t dor = a.d_out[r], dir = a.d_in[r];
-  // the uniform draw's block, the proposal in most cases: its row and
-  // degrees load with r's
-  const int32_t s_pre = (int32_t)usap::idx_of(x[2], B);
-  const Row sM_pre = m_row(a.M, s_pre);
+  const int32_t s_pre = (int32_t)idx32(x[2], (uint32_t)B);
+  const Row pM = m_row<kD>(M, s_pre);
   const int32_t dos_pre = a.d_out[s_pre], dis_pre = a.d_in[s_pre];
-  int64_t k_out = kco, k_in = kci;
-  if (g.out_w) {
-    long so = 0, si = 0;
-    for (int64_t j = lane; j < kco; j += kWave) so += g.out_w[o0 + j];
-    for (int64_t j = lane; j < kci; j += kWave) si += g.in_w[i0 + j];
-    k_out = wave_sum(so);
-    k_in = wave_sum(si);
+  int32_t v[U], w[U];
+#pragma unroll
+  for (int q = 0; q < U; ++q) {
+    const int32_t j = q * kWave + lane;
+    v[q] = -1;
+    w[q] = kW ? 0 : 1;
+    if (j < kco) {
+      v[q] = g.out_idx[o0 + j];
+      if (kW) w[q] = g.out_w[o0 + j];
+    } else if (j < kc) {
+      v[q] = g.in_idx[i0 + (j - kco)];
+      if (kW) w[q] = g.in_w[i0 + (j - kco)];
+    }
   }
-  const int64_t k = k_out + k_in;
-  // list offsets, own label, outputs (s, dS, inf, accept, r) (+ weights)
-  long bytes = 32 + 4 + 32 + (g.out_w ? 4 * kc : 0);
-  const Table T = tab_open<kBig>(tab, a.big_off, a.big_tab, n, kc);
-  const uint32_t mask = (uint32_t)T.cap - 1;
-  // the drawn neighbour (graph_parallel.hpp:1010-1027): unit t of the list
-  const int64_t t = k > 0 ? (int64_t)usap::idx_of(x[0], k) : 0;
-  int32_t vpick = -1;
+  constexpr int kCap = 128 * U;  // at least twice the units
+  static_assert(2 * kCap <= kLdsWave, "unit table exceeds the wavefront's LDS");
+  uint32_t* tk = reinterpret_cast<uint32_t*>(lds);
+  int32_t* tw = lds + kCap;
+  for (int j = 4 * lane; j < 2 * kCap; j += 4 * kWave) {
+    const int32_t z = j < kCap ? -1 : 0;
+    *reinterpret_cast<int4*>(lds + j) = make_int4(z, z, z, z);
+  }
+  lds_order();
+  // n's weights, and unit t of its list (graph_parallel.hpp:1010-1027)
+  int32_t k_out = kco, k_in = kc - kco;
+  if (kW) {
+    uint32_t so = 0, si = 0;
+#pragma unroll
+    for (int q = 0; q < U; ++q) (q * kWave + lane < kco ? so : si) += (uint32_t)w[q];
+    k_out = (int32_t)wave_sum32(so);
+    k_in = (int32_t)wave_sum32(si);
+  }
+  const uint32_t k = (uint32_t)k_out + (uint32_t)k_in;
+  int pq = 0, pl = 0;
   if (k > 0) {
-    if (g.out_w)
-      vpick = pick_neighbor(g, o0, kco, i0, kci, t);
-    else if (t >= kEdgeRegs * kWave)
-      vpick = t < kco ? g.out_idx[o0 + t] : g.in_idx[i0 + (t - kco)];
-  }
-  int32_t u = -1;
-  int64_t da = 0;
-  long wself = 0;
-  for (int64_t base = 0; base < kc; base += kEdgeRegs * kWave) {
-    int32_t v[kEdgeRegs], ww[kEdgeRegs], lb[kEdgeRegs];
+    const uint32_t t = idx32(x[0], k);
+    if (!kW) {
+      pq = (int)(t / kWave);
+      pl = (int)(t % kWave);
+    } else {
+      uint32_t sum = 0;
+      bool found = false;
 #pragma unroll
-    for (int q = 0; q < kEdgeRegs; ++q)
-      list_entry(g, o0, kco, i0, kc, base + q * kWave + lane, v[q], ww[q]);
-    if (base == 0 && k > 0 && vpick < 0) {  // unweighted, t < 256: lane t % 64 holds it
-      int32_t vv = v[0];
-#pragma unroll
-      for (int q = 1; q < kEdgeRegs; ++q)
-        if ((t >> 6) == q) vv = v[q];
-      vpick = __shfl(vv, (int)(t & (kWave - 1)));
-    }
-#pragma unroll
-    for (int q = 0; q < kEdgeRegs; ++q) lb[q] = v[q] >= 0 ? a.labels[v[q]] : -1;
-    if (base == 0 && k > 0) {
-      u = a.labels[vpick];
-      da = (int64_t)a.d_out[u] + a.d_in[u];
-    }
-#pragma unroll
-    for (int q = 0; q < kEdgeRegs; ++q) {
-      if (v[q] < 0) continue;
-      if (base + q * kWave + lane < kco) {
-        if (v[q] == n) wself += ww[q];
-        tab_add(T.tk, T.two, mask, lb[q], ww[q]);
-      } else {
-        tab_add(T.tk, T.twi, mask, lb[q], ww[q]);
+      for (int q = 0; q < U; ++q) {
+        const uint32_t inc = wave_incl_scan32((uint32_t)w[q]);
+        const unsigned long long hit = __ballot(sum + inc > t);
+        if (!found && hit) {
+          found = true;
+          pq = q;
+          pl = __ffsll(hit) - 1;
+        }
+        sum += read_lane32(inc, kWave - 1);
       }
     }
   }
-  int32_t s;
-  if (k == 0) {
-    s = (int32_t)usap::idx_of(x[2], B);
-  } else {
+  int32_t lb[U];
+#pragma unroll
+  for (int q = 0; q < U; ++q) lb[q] = v[q] >= 0 ? a.labels[v[q]] : -1;
+  int32_t lv = lb[0];
+#pragma unroll
+  for (int q = 1; q < U; ++q) lv = pq == q ? lb[q] : lv;
+  const int32_t u = k > 0 ? __builtin_amdgcn_readlane(lv, pl) : r;
+  const uint32_t da = (uint32_t)a.d_out[u] + (uint32_t)a.d_in[u];
+  Sums bk;
+  if (kD) bk = load_sums(M, u);
+  Probe p0[U];
+  int32_t ks[U];  // row s's key at the block's home slot
+  const bool pdir = kD || pM.c == B;
+#pragma unroll
+  for (int q = 0; q < U; ++q) {
+    p0[q] = Probe{0, -1, {0, 0}};
+    ks[q] = lb[q];
+    if (v[q] >= 0) {
+      p0[q] = m_probe<kD>(M, rM, lb[q]);
+      if (!pdir) ks[q] = M.key[pM.o + m_home(M, pM, lb[q])];
+    }
+  }
+  const Probe pRR = m_probe<kD>(M, rM, r);
+  Probe pRS, pSS;
+  if (!kD) {
+    pRS = m_probe(M, rM, s_pre);
+    pSS = m_probe(M, pM, s_pre);
+  }
+  // units: the owner of each (block, direction), its summed weight
+  uint32_t hs[U];
+  bool own[U];
+#pragma unroll
+  for (int q = 0; q < U; ++q) {
+    own[q] = false;
+    hs[q] = 0;
+    if (v[q] >= 0) {
+      const uint32_t key = unit_key(lb[q], q * kWave + lane >= kco);
+      uint32_t h = hash32((int32_t)key) & (kCap - 1);
+      for (;;) {
+        const uint32_t old = atomicCAS(&tk[h], kNoUnit, key);
+        own[q] = old == kNoUnit;
+        if (own[q] || old == key) break;
+        h = (h + 1) & (kCap - 1);
+      }
+      hs[q] = h;
+      atomicAdd(&tw[h], w[q]);
+    }
+  }
+  lds_order();
+  int32_t wself = 0;
+  if (a.exact) {
+    uint32_t ws = 0;
+#pragma unroll
+    for (int q = 0; q < U; ++q)
+      if (q * kWave + lane < kco && v[q] == n) ws += (uint32_t)w[q];
+    if (__ballot(ws != 0)) wself = (int32_t)wave_sum32(ws);  // self-loops are rare
+  }
+#pragma unroll
+  for (int q = 0; q < U; ++q) w[q] = own[q] ? tw[hs[q]] : 0;
+  lds_order();  // the table's LDS may hold a key bucket next
+  // list offsets, own label, outputs (s, dS, inf, accept, r) (+ weights)
+  long bytes = 32 + 4 + 32 + (kW ? 4 * (long)kc : 0);
+  int32_t s = s_pre;
+  if (k > 0) {
     bytes += 16;  // drawn neighbour id, its label, d_out[u], d_in[u]
-    if (usap::uniform_branch(x[1], da, B))
-      s = (int32_t)usap::idx_of(x[2], B);
+    if (!usap::uniform_branch(x[1], da, B)) {
+      if (!kD) bk = load_sums(M, u);
+      s = select_combined<kD>(M, u, idx32(x[3], da), -1, bk, lds, kLdsWave, bytes);
+    }
+  }
+  out.s = s;
+  out.u = k > 0 ? u : -1;
+  out.acc = 0;
+  out.inf = false;
+  out.dS = 0;
+  if (s == r) {
+    out.bytes = bytes;
+    return;
+  }
+  const bool pre = s == s_pre;
+  const Row sM = pre ? pM : m_row<kD>(M, s);
+  const int32_t dos = pre ? dos_pre : a.d_out[s], dis = pre ? dis_pre : a.d_in[s];
+  const bool sdir = kD || sM.c == B;
+  if (kD || !pre) {
+    pRS = m_probe<kD>(M, rM, s);
+    pSS = m_probe<kD>(M, sM, s);
+  }
+  Cnt cs[U];
+  int32_t wor = 0, wir = 0, wos = 0, wis = 0, units = 0;
+#pragma unroll
+  for (int q = 0; q < U; ++q) {
+    const bool in = q * kWave + lane >= kco;
+    const bool isr = own[q] && lb[q] == r, iss = own[q] && lb[q] == s;
+    const unsigned long long mr = __ballot(isr), ms = __ballot(iss);
+    if (mr) {  // at most one owner per direction
+      const unsigned long long o = __ballot(isr && !in), i = __ballot(isr && in);
+      if (o) wor = __builtin_amdgcn_readlane(w[q], __ffsll(o) - 1);
+      if (i) wir = __builtin_amdgcn_readlane(w[q], __ffsll(i) - 1);
+    }
+    if (ms) {
+      const unsigned long long o = __ballot(iss && !in), i = __ballot(iss && in);
+      if (o) wos = __builtin_amdgcn_readlane(w[q], __ffsll(o) - 1);
+      if (i) wis = __builtin_amdgcn_readlane(w[q], __ffsll(i) - 1);
+    }
+    own[q] = own[q] && !isr && !iss;
+    units += __popcll(__ballot(own[q]));
+    cs[q] = Cnt{0, 0};
+    if (own[q]) {
+      if (sdir) {
+        cs[q] = M.cnt[sM.o + lb[q]];
+      } else {
+        const uint32_t h = m_home(M, sM, lb[q]);
+        if (!pre) ks[q] = M.key[sM.o + h];
+        if (ks[q] == lb[q])
+          cs[q] = M.cnt[sM.o + h];
+        else if (ks[q] >= 0)
+          cs[q] = m_value_more(M, sM, lb[q], h);
+      }
+    }
+  }
+  // ids + labels (+ weights); rows (offset + capacity) and degrees of r and s;
+  // 2 block-row lookups (key + two counts) per unit and 3 corner lookups
+  bytes += (kW ? 12 : 8) * (long)kc + 24 + 16 + 12 * (long)(2 * units + 3);
+  out.bytes = bytes;
+  Acc acc{0, 0};
+  int64_t L[U][4];
+  int32_t m0[U], m1[U];
+  bool neg = false;
+#pragma unroll
+  for (int q = 0; q < U; ++q) {
+    const bool in = q * kWave + lane >= kco;
+    Cnt cr{0, 0};
+    if (own[q])
+      cr = m_value<kD>(M, rM, lb[q], p0[q]);
     else
-      s = select_combined(a.M, u, usap::idx_of(x[3], da), -1, scr, kScrNodal, bytes);
+      w[q] = 0;
+    m0[q] = in ? cr.i : cr.o;
+    m1[q] = in ? cs[q].i : cs[q].o;
+    neg |= m0[q] < w[q];
+    L[q][0] = lam_of(a.lam, m0[q]);
+    L[q][1] = lam_of(a.lam, m1[q]);
+    L[q][2] = lam_of(a.lam, m0[q] - w[q]);
+    L[q][3] = lam_of(a.lam, m1[q] + w[q]);
   }
-  i128 dS = 0;
-  bool inf = false;
-  int32_t acc = 0;
-  if (s != r) {
-    wave_fence();  // the table is complete
-    dS = nodal_delta(a, T, r, s, rM, dor, dir, kc, (int32_t)k_out, (int32_t)k_in, wself, inf,
-                     bytes, s_pre, sM_pre, dos_pre, dis_pre);
-    acc = (inf || dS < 0) ? 1 : 0;
-  }
-  if (lane == 0) {
-    a.prop_s[item] = s;
-    a.prop_hi[item] = (long)(dS >> 64);
-    a.prop_lo[item] = (unsigned long)(u128)dS;
-    a.prop_inf[item] = inf ? -1 : 0;
-    a.prop_acc[item] = acc;
-    a.prop_r[item] = r;
-    if (a.prop_u) a.prop_u[item] = u;
-  }
-  acc_out = acc;
-  inf_out = inf ? 1 : 0;
-  dS_out = dS;
-  return bytes;
+  const Cnt crs = m_value<kD>(M, rM, s, pRS);
+  const Corner c{m_value<kD>(M, rM, r, pRR).o, crs.o, crs.i, m_value<kD>(M, sM, s, pSS).o,
+                 dor, dir, dos, dis, k_out, k_in, wor, wir, wos, wis, wself};
+  corner_terms(a, c, acc, out.inf);
+#pragma unroll
+  for (int q = 0; q < U; ++q) unit_terms(acc, L[q], m0[q], m1[q], w[q]);
+  if (neg) atomicOr(&a.status->flags, kFlagNegative);
+  acc.h = wave_sum(acc.h);
+  acc.l = wave_sum(acc.l);
+  out.dS = acc_value(acc);
+  out.acc = (out.inf || out.dS < 0) ? 1 : 0;
 }
 
-__global__ __launch_bounds__(kWave* kNodalWaves) void k_nodal(NodalArgs a) {
-  __shared__ int32_t s_tab[kNodalWaves][3 * kTab];
-  __shared__ __align__(8) int32_t s_scr[kNodalWaves][kScrNodal];
+// Workgroup scratch of nodal_hub.
+struct HubShared {
+  long h[kNodalWaves], l[kNodalWaves];
+  uint32_t sum[2];
+  int32_t s, u, units, wself;
+  int32_t w[4];  // weights into r (out, in) and s (out, in)
+  long bytes;
+};
+
+// The unit table of a node a whole workgroup handles: in LDS, or, when its
+// units may exceed that, in the node's global table.  Slots are read by
+// relaxed atomic loads (the table may sit in global memory, where the atomics
+// that build it bypass the CU's cache).
+constexpr int kHubCap = kNodalWaves * kLdsWave / 2;  // slots of the LDS table
+constexpr int kHubUnits = kHubCap * 3 / 4;
+
+template <bool kD, bool kW, bool kBig>
+__device__ __forceinline__ void hub_terms(const NodalArgs& a, int32_t n, int32_t r, int32_t s,
+                                          int64_t o0, int64_t i0, int32_t kco, int32_t kc,
+                                          int32_t* lds, HubShared& hub, Row rM, Row sM, Acc& acc) {
+  const GraphView& g = a.g;
+  const MView& M = a.M;
+  int32_t cap = kHubCap;
+  uint32_t* tk = reinterpret_cast<uint32_t*>(lds);
+  int32_t* tw = lds + kHubCap;
+  if (kBig) {
+    cap = 1;
+    while (cap < 2 * kc) cap <<= 1;
+    tk = reinterpret_cast<uint32_t*>(a.big_tab + a.big_off[n]);
+    tw = a.big_tab + a.big_off[n] + cap;
+  }
+  const uint32_t mask = (uint32_t)cap - 1;
+  for (int32_t i = threadIdx.x; i < cap; i += blockDim.x) {
+    tk[i] = kNoUnit;
+    tw[i] = 0;
+  }
+  __syncthreads();
+  uint32_t ws = 0;
+  constexpr int kQ = 2;  // entries and slots in flight per thread
+#pragma unroll 1
+  for (int32_t base = threadIdx.x; base < kc; base += kQ * blockDim.x) {
+    int32_t v[kQ], w[kQ], lb[kQ];
+#pragma unroll
+    for (int q = 0; q < kQ; ++q)
+      list_entry(g, o0, kco, i0, kc, base + q * (int32_t)blockDim.x, v[q], w[q]);
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) lb[q] = v[q] >= 0 ? a.labels[v[q]] : -1;
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      if (v[q] < 0) continue;
+      const bool in = base + q * (int32_t)blockDim.x >= kco;
+      if (!in && v[q] == n) ws += (uint32_t)w[q];
+      const uint32_t key = unit_key(lb[q], in);
+      uint32_t h = hash32((int32_t)key) & mask;
+      for (;;) {
+        const uint32_t old = atomicCAS(&tk[h], kNoUnit, key);
+        if (old == kNoUnit || old == key) break;
+        h = (h + 1) & mask;
+      }
+      atomicAdd(&tw[h], w[q]);
+    }
+  }
+  if (ws) atomicAdd(reinterpret_cast<uint32_t*>(&hub.wself), ws);
+  __syncthreads();
+  bool neg = false;
+#pragma unroll 1
+  for (int32_t base = threadIdx.x; base < cap; base += kQ * (int32_t)blockDim.x) {
+    uint32_t key[kQ];
+    int32_t w[kQ];
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      const int32_t i = base + q * (int32_t)blockDim.x;
+      key[q] = kNoUnit;
+      w[q] = 0;
+      if (i < cap) {
+        key[q] = __hip_atomic_load(&tk[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        w[q] = __hip_atomic_load(&tw[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    Probe p0[kQ], p1[kQ];
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      const int32_t b = (int32_t)(key[q] >> 1);
+      if (key[q] == kNoUnit) continue;
+      if (b == r || b == s) {
+        hub.w[2 * (b == s) + (int)(key[q] & 1u)] = w[q];
+        key[q] = kNoUnit;
+        continue;
+      }
+      p0[q] = m_probe<kD>(M, rM, b);
+      p1[q] = m_probe<kD>(M, sM, b);
+    }
+    int32_t m0[kQ], m1[kQ];
+    int64_t L[kQ][4];
+    int32_t live = 0;
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      m0[q] = m1[q] = 0;
+      if (key[q] != kNoUnit) {
+        const int32_t b = (int32_t)(key[q] >> 1);
+        const Cnt cr = m_value<kD>(M, rM, b, p0[q]), cs = m_value<kD>(M, sM, b, p1[q]);
+        const bool in = key[q] & 1u;
+        m0[q] = in ? cr.i : cr.o;
+        m1[q] = in ? cs.i : cs.o;
+        ++live;
+      } else {
+        w[q] = 0;
+      }
+      neg |= m0[q] < w[q];
+      L[q][0] = lam_of(a.lam, m0[q]);
+      L[q][1] = lam_of(a.lam, m1[q]);
+      L[q][2] = lam_of(a.lam, m0[q] - w[q]);
+      L[q][3] = lam_of(a.lam, m1[q] + w[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) unit_terms(acc, L[q], m0[q], m1[q], w[q]);
+    if (a.tstamp && live) atomicAdd(&hub.units, live);
+  }
+  if (neg) atomicOr(&a.status->flags, kFlagNegative);
+}
+
+// One nodal proposal by the whole workgroup, for a node with more list entries
+// than a wavefront's registers take (one wavefront alone set the length of the
+// launch: N = 3001 with four 1200-entry hubs 50.6 -> 13.9 us a launch).
+// The first wavefront draws; the result is in thread 0's out.
+template <bool kD, bool kW>
+__device__ __forceinline__ void nodal_hub(const NodalArgs& a, int32_t n, int32_t* lds,
+                                          HubShared& hub, Nodal& out) {
+  const int lane = lane_id(), w = threadIdx.x / kWave;
+  const GraphView& g = a.g;
+  const MView& M = a.M;
+  const int32_t B = a.B;
+  const int32_t r = a.labels[n];
+  const int64_t o0 = g.out_ptr[n], i0 = g.in_ptr[n];
+  const int32_t kco = (int32_t)(g.out_ptr[n + 1] - o0);
+  const int32_t kc = kco + (int32_t)(g.in_ptr[n + 1] - i0);
+  uint64_t x[4];
+  predrawn(a.draws, (a.predrawn ? a.sweep->stream0 : 0) + (uint64_t)n, x);
+  if (threadIdx.x == 0) {
+    hub.sum[0] = hub.sum[1] = 0;
+    hub.units = hub.wself = 0;
+    hub.w[0] = hub.w[1] = hub.w[2] = hub.w[3] = 0;
+  }
+  __syncthreads();
+  int32_t k_out = kco, k_in = kc - kco;
+  if (kW) {
+    uint32_t so = 0, si = 0;
+    for (int32_t j = threadIdx.x; j < kc; j += blockDim.x) {
+      if (j < kco)
+        so += (uint32_t)g.out_w[o0 + j];
+      else
+        si += (uint32_t)g.in_w[i0 + (j - kco)];
+    }
+    so = wave_sum32(so);
+    si = wave_sum32(si);
+    if (lane == 0) {
+      atomicAdd(&hub.sum[0], so);
+      atomicAdd(&hub.sum[1], si);
+    }
+    __syncthreads();
+    k_out = (int32_t)hub.sum[0];
+    k_in = (int32_t)hub.sum[1];
+  }
+  const uint32_t k = (uint32_t)k_out + (uint32_t)k_in;
+  if (w == 0) {
+    long bytes = 32 + 4 + 32 + (kW ? 4 * (long)kc : 0);
+    int32_t u = -1, s = (int32_t)idx32(x[2], (uint32_t)B);
+    if (k > 0) {
+      u = a.labels[pick_neighbor(g, o0, kco, i0, kc - kco, (int64_t)idx32(x[0], k))];
+      const uint32_t da = (uint32_t)a.d_out[u] + (uint32_t)a.d_in[u];
+      bytes += 16;
+      if (!usap::uniform_branch(x[1], da, B))
+        s = select_combined<kD>(M, u, idx32(x[3], da), -1, load_sums(M, u), lds, kLdsWave, bytes);
+    }
+    if (lane == 0) {
+      hub.s = s;
+      hub.u = u;
+      hub.bytes = bytes;
+    }
+  }
+  __syncthreads();
+  const int32_t s = hub.s;
+  out.s = s;
+  out.u = hub.u;
+  out.acc = 0;
+  out.inf = false;
+  out.dS = 0;
+  out.bytes = hub.bytes;
+  if (s == r) return;  // the same for every thread
+  const Row rM = m_row<kD>(M, r), sM = m_row<kD>(M, s);
+  Acc acc{0, 0};
+  const int64_t most = min((int64_t)kc, 2 * (int64_t)B);  // units
+  if (most <= kHubUnits)
+    hub_terms<kD, kW, false>(a, n, r, s, o0, i0, kco, kc, lds, hub, rM, sM, acc);
+  else
+    hub_terms<kD, kW, true>(a, n, r, s, o0, i0, kco, kc, lds, hub, rM, sM, acc);
+  acc.h = wave_sum(acc.h);
+  acc.l = wave_sum(acc.l);
+  if (lane == 0) {
+    hub.h[w] = acc.h;
+    hub.l[w] = acc.l;
+  }
+  __syncthreads();
+  if (w == 0) {
+    const Cnt crs = m_value<kD>(M, rM, s, m_probe<kD>(M, rM, s));
+    const Corner c{m_value<kD>(M, rM, r, m_probe<kD>(M, rM, r)).o, crs.o, crs.i,
+                   m_value<kD>(M, sM, s, m_probe<kD>(M, sM, s)).o,
+                   a.d_out[r], a.d_in[r], a.d_out[s], a.d_in[s], k_out, k_in,
+                   hub.w[0], hub.w[1], hub.w[2], hub.w[3], hub.wself};
+    Acc t{0, 0};
+    corner_terms(a, c, t, out.inf);
+    t.h = wave_sum(t.h);
+    t.l = wave_sum(t.l);
+    for (int i = 0; i < kNodalWaves; ++i) {
+      t.h += hub.h[i];
+      t.l += hub.l[i];
+    }
+    out.dS = acc_value(t);
+    out.acc = (out.inf || out.dS < 0) ? 1 : 0;
+    out.bytes += (kW ? 12 : 8) * (long)kc + 24 + 16 + 12 * (long)(2 * hub.units + 3);
+  }
+}
+
+// Batch nodes [beg, end), four to a workgroup, one wavefront each; nodes too
+// large for a wavefront are left to the whole workgroup afterwards (kHub: the
+// graph has such nodes; their code costs registers).
+template <bool kD, bool kW, bool kHub>
+__global__ __launch_bounds__(kWave* kNodalWaves, 4) void k_nodal(NodalArgs a) {
+  __shared__ __align__(16) int32_t s_lds[kNodalWaves][kLdsWave];
+  __shared__ unsigned long long s_p[kNodalWaves][6];
+  __shared__ int32_t s_large[kNodalWaves];
   const int w = threadIdx.x / kWave;
   if (a.tstamp && threadIdx.x == 0) a.tstamp[blockIdx.x] = wall_clock64();
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -2014,52 +2386,76 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_nodal(NodalArgs a) {
     // updates stop meanwhile
     a.sweep->stop_n = a.sweep->stop;
   }
-  const int64_t item = (int64_t)xcd_block(blockIdx.x, gridDim.x) * kNodalWaves + w;
+  const int64_t item0 = (int64_t)xcd_block(blockIdx.x, gridDim.x) * kNodalWaves;
+  const int64_t item = item0 + w;
   const int64_t n64 = (int64_t)a.beg + item;
-  long bytes = 0, abytes = 0;
-  int32_t acc = 0, inf = 0;
-  i128 dS = 0;
+  // this node's proposal to memory, and its share of the batch sums: accepted
+  // moves, the exact sum of their finite dS, the -inf ones, byte tallies
+  auto store = [&](int64_t it, int wv, int32_t r, int32_t kc, const Nodal& p) {
+    a.prop[it] = Prop{p.s, r, p.acc, p.inf ? -1 : 0};
+    a.prop_ds[it] = PropDs{(long)(p.dS >> 64), (unsigned long)(u128)p.dS};
+    if (a.prop_u) a.prop_u[it] = p.u;
+    const u128 d = (p.acc && !p.inf) ? (u128)p.dS : (u128)0;
+    s_p[wv][0] = (unsigned long long)p.bytes;
+    s_p[wv][1] = p.acc ? (unsigned long long)apply_tally(kc) : 0ull;
+    s_p[wv][2] = (unsigned long long)d;
+    s_p[wv][3] = (unsigned long long)(d >> 64);
+    s_p[wv][4] = (unsigned long long)p.acc;
+    s_p[wv][5] = (unsigned long long)(p.acc && p.inf);
+  };
+  bool large = false;
+  if (lane_id() == 0)
+    for (int i = 0; i < 6; ++i) s_p[w][i] = 0;
   if (n64 < a.end) {
     // the sweep's stop flag is read together with the node's first loads
     const int32_t n = (int32_t)n64;
     const int32_t stop = a.sweep->stop;
-    const uint64_t stream0 = a.sweep->stream0;
+    uint64_t x[4];
+    predrawn(a.draws, (a.predrawn ? a.sweep->stream0 : 0) + (uint64_t)n, x);
     const int32_t r = a.labels[n];
     const int64_t o0 = a.g.out_ptr[n], i0 = a.g.in_ptr[n];
-    const int64_t kco = a.g.out_ptr[n + 1] - o0, kci = a.g.in_ptr[n + 1] - i0;
+    const int64_t kco = a.g.out_ptr[n + 1] - o0, kc = kco + (a.g.in_ptr[n + 1] - i0);
     if (!stop) {
-      bytes = kco + kci > kTabMaxDeg
-                  ? nodal_one<true>(a, item, n, r, o0, kco, i0, kci, stream0, s_tab[w], s_scr[w],
-                                    acc, inf, dS)
-                  : nodal_one<false>(a, item, n, r, o0, kco, i0, kci, stream0, s_tab[w],
-                                     s_scr[w], acc, inf, dS);
-      if (acc) abytes = apply_tally(kco + kci);
+      large = kHub && kc > kRegUnits * kWave;
+      if (!large) {
+        Nodal p;
+        const int32_t ko = (int32_t)kco, kk = (int32_t)kc;
+        if (kk <= kWave)
+          nodal_regs<kD, kW, 1>(a, n, r, o0, i0, ko, kk, x, s_lds[w], p);
+        else if (kk <= 2 * kWave)
+          nodal_regs<kD, kW, 2>(a, n, r, o0, i0, ko, kk, x, s_lds[w], p);
+        else
+          nodal_regs<kD, kW, kRegUnits>(a, n, r, o0, i0, ko, kk, x, s_lds[w], p);
+        if (lane_id() == 0) store(item, w, r, kk, p);
+      }
     }
   }
-  __syncthreads();  // every wavefront is done with its scratch
-  // this block's share of the batch sums: accepted moves, the exact sum of
-  // their finite dS, the -inf ones, byte tallies
-  unsigned long long* s_p = reinterpret_cast<unsigned long long*>(&s_scr[0][0]);
-  if (lane_id() == 0) {
-    const u128 d = (acc && !inf) ? (u128)dS : (u128)0;
-    s_p[6 * w + 0] = (unsigned long long)bytes;
-    s_p[6 * w + 1] = (unsigned long long)abytes;
-    s_p[6 * w + 2] = (unsigned long long)d;
-    s_p[6 * w + 3] = (unsigned long long)(d >> 64);
-    s_p[6 * w + 4] = (unsigned long long)acc;
-    s_p[6 * w + 5] = (unsigned long long)(acc && inf);
+  if (kHub && lane_id() == 0) s_large[w] = large;
+  __syncthreads();  // every wavefront is done with its LDS
+  if (kHub) {
+    __shared__ HubShared s_hub;
+    for (int i = 0; i < kNodalWaves; ++i) {
+      if (!s_large[i]) continue;
+      const int32_t n = (int32_t)((int64_t)a.beg + item0 + i);
+      Nodal p;
+      nodal_hub<kD, kW>(a, n, &s_lds[0][0], s_hub, p);
+      if (threadIdx.x == 0)
+        store(item0 + i, i, a.labels[n],
+              (int32_t)((a.g.out_ptr[n + 1] - a.g.out_ptr[n]) + (a.g.in_ptr[n + 1] - a.g.in_ptr[n])),
+              p);
+      __syncthreads();
+    }
   }
-  __syncthreads();
   if (threadIdx.x == 0) {
     unsigned long long nb = 0, ab = 0;
     u128 sum = 0;
     int32_t moves = 0, ninf = 0;
     for (int i = 0; i < kNodalWaves; ++i) {
-      nb += s_p[6 * i + 0];
-      ab += s_p[6 * i + 1];
-      sum += ((u128)s_p[6 * i + 3] << 64) | (u128)s_p[6 * i + 2];
-      moves += (int32_t)s_p[6 * i + 4];
-      ninf += (int32_t)s_p[6 * i + 5];
+      nb += s_p[i][0];
+      ab += s_p[i][1];
+      sum += ((u128)s_p[i][3] << 64) | (u128)s_p[i][2];
+      moves += (int32_t)s_p[i][4];
+      ninf += (int32_t)s_p[i][5];
     }
     BlockPart& P = a.part[blockIdx.x];
     P.sum_lo = (unsigned long)sum;
@@ -2090,10 +2486,8 @@ struct AqArgs {
   GraphView g;
   MView M;
   int32_t beg, end;
-  const int32_t* prop_r;
-  const int32_t* prop_s;
+  const Prop* prop;
   const int32_t* prop_u;
-  const int32_t* prop_acc;
   int32_t* mark;
   int32_t stamp;
   const Sweep* sweep;
@@ -2109,8 +2503,8 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_aq(AqArgs a) {
   const int64_t kc =
       live ? (a.g.out_ptr[n + 1] - a.g.out_ptr[n]) + (a.g.in_ptr[n + 1] - a.g.in_ptr[n]) : 0;
   int32_t b = -1;
-  if (live && lane == 0) b = a.prop_r[item];
-  if (live && lane == 1) b = a.prop_s[item];
+  if (live && lane == 0) b = a.prop[item].r;
+  if (live && lane == 1) b = a.prop[item].s;
   if (live && lane == 2) b = a.prop_u[item];
   const bool first = b >= 0 && atomicMax(&a.mark[b], a.stamp) < a.stamp;
   unsigned long long rows = __ballot(first);
@@ -2135,7 +2529,7 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_aq(AqArgs a) {
     if (live) {
       node = 16 + 4 + 8 * (unsigned long long)kc + 12;
       if (a.g.out_w) node += 4 * (unsigned long long)kc;
-      if (a.prop_acc[item]) node += 4 + 16 * (unsigned long long)kc;
+      if (a.prop[item].acc) node += 4 + 16 * (unsigned long long)kc;
     }
     s_node[w] = node;
     s_blk[w] = blk;
@@ -2226,12 +2620,7 @@ struct ApplyArgs {
   int32_t beg, end;
   const int64_t* big_off;
   int32_t* big_tab;
-  const int32_t* prop_s;
-  const long* prop_hi;
-  const unsigned long* prop_lo;
-  const int32_t* prop_inf;
-  const int32_t* prop_acc;
-  const int32_t* prop_r;
+  const Prop* prop;
   const BlockPart* part;  // k_nodal's per-workgroup shares of the batch
   uint32_t nparts;
   Status* status;
@@ -2300,7 +2689,7 @@ __device__ void sweep_tail(Sweep* sw, u128 sum, int32_t ninf, int32_t moves,
 // edges b -> n), so each changed pair of counts gets one 64-bit atomic per
 // node (apply_entry); edges to neighbours that move in the same batch are
 // applied here, one by one.  Also moves the node's degrees and writes its
-// label.  Old labels of nodes inside the batch come from prop_r, so writing
+// label.  Old labels of nodes inside the batch come from prop, so writing
 // labels cannot race with their reads.  Returns the table, compacted to its
 // nent entries (nent = 0 when none is left).
 template <bool kBig>
@@ -2325,8 +2714,9 @@ __device__ __forceinline__ Table apply_table(const ApplyArgs& a, int32_t n, int3
       if (v[q] < 0) continue;
       if (v[q] >= a.beg && v[q] < a.end) {
         const int32_t x = v[q] - a.beg;
-        bo[q] = a.prop_r[x];
-        bn[q] = a.prop_acc[x] ? a.prop_s[x] : -2;
+        const Prop p = a.prop[x];
+        bo[q] = p.r;
+        bn[q] = p.acc ? p.s : -2;
       } else {
         bo[q] = a.labels[v[q]];
         bn[q] = -2;
@@ -2480,8 +2870,8 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_apply(ApplyArgs a) {
   // whether the batch runs, the proposal and the node's list bounds in one
   // round of loads
   const int32_t stop = a.sweep->stop_n;  // the same for every block of this launch
-  const int32_t acc = in ? a.prop_acc[item] : 0;
-  const int32_t pr = in ? a.prop_r[item] : 0, ps = in ? a.prop_s[item] : 0;
+  const Prop p = in ? a.prop[item] : Prop{0, 0, 0, 0};
+  const int32_t acc = p.acc, pr = p.r, ps = p.s;
   const int64_t o0 = a.g.out_ptr[n], i0 = a.g.in_ptr[n];
   const int64_t kco = a.g.out_ptr[n + 1] - o0, kci = a.g.in_ptr[n + 1] - i0;
   if (stop) return;
@@ -2890,11 +3280,9 @@ struct usap_engine {
   void* sort_tmp = nullptr;
   size_t sort_tmp_bytes = 0;
   // nodal
-  int32_t* prop_s = nullptr;
-  long* prop_hi = nullptr;
-  unsigned long* prop_lo = nullptr;
-  int32_t* prop_inf = nullptr;
-  int32_t* prop_acc = nullptr;
+  Prop* prop = nullptr;
+  PropDs* prop_ds = nullptr;
+  uint64_t* draws = nullptr;  // the sweep's (or batch's) Philox words, 4 per node
   int32_t last_beg = 0, last_end = 0;
   // pre-drawn uniform stream (usap_set_uniforms): 4 words per draw, or null
   uint64_t* uni = nullptr;
@@ -2906,7 +3294,6 @@ struct usap_engine {
   Sweep* h_sweep = nullptr;   // pinned host copy
   Sweep* h_chunk[2] = {nullptr, nullptr};  // sweep state after alternate launch chunks
   hipEvent_t chunk_ev[2] = {nullptr, nullptr};
-  int32_t* prop_r = nullptr;  // old label of each batch node
   // reference-algorithm byte counts (profiling): drawn neighbour's block per
   // batch node, per-block batch stamps, device totals [nodal per-node,
   // nodal per-block, merge non-zeros]
@@ -2931,6 +3318,7 @@ struct usap_engine {
   size_t pair_tmp_bytes = 0;
   int64_t* big_off = nullptr;
   int32_t* big_tab = nullptr;
+  int64_t max_list = 0;  // list entries of the largest node
   // entropy
   long* ent_part = nullptr;
   long* h_ent_part = nullptr;
@@ -3429,15 +3817,12 @@ int usap_destroy(usap_engine* e) {
     dfree(e, e->sort_idx[i]);
   }
   dfree(e, e->sort_tmp);
-  dfree(e, e->prop_s);
-  dfree(e, e->prop_hi);
-  dfree(e, e->prop_lo);
-  dfree(e, e->prop_inf);
-  dfree(e, e->prop_acc);
+  dfree(e, e->prop);
+  dfree(e, e->prop_ds);
+  dfree(e, e->draws);
   dfree(e, e->part);
   dfree(e, e->status);
   dfree(e, e->sweep);
-  dfree(e, e->prop_r);
   dfree(e, e->prop_u);
   dfree(e, e->aq_mark);
   dfree(e, e->aq_acc);
@@ -3572,8 +3957,10 @@ int load_graph(usap_engine* e, const usap_graph* g, int64_t wtot) {
   // global-memory neighbour tables of the nodes too large for LDS
   std::vector<int64_t> big((size_t)N, -1);
   int64_t big_total = 0;
+  e->max_list = 0;
   for (int32_t x = 0; x < N; ++x) {
     const int64_t k = (g->out_ptr[x + 1] - g->out_ptr[x]) + (g->in_ptr[x + 1] - g->in_ptr[x]);
+    e->max_list = std::max(e->max_list, k);
     if (k > kTabMaxDeg) {
       int64_t cap = 1;
       while (cap < 2 * k) cap <<= 1;
@@ -3608,8 +3995,10 @@ int build_big_tables(usap_engine* e) {
   const int32_t N = e->N;
   std::vector<int64_t> big((size_t)N, -1);
   int64_t big_total = 0;
+  e->max_list = 0;
   for (int32_t x = 0; x < N; ++x) {
     const int64_t k = (e->h_out_ptr[x + 1] - e->h_out_ptr[x]) + (e->h_in_ptr[x + 1] - e->h_in_ptr[x]);
+    e->max_list = std::max(e->max_list, k);
     if (k > kTabMaxDeg) {
       int64_t cap = 1;
       while (cap < 2 * k) cap <<= 1;
@@ -3828,15 +4217,12 @@ int alloc_state(usap_engine* e) {
   TRY(dalloc(e, &e->best_hi, N));
   TRY(dalloc(e, &e->best_lo, N));
   TRY(dalloc(e, &e->map, N));
-  TRY(dalloc(e, &e->prop_s, N));
-  TRY(dalloc(e, &e->prop_hi, N));
-  TRY(dalloc(e, &e->prop_lo, N));
-  TRY(dalloc(e, &e->prop_inf, N));
-  TRY(dalloc(e, &e->prop_acc, N));
+  TRY(dalloc(e, &e->prop, N));
+  TRY(dalloc(e, &e->prop_ds, N));
+  TRY(dalloc(e, &e->draws, (size_t)4 * N));
   TRY(dalloc(e, &e->status, 1));
   TRY(dalloc(e, &e->part, blocks_for(N, kNodalWaves)));
   TRY(dalloc(e, &e->sweep, 1));
-  TRY(dalloc(e, &e->prop_r, N));
   TRY(dalloc(e, &e->build_flags, 3));
   TRY(dalloc(e, &e->ent_part, 2 * kEntropyBlocks));
   e->h_sweep = (Sweep*)pin_get(sizeof(Sweep));
@@ -4449,10 +4835,29 @@ int prof_end(usap_engine* e, size_t executed) {
   return USAP_OK;
 }
 
-// Launches k_nodal + k_apply + k_grow for nodes [beg, end), batch bidx of the
-// sweep (random stream sweep->stream0 + bidx).
-int launch_batch(usap_engine* e, int32_t beg, int32_t end, int32_t bidx, size_t ev_slot,
-                 bool grow = true) {
+// k_nodal for M all direct or not, a weighted graph or not, with nodes beyond a
+// wavefront's registers or without.
+typedef void (*NodalKernel)(NodalArgs);
+NodalKernel nodal_kernel(bool dense, bool weighted, bool hubs) {
+  static const NodalKernel k[8] = {
+      k_nodal<false, false, false>, k_nodal<false, false, true>, k_nodal<false, true, false>,
+      k_nodal<false, true, true>,   k_nodal<true, false, false>, k_nodal<true, false, true>,
+      k_nodal<true, true, false>,   k_nodal<true, true, true>};
+  return k[4 * dense + 2 * weighted + hubs];
+}
+
+// The Philox words of nodes [beg, end) in batches of `batch` (batch i: stream
+// sweep->stream0 + i), before their first batch (pre-drawn mode has its own).
+int launch_draws(usap_engine* e, int32_t beg, int32_t end, int32_t batch) {
+  if (e->uni) return USAP_OK;
+  k_draw<<<blocks_for((int64_t)end - beg, 256), 256, 0, e->stream>>>(beg, end, batch, e->p.seed,
+                                                                     e->sweep, e->draws);
+  HIPCHK(hipGetLastError());
+  return USAP_OK;
+}
+
+// Launches k_nodal + k_apply + k_grow for nodes [beg, end).
+int launch_batch(usap_engine* e, int32_t beg, int32_t end, size_t ev_slot, bool grow = true) {
   const int32_t B = e->B;
   hipStream_t st = e->stream;
   NodalArgs a;
@@ -4466,8 +4871,6 @@ int launch_batch(usap_engine* e, int32_t beg, int32_t end, int32_t bidx, size_t 
   a.beg = beg;
   a.end = end;
   a.exact = e->p.ds_mode == USAP_DS_EXACT;
-  a.seed = e->p.seed;
-  a.bidx = bidx;
   // profiled: this slot's workgroup stamps (k_nodal: G starts + G ends;
   // k_apply: G + 1 each; k_grow: kGrowBlocks each)
   const int32_t G = e->tstamp_G;
@@ -4477,14 +4880,11 @@ int launch_batch(usap_engine* e, int32_t beg, int32_t end, int32_t bidx, size_t 
   a.tstride = G;
   a.big_off = e->big_off;
   a.big_tab = e->big_tab;
-  a.prop_s = e->prop_s;
-  a.prop_hi = e->prop_hi;
-  a.prop_lo = e->prop_lo;
-  a.prop_inf = e->prop_inf;
-  a.prop_acc = e->prop_acc;
-  a.prop_r = e->prop_r;
+  a.prop = e->prop;
+  a.prop_ds = e->prop_ds;
   a.prop_u = e->prof ? e->prop_u : nullptr;
-  a.uni = e->uni;
+  a.draws = e->uni ? e->uni : e->draws;
+  a.predrawn = e->uni != nullptr;
   a.part = e->part;
   a.status = e->status;
   a.sweep = e->sweep;
@@ -4497,12 +4897,7 @@ int launch_batch(usap_engine* e, int32_t beg, int32_t end, int32_t bidx, size_t 
   b.bsize = e->bsize;
   b.beg = beg;
   b.end = end;
-  b.prop_s = e->prop_s;
-  b.prop_hi = e->prop_hi;
-  b.prop_lo = e->prop_lo;
-  b.prop_inf = e->prop_inf;
-  b.prop_acc = e->prop_acc;
-  b.prop_r = e->prop_r;
+  b.prop = e->prop;
   b.big_off = e->big_off;
   b.big_tab = e->big_tab;
   const unsigned grid = blocks_for((int64_t)end - beg, kNodalWaves);
@@ -4535,17 +4930,16 @@ int launch_batch(usap_engine* e, int32_t beg, int32_t end, int32_t bidx, size_t 
   ga.tstride = kGrowBlocks;
   if (e->prof && (int64_t)grid > G)
     return set_err(e, USAP_ESTATE, "profiled batch larger than its stamp slot");
-  k_nodal<<<grid, kWave * kNodalWaves, 0, st>>>(a);
+  nodal_kernel(e->all_direct, e->weighted, e->max_list > kRegUnits * kWave)<<<
+      grid, kWave * kNodalWaves, 0, st>>>(a);
   if (e->prof) {  // the reference algorithm's bytes for this batch (M not yet changed)
     AqArgs q;
     q.g = a.g;
     q.M = a.M;
     q.beg = beg;
     q.end = end;
-    q.prop_r = e->prop_r;
-    q.prop_s = e->prop_s;
+    q.prop = e->prop;
     q.prop_u = e->prop_u;
-    q.prop_acc = e->prop_acc;
     q.mark = e->aq_mark;
     q.stamp = e->aq_stamp++;
     q.sweep = e->sweep;
@@ -4573,11 +4967,11 @@ int sweep_graph(usap_engine* e, int32_t batch, int32_t nb) {
       e->gexec = nullptr;
     }
     HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    int rc = USAP_OK;
+    int rc = launch_draws(e, 0, e->N, batch);
     for (int32_t i = 0; i < nb && rc == USAP_OK; ++i) {
       const int32_t beg = i * batch;
       const int32_t end = std::min<int64_t>((int64_t)beg + batch, e->N);
-      rc = launch_batch(e, beg, end, i, 0);
+      rc = launch_batch(e, beg, end, 0);
     }
     hipGraph_t graph = nullptr;
     const hipError_t ce = hipStreamEndCapture(st, &graph);
@@ -4620,6 +5014,8 @@ int run_sweep(usap_engine* e, int32_t batch, int32_t first, int32_t last, int32_
     } else {
       if (e->prof)
         if (int rc = prof_begin(e, (size_t)(last - next), batch)) return rc;
+      if (next == 0)  // a resumed round still has the sweep's draws
+        if (int rc = launch_draws(e, 0, e->N, batch)) return rc;
       // A sweep whose convergence test is active stops at a batch nobody
       // knows in advance, and the batches launched after it exit at once
       // (a few us each).  Such a sweep goes out in chunks of kChunk batches,
@@ -4637,7 +5033,7 @@ int run_sweep(usap_engine* e, int32_t batch, int32_t first, int32_t last, int32_
           // with every row direct, the chunk's last k_grow folds the error
           // flags of all its batches (they only report inconsistent M)
           const bool grow = !e->all_direct || e->prof || i == upto - 1;
-          if (int rc = launch_batch(e, beg, end, i, slot, grow)) return rc;
+          if (int rc = launch_batch(e, beg, end, slot, grow)) return rc;
         }
         i0 = upto;
         if (!chunked) break;
@@ -4708,7 +5104,8 @@ int usap_nodal_batch(usap_engine* e, int32_t begin, int32_t end, uint64_t stream
     // "batch" starts at begin
     if (e->prof)
       if (int rc = prof_begin(e, 1, end - begin)) return rc;
-    if (int rc = launch_batch(e, begin, end, 0, 0)) return rc;
+    if (int rc = launch_draws(e, begin, end, end - begin)) return rc;
+    if (int rc = launch_batch(e, begin, end, 0)) return rc;
     Sweep& hs = *e->h_sweep;
     HIPCHK(hipMemcpyAsync(&hs, e->sweep, sizeof(Sweep), hipMemcpyDeviceToHost, e->stream));
     HIPCHK(hipStreamSynchronize(e->stream));
@@ -4833,12 +5230,18 @@ int usap_nodal_detail(usap_engine* e, int32_t* s, int64_t* hi, uint64_t* lo, int
   const int64_t n = e->last_end - e->last_beg;
   hipStream_t st = e->stream;
   if (n > 0) {
-    if (s) HIPCHK(hipMemcpyAsync(s, e->prop_s, sizeof(int32_t) * n, hipMemcpyDeviceToHost, st));
-    if (hi) HIPCHK(hipMemcpyAsync(hi, e->prop_hi, sizeof(int64_t) * n, hipMemcpyDeviceToHost, st));
-    if (lo) HIPCHK(hipMemcpyAsync(lo, e->prop_lo, sizeof(uint64_t) * n, hipMemcpyDeviceToHost, st));
-    if (inf) HIPCHK(hipMemcpyAsync(inf, e->prop_inf, sizeof(int32_t) * n, hipMemcpyDeviceToHost, st));
-    if (accept) HIPCHK(hipMemcpyAsync(accept, e->prop_acc, sizeof(int32_t) * n, hipMemcpyDeviceToHost, st));
+    std::vector<Prop> p((size_t)n);
+    std::vector<PropDs> d((size_t)n);
+    HIPCHK(hipMemcpyAsync(p.data(), e->prop, sizeof(Prop) * n, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync(d.data(), e->prop_ds, sizeof(PropDs) * n, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
+    for (int64_t i = 0; i < n; ++i) {
+      if (s) s[i] = p[i].s;
+      if (hi) hi[i] = d[i].hi;
+      if (lo) lo[i] = d[i].lo;
+      if (inf) inf[i] = p[i].inf;
+      if (accept) accept[i] = p[i].acc;
+    }
   }
   return USAP_OK;
 }
