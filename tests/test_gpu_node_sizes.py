@@ -52,3 +52,4 @@ def test_list_sizes(usap, orc, weighted, mode, B):
         assert r["sum"] == ro["sum"]
         np.testing.assert_array_equal(eng.labels(), o.labels())
     assert eng.entropy()[0] == o.entropy()[0]
+    np.testing.assert_array_equal(eng.M_dense(), o.M_dense())

@@ -89,7 +89,6 @@ static __device__ __align__(256) long scratch[2 * kEntropyBlocks];
 constexpr int kNumSnap = 4;
 
 enum : int32_t {
-  kFlagLoad = 1,      // a hashed row passed 3/4 load
   kFlagFull = 2,      // an insertion found no free slot (increment lost)
   kFlagMissing = 4,   // a decrement did not find its key (bug)
   kFlagNegative = 8,  // a negative count reached an entropy term (bug)
@@ -139,10 +138,10 @@ struct __align__(8) Cnt {
 struct MView {
   const int64_t* off;
   const int32_t* cap;
-  int32_t* nkeys;
+  int32_t* gmark;  // [B]: > 0: k_grow looks at the row (kMarked, room_mark)
   int32_t* key;    // row slabs: keys (-1 empty; unused in a direct row) ...
   Cnt* cnt;        // ... and the counts of each slot
-  int32_t* bs;     // [B][kNBK]: sum of the row's o + i per key bucket
+  int32_t* bs;     // [B][kNBK]: sum of the row's o + i per key bucket (rows with row_sums)
   int32_t* gpend;  // [B]: increments of the row waiting in the overflow buffer
   int32_t* ovf;    // [4][ovf_cap]: (row, key, do, di) increments that found no free slot
   int32_t ovf_cap;
@@ -154,15 +153,23 @@ struct MView {
 
 // Rows to grow between two batches; slabs for grown rows come from the free
 // tail of the pool.
+constexpr int kGrowBlocks = 768;  // k_grow's grid: three workgroups of 52 KB of LDS per CU
+
+// A k_grow workgroup's piece of the free tail: slots [pos, end), their counts 0;
+// and what the workgroup did since the engine was created.
+struct GrowChunk {
+  long long pos, end;
+  unsigned long long grows;        // rows grown or compacted
+  unsigned long long compactions;  // of them in place
+};
+
 struct GrowState {
-  int32_t n;                  // unused (rows to grow are found by k_grow's scan)
   int32_t nospace;            // the pool ran out: the host rebuilds M
   int32_t ovf_n;              // entries in the overflow buffer
   unsigned long long used;    // pool slots in use
-  unsigned long long grows;   // rows grown or compacted since the engine was created
   unsigned long long full;    // insertions that found no free slot
   unsigned long long nospace_events;
-  unsigned long long compactions;
+  GrowChunk chunk[kGrowBlocks];
 };
 
 __device__ __forceinline__ uint32_t hash32(int32_t b) {
@@ -250,90 +257,35 @@ __device__ __forceinline__ void cnt_add(Cnt* q, int32_t dout, int32_t din) {
   atomicAdd(reinterpret_cast<unsigned long long*>(q), (unsigned long long)d);
 }
 
-constexpr int32_t kMaxWalk = 16;  // probes before a nodal-batch increment is parked
-
-// M[a][b] += dout and M[b][a] += din in row R of a (negative only for a key
-// that exists), given the key k read at the first probed slot `slot`.  Keys
-// only go from empty to set, so an earlier read is a valid first read: a
-// stale "empty" makes the claim fail and return the key that is there.
-// kBuckets also updates the row's bucket sum, and leaves a crowded row to
-// k_grow (by its key count, or a parked increment) instead of flagging a
-// rebuild.
-template <bool kBuckets>
-__device__ __forceinline__ void m_add_at(const MView& m, int32_t a, Row R, int32_t b, int32_t dout,
-                                         int32_t din, int64_t slot, int32_t k, int32_t* flags) {
-  if (kBuckets && dout + din != 0)
-    atomicAdd(&m.bs[(int64_t)a * kNBK + (b >> m.bshift)], dout + din);
-  if (R.c == m.B || k == b) {
-    cnt_add(&m.cnt[slot], dout, din);
-    return;
-  }
-  const bool dec = dout < 0 || din < 0;
-  const int64_t o = R.o;
-  const int32_t c = R.c;
-  const uint32_t mask = (uint32_t)c - 1;
-  uint32_t h = (uint32_t)(slot - o);
-  for (int32_t probe = 0; probe < c; ++probe) {
-    // an increment whose key is still absent after kMaxWalk slots is parked
-    // (k_grow grows the row) rather than walking a crowded row
-    if (kBuckets && !dec && probe >= kMaxWalk) break;
-    if (probe > 0) k = ld_relaxed(&m.key[o + h]);
-    if (k < 0) {
-      if (dec) {
-        atomicOr(flags, kFlagMissing);
-        return;
-      }
-      k = atomicCAS(&m.key[o + h], -1, b);
-      if (k == -1) {
-        if (kBuckets) {
-          // the counts and the key count without waiting for either: k_grow
-          // finds the rows past 1/slack load (short probe chains for the
-          // lookups, most of which miss) from the key counts themselves
-          cnt_add(&m.cnt[o + h], dout, din);
-          atomicAdd(&m.nkeys[a], 1);
-          return;
-        }
-        // past 3/4 load in a build: rebuild
-        if (4 * (atomicAdd(&m.nkeys[a], 1) + 1) > 3 * c) atomicOr(flags, kFlagLoad);
-        k = b;
-      }
-    }
-    if (k == b) {
-      cnt_add(&m.cnt[o + h], dout, din);
-      return;
-    }
-    h = (h + 1) & mask;
-  }
-  if (kBuckets && !dec) {  // no free slot near: park the increment until k_grow has grown the row
-    atomicAdd(&m.gst->full, 1ull);
-    const int32_t i = atomicAdd(&m.gst->ovf_n, 1);
-    if (i < m.ovf_cap) {
-      m.ovf[i] = a;
-      m.ovf[m.ovf_cap + i] = b;
-      m.ovf[2 * m.ovf_cap + i] = dout;
-      m.ovf[3 * m.ovf_cap + i] = din;
-      atomicAdd(&m.gpend[a], 1);  // k_grow grows every row with parked increments
-      return;
-    }
-  }
-  atomicOr(flags, dec ? kFlagMissing : kFlagFull);
+constexpr uint32_t kMaxWalk = 32;  // probes before a nodal-batch increment is parked
+constexpr uint32_t kMarkWalk = 4;  // slots from home at which a new key marks its row for k_grow
+// MView::gmark: k_grow looks at rows where it is positive.  A small hashed row's
+// is 0 or kMarked; one of more than kScanRow slots (whose long chains would
+// mark it in nearly every batch, and whose slab takes a workgroup to count)
+// counts new keys up from minus the keys that fit 1/slack load (room_mark).
+constexpr int32_t kMarked = 1 << 30;
+constexpr int32_t kScanRow = 512;  // slots up to which a hashed slab is read whole
+__device__ __forceinline__ int32_t room_mark(int32_t keys, int32_t c, int32_t slack) {
+  return c > kScanRow ? min(0, keys - c / slack) : 0;
 }
 
-// Where m_add_at starts for key b in row R: the keys of kWin slots from b's
-// home slot are read at once (two 16-byte loads; one memory latency for most
-// probe chains) and the first that holds b or is empty is returned with its
-// slot; if none does, the window's last slot, from which m_add_at walks on.
-// The window ends at the slab's end at the latest.  Keys only go from empty
-// to set, so a plain load is as good as a relaxed atomic one.
+// Whether a row of capacity c keeps bucket sums.  The pick reads a direct row
+// of at most kNBK keys and a hashed slab of at most kScanRow slots whole (in
+// one round of loads, as the sums would be), so those rows' counts cost
+// k_apply one atomic less per update and a rebuild 2 KB less per row.
+__device__ __forceinline__ bool row_sums(const MView& m, int32_t c) {
+  return c == m.B ? m.B > kNBK : c > kScanRow;
+}
+
+// The keys of kWin slots of hashed row R from slot h on are read at once (two
+// 16-byte loads; one memory latency for most probe chains); returns the first
+// that holds b or is empty, with its slot in h, or, if none does, the
+// window's last.  The window ends at the slab's end at the latest.  Keys only
+// go from empty to set, so a plain load is as good as a relaxed atomic one.
 constexpr int kWin = 8;
 typedef int32_t Key4 __attribute__((ext_vector_type(4), aligned(4)));  // 4-byte aligned
-__device__ __forceinline__ int32_t m_first_key(const MView& m, Row R, int32_t b, int64_t& slot) {
-  if (R.c == m.B) {
-    slot = R.o + b;
-    return b;
-  }
-  const uint32_t h = hash32(b) & ((uint32_t)R.c - 1);  // hashed rows hold >= 32 slots
-  const uint32_t w0 = min(h, (uint32_t)R.c - kWin);
+__device__ __forceinline__ int32_t m_window(const MView& m, Row R, int32_t b, uint32_t& h) {
+  const uint32_t w0 = min(h, (uint32_t)R.c - kWin);  // hashed rows hold >= 32 slots
   const Key4* w = reinterpret_cast<const Key4*>(m.key + R.o + w0);
   const Key4 lo = w[0], hi = w[1];
   const int32_t k[kWin] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
@@ -346,18 +298,97 @@ __device__ __forceinline__ int32_t m_first_key(const MView& m, Row R, int32_t b,
       pos = w0 + q;
     }
   }
-  slot = R.o + pos;
+  h = pos;
   return kk;
 }
 
-// M[a][b] += dout, M[b][a] += din in row a
-template <bool kBuckets>
+// Where m_add_at starts for key b in row R: the end of its probe chain, or as
+// far along it as one window reaches.
+template <bool kD = false>
+__device__ __forceinline__ int32_t m_first_key(const MView& m, Row R, int32_t b, int64_t& slot) {
+  if (kD || R.c == m.B) {
+    slot = R.o + b;
+    return b;
+  }
+  uint32_t h = hash32(b) & ((uint32_t)R.c - 1);
+  const int32_t k = m_window(m, R, b, h);
+  slot = R.o + h;
+  return k;
+}
+
+// M[a][b] += dout and M[b][a] += din in row R of a (negative only for a key
+// that exists), given the key k read at the first probed slot `slot`.  Keys
+// only go from empty to set, so an earlier read is a valid first read: a
+// stale "empty" makes the claim fail and return the key that is there.
+// kBatch (k_apply) also updates the row's bucket sum, and leaves a crowded row
+// to k_grow (by a mark, or a parked increment) instead of flagging a rebuild.
+template <bool kBatch, bool kD = false>
+__device__ __forceinline__ void m_add_at(const MView& m, int32_t a, Row R, int32_t b, int32_t dout,
+                                         int32_t din, int64_t slot, int32_t k, int32_t* flags) {
+  if (kBatch && dout + din != 0 && row_sums(m, R.c))
+    atomicAdd(&m.bs[(int64_t)a * kNBK + (b >> m.bshift)], dout + din);
+  if (kD || R.c == m.B || k == b) {
+    cnt_add(&m.cnt[slot], dout, din);
+    return;
+  }
+  const bool dec = dout < 0 || din < 0;
+  const int64_t o = R.o;
+  const int32_t c = R.c;
+  const uint32_t mask = (uint32_t)c - 1, home = hash32(b) & mask;
+  uint32_t h = (uint32_t)(slot - o);
+  // an increment whose key is still absent after kMaxWalk slots is parked
+  // (k_grow grows the row) rather than walking a crowded row
+  const uint32_t most = kBatch && !dec ? min(kMaxWalk, (uint32_t)c) : (uint32_t)c;
+  for (;;) {
+    if (k < 0) {
+      if (dec) {
+        atomicOr(flags, kFlagMissing);
+        return;
+      }
+      k = atomicCAS(&m.key[o + h], -1, b);
+      if (k == -1) {
+        cnt_add(&m.cnt[o + h], dout, din);
+        // a new key kMarkWalk slots or more from home: the row is (or will
+        // soon be) past 1/slack load; a large row's new keys are counted
+        if (kBatch && c > kScanRow)
+          atomicAdd(&m.gmark[a], 1);
+        else if (kBatch && ((h - home) & mask) >= kMarkWalk)
+          m.gmark[a] = kMarked;
+        return;
+      }
+    }
+    if (k == b) {
+      cnt_add(&m.cnt[o + h], dout, din);
+      return;
+    }
+    const uint32_t walked = ((h - home) & mask) + 1;  // slots found taken
+    if (walked >= most) break;
+    h = (h + 1) & mask;
+    k = m_window(m, R, b, h);
+    if (((h - home) & mask) < walked) break;  // past the whole slab
+  }
+  if (kBatch && !dec) {  // no free slot near: park the increment until k_grow has grown the row
+    const int32_t i = atomicAdd(&m.gst->ovf_n, 1);
+    if (i < m.ovf_cap) {
+      m.ovf[i] = a;
+      m.ovf[m.ovf_cap + i] = b;
+      m.ovf[2 * m.ovf_cap + i] = dout;
+      m.ovf[3 * m.ovf_cap + i] = din;
+      atomicAdd(&m.gpend[a], 1);  // k_grow grows every row with parked increments
+      m.gmark[a] = kMarked;
+      return;
+    }
+  }
+  atomicOr(flags, dec ? kFlagMissing : kFlagFull);
+}
+
+// M[a][b] += dout, M[b][a] += din in row a (M builds)
 __device__ __forceinline__ void m_add(const MView& m, int32_t a, int32_t b, int32_t dout,
                                       int32_t din, int32_t* flags) {
   const Row R = m_row(m, a);
   int64_t slot;
   const int32_t k = m_first_key(m, R, b, slot);
-  m_add_at<kBuckets>(m, a, R, b, dout, din, slot, k, flags);
+  m_add_at<false>(m, a, R, b, dout, din, slot, k, flags);
 }
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (kWave - 1); }
@@ -630,52 +661,37 @@ __device__ __forceinline__ void lookup_bucket(const MView& m, Row R, int32_t lo,
   }
 }
 
-// A row's kNBK bucket sums, kNBK / 64 consecutive ones per lane (buckets past
-// the last key are 0).
+// A row's weight per key bucket, `per` consecutive buckets per lane (buckets
+// past the last key are 0).
 constexpr int kBkLane = kNBK / kWave;
 struct Sums {
+  int per;
   uint32_t w[kBkLane];
 };
 
-__device__ __forceinline__ Sums load_sums(const MView& M, int32_t u) {
+// Of a row that keeps bucket sums (row_sums), or a direct row of at most kNBK
+// keys (a bucket is one key: its counts).
+__device__ __forceinline__ Sums load_sums(const MView& M, int32_t u, Row R) {
   static_assert(kBkLane == 8, "two 16-byte loads per lane");
-  const uint4* p = reinterpret_cast<const uint4*>(M.bs + (int64_t)u * kNBK) + 2 * lane_id();
-  const uint4 a = p[0], b = p[1];
-  return Sums{{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}};
-}
-
-// Inverse-CDF pick over the combined weights M[u][i] + M[i][u] (block row
-// u: o + i), ascending i, skipping i == excl: the first i whose running sum
-// exceeds t (graph_parallel.hpp:849-850 / :1061-1062 with exact integer
-// weights; a row's weights sum to less than 2^32).  The caller guarantees t <
-// total weight and has loaded the row's bucket sums.  Two levels: the bucket
-// sums locate the key bucket [lo, hi); the bucket's weights then come from
-// one load per key when the row is direct, else they are gathered into the
-// wavefront's LDS scratch `scr` (scr_cap ints) -- a hashed row by scanning its
-// slab, which costs a few loads per lane where looking up each absent key
-// would walk a probe chain, or, when the slab holds kLookupRatio times the
-// bucket's keys or more, by looking each key up (a whole-slab scan of a
-// 16384-slot row took one wavefront ~120 us) -- and searched 512 keys at a
-// time.
-template <bool kD>
-__device__ __forceinline__ int32_t select_combined(const MView& M, int32_t u, uint32_t t,
-                                                   int32_t excl, Sums S, int32_t* scr,
-                                                   int32_t scr_cap, long& bytes) {
   const int lane = lane_id();
-  const int32_t B = M.B;
-  const int sh = M.bshift;
-  const int32_t nbk = ((B - 1) >> sh) + 1;
-  const Row RM = m_row<kD>(M, u);
-  bytes += 12 + 4 * (long)nbk;
-  if (excl >= 0) {
-    const Cnt x = m_value<kD>(M, RM, excl, m_probe<kD>(M, RM, excl));
-    bytes += 12;
-    const int32_t xb = excl >> sh;
+  if (M.B <= kNBK) {
+    Sums S{(M.B + kWave - 1) / kWave, {0, 0, 0, 0, 0, 0, 0, 0}};
 #pragma unroll
     for (int q = 0; q < kBkLane; ++q)
-      if (lane * kBkLane + q == xb) S.w[q] -= (uint32_t)x.o + (uint32_t)x.i;
+      if (q < S.per && lane * S.per + q < M.B) {
+        const Cnt x = M.cnt[R.o + lane * S.per + q];
+        S.w[q] = (uint32_t)x.o + (uint32_t)x.i;
+      }
+    return S;
   }
-  // level 1: bucket jb holding the t-th unit
+  const uint4* p = reinterpret_cast<const uint4*>(M.bs + (int64_t)u * kNBK) + 2 * lane;
+  const uint4 a = p[0], b = p[1];
+  return Sums{kBkLane, {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}};
+}
+
+// The bucket holding unit t; t becomes the unit within it.
+__device__ __forceinline__ int32_t pick_bucket(const Sums& S, uint32_t& t) {
+  const int lane = lane_id();
   uint32_t own = 0;
 #pragma unroll
   for (int q = 0; q < kBkLane; ++q) own += S.w[q];
@@ -683,7 +699,8 @@ __device__ __forceinline__ int32_t select_combined(const MView& M, int32_t u, ui
   const unsigned long long past = __ballot(inc > t);
   const int f = past ? __ffsll(past) - 1 : kWave - 1;
   int j = 0;
-  uint32_t rest = t - (inc - own), before = 0;  // in lane f: the units before t in its buckets
+  const uint32_t rest = t - (inc - own);  // in lane f: the unit within its buckets
+  uint32_t before = 0;
 #pragma unroll
   for (int q = 0; q < kBkLane - 1; ++q) {
     before += S.w[q];
@@ -693,9 +710,98 @@ __device__ __forceinline__ int32_t select_combined(const MView& M, int32_t u, ui
 #pragma unroll
   for (int q = 0; q < kBkLane - 1; ++q)
     if (q < j) before += S.w[q];
-  const int32_t jb = min((int32_t)read_lane32((uint32_t)(lane * kBkLane + j), f), nbk - 1);
   t = read_lane32(rest - before, f);
-  // level 2: keys [lo, hi) of that bucket in ascending order
+  return (int32_t)read_lane32((uint32_t)(lane * S.per + j), f);
+}
+
+// The t-th unit among `width` weights, weight(i) for 0 <= i < width in lane i
+// % 64, 512 of them in flight at a time; width - 1 if there is none.
+template <typename F>
+__device__ __forceinline__ int32_t pick_scan(int32_t width, uint32_t t, F weight) {
+  const int lane = lane_id();
+  for (int32_t base = 0; base < width; base += 8 * kWave) {
+    uint32_t v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int32_t i = base + q * kWave + lane;
+      v[q] = i < width ? weight(i) : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      if (base + q * kWave >= width) break;
+      const uint32_t c = wave_incl_scan32(v[q]);
+      const unsigned long long hit = __ballot(c > t);
+      if (hit) return base + q * kWave + __ffsll(hit) - 1;
+      t -= read_lane32(c, kWave - 1);
+    }
+  }
+  return width - 1;
+}
+
+// Inverse-CDF pick over the combined weights M[u][i] + M[i][u] (block row
+// u: o + i), ascending i, skipping i == excl: the first i whose running sum
+// exceeds t (graph_parallel.hpp:849-850 / :1061-1062 with exact integer
+// weights; a row's weights sum to less than 2^32).  The caller guarantees t <
+// total weight.  Two levels: the weight per key bucket locates the bucket [lo,
+// hi), then the bucket's keys are searched.  `pre`: the row's sums, loaded
+// ahead (a direct row's), or null.
+//   direct row: sums as load_sums; one load per key of the bucket.
+//   hashed, at most kScanRow slots: the slab is read once, eight slots a lane,
+//     and histogrammed over the buckets in the wavefront's LDS scratch `scr`
+//     (scr_cap >= kNBK ints), then the bucket's entries gathered there.
+//   larger hashed: its bucket sums; then the bucket's weights gathered into scr
+//     by a scan of the slab, or, when it holds kLookupRatio times the bucket's
+//     keys or more, by looking each key up (a whole-slab scan of a 16384-slot
+//     row took one wavefront ~120 us).
+template <bool kD>
+__device__ __forceinline__ int32_t select_combined(const MView& M, int32_t u, uint32_t t,
+                                                   int32_t excl, const Sums* pre, int32_t* scr,
+                                                   int32_t scr_cap, long& bytes) {
+  const int lane = lane_id();
+  const int32_t B = M.B;
+  const int sh = M.bshift;
+  const int32_t nbk = ((B - 1) >> sh) + 1;
+  const Row RM = m_row<kD>(M, u);
+  const bool direct = kD || RM.c == B;
+  const bool small = !direct && !row_sums(M, RM.c);
+  Sums S;
+  if (small) {
+    constexpr int kQ = kScanRow / kWave;
+    for (int32_t i = lane; i < kNBK; i += kWave) scr[i] = 0;
+    int32_t key[kQ];
+    uint32_t wt[kQ];
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      const int32_t j = q * kWave + lane;
+      key[q] = -1;
+      wt[q] = 0;
+      if (j < RM.c) {
+        key[q] = M.key[RM.o + j];
+        const Cnt x = M.cnt[RM.o + j];
+        wt[q] = (uint32_t)x.o + (uint32_t)x.i;
+      }
+    }
+    wave_fence();
+#pragma unroll
+    for (int q = 0; q < kQ; ++q)
+      if (key[q] >= 0 && key[q] != excl && wt[q]) atomicAdd(&scr[key[q] >> sh], (int32_t)wt[q]);
+    wave_fence();
+    S.per = kBkLane;
+#pragma unroll
+    for (int q = 0; q < kBkLane; ++q) S.w[q] = (uint32_t)scr[lane * kBkLane + q];
+    bytes += 12 + 12 * (long)RM.c;
+  } else {
+    S = pre ? *pre : load_sums(M, u, RM);
+    bytes += 12 + 4 * (long)nbk;
+    if (excl >= 0) {
+      const Cnt x = m_value<kD>(M, RM, excl, m_probe<kD>(M, RM, excl));
+      bytes += 12;
+#pragma unroll
+      for (int q = 0; q < kBkLane; ++q)
+        if (lane * S.per + q == excl >> sh && q < S.per) S.w[q] -= (uint32_t)x.o + (uint32_t)x.i;
+    }
+  }
+  const int32_t jb = min(pick_bucket(S, t), nbk - 1);
   const int32_t lo = jb << sh;
   const int32_t hi = min(B, lo + (1 << sh));
   const int32_t width = hi - lo;
@@ -703,8 +809,15 @@ __device__ __forceinline__ int32_t select_combined(const MView& M, int32_t u, ui
   // that key's weight, so the bucket is the pick (the scans below would
   // return lo too, also for the excluded key's emptied bucket)
   if (width == 1) return lo;
-  const bool direct = kD || RM.c == B;
-  if (!direct && width > scr_cap) {  // wider than the scratch: bisection inside the bucket
+  if (direct) {
+    bytes += 8 * (long)width;
+    return lo + pick_scan(width, t, [&](int32_t i) -> uint32_t {
+             if (lo + i == excl) return 0;
+             const Cnt x = M.cnt[RM.o + lo + i];
+             return (uint32_t)x.o + (uint32_t)x.i;
+           });
+  }
+  if (width > scr_cap) {  // wider than the scratch: bisection inside the bucket
     int32_t a = lo, b = hi - 1;
     while (a < b) {
       const int32_t mid = a + (b - a) / 2;
@@ -716,43 +829,18 @@ __device__ __forceinline__ int32_t select_combined(const MView& M, int32_t u, ui
     }
     return a;
   }
-  if (!direct) {
-    if (RM.c >= kLookupRatio * width) {
-      lookup_bucket(M, RM, lo, hi, scr, bytes);
-    } else {
-      for (int32_t i = lane; i < width; i += kWave) scr[i] = 0;
-      wave_fence();
-      gather_row(M, RM, lo, hi, scr, bytes);
-    }
-    wave_fence();
+  wave_fence();  // the reads of the histogram are done
+  if (!small && RM.c >= kLookupRatio * width) {
+    lookup_bucket(M, RM, lo, hi, scr, bytes);
   } else {
-    bytes += 8 * (long)width;
+    for (int32_t i = lane; i < width; i += kWave) scr[i] = 0;
+    wave_fence();
+    gather_row(M, RM, lo, hi, scr, bytes);
   }
-  for (int32_t base = 0; base < width; base += 8 * kWave) {
-    uint32_t v[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int32_t i = base + q * kWave + lane;
-      v[q] = 0;
-      if (i < width && lo + i != excl) {
-        if (direct) {
-          const Cnt x = M.cnt[RM.o + lo + i];
-          v[q] = (uint32_t)x.o + (uint32_t)x.i;
-        } else {
-          v[q] = (uint32_t)scr[i];
-        }
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      if (base + q * kWave >= width) break;
-      const uint32_t c = wave_incl_scan32(v[q]);
-      const unsigned long long hit = __ballot(c > t);
-      if (hit) return lo + base + q * kWave + __ffsll(hit) - 1;
-      t -= read_lane32(c, kWave - 1);
-    }
-  }
-  return hi - 1;
+  wave_fence();
+  return lo + pick_scan(width, t, [&](int32_t i) -> uint32_t {
+           return lo + i == excl ? 0u : (uint32_t)scr[i];
+         });
 }
 
 // t-th unit of the node's neighbour list (out-neighbours then in-neighbours,
@@ -885,10 +973,10 @@ __global__ void k_insert_edges(int64_t E, const int32_t* __restrict__ src,
     const bool ia = !kSkipLds || !lds_row(M.cap[a], M.B);
     const bool ib = !kSkipLds || !lds_row(M.cap[b], M.B);
     if (a == b) {
-      if (ia) m_add<false>(M, a, a, ww, ww, flags);
+      if (ia) m_add(M, a, a, ww, ww, flags);
     } else {
-      if (ia) m_add<false>(M, a, b, ww, 0, flags);
-      if (ib) m_add<false>(M, b, a, 0, ww, flags);
+      if (ia) m_add(M, a, b, ww, 0, flags);
+      if (ib) m_add(M, b, a, 0, ww, flags);
     }
   }
 }
@@ -935,7 +1023,6 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_build_rows(
   }
   const uint32_t mask = (uint32_t)c - 1;
   const int32_t n0 = bl_off[a], n1 = a + 1 < M.B ? bl_off[a + 1] : g.N;
-  long nk = 0;  // keys this lane placed in the LDS slab
   bool full = false;
   for (int32_t base = n0; base < n1; base += kWave) {  // 64 nodes at a time
     const int32_t j = base + lane;
@@ -984,10 +1071,7 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_build_rows(
         int32_t k = __hip_atomic_load(&tk[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
         if (k < 0) {
           k = atomicCAS(&tk[h], -1, b);
-          if (k == -1) {
-            k = b;
-            ++nk;
-          }
+          if (k == -1) k = b;
         }
         if (k == b) {
           atomicAdd(out ? &to[h] : &ti[h], wt);
@@ -1003,8 +1087,6 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_build_rows(
     M.key[o + j] = tk[j];
     M.cnt[o + j] = Cnt{to[j], ti[j]};
   }
-  nk = wave_sum(nk);
-  if (lane == 0) M.nkeys[a] = (int32_t)nk;
   if (__ballot(full)) {
     if (lane == 0) atomicOr(flags, kFlagFull);
   }
@@ -1061,10 +1143,10 @@ __global__ void k_insert_pairs(int64_t E, const uint32_t* __restrict__ key,
     const int32_t a = (int32_t)(key[e] / (uint32_t)M.B), b = (int32_t)(key[e] % (uint32_t)M.B);
     const int32_t w = val[e];
     if (a == b) {
-      m_add<false>(M, a, a, w, w, flags);
+      m_add(M, a, a, w, w, flags);
     } else {
-      m_add<false>(M, a, b, w, 0, flags);
-      m_add<false>(M, b, a, 0, w, flags);
+      m_add(M, a, b, w, 0, flags);
+      m_add(M, b, a, 0, w, flags);
     }
   }
 }
@@ -1075,26 +1157,57 @@ __global__ void k_count_nonsingle(int32_t B, const int32_t* __restrict__ bsize, 
     if (bsize[i] != 1) atomicAdd(out, 1);
 }
 
-// Bucket sums (o + i) of every block row (one wavefront per row).
+// Bucket sums (o + i) of the block rows that keep them: kSumRows rows to a
+// workgroup, which handles those of them one by one (a block that absorbed
+// thousands of nodes has a slab of 16384 slots or more: 4 wavefronts with 8
+// slots a thread in flight, where one with one slot a lane took 0.8 ms).  Sets
+// the hashed ones' marks too (room_mark).
+constexpr int kSumRows = 64;
 __global__ __launch_bounds__(256) void k_bucket_sums(MView m) {
-  __shared__ int32_t s_b[4][kNBK];
-  const int w = threadIdx.x / kWave, lane = lane_id();
-  const int64_t a = (int64_t)blockIdx.x * 4 + w;
-  if (a >= m.B) return;
-  int32_t* bk = s_b[w];
-  for (int i = lane; i < kNBK; i += kWave) bk[i] = 0;
-  wave_fence();
-  const int64_t o = m.off[a];
-  const int32_t c = m.cap[a];
-  const bool direct = c == m.B;
-  for (int32_t j = lane; j < c; j += kWave) {
-    const Cnt q = m.cnt[o + j];
-    const int32_t k = direct ? j : m.key[o + j];
-    const int32_t v = q.o + q.i;
-    if (k >= 0 && v != 0) atomicAdd(&bk[k >> m.bshift], v);
+  __shared__ int32_t s_b[kNBK];
+  __shared__ int32_t s_keys;
+  const int lane = lane_id();
+  const int64_t a0 = (int64_t)blockIdx.x * kSumRows;
+  const int32_t cl = a0 + lane < m.B ? m.cap[a0 + lane] : 0;
+  unsigned long long todo = __ballot(cl > 0 && row_sums(m, cl));  // the same in every wavefront
+  while (todo) {
+    const int l = __ffsll(todo) - 1;
+    todo &= todo - 1ull;
+    const int64_t a = a0 + l;
+    const int32_t c = __shfl(cl, l);
+    for (int i = threadIdx.x; i < kNBK; i += blockDim.x) s_b[i] = 0;
+    if (threadIdx.x == 0) s_keys = 0;
+    __syncthreads();
+    int32_t keys = 0;
+    const int64_t o = m.off[a];
+    const bool direct = c == m.B;
+    constexpr int kQ = 8;
+    for (int32_t j0 = threadIdx.x; j0 < c; j0 += kQ * blockDim.x) {
+      int32_t k[kQ];
+      Cnt x[kQ];
+#pragma unroll
+      for (int q = 0; q < kQ; ++q) {
+        const int32_t j = j0 + q * (int32_t)blockDim.x;
+        k[q] = -1;
+        x[q] = Cnt{0, 0};
+        if (j < c) {
+          k[q] = direct ? j : m.key[o + j];
+          x[q] = m.cnt[o + j];
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < kQ; ++q) {
+        const int32_t v = x[q].o + x[q].i;
+        keys += k[q] >= 0;
+        if (k[q] >= 0 && v != 0) atomicAdd(&s_b[k[q] >> m.bshift], v);
+      }
+    }
+    atomicAdd(&s_keys, keys);
+    __syncthreads();
+    for (int i = threadIdx.x; i < kNBK; i += blockDim.x) m.bs[a * kNBK + i] = s_b[i];
+    if (threadIdx.x == 0 && !direct) m.gmark[a] = room_mark(s_keys, c, m.slack);
+    __syncthreads();
   }
-  wave_fence();
-  for (int i = lane; i < kNBK; i += kWave) m.bs[a * kNBK + i] = bk[i];
 }
 
 // Workgroup stamps of profiled batch launches (100 MHz wall clock; 0 = the
@@ -1104,7 +1217,7 @@ __global__ __launch_bounds__(256) void k_bucket_sums(MView m) {
 // kernel's own tail.  Per batch slot: k_nodal's starts and ends (G each),
 // k_apply's (G + 1 each), k_grow's (kGrowBlocks each).
 // The per-block counters and flags a rebuild starts from, zeroed in one
-// launch (degrees, edge counts, sizes, key counts, growth marks, parked
+// launch (degrees, edge counts, sizes, growth marks, parked
 // counts: B entries each; build_flags[0..2]).
 constexpr int kClearArrays = 8;
 struct ClearArgs {
@@ -1161,10 +1274,13 @@ __global__ __launch_bounds__(256) void k_stamp_reduce(const unsigned long long* 
 // Growth state after a rebuild: nothing parked, the pool used up to
 // the new slabs' end (the event counters are kept).
 __global__ void k_reset_grow(GrowState* g, unsigned long long used) {
-  g->n = 0;
-  g->nospace = 0;
-  g->ovf_n = 0;
-  g->used = used;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < kGrowBlocks) g->chunk[i].pos = g->chunk[i].end = 0;
+  if (i == 0) {
+    g->nospace = 0;
+    g->ovf_n = 0;
+    g->used = used;
+  }
 }
 
 __global__ void k_relabel(int32_t N, int32_t* labels, const int32_t* __restrict__ map) {
@@ -1468,7 +1584,7 @@ __device__ void merge_one(const MergeArgs& a, int32_t r, int32_t idx, int32_t* s
   } else {
     long bytes = 0;
     const int64_t t0 = (int64_t)usap::idx_of(x[0], k);
-    const int32_t u = L.n >= 0 ? rowlds_pick(L, t0) : select_combined<false>(a.M, r, (uint32_t)t0, -1, load_sums(a.M, r), scr, kScr, bytes);
+    const int32_t u = L.n >= 0 ? rowlds_pick(L, t0) : select_combined<false>(a.M, r, (uint32_t)t0, -1, nullptr, scr, kScr, bytes);
     const int64_t da = (int64_t)a.d_out[u] + a.d_in[u];
     if (usap::uniform_branch(x[1], da, B)) {
       s = usap::uniform_not_r(x[2], r, B);
@@ -1476,7 +1592,7 @@ __device__ void merge_one(const MergeArgs& a, int32_t r, int32_t idx, int32_t* s
       const Cnt ur = m_get(a.M, u, r);  // M[u][r], M[r][u]
       const int64_t W2 = da - ur.o - ur.i;
       s = W2 == 0 ? usap::uniform_not_r(x[2], r, B)
-                  : select_combined<false>(a.M, u, idx32(x[3], (uint32_t)W2), r, load_sums(a.M, u), scr, kScr, bytes);
+                  : select_combined<false>(a.M, u, idx32(x[3], (uint32_t)W2), r, nullptr, scr, kScr, bytes);
     }
   }
   s_out = s;
@@ -1618,7 +1734,6 @@ __global__ __launch_bounds__(kWave* kMergeWaves, 5) void k_merge(MergeArgs a) {
 // Nodal proposal, graph_parallel.hpp:990-1222
 // ---------------------------------------------------------------------------
 
-constexpr int kEdgeRegs = 4;     // list entries per lane per pass (256 per wavefront)
 
 // Workgroups are dispatched to the GPU's 8 XCDs (each with its own L2) in
 // turn: workgroup b runs on XCD b % 8.  Block b of a batch kernel takes item
@@ -1999,7 +2114,7 @@ __device__ __forceinline__ void nodal_regs(const NodalArgs& a, int32_t n, int32_
   const int32_t u = k > 0 ? __builtin_amdgcn_readlane(lv, pl) : r;
   const uint32_t da = (uint32_t)a.d_out[u] + (uint32_t)a.d_in[u];
   Sums bk;
-  if (kD) bk = load_sums(M, u);
+  if (kD) bk = load_sums(M, u, m_row<kD>(M, u));
   Probe p0[U];
   int32_t ks[U];  // row s's key at the block's home slot
   const bool pdir = kD || pM.c == B;
@@ -2055,10 +2170,8 @@ __device__ __forceinline__ void nodal_regs(const NodalArgs& a, int32_t n, int32_
   int32_t s = s_pre;
   if (k > 0) {
     bytes += 16;  // drawn neighbour id, its label, d_out[u], d_in[u]
-    if (!usap::uniform_branch(x[1], da, B)) {
-      if (!kD) bk = load_sums(M, u);
-      s = select_combined<kD>(M, u, idx32(x[3], da), -1, bk, lds, kLdsWave, bytes);
-    }
+    if (!usap::uniform_branch(x[1], da, B))
+      s = select_combined<kD>(M, u, idx32(x[3], da), -1, kD ? &bk : nullptr, lds, kLdsWave, bytes);
   }
   out.s = s;
   out.u = k > 0 ? u : -1;
@@ -2319,7 +2432,7 @@ __device__ __forceinline__ void nodal_hub(const NodalArgs& a, int32_t n, int32_t
       const uint32_t da = (uint32_t)a.d_out[u] + (uint32_t)a.d_in[u];
       bytes += 16;
       if (!usap::uniform_branch(x[1], da, B))
-        s = select_combined<kD>(M, u, idx32(x[3], da), -1, load_sums(M, u), lds, kLdsWave, bytes);
+        s = select_combined<kD>(M, u, idx32(x[3], da), -1, nullptr, lds, kLdsWave, bytes);
     }
     if (lane == 0) {
       hub.s = s;
@@ -2586,7 +2699,7 @@ __device__ __forceinline__ void build_single_one(const GraphView& g, const int32
   wave_fence();
   long x0 = 0, x1 = 0, x2 = 0, x3 = 0;
   const int32_t nent = tab_compact(T, -2, -2, x0, x1, x2, x3);
-  for (int32_t j = lane; j < nent; j += kWave) m_add<false>(M, a, T.tk[j], T.two[j], T.twi[j], flags);
+  for (int32_t j = lane; j < nent; j += kWave) m_add(M, a, T.tk[j], T.two[j], T.twi[j], flags);
 }
 
 __global__ __launch_bounds__(kWave* kNodalWaves) void k_build_single(GraphView g,
@@ -2618,8 +2731,6 @@ struct ApplyArgs {
   int32_t* d_in;
   int32_t* bsize;
   int32_t beg, end;
-  const int64_t* big_off;
-  int32_t* big_tab;
   const Prop* prop;
   const BlockPart* part;  // k_nodal's per-workgroup shares of the batch
   uint32_t nparts;
@@ -2683,114 +2794,202 @@ __device__ void sweep_tail(Sweep* sw, u128 sum, int32_t ninf, int32_t moves,
   if (sw->check && -sw->mean < sw->thr * sw->S) atomicExch(&sw->stop, 1);
 }
 
-// Moves accepted node n from block r to s: its edges' counts leave row and
-// column r for row and column s.  Edges to neighbours that stay put are first
-// summed per neighbour block b in the node's table (wo = edges n -> b, wi =
-// edges b -> n), so each changed pair of counts gets one 64-bit atomic per
-// node (apply_entry); edges to neighbours that move in the same batch are
-// applied here, one by one.  Also moves the node's degrees and writes its
-// label.  Old labels of nodes inside the batch come from prop, so writing
-// labels cannot race with their reads.  Returns the table, compacted to its
-// nent entries (nent = 0 when none is left).
-template <bool kBig>
-__device__ __forceinline__ Table apply_table(const ApplyArgs& a, int32_t n, int32_t r, int32_t s,
-                                             int64_t o0, int64_t kco, int64_t i0, int64_t kci,
-                                             int32_t* tab, int32_t& nent) {
-  const int lane = lane_id();
-  const GraphView& g = a.g;
+// One record of an accepted move r -> s: n's edges to (wo) and from (wi) the
+// neighbours of block x, or, for a neighbour that moves in the same batch, its
+// edge n -> neighbour (wo) whose other end goes from block x to y (else y = x).
+// Block row r at key x loses (wo, wi), row s at y gains them, row x at r loses
+// (wi, wo) and row y at s gains them: four 64-bit atomics on (o, i).  M all
+// direct, nothing is read for them; else the four rows' headers, then the four
+// key windows, are read together before the adds.
+template <bool kD>
+__device__ __forceinline__ void apply_record(const ApplyArgs& a, int32_t r, int32_t s, int32_t x,
+                                             int32_t y, int32_t wo, int32_t wi) {
+  const MView& M = a.M;
   int32_t* flags = &a.status->flags;
-  const int64_t kc = kco + kci;
-  const Table T = tab_open<kBig>(tab, a.big_off, a.big_tab, n, kc);
-  const uint32_t mask = (uint32_t)T.cap - 1;
-  long wo_sum = 0, wi_sum = 0;
-  for (int64_t base = 0; base < kc; base += kEdgeRegs * kWave) {
-    int32_t v[kEdgeRegs], ww[kEdgeRegs], bo[kEdgeRegs], bn[kEdgeRegs];
-#pragma unroll
-    for (int q = 0; q < kEdgeRegs; ++q)
-      list_entry(g, o0, kco, i0, kc, base + q * kWave + lane, v[q], ww[q]);
-#pragma unroll
-    for (int q = 0; q < kEdgeRegs; ++q) {
-      bo[q] = bn[q] = -1;
-      if (v[q] < 0) continue;
-      if (v[q] >= a.beg && v[q] < a.end) {
-        const int32_t x = v[q] - a.beg;
-        const Prop p = a.prop[x];
-        bo[q] = p.r;
-        bn[q] = p.acc ? p.s : -2;
-      } else {
-        bo[q] = a.labels[v[q]];
-        bn[q] = -2;
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < kEdgeRegs; ++q) {
-      if (v[q] < 0) continue;
-      const int32_t w = ww[q];
-      if (base + q * kWave + lane < kco) {
-        wo_sum += w;
-        if (bn[q] == -2) {
-          tab_add(T.tk, T.two, mask, bo[q], w);
-        } else {  // the neighbour moved in this batch too: bo -> bn
-          // four independent updates: their rows, then their first keys,
-          // are read together before the adds
-          const int32_t ra[4] = {r, bo[q], s, bn[q]}, kb[4] = {bo[q], r, bn[q], s};
-          const int32_t dO[4] = {-w, 0, w, 0}, dI[4] = {0, -w, 0, w};
-          Row R4[4];
-          int64_t sl[4];
-          int32_t k4[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) R4[i] = m_row(a.M, ra[i]);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) k4[i] = m_first_key(a.M, R4[i], kb[i], sl[i]);
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            m_add_at<true>(a.M, ra[i], R4[i], kb[i], dO[i], dI[i], sl[i], k4[i], flags);
-        }
-      } else {
-        wi_sum += w;
-        if (bn[q] == -2) tab_add(T.tk, T.twi, mask, bo[q], w);
-        // else: moved as the neighbour's out-edge
-      }
-    }
-  }
-  wave_fence();
-  long x0 = 0, x1 = 0, x2 = 0, x3 = 0;
-  nent = tab_compact(T, -2, -2, x0, x1, x2, x3);
-  wo_sum = wave_sum(wo_sum);
-  wi_sum = wave_sum(wi_sum);
-  if (lane == 0) {
-    if (wo_sum) {
-      atomicSub(&a.d_out[r], (int32_t)wo_sum);
-      atomicAdd(&a.d_out[s], (int32_t)wo_sum);
-    }
-    if (wi_sum) {
-      atomicSub(&a.d_in[r], (int32_t)wi_sum);
-      atomicAdd(&a.d_in[s], (int32_t)wi_sum);
-    }
-    atomicSub(&a.bsize[r], 1);
-    atomicAdd(&a.bsize[s], 1);
-    a.labels[n] = s;
-  }
-  return T;
-}
-
-// One entry (b, wo, wi) of a moving node's table, node moving r -> s: block
-// row r at key b (-wo, -wi), row s at b (+wo, +wi), row b at r (-wi, -wo)
-// and at s (+wi, +wo); the four first keys are read together before the adds.
-__device__ __forceinline__ void apply_entry(const ApplyArgs& a, int32_t r, Row rM, int32_t s,
-                                            Row sM, int32_t b, int32_t wo, int32_t wi) {
-  int32_t* flags = &a.status->flags;
-  const Row bM = m_row(a.M, b);
+  const Row rM = m_row<kD>(M, r), sM = m_row<kD>(M, s);
+  const Row xM = m_row<kD>(M, x), yM = m_row<kD>(M, y);
   int64_t sl[4];
   int32_t k[4];
-  k[0] = m_first_key(a.M, rM, b, sl[0]);  // (M[r][b], M[b][r]) -= (wo, wi)
-  k[1] = m_first_key(a.M, sM, b, sl[1]);  // (M[s][b], M[b][s]) += (wo, wi)
-  k[2] = m_first_key(a.M, bM, r, sl[2]);  // (M[b][r], M[r][b]) -= (wi, wo)
-  k[3] = m_first_key(a.M, bM, s, sl[3]);  // (M[b][s], M[s][b]) += (wi, wo)
-  m_add_at<true>(a.M, r, rM, b, -wo, -wi, sl[0], k[0], flags);
-  m_add_at<true>(a.M, s, sM, b, wo, wi, sl[1], k[1], flags);
-  m_add_at<true>(a.M, b, bM, r, -wi, -wo, sl[2], k[2], flags);
-  m_add_at<true>(a.M, b, bM, s, wi, wo, sl[3], k[3], flags);
+  k[0] = m_first_key<kD>(M, rM, x, sl[0]);
+  k[1] = m_first_key<kD>(M, sM, y, sl[1]);
+  k[2] = m_first_key<kD>(M, xM, r, sl[2]);
+  k[3] = m_first_key<kD>(M, yM, s, sl[3]);
+  m_add_at<true, kD>(M, r, rM, x, -wo, -wi, sl[0], k[0], flags);
+  m_add_at<true, kD>(M, s, sM, y, wo, wi, sl[1], k[1], flags);
+  m_add_at<true, kD>(M, x, xM, r, -wi, -wo, sl[2], k[2], flags);
+  m_add_at<true, kD>(M, y, yM, s, wi, wo, sl[3], k[3], flags);
+}
+
+// Node n's label and the degrees and sizes of r and s, by lanes 0..5 of one
+// wavefront.
+__device__ __forceinline__ void move_node(const ApplyArgs& a, int32_t n, int32_t r, int32_t s,
+                                          int32_t wo, int32_t wi) {
+  const int lane = lane_id();
+  if (lane < 6) {
+    int32_t* p = lane < 2 ? a.d_out : lane < 4 ? a.d_in : a.bsize;
+    const int32_t w = lane < 2 ? wo : lane < 4 ? wi : 1;
+    if (w) atomicAdd(&p[lane & 1 ? s : r], lane & 1 ? w : -w);
+  }
+  if (lane == 0) a.labels[n] = s;
+}
+
+// The block v's edges leave (x) and, if v moved in this batch, go to (y; else
+// y = x).  Nodes of the batch are read from their proposals: their labels are
+// being written.
+__device__ __forceinline__ void ends_of(const ApplyArgs& a, int32_t v, int32_t& x, int32_t& y,
+                                        bool& moved) {
+  if (v >= a.beg && v < a.end) {
+    const Prop p = a.prop[v - a.beg];
+    x = p.r;
+    moved = p.acc != 0;
+    y = moved ? p.s : p.r;
+  } else {
+    x = y = a.labels[v];
+    moved = false;
+  }
+}
+
+constexpr int kMaxRec = kRegUnits * kWave;  // records of a node one wavefront handles
+constexpr int kApplyLds = 6 * kMaxRec;      // LDS ints per wavefront
+
+// The records of accepted node n (at most 64 U list entries), by one
+// wavefront: its entries to neighbours that stay put, summed per block (so each
+// changed pair of counts gets one atomic per node; in registers, an LDS hash
+// deciding which entry owns a block), and one per out-edge to a neighbour that
+// moves too (the edge's other end leaves it to this one).  They are left in
+// the wavefront's LDS as x, y, wo, wi, kMaxRec each; returns their number.
+template <bool kW, int U>
+__device__ __forceinline__ int32_t apply_records(const ApplyArgs& a, int32_t n, int32_t r,
+                                                 int32_t s, int64_t o0, int64_t i0, int32_t kco,
+                                                 int32_t kc, int32_t* lds) {
+  const int lane = lane_id();
+  const GraphView& g = a.g;
+  int32_t v[U], w[U];
+#pragma unroll
+  for (int q = 0; q < U; ++q) {
+    const int32_t j = q * kWave + lane;
+    v[q] = -1;
+    w[q] = kW ? 0 : 1;
+    if (j < kco) {
+      v[q] = g.out_idx[o0 + j];
+      if (kW) w[q] = g.out_w[o0 + j];
+    } else if (j < kc) {
+      v[q] = g.in_idx[i0 + (j - kco)];
+      if (kW) w[q] = g.in_w[i0 + (j - kco)];
+    }
+  }
+  constexpr int kCap = 128 * U;  // at least twice the blocks
+  static_assert(3 * kCap <= kApplyLds && 4 * kMaxRec <= kApplyLds, "LDS per wavefront");
+  int32_t *tk = lds, *two = lds + kCap, *twi = lds + 2 * kCap;
+  for (int j = 4 * lane; j < 3 * kCap; j += 4 * kWave) {
+    const int32_t z = j < kCap ? -1 : 0;
+    *reinterpret_cast<int4*>(lds + j) = make_int4(z, z, z, z);
+  }
+  lds_order();
+  int32_t wo_sum = kco, wi_sum = kc - kco;
+  if (kW) {
+    uint32_t so = 0, si = 0;
+#pragma unroll
+    for (int q = 0; q < U; ++q) (q * kWave + lane < kco ? so : si) += (uint32_t)w[q];
+    wo_sum = (int32_t)wave_sum32(so);
+    wi_sum = (int32_t)wave_sum32(si);
+  }
+  int32_t x[U], y[U];
+  bool moved[U];
+#pragma unroll
+  for (int q = 0; q < U; ++q) {
+    x[q] = y[q] = -1;
+    moved[q] = false;
+    if (v[q] >= 0) ends_of(a, v[q], x[q], y[q], moved[q]);
+  }
+  uint32_t hs[U];
+  bool own[U];
+#pragma unroll
+  for (int q = 0; q < U; ++q) {
+    const bool in = q * kWave + lane >= kco;
+    own[q] = false;
+    hs[q] = 0;
+    if (v[q] >= 0 && !moved[q]) {
+      uint32_t h = hash32(x[q]) & (kCap - 1);
+      for (;;) {
+        const int32_t old = atomicCAS(&tk[h], -1, x[q]);
+        own[q] = old == -1;
+        if (own[q] || old == x[q]) break;
+        h = (h + 1) & (kCap - 1);
+      }
+      hs[q] = h;
+      atomicAdd(in ? &twi[h] : &two[h], w[q]);
+    }
+  }
+  lds_order();
+  int32_t wo[U], wi[U];
+#pragma unroll
+  for (int q = 0; q < U; ++q) {
+    wo[q] = own[q] ? two[hs[q]] : w[q];
+    wi[q] = own[q] ? twi[hs[q]] : 0;
+  }
+  lds_order();  // the records take the table's place
+  int32_t nrec = 0;
+#pragma unroll
+  for (int q = 0; q < U; ++q) {
+    const bool emit = own[q] || (moved[q] && q * kWave + lane < kco);
+    const unsigned long long m = __ballot(emit);
+    if (emit) {
+      const int32_t j = nrec + __popcll(m & ((1ull << lane) - 1ull));
+      lds[j] = x[q];
+      lds[kMaxRec + j] = y[q];
+      lds[2 * kMaxRec + j] = wo[q];
+      lds[3 * kMaxRec + j] = wi[q];
+    }
+    nrec += __popcll(m);
+  }
+  move_node(a, n, r, s, wo_sum, wi_sum);
+  return nrec;
+}
+
+// An accepted node with more list entries than a wavefront's registers take, by
+// the whole workgroup: edges to neighbours that stay put are summed per block
+// in LDS where the blocks are few, else each list entry is a record.
+constexpr int kHubBlocks = kNodalWaves * kApplyLds / 2;  // blocks whose two sums fit in LDS
+
+template <bool kD, bool kW>
+__device__ __forceinline__ void apply_hub(const ApplyArgs& a, int32_t n, int32_t r, int32_t s,
+                                          int32_t* lds, int32_t* sums) {
+  const GraphView& g = a.g;
+  const int32_t B = a.M.B;
+  const int64_t o0 = g.out_ptr[n], i0 = g.in_ptr[n];
+  const int64_t kco = g.out_ptr[n + 1] - o0, kc = kco + (g.in_ptr[n + 1] - i0);
+  const bool few = B <= kHubBlocks;
+  if (few)
+    for (int32_t b = threadIdx.x; b < 2 * B; b += blockDim.x) lds[b] = 0;
+  if (threadIdx.x == 0) sums[0] = sums[1] = 0;
+  __syncthreads();
+  int32_t so = 0, si = 0;
+  for (int64_t j = threadIdx.x; j < kc; j += blockDim.x) {
+    int32_t v, w, x, y;
+    bool moved;
+    list_entry(g, o0, kco, i0, kc, j, v, w);
+    const bool in = j >= kco;
+    (in ? si : so) += w;
+    ends_of(a, v, x, y, moved);
+    if (moved) {
+      if (!in) apply_record<kD>(a, r, s, x, y, w, 0);
+    } else if (few) {
+      atomicAdd(&lds[2 * x + in], w);
+    } else {
+      apply_record<kD>(a, r, s, x, x, in ? 0 : w, in ? w : 0);
+    }
+  }
+  atomicAdd(&sums[0], so);
+  atomicAdd(&sums[1], si);
+  __syncthreads();
+  if (few)
+    for (int32_t b = threadIdx.x; b < B; b += blockDim.x) {
+      const int32_t wo = lds[2 * b], wi = lds[2 * b + 1];
+      if (wo != 0 || wi != 0) apply_record<kD>(a, r, s, b, b, wo, wi);
+    }
+  if (threadIdx.x < kWave) move_node(a, n, r, s, sums[0], sums[1]);
+  __syncthreads();
 }
 
 // The batch's sums over all workgroups' shares (nparts of them), by one
@@ -2841,17 +3040,18 @@ __device__ __forceinline__ void batch_tail(const BlockPart* part, uint32_t npart
   __syncthreads();
 }
 
-// Block 0 runs the batch's update step from k_nodal's shares while blocks
-// 1.. apply the moves of items (block - 1) * kNodalWaves + wave.
 // Block 0 runs the batch's update step; every other block applies the moves
-// of its four batch nodes: each moving node's wavefront builds its table,
-// then the entries of all the block's tables are spread over all its
-// threads (a block holds 0-4 moving nodes, most often 0 or 1, so a node's
-// entries no longer wait for its own 64 lanes only).
-__global__ __launch_bounds__(kWave* kNodalWaves) void k_apply(ApplyArgs a) {
-  __shared__ int32_t s_tab[kNodalWaves][3 * kTab];
-  __shared__ int32_t* s_tk[kNodalWaves];  // each moving node's compacted table (LDS or global)
-  __shared__ int32_t s_stride[kNodalWaves];
+// of its four batch nodes: each moving node's wavefront writes its records,
+// then all the block's records are spread over all its threads (a block holds
+// 0-4 moving nodes, most often 0 or 1, so a node's records do not wait for its
+// own 64 lanes only).  kHub: the graph has nodes larger than kMaxRec entries.
+// Its time is one mover's chain of loads, and with 2000 movers of 45 edges a
+// batch (B = 100000, after a merge) its atomics: four on counts per record,
+// and a claim per new key (key counts and a bucket sum per update doubled
+// them).  62.0 -> 42.6 us a launch there; N = 50000 dense 11.2 -> 7.4.
+template <bool kD, bool kW, bool kHub>
+__global__ __launch_bounds__(kWave* kNodalWaves, 4) void k_apply(ApplyArgs a) {
+  __shared__ __align__(16) int32_t s_lds[kNodalWaves][kApplyLds];
   __shared__ int32_t s_n[kNodalWaves], s_r[kNodalWaves], s_s[kNodalWaves];
   if (blockIdx.x == 0) {
     if (a.tstamp && threadIdx.x == 0) a.tstamp[0] = wall_clock64();
@@ -2863,51 +3063,57 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_apply(ApplyArgs a) {
     return;
   }
   const int w = threadIdx.x / kWave;
-  const int64_t item = (int64_t)xcd_block(blockIdx.x - 1, gridDim.x - 1) * kNodalWaves + w;
-  const int64_t n64 = (int64_t)a.beg + item;
+  const int64_t item0 = (int64_t)xcd_block(blockIdx.x - 1, gridDim.x - 1) * kNodalWaves;
+  const int64_t n64 = (int64_t)a.beg + item0 + w;
   const bool in = n64 < a.end;
   const int32_t n = in ? (int32_t)n64 : a.beg;
   // whether the batch runs, the proposal and the node's list bounds in one
   // round of loads
   const int32_t stop = a.sweep->stop_n;  // the same for every block of this launch
-  const Prop p = in ? a.prop[item] : Prop{0, 0, 0, 0};
-  const int32_t acc = p.acc, pr = p.r, ps = p.s;
+  const Prop p = in ? a.prop[item0 + w] : Prop{0, 0, 0, 0};
   const int64_t o0 = a.g.out_ptr[n], i0 = a.g.in_ptr[n];
-  const int64_t kco = a.g.out_ptr[n + 1] - o0, kci = a.g.in_ptr[n + 1] - i0;
+  const int64_t kco = a.g.out_ptr[n + 1] - o0, kc = kco + (a.g.in_ptr[n + 1] - i0);
   if (stop) return;
   if (a.tstamp && threadIdx.x == 0) a.tstamp[blockIdx.x] = wall_clock64();
-  int32_t nent = 0;
-  Table T{s_tab[w], s_tab[w] + kTab, s_tab[w] + 2 * kTab, kTab};
-  if (in && acc) {
-    if (kco + kci > kTabMaxDeg)
-      T = apply_table<true>(a, n, pr, ps, o0, kco, i0, kci, s_tab[w], nent);
+  int32_t nrec = 0;
+  if (in && p.acc) {
+    const int32_t ko = (int32_t)kco, kk = (int32_t)kc;
+    if (kHub && kc > kMaxRec)
+      nrec = -1;
+    else if (kk <= kWave)
+      nrec = apply_records<kW, 1>(a, n, p.r, p.s, o0, i0, ko, kk, s_lds[w]);
+    else if (kk <= 2 * kWave)
+      nrec = apply_records<kW, 2>(a, n, p.r, p.s, o0, i0, ko, kk, s_lds[w]);
     else
-      T = apply_table<false>(a, n, pr, ps, o0, kco, i0, kci, s_tab[w], nent);
+      nrec = apply_records<kW, kRegUnits>(a, n, p.r, p.s, o0, i0, ko, kk, s_lds[w]);
   }
   if (lane_id() == 0) {
-    s_n[w] = nent;
-    s_r[w] = pr;
-    s_s[w] = ps;
-    s_tk[w] = T.tk;
-    s_stride[w] = (int32_t)(T.two - T.tk);
+    s_n[w] = nrec;
+    s_r[w] = p.r;
+    s_s[w] = p.s;
   }
   __syncthreads();
   int32_t off[kNodalWaves + 1];
   off[0] = 0;
 #pragma unroll
-  for (int i = 0; i < kNodalWaves; ++i) off[i + 1] = off[i] + s_n[i];
-  const int32_t total = off[kNodalWaves];
-  for (int32_t e = threadIdx.x; e < total; e += blockDim.x) {
+  for (int i = 0; i < kNodalWaves; ++i) off[i + 1] = off[i] + max(s_n[i], 0);
+  for (int32_t e = threadIdx.x; e < off[kNodalWaves]; e += blockDim.x) {
     int wv = 0;
 #pragma unroll
     for (int i = 1; i < kNodalWaves; ++i) wv += e >= off[i];
-    const int32_t j = e - off[wv];
-    const int32_t* tk = s_tk[wv];
-    const int32_t st = s_stride[wv];
-    const int32_t b = tk[j], wo = tk[st + j], wi = tk[2 * st + j];
-    if (wo == 0 && wi == 0) continue;
-    const int32_t r = s_r[wv], s = s_s[wv];
-    apply_entry(a, r, m_row(a.M, r), s, m_row(a.M, s), b, wo, wi);
+    const int32_t* rec = s_lds[wv] + (e - off[wv]);
+    const int32_t wo = rec[2 * kMaxRec], wi = rec[3 * kMaxRec];
+    if (wo != 0 || wi != 0)
+      apply_record<kD>(a, s_r[wv], s_s[wv], rec[0], rec[kMaxRec], wo, wi);
+  }
+  if (kHub) {
+    __shared__ int32_t s_sum[2];
+    for (int i = 0; i < kNodalWaves; ++i) {
+      if (s_n[i] >= 0) continue;
+      __syncthreads();  // the records above are read
+      apply_hub<kD, kW>(a, (int32_t)((int64_t)a.beg + item0 + i), s_r[i], s_s[i], &s_lds[0][0],
+                        s_sum);
+    }
   }
   if (a.tstamp) {
     __syncthreads();
@@ -2915,38 +3121,72 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_apply(ApplyArgs a) {
   }
 }
 
-// Rows whose key count passed 1/slack of the slab or that have parked
-// increments (each of the 512 workgroups scans its slice of the rows),
-// handled between two batches, dead keys (both counts 0) dropped: a
-// row whose live keys and parked increments fit 1/(2 slack) of its slab (and
-// at most kCompact slots) is compacted in place through LDS; any other row
+// k_grow: the rows marked by k_apply (a new key far from home, a large row past
+// 1/slack load, parked increments), handled between two batches.  A row whose keys are not past
+// 1/slack of its slab and that has nothing parked is only unmarked.  Else its
+// dead keys (both counts 0) are dropped: a row whose live keys and parked
+// increments fit 1/(2 slack) of its slab is rewritten in place, any other
 // moves to a slab >= 2*slack*live+16 (direct once that reaches B/8) at the
-// free tail of the pool, and the row's parked increments are replayed into it.  A
-// new slab of at most kGrowLds slots is laid out in LDS (its slots claimed
-// meanwhile) and written out whole; the old one is left as zeros.  Bucket
-// sums are unchanged.  Block 0 also acts on the batch's flags.
-constexpr int kCompact = 4096;
-constexpr int kGrowLds = 2048;    // slabs up to this many slots are laid out in LDS
-constexpr int kGrowBlocks = 512;  // k_grow's grid
-constexpr int kGrowScan = 1024;   // rows a k_grow workgroup checks per round (4 per thread)
+// free tail of the pool, and its parked increments go in with the rest; the
+// old slab's counts are left as zeros.  A slab that is the row's first to keep
+// bucket sums gets them here.  Block 0 also acts on the batch's flags.
+//
+// Right after a merge phase a batch marks thousands of rows (2000 movers of 45
+// edges at B = 100000), nearly all of them slabs of 128 to 512 slots: such a
+// row is one wavefront's, read once into registers, laid out in LDS and
+// written out whole.  The others are the workgroup's, one after another.
+// 72.6 -> 20.0 us a launch there (every row by a workgroup, one counter for
+// every slab, bucket sums and key counts kept for every row before).
+constexpr int kWaveRow = 512;     // slots of a row one wavefront handles (8 per lane)
+constexpr int kWaveSlab = 1024;   // and of its new slab
+constexpr int kCompact = 4096;    // slots up to which the workgroup compacts in place
+constexpr int kGrowLds = 2048;    // entries staged, and slots laid out, in LDS by the workgroup
+constexpr int kGrowScan = 512;    // rows a k_grow workgroup checks per round (2 per thread)
 constexpr int32_t kOvfCap = 1 << 22;  // parked increments
+static_assert(kNodalWaves * 3 * kWaveSlab == 6 * kGrowLds, "one LDS pool for both paths");
 
 struct GrowSide {
   int64_t* off;
   int32_t* cap;
-  int32_t* nkeys;
+  int32_t* gmark;
   int32_t* key;
   Cnt* cnt;
+  int32_t* bs;
   int32_t* gpend;
   const int32_t* ovf;
   int32_t ovf_cap;
   GrowState* gst;
   int64_t P;
   int32_t slack;
+  int32_t chunk;  // slots a workgroup takes from the free tail at a time (0: each row its own)
 };
+
+// Slots of the pool for grown rows.  One counter gives out the free tail, and
+// an atomic on it costs ~30 ns, one after another: 1500 rows growing after one
+// batch (B = 100000, right after a merge) waited 40 us on it.  So a workgroup
+// takes `chunk` slots at a time and keeps what is left for later batches.
+struct GrowAlloc {
+  long long pos, end;    // the workgroup's chunk
+  long long last;        // end of what was taken from it
+  int32_t grows, compactions;
+};
+
+__device__ __forceinline__ long long grow_alloc(const GrowSide& g, GrowAlloc& al, int32_t n) {
+  const long long p = (long long)atomicAdd(reinterpret_cast<unsigned long long*>(&al.pos),
+                                           (unsigned long long)n);
+  if (p + n <= al.end) {
+    atomicMax(reinterpret_cast<unsigned long long*>(&al.last), (unsigned long long)(p + n));
+    return p;
+  }
+  const long long q = (long long)atomicAdd(&g.gst->used, (unsigned long long)n);
+  if (q + n <= g.P) return q;
+  atomicAdd(&g.gst->used, (unsigned long long)(-(long long)n));  // give the slots back
+  return -1;
+}
 
 struct GrowArgs {
   GrowSide side;
+  MView M;
   int32_t B;
   Sweep* sweep;
   Status* status;
@@ -2954,17 +3194,171 @@ struct GrowArgs {
   int32_t tstride;
 };
 
-// Replays the parked increments of row a into its slab (o, c) (the only block
-// touching row a in this launch); an increment that still finds no slot asks
-// the host for a rebuild.
-__device__ void replay_row(const GrowSide& g, int32_t a, int64_t o, int32_t c, int32_t B,
-                           Sweep* sw) {
+// Slots of the new slab of a row of c slots with `need` keys to hold.
+__device__ __forceinline__ int64_t grown_cap(int64_t need, int32_t c, int32_t slack, int32_t B) {
+  int64_t nc = 32;
+  while (nc < 2 * slack * need + 16) nc <<= 1;
+  if (nc < 2 * (int64_t)c) nc = 2 * (int64_t)c;
+  return 8 * nc >= B ? B : nc;
+}
+
+// The pool ran out: the host rebuilds M from the labels (parked increments
+// and all).
+__device__ __forceinline__ void grow_nospace(const GrowSide& g, Sweep* sw) {
+  g.gst->nospace = 1;
+  atomicAdd(&g.gst->nospace_events, 1ull);
+  atomicOr(&sw->flags, kFlagFull);
+  atomicCAS(&sw->stop, 0, 2);
+}
+
+// (key, do, di) into an LDS slab, direct or hashed (never full: it is sized for
+// the row's live keys and parked increments).
+__device__ __forceinline__ void lds_slab_add(int32_t* tk, int32_t* to, int32_t* ti, uint32_t mask,
+                                             bool direct, int32_t k, int32_t dout, int32_t din) {
+  uint32_t h = (uint32_t)k;
+  if (!direct) {
+    h = hash32(k) & mask;
+    for (;;) {
+      const int32_t old = atomicCAS(&tk[h], -1, k);
+      if (old == -1 || old == k) break;
+      h = (h + 1) & mask;
+    }
+  }
+  if (dout) atomicAdd(&to[h], dout);
+  if (din) atomicAdd(&ti[h], din);
+}
+
+// Row a by one wavefront, with 3 * kWaveSlab ints of LDS; false: the row is
+// the workgroup's.
+__device__ __forceinline__ bool grow_wave(const GrowArgs& ga, int32_t a, int32_t* lds,
+                                          GrowAlloc& al) {
+  const GrowSide& g = ga.side;
+  const int lane = lane_id();
+  const int32_t B = ga.B;
+  const int64_t o = g.off[a];
+  const int32_t c = g.cap[a];
+  const int32_t pend = g.gpend[a];  // parked increments (at most one new key each)
+  if (c == B || c > kWaveRow) return false;
+  constexpr int kQ = kWaveRow / kWave;
+  int32_t k[kQ];
+  Cnt x[kQ];
+#pragma unroll
+  for (int q = 0; q < kQ; ++q) {
+    const int32_t j = q * kWave + lane;
+    k[q] = -1;
+    x[q] = Cnt{0, 0};
+    if (j < c) {
+      k[q] = g.key[o + j];
+      x[q] = g.cnt[o + j];
+    }
+  }
+  int32_t keys = 0, live = 0;
+#pragma unroll
+  for (int q = 0; q < kQ; ++q) {
+    keys += __popcll(__ballot(k[q] >= 0));
+    if (x[q].o == 0 && x[q].i == 0) k[q] = -1;
+    live += __popcll(__ballot(k[q] >= 0));
+  }
+  if (pend == 0 && (int64_t)g.slack * keys <= c) {  // not past 1/slack load yet
+    if (lane == 0) g.gmark[a] = 0;
+    return true;
+  }
+  const bool inplace = 2 * (int64_t)g.slack * (live + pend) <= c;
+  const int64_t nc64 = inplace ? c : grown_cap((int64_t)live + pend, c, g.slack, B);
+  if (nc64 > kWaveSlab || nc64 == B) return false;
+  const int32_t nc = (int32_t)nc64;
+  long long base = 0;  // the slots are taken while the slab is laid out
+  if (!inplace && lane == 0) base = grow_alloc(g, al, nc);
+  int32_t *tk = lds, *to = lds + kWaveSlab, *ti = lds + 2 * kWaveSlab;
+  for (int32_t j = lane; j < nc; j += kWave) {
+    tk[j] = -1;
+    to[j] = 0;
+    ti[j] = 0;
+  }
+  lds_order();
+  const uint32_t mask = (uint32_t)nc - 1;
+#pragma unroll
+  for (int q = 0; q < kQ; ++q)
+    if (k[q] >= 0) lds_slab_add(tk, to, ti, mask, false, k[q], x[q].o, x[q].i);
+  if (pend > 0) {
+    const int32_t no = min(g.gst->ovf_n, g.ovf_cap);
+    constexpr int kP = 8;  // entries in flight per lane: a batch may park thousands
+    for (int32_t i0 = lane; i0 < no; i0 += kP * kWave) {
+      int32_t row[kP];
+#pragma unroll
+      for (int q = 0; q < kP; ++q) row[q] = i0 + q * kWave < no ? g.ovf[i0 + q * kWave] : -1;
+#pragma unroll
+      for (int q = 0; q < kP; ++q) {
+        if (row[q] != a) continue;
+        const int32_t* e = g.ovf + i0 + q * kWave;
+        lds_slab_add(tk, to, ti, mask, false, e[g.ovf_cap], e[2 * (int64_t)g.ovf_cap],
+                     e[3 * (int64_t)g.ovf_cap]);
+      }
+    }
+  }
+  lds_order();
+  int64_t nb = o;
+  bool ok = true;
+  if (!inplace) {
+    nb = read_lane((long)base, 0);
+    ok = nb >= 0;
+    if (!ok && lane == 0) grow_nospace(g, ga.sweep);
+  }
+  if (ok) {
+    for (int32_t j = lane; j < nc; j += kWave) {
+      g.key[nb + j] = tk[j];
+      g.cnt[nb + j] = Cnt{to[j], ti[j]};
+    }
+    if (!inplace)
+      for (int32_t j = lane; j < c; j += kWave) g.cnt[o + j] = Cnt{0, 0};
+    if (row_sums(ga.M, nc) && !row_sums(ga.M, c)) {  // the row's first bucket sums
+      constexpr int kS = kWaveSlab / kWave;
+      int32_t sk[kS], sv[kS];
+#pragma unroll
+      for (int q = 0; q < kS; ++q) {
+        const int32_t j = q * kWave + lane;
+        sk[q] = j < nc ? tk[j] : -1;
+        sv[q] = j < nc ? to[j] + ti[j] : 0;
+      }
+      lds_order();
+      for (int32_t j = lane; j < kNBK; j += kWave) tk[j] = 0;
+      lds_order();
+#pragma unroll
+      for (int q = 0; q < kS; ++q)
+        if (sk[q] >= 0 && sv[q] != 0) atomicAdd(&tk[sk[q] >> ga.M.bshift], sv[q]);
+      lds_order();
+      for (int32_t j = lane; j < kNBK; j += kWave) g.bs[(int64_t)a * kNBK + j] = tk[j];
+    }
+  }
+  if (lane == 0) {
+    if (ok) {
+      if (!inplace) {
+        g.off[a] = nb;
+        g.cap[a] = nc;
+      } else {
+        atomicAdd(&al.compactions, 1);
+      }
+      atomicAdd(&al.grows, 1);
+    }
+    g.gpend[a] = 0;
+    g.gmark[a] = ok ? room_mark(live + pend, nc, g.slack) : 0;
+  }
+  lds_order();  // the next row's slab takes this one's LDS
+  return true;
+}
+
+// Parked increments of row a into its slab (o, c) in the pool (the only block
+// touching row a in this launch); an increment that finds no slot asks the
+// host for a rebuild.  sums: the row's bucket sums lack them too.
+__device__ void replay_row(const GrowArgs& ga, int32_t a, int64_t o, int32_t c, bool sums) {
+  const GrowSide& g = ga.side;
   const int32_t no = min(g.gst->ovf_n, g.ovf_cap);
   for (int32_t i = threadIdx.x; i < no; i += blockDim.x) {
     if (g.ovf[i] != a) continue;
     const int32_t b = g.ovf[g.ovf_cap + i];
     const int32_t dout = g.ovf[2 * g.ovf_cap + i], din = g.ovf[3 * g.ovf_cap + i];
-    if (c == B) {
+    if (sums) atomicAdd(&g.bs[(int64_t)a * kNBK + (b >> ga.M.bshift)], dout + din);
+    if (c == ga.B) {
       cnt_add(&g.cnt[o + b], dout, din);
       continue;
     }
@@ -2975,10 +3369,7 @@ __device__ void replay_row(const GrowSide& g, int32_t a, int64_t o, int32_t c, i
       int32_t k = ld_relaxed(&g.key[o + h]);
       if (k < 0) {
         k = atomicCAS(&g.key[o + h], -1, b);
-        if (k == -1) {
-          atomicAdd(&g.nkeys[a], 1);
-          k = b;
-        }
+        if (k == -1) k = b;
       }
       if (k == b) {
         cnt_add(&g.cnt[o + h], dout, din);
@@ -2987,8 +3378,8 @@ __device__ void replay_row(const GrowSide& g, int32_t a, int64_t o, int32_t c, i
       h = (h + 1) & mask;
     }
     if (!done) {  // no room (the pool ran out): rebuild M
-      atomicOr(&sw->flags, kFlagFull);
-      atomicCAS(&sw->stop, 0, 2);
+      atomicOr(&ga.sweep->flags, kFlagFull);
+      atomicCAS(&ga.sweep->stop, 0, 2);
     }
   }
 }
@@ -3005,32 +3396,196 @@ __device__ void lds_slab(const int32_t* s_k, const int32_t* s_o, const int32_t* 
     t_i[j] = 0;
   }
   __syncthreads();
-  const uint32_t mask = (uint32_t)nc - 1;
-  for (int32_t i = threadIdx.x; i < live; i += blockDim.x) {
-    const int32_t k = s_k[i];
-    uint32_t h = (uint32_t)k;
-    if (!direct) {
-      h = hash32(k) & mask;
-      while (atomicCAS(&t_k[h], -1, k) != -1) h = (h + 1) & mask;
+  for (int32_t i = threadIdx.x; i < live; i += blockDim.x)
+    lds_slab_add(t_k, t_o, t_i, (uint32_t)nc - 1, direct, s_k[i], s_o[i], s_i[i]);
+  __syncthreads();
+}
+
+// Row a by the whole workgroup.
+__device__ void grow_block(const GrowArgs& ga, int32_t a, int32_t* pool, GrowAlloc& al) {
+  __shared__ long long s_base;
+  __shared__ int32_t s_cap, s_live, s_keys;
+  int32_t *s_k = pool, *s_o = pool + kGrowLds, *s_i = pool + 2 * kGrowLds;  // live entries
+  int32_t *t_k = pool + 3 * kGrowLds, *t_o = t_k + kGrowLds, *t_i = t_o + kGrowLds;  // new slab
+  const GrowSide& g = ga.side;
+  const int32_t B = ga.B;
+  const int64_t o = g.off[a];
+  const int32_t c = g.cap[a];
+  const int32_t pend = g.gpend[a];
+  const bool dold = c == B;  // a direct row never moves
+  if (threadIdx.x == 0) s_live = s_keys = 0;
+  __syncthreads();
+  constexpr int kQ = 4;
+  int32_t keys = 0;
+  for (int32_t j0 = threadIdx.x; j0 < c && !dold; j0 += kQ * blockDim.x) {
+    int32_t k[kQ];
+    Cnt x[kQ];
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      const int32_t j = j0 + q * (int32_t)blockDim.x;
+      k[q] = j < c ? g.key[o + j] : -1;
+      x[q] = j < c ? g.cnt[o + j] : Cnt{0, 0};
     }
-    t_o[h] = s_o[i];
-    t_i[h] = s_i[i];
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      keys += k[q] >= 0;
+      if (k[q] >= 0 && (x[q].o != 0 || x[q].i != 0)) {
+        const int32_t i = atomicAdd(&s_live, 1);
+        if (i < kGrowLds) {
+          s_k[i] = k[q];
+          s_o[i] = x[q].o;
+          s_i[i] = x[q].i;
+        }
+      }
+    }
+  }
+  if (keys) atomicAdd(&s_keys, keys);
+  __syncthreads();
+  const int32_t live = s_live;
+  const bool staged = live <= kGrowLds;
+  bool fresh = false;  // bucket sums just computed, without the parked increments
+  bool moved = false;  // dead keys dropped
+  int64_t o2 = o;      // the row's slab after this step
+  int32_t c2 = c;
+  if (dold || (pend == 0 && (int64_t)g.slack * s_keys <= c)) {
+    // nothing to move
+  } else if (staged && c <= kCompact && 2 * (int64_t)g.slack * (live + pend) <= c) {
+    // in place: the slab rewritten with the live entries only
+    moved = true;
+    if (c <= kGrowLds) {
+      lds_slab(s_k, s_o, s_i, live, t_k, t_o, t_i, c, false);
+      for (int32_t j = threadIdx.x; j < c; j += blockDim.x) {
+        g.key[o + j] = t_k[j];
+        g.cnt[o + j] = Cnt{t_o[j], t_i[j]};
+      }
+    } else {
+      for (int32_t j = threadIdx.x; j < c; j += blockDim.x) {
+        g.key[o + j] = -1;
+        g.cnt[o + j] = Cnt{0, 0};
+      }
+      __threadfence_block();
+      __syncthreads();
+      const uint32_t mask = (uint32_t)c - 1;
+      for (int32_t i = threadIdx.x; i < live; i += blockDim.x) {
+        uint32_t h = hash32(s_k[i]) & mask;
+        while (atomicCAS(&g.key[o + h], -1, s_k[i]) != -1) h = (h + 1) & mask;
+        g.cnt[o + h] = Cnt{s_o[i], s_i[i]};
+      }
+    }
+    __threadfence_block();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      atomicAdd(&al.grows, 1);
+      atomicAdd(&al.compactions, 1);
+    }
+  } else {
+    const int64_t nc = grown_cap((int64_t)live + pend, c, g.slack, B);
+    // the slots are taken while the new slab is laid out in LDS
+    long long base = 0;
+    if (threadIdx.x == 0) base = grow_alloc(g, al, (int32_t)nc);
+    const bool inlds = staged && nc <= kGrowLds;
+    if (inlds) lds_slab(s_k, s_o, s_i, live, t_k, t_o, t_i, (int32_t)nc, nc == B);
+    if (threadIdx.x == 0) {
+      s_cap = 0;
+      if (base < 0) {
+        grow_nospace(g, ga.sweep);
+      } else {
+        s_cap = (int32_t)nc;
+        s_base = base;
+      }
+    }
+    __syncthreads();
+    const int32_t ncap = s_cap;
+    if (ncap > 0) {
+      const int64_t nb = s_base;
+      if (inlds) {
+        for (int32_t j = threadIdx.x; j < ncap; j += blockDim.x) {
+          g.key[nb + j] = t_k[j];
+          g.cnt[nb + j] = Cnt{t_o[j], t_i[j]};
+        }
+        // the old slab's counts stay in the pool as zeros until a rebuild
+        for (int32_t j = threadIdx.x; j < c; j += blockDim.x) g.cnt[o + j] = Cnt{0, 0};
+      } else {
+        for (int32_t i = threadIdx.x; i < ncap; i += blockDim.x) {
+          g.key[nb + i] = -1;
+          g.cnt[nb + i] = Cnt{0, 0};
+        }
+        __threadfence_block();
+        __syncthreads();
+        const bool dnew = ncap == B;
+        const uint32_t mask = (uint32_t)ncap - 1;
+        for (int32_t j0 = threadIdx.x; j0 < c; j0 += kQ * blockDim.x) {
+          int32_t k[kQ];
+          Cnt x[kQ];
+#pragma unroll
+          for (int q = 0; q < kQ; ++q) {
+            const int32_t j = j0 + q * (int32_t)blockDim.x;
+            k[q] = j < c ? g.key[o + j] : -1;
+            x[q] = j < c ? g.cnt[o + j] : Cnt{0, 0};
+          }
+#pragma unroll
+          for (int q = 0; q < kQ; ++q) {
+            if (k[q] < 0 || (x[q].o == 0 && x[q].i == 0)) continue;
+            g.cnt[o + j0 + q * (int32_t)blockDim.x] = Cnt{0, 0};
+            if (dnew) {
+              g.cnt[nb + k[q]] = x[q];
+              continue;
+            }
+            uint32_t h = hash32(k[q]) & mask;
+            while (atomicCAS(&g.key[nb + h], -1, k[q]) != -1) h = (h + 1) & mask;
+            g.cnt[nb + h] = x[q];
+          }
+        }
+      }
+      __threadfence_block();
+      __syncthreads();
+      // the new slab's bucket sums, if it is the first to keep them (parked
+      // increments added theirs only to a slab that kept them)
+      if (row_sums(ga.M, ncap) && !row_sums(ga.M, c)) {
+        for (int32_t j = threadIdx.x; j < kNBK; j += blockDim.x) s_k[j] = 0;
+        __syncthreads();
+        for (int32_t j = threadIdx.x; j < ncap; j += blockDim.x) {
+          const int32_t k = ncap == B ? j : ld_relaxed(&g.key[nb + j]);
+          const Cnt x = g.cnt[nb + j];
+          if (k >= 0 && (x.o != 0 || x.i != 0)) atomicAdd(&s_k[k >> ga.M.bshift], x.o + x.i);
+        }
+        __syncthreads();
+        for (int32_t j = threadIdx.x; j < kNBK; j += blockDim.x)
+          g.bs[(int64_t)a * kNBK + j] = s_k[j];
+        __threadfence_block();
+        __syncthreads();
+        fresh = true;
+      }
+      if (threadIdx.x == 0) {
+        g.off[a] = nb;
+        g.cap[a] = ncap;
+        atomicAdd(&al.grows, 1);
+      }
+      moved = true;
+      o2 = nb;
+      c2 = ncap;
+    }
+  }
+  if (pend > 0) replay_row(ga, a, o2, c2, fresh);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    g.gpend[a] = 0;
+    g.gmark[a] = dold ? 0 : room_mark(moved ? live + pend : s_keys, c2, g.slack);
   }
   __syncthreads();
 }
 
 __global__ __launch_bounds__(256) void k_grow(GrowArgs ga) {
-  __shared__ int32_t s_k[kCompact];  // the row's live entries
-  __shared__ int32_t s_o[kCompact];
-  __shared__ int32_t s_i[kCompact];
-  __shared__ int32_t t_k[kGrowLds];  // its new slab, when it fits
-  __shared__ int32_t t_o[kGrowLds];
-  __shared__ int32_t t_i[kGrowLds];
-  __shared__ int32_t s_q[kGrowScan];  // rows of the scanned chunk to handle
-  __shared__ long long s_base;
-  __shared__ int32_t s_cap, s_live, s_nq;
+  __shared__ __align__(16) int32_t s_pool[6 * kGrowLds];
+  __shared__ int32_t s_q[kGrowScan];    // marked rows of the scanned chunk
+  __shared__ int32_t s_big[kGrowScan];  // those left to the workgroup
+  __shared__ int32_t s_nq, s_nbig;
+  __shared__ GrowAlloc s_al;
+  __shared__ bool s_taken;  // a chunk was taken in this round
   const int32_t B = ga.B;
   const GrowSide& g = ga.side;
+  const int w = threadIdx.x / kWave;
+  bool any = false;  // thread 0: s_al is loaded
   if (ga.tstamp && threadIdx.x == 0) ga.tstamp[blockIdx.x] = wall_clock64();
   // the batch's flags (raised by its k_nodal and k_apply, both complete):
   // errors override convergence, which overrides a rebuild request, as the
@@ -3045,167 +3600,65 @@ __global__ __launch_bounds__(256) void k_grow(GrowArgs ga) {
         atomicCAS(&ga.sweep->stop, 0, 2);
       ga.status->flags = 0;
     }
+    g.gst->full += (unsigned long long)g.gst->ovf_n;
   }
-  // the rows to grow or compact, found by a scan of this workgroup's slice
-  // of the rows: hashed rows past 1/slack load, or with parked increments
-  // (k_apply only counts keys and parked increments; it queues nothing)
   const int32_t per = (B + (int32_t)gridDim.x - 1) / (int32_t)gridDim.x;
   const int32_t lo = (int32_t)blockIdx.x * per, hi = min(B, lo + per);
   for (int32_t base = lo; base < hi; base += kGrowScan) {
-    if (threadIdx.x == 0) s_nq = 0;
+    if (threadIdx.x == 0) s_nq = s_nbig = 0;
     __syncthreads();
-    int32_t cq[kGrowScan / 256], nq_k[kGrowScan / 256], pq[kGrowScan / 256];
+    int32_t mq[kGrowScan / 256];
 #pragma unroll
     for (int q = 0; q < kGrowScan / 256; ++q) {
       const int32_t r = base + q * 256 + (int32_t)threadIdx.x;
-      cq[q] = B;
-      nq_k[q] = 0;
-      pq[q] = 0;
-      if (r < hi) {
-        cq[q] = g.cap[r];
-        nq_k[q] = g.nkeys[r];
-        pq[q] = g.gpend[r];
-      }
+      mq[q] = r < hi ? g.gmark[r] : 0;
     }
 #pragma unroll
     for (int q = 0; q < kGrowScan / 256; ++q)
-      if (cq[q] < B && ((int64_t)g.slack * nq_k[q] > cq[q] || pq[q] > 0))
-        s_q[atomicAdd(&s_nq, 1)] = base + q * 256 + (int32_t)threadIdx.x;
+      if (mq[q] > 0) s_q[atomicAdd(&s_nq, 1)] = base + q * 256 + (int32_t)threadIdx.x;
     __syncthreads();
     const int32_t nq = s_nq;
-    for (int32_t qi = 0; qi < nq; ++qi) {
-    const int32_t a = s_q[qi];
-    const int64_t o = g.off[a];
-    const int32_t c = g.cap[a];
-    const int32_t pend = g.gpend[a];  // parked increments (at most one new key each)
-    const bool dold = c == B;
-    // a hashed slab of at most kCompact slots has its live entries gathered
-    // into LDS by the counting pass
-    const bool gather = !dold && c <= kCompact;
-    if (threadIdx.x == 0) s_live = 0;
-    __syncthreads();
-    for (int32_t j = threadIdx.x; j < c; j += blockDim.x) {
-      const Cnt x = g.cnt[o + j];
-      const int32_t k = dold ? j : g.key[o + j];
-      if (k >= 0 && (x.o != 0 || x.i != 0)) {
-        const int32_t i = atomicAdd(&s_live, 1);
-        if (gather) {
-          s_k[i] = k;
-          s_o[i] = x.o;
-          s_i[i] = x.i;
-        }
+    if (nq == 0) continue;  // the same for every thread; s_nq is next written by thread 0
+    if (threadIdx.x == 0) {
+      s_taken = false;
+      if (!any) {
+        const GrowChunk c = g.gst->chunk[blockIdx.x];
+        s_al = GrowAlloc{c.pos, c.end, c.pos, 0, 0};
+        any = true;
       }
-    }
-    __syncthreads();
-    const int32_t live = s_live;
-    int64_t o2 = o;  // the row's slab after this step
-    int32_t c2 = c;
-    if (gather && 2 * g.slack * (live + pend) <= c) {
-      // in place: the slab rewritten with the live entries only
-      if (c <= kGrowLds) {
-        lds_slab(s_k, s_o, s_i, live, t_k, t_o, t_i, c, false);
-        for (int32_t j = threadIdx.x; j < c; j += blockDim.x) {
-          g.key[o + j] = t_k[j];
-          g.cnt[o + j] = Cnt{t_o[j], t_i[j]};
-        }
-      } else {
-        for (int32_t j = threadIdx.x; j < c; j += blockDim.x) {
-          g.key[o + j] = -1;
-          g.cnt[o + j] = Cnt{0, 0};
-        }
-        __threadfence_block();
-        __syncthreads();
-        const uint32_t mask = (uint32_t)c - 1;
-        for (int32_t i = threadIdx.x; i < live; i += blockDim.x) {
-          uint32_t h = hash32(s_k[i]) & mask;
-          while (atomicCAS(&g.key[o + h], -1, s_k[i]) != -1) h = (h + 1) & mask;
-          g.cnt[o + h] = Cnt{s_o[i], s_i[i]};
-        }
-      }
-      __threadfence_block();
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        g.nkeys[a] = live;
-        g.gst->grows += 1;
-        g.gst->compactions += 1;
-      }
-    } else {
-      int64_t nc = 32;
-      while (nc < 2 * g.slack * ((int64_t)live + pend) + 16) nc <<= 1;
-      if (nc < 2 * (int64_t)c) nc = 2 * (int64_t)c;
-      if (8 * nc >= B) nc = B;
-      // the slots are claimed while the new slab is laid out in LDS; a
-      // direct row never moves
-      unsigned long long base = 0;
-      if (threadIdx.x == 0 && !dold) base = atomicAdd(&g.gst->used, (unsigned long long)nc);
-      const bool inlds = gather && nc <= kGrowLds;
-      if (inlds) lds_slab(s_k, s_o, s_i, live, t_k, t_o, t_i, (int32_t)nc, nc == B);
-      if (threadIdx.x == 0) {
-        s_cap = 0;
-        if (!dold) {
-          if ((int64_t)base + nc > g.P) {
-            atomicAdd(&g.gst->used, (unsigned long long)(-nc));  // give the slots back
-            g.gst->nospace = 1;
-            g.gst->nospace_events += 1;
-            atomicOr(&ga.sweep->flags, kFlagFull);
-            atomicCAS(&ga.sweep->stop, 0, 2);
-          } else {
-            s_cap = (int32_t)nc;
-            s_base = (long long)base;
-          }
-        }
-      }
-      __syncthreads();
-      const int32_t ncap = s_cap;
-      if (ncap > 0) {
-        const int64_t nb = s_base;
-        if (inlds) {
-          for (int32_t j = threadIdx.x; j < ncap; j += blockDim.x) {
-            g.key[nb + j] = t_k[j];
-            g.cnt[nb + j] = Cnt{t_o[j], t_i[j]};
-          }
-          // the old slab's counts stay in the pool as zeros until a rebuild
-          for (int32_t j = threadIdx.x; j < c; j += blockDim.x) g.cnt[o + j] = Cnt{0, 0};
+      if (g.chunk > 0 && s_al.end - s_al.last < kWaveSlab) {
+        const long long p = (long long)atomicAdd(&g.gst->used, (unsigned long long)g.chunk);
+        if (p + g.chunk <= g.P) {
+          s_al.pos = s_al.last = p;
+          s_al.end = p + g.chunk;
+          s_taken = true;
         } else {
-          for (int32_t i = threadIdx.x; i < ncap; i += blockDim.x) {
-            g.key[nb + i] = -1;
-            g.cnt[nb + i] = Cnt{0, 0};
-          }
-          __threadfence_block();
-          __syncthreads();
-          const bool dnew = ncap == B;
-          const uint32_t mask = (uint32_t)ncap - 1;
-          for (int32_t j = threadIdx.x; j < c; j += blockDim.x) {
-            const int32_t k = g.key[o + j];
-            const Cnt x = g.cnt[o + j];
-            if (k < 0 || (x.o == 0 && x.i == 0)) continue;
-            g.cnt[o + j] = Cnt{0, 0};
-            if (dnew) {
-              g.cnt[nb + k] = x;
-              continue;
-            }
-            uint32_t h = hash32(k) & mask;
-            while (atomicCAS(&g.key[nb + h], -1, k) != -1) h = (h + 1) & mask;
-            g.cnt[nb + h] = x;
-          }
+          atomicAdd(&g.gst->used, (unsigned long long)(-(long long)g.chunk));
         }
-        __threadfence_block();
-        __syncthreads();
-        if (threadIdx.x == 0) {
-          g.off[a] = nb;
-          g.cap[a] = ncap;
-          g.nkeys[a] = live;
-          g.gst->grows += 1;
-        }
-        o2 = nb;
-        c2 = ncap;
       }
     }
-    if (pend > 0) replay_row(g, a, o2, c2, B, ga.sweep);
     __syncthreads();
-    if (threadIdx.x == 0) g.gpend[a] = 0;
-    __syncthreads();
+    for (int32_t i = w; i < nq; i += kNodalWaves) {
+      const int32_t a = s_q[i];
+      if (!grow_wave(ga, a, s_pool + w * 3 * kWaveSlab, s_al) && lane_id() == 0)
+        s_big[atomicAdd(&s_nbig, 1)] = a;
     }
+    __syncthreads();
+    for (int32_t i = 0; i < s_nbig; ++i) grow_block(ga, s_big[i], s_pool, s_al);
+    __syncthreads();
+    if (s_taken)  // the MDL scan reads the whole used pool
+      for (long long j = s_al.last + threadIdx.x; j < s_al.end; j += blockDim.x)
+        g.cnt[j] = Cnt{0, 0};
+    __threadfence_block();
+    __syncthreads();
+    if (threadIdx.x == 0) s_al.pos = s_al.last;  // a request that did not fit took nothing
+  }
+  if (threadIdx.x == 0 && any) {
+    GrowChunk& c = g.gst->chunk[blockIdx.x];
+    c.pos = s_al.last;
+    c.end = s_al.end;
+    c.grows += (unsigned long long)s_al.grows;
+    c.compactions += (unsigned long long)s_al.compactions;
   }
   if (ga.tstamp) {
     __syncthreads();
@@ -3222,7 +3675,7 @@ __global__ __launch_bounds__(256) void k_grow(GrowArgs ga) {
 struct DevSpM {
   int64_t* off = nullptr;
   int32_t* cap = nullptr;
-  int32_t* nkeys = nullptr;
+  int32_t* gmark = nullptr;  // [N]
   int32_t* key = nullptr;  // row slabs [P]: keys
   Cnt* cnt = nullptr;      // and counts
   int32_t* bs = nullptr;  // [bs_rows][kNBK]
@@ -3453,7 +3906,7 @@ MView view(const DevSpM& m, int32_t B) {
   MView v;
   v.off = m.off;
   v.cap = m.cap;
-  v.nkeys = m.nkeys;
+  v.gmark = m.gmark;
   v.key = m.key;
   v.cnt = m.cnt;
   v.bs = m.bs;
@@ -3588,7 +4041,7 @@ int rebuild_M(usap_engine* e) {
   {
     ClearArgs c;
     int32_t* arr[kClearArrays] = {e->d_out, e->d_in, e->ecnt_out, e->ecnt_in,
-                                  e->bsize, e->M.nkeys, e->M.gpend, e->bl_cur};
+                                  e->bsize, e->M.gmark, e->M.gpend, e->bl_cur};
     for (int i = 0; i < kClearArrays; ++i) c.p[i] = arr[i];
     c.n = B;
     c.flags = e->build_flags;
@@ -3642,8 +4095,8 @@ int rebuild_M(usap_engine* e) {
   }
   if (m.total > 0) k_fill<<<std::min<int64_t>(blocks_for(m.total, 256), 8192), 256, 0, st>>>(
       e->all_direct ? nullptr : m.key, m.cnt, m.total);
-  k_reset_grow<<<1, 1, 0, st>>>(m.gst, (unsigned long long)m.total);
-  if (m.bs_rows < B) {
+  k_reset_grow<<<blocks_for(kGrowBlocks, 256), 256, 0, st>>>(m.gst, (unsigned long long)m.total);
+  if (B > kNBK && m.bs_rows < B) {
     dfree(e, m.bs);
     if (int rc = dalloc(e, &m.bs, (size_t)B * kNBK)) return rc;
     m.bs_rows = B;
@@ -3664,7 +4117,7 @@ int rebuild_M(usap_engine* e) {
       if (int rc = build_rows(e)) return rc;
     }
   }
-  k_bucket_sums<<<blocks_for(B, 4), 256, 0, st>>>(view(e->M, B));
+  if (B > kNBK) k_bucket_sums<<<blocks_for(B, kSumRows), 256, 0, st>>>(view(e->M, B));
   HIPCHK(hipGetLastError());
   ev_rec(e, 1);
   int32_t flags = 0;
@@ -3721,25 +4174,29 @@ const usap_params* engine_params(const usap_engine* e) { return &e->p; }
 int32_t engine_rebuilds(const usap_engine* e) { return e->rebuilds; }
 // Growth counters, read on the engine's own stream (never the legacy null
 // stream, which other engines' threads must not see).
-static bool read_grow_state(usap_engine* e, GrowState* g) {
+static bool read_grow_state(usap_engine* e, GrowState* g, long long* grows, long long* compactions) {
   if (hipMemcpyAsync(g, e->M.gst, sizeof(GrowState), hipMemcpyDeviceToHost, e->stream) !=
       hipSuccess)
     return false;
-  return hipStreamSynchronize(e->stream) == hipSuccess;
+  if (hipStreamSynchronize(e->stream) != hipSuccess) return false;
+  *grows = *compactions = 0;
+  for (const GrowChunk& c : g->chunk) {
+    *grows += (long long)c.grows;
+    *compactions += (long long)c.compactions;
+  }
+  return true;
 }
 void engine_grow_debug(usap_engine* e, long long out[4]) {
   out[0] = out[1] = out[2] = out[3] = 0;
   GrowState g{};
-  if (!read_grow_state(e, &g)) return;
-  out[0] = (long long)g.grows;
-  out[1] = (long long)g.compactions;
+  if (!read_grow_state(e, &g, &out[0], &out[1])) return;
   out[2] = (long long)g.full;
   out[3] = (long long)g.nospace_events;
 }
 int64_t engine_grows(usap_engine* e) {
   GrowState g{};
-  if (!read_grow_state(e, &g)) return 0;
-  return (int64_t)g.grows;
+  long long n = 0, c = 0;
+  return read_grow_state(e, &g, &n, &c) ? (int64_t)n : 0;
 }
 void engine_set_error(usap_engine* e, const char* msg) { e->err = msg; }
 }  // namespace usap
@@ -3798,7 +4255,7 @@ int usap_destroy(usap_engine* e) {
   for (DevSpM* m : {&e->M}) {
     dfree(e, m->off);
     dfree(e, m->cap);
-    dfree(e, m->nkeys);
+    dfree(e, m->gmark);
     dfree(e, m->key);
     dfree(e, m->cnt);
     dfree(e, m->bs);
@@ -4206,7 +4663,7 @@ int alloc_state(usap_engine* e) {
   for (DevSpM* m : {&e->M}) {
     TRY(dalloc(e, &m->off, (size_t)N + 1));
     TRY(dalloc(e, &m->cap, N));
-    TRY(dalloc(e, &m->nkeys, N));
+    TRY(dalloc(e, &m->gmark, N));
     TRY(dalloc(e, &m->gpend, N));
     m->ovf_cap = (int32_t)std::min<int64_t>(kOvfCap, 2 * e->E + 4096);
     TRY(dalloc(e, &m->ovf, (size_t)4 * m->ovf_cap));
@@ -4846,6 +5303,15 @@ NodalKernel nodal_kernel(bool dense, bool weighted, bool hubs) {
   return k[4 * dense + 2 * weighted + hubs];
 }
 
+typedef void (*ApplyKernel)(ApplyArgs);
+ApplyKernel apply_kernel(bool dense, bool weighted, bool hubs) {
+  static const ApplyKernel k[8] = {
+      k_apply<false, false, false>, k_apply<false, false, true>, k_apply<false, true, false>,
+      k_apply<false, true, true>,   k_apply<true, false, false>, k_apply<true, false, true>,
+      k_apply<true, true, false>,   k_apply<true, true, true>};
+  return k[4 * dense + 2 * weighted + hubs];
+}
+
 // The Philox words of nodes [beg, end) in batches of `batch` (batch i: stream
 // sweep->stream0 + i), before their first batch (pre-drawn mode has its own).
 int launch_draws(usap_engine* e, int32_t beg, int32_t end, int32_t batch) {
@@ -4898,8 +5364,6 @@ int launch_batch(usap_engine* e, int32_t beg, int32_t end, size_t ev_slot, bool 
   b.beg = beg;
   b.end = end;
   b.prop = e->prop;
-  b.big_off = e->big_off;
-  b.big_tab = e->big_tab;
   const unsigned grid = blocks_for((int64_t)end - beg, kNodalWaves);
   b.part = e->part;
   b.nparts = grid;
@@ -4913,7 +5377,11 @@ int launch_batch(usap_engine* e, int32_t beg, int32_t end, size_t ev_slot, bool 
     GrowSide& gs = ga.side;
     gs.off = m.off;
     gs.cap = m.cap;
-    gs.nkeys = m.nkeys;
+    gs.gmark = m.gmark;
+    // an eighth of the tail left by the rebuild, over the workgroups
+    const int64_t share = (m.P - m.total) / (8 * kGrowBlocks) / 32 * 32;
+    gs.chunk = share < kWaveSlab ? 0 : (int32_t)std::min<int64_t>(share, 8192);
+    gs.bs = m.bs;
     gs.key = m.key;
     gs.cnt = m.cnt;
     gs.gpend = m.gpend;
@@ -4923,7 +5391,8 @@ int launch_batch(usap_engine* e, int32_t beg, int32_t end, size_t ev_slot, bool 
     gs.P = m.P;
     gs.slack = m.slack;
   }
-  ga.B = B;
+  ga.M = a.M;
+  ga.B = e->all_direct ? 0 : B;  // no row grows while all are direct: only the flags
   ga.sweep = e->sweep;
   ga.status = e->status;
   ga.tstamp = ts ? ts + 4 * (size_t)G + 2 : nullptr;
@@ -4946,8 +5415,9 @@ int launch_batch(usap_engine* e, int32_t beg, int32_t end, size_t ev_slot, bool 
     q.acc = e->aq_acc;
     k_aq<<<grid, kWave * kNodalWaves, 0, st>>>(q);
   }
-  k_apply<<<grid + 1, kWave * kNodalWaves, 0, st>>>(b);  // block 0: the update step
-  if (grow) k_grow<<<kGrowBlocks, 256, 0, st>>>(ga);
+  apply_kernel(e->all_direct, e->weighted, e->max_list > kRegUnits * kWave)<<<
+      grid + 1, kWave * kNodalWaves, 0, st>>>(b);  // block 0: the update step
+  if (grow) k_grow<<<e->all_direct ? 1 : kGrowBlocks, 256, 0, st>>>(ga);
   HIPCHK(hipGetLastError());
   return USAP_OK;
 }
@@ -5051,7 +5521,7 @@ int run_sweep(usap_engine* e, int32_t batch, int32_t first, int32_t last, int32_
     if (e->prof)
       if (int rc = prof_end(e, (size_t)executed)) return rc;
     if (hs.stop == 3) return set_err(e, USAP_ESTATE, "inconsistent M during a nodal batch");
-    if (hs.flags & (kFlagLoad | kFlagFull)) {
+    if (hs.flags & kFlagFull) {
       if (int rc = rebuild_M(e)) return rc;
       if (rebuilds) ++*rebuilds;
     }
@@ -5116,7 +5586,7 @@ int usap_nodal_batch(usap_engine* e, int32_t begin, int32_t end, uint64_t stream
     }
     if (hs.stop == 3) return set_err(e, USAP_ESTATE, "inconsistent M during a nodal batch");
     if (e->uni) e->uni_pos += end - begin;
-    if (hs.flags & (kFlagLoad | kFlagFull))
+    if (hs.flags & kFlagFull)
       if (int rc = rebuild_M(e)) return rc;
   }
   const Sweep& hs = *e->h_sweep;
