@@ -81,7 +81,7 @@ constexpr int kNBK = 512;                // bucket sums per block row
 constexpr int kLookupRatio = 8;          // a hashed slab this many times a bucket is looked up per key
 constexpr int kScr = 3 * kTab;           // per-wavefront LDS scratch (ints) for one bucket
 constexpr int kDegLds = 1024;            // k_degrees privatises its counters for B <= this
-constexpr int kSmallB = 128;             // k_insert_small: B*B counts in LDS
+constexpr int kHistB = 256;              // M is built by histograms in LDS up to here
 constexpr int kEntropyBlocks = 4096;  // k_entropy grid at most
 // Partials of the allocation-free MDL (usap_entropy_noalloc): 2 words per
 // k_entropy workgroup, 64 KiB per GPU.
@@ -1092,31 +1092,138 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_build_rows(
   }
 }
 
-// M build for B <= kSmallB (every row direct): per-workgroup B*B counts in
-// LDS, flushed once, so the few hot cells are not hammered by atomics.
-__global__ __launch_bounds__(256) void k_insert_small(int64_t E, const int32_t* __restrict__ src,
-                                                      const int32_t* __restrict__ dst,
-                                                      const int32_t* __restrict__ w,
-                                                      const int32_t* __restrict__ labels,
-                                                      MView M) {
-  __shared__ int32_t s_h[kSmallB * kSmallB];
-  const int32_t B = M.B;
-  for (int i = threadIdx.x; i < B * B; i += blockDim.x) s_h[i] = 0;
+// M build for B <= kHistB (every row is direct there: 8 times the smallest
+// hashed slab reaches B): workgroup (g, half) counts the block pairs of its
+// share of the edges, of the rows of its half, in LDS, and the degrees and
+// sizes with them, and writes its counts out whole; k_hist_sum adds them up.
+// No counter is cleared or added to in memory, no row header is needed
+// first, and the host waits for nothing.  (Every workgroup's counts by atomics
+// on M, and before B = 128 a sort of the edges' pairs: E = 1 M at B = 76 46 us
+// in the insert alone, E = 4 M at B = 132 ~250 us.)
+constexpr int kHistThreads = 1024;
+constexpr int kHistOne = 200;  // B up to which one workgroup's LDS holds every row
+struct HistArgs {
+  GraphView g;
+  const int32_t* src;  // edge sources
+  const int32_t* labels;
+  int64_t E;
+  int32_t B, G, rows;  // rows per workgroup
+  int32_t* part;       // [G][B * B] counts
+  int32_t* part_d;     // [G * halves][3][kHistB] d_out, d_in, sizes
+};
+
+template <int kCells>
+__global__ __launch_bounds__(kHistThreads) void k_hist(HistArgs a) {
+  __shared__ int32_t s_h[kCells];
+  __shared__ int32_t s_size[kHistB];
+  const int32_t B = a.B, t = threadIdx.x;
+  const int32_t g = blockIdx.x, half = blockIdx.y;
+  const int32_t r0 = half * a.rows, nr = min(a.rows, B - r0), cells = nr * B;
+  for (int32_t i = t; i < cells; i += kHistThreads) s_h[i] = 0;
+  if (t < kHistB) s_size[t] = 0;
   __syncthreads();
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < E;
-       e += (int64_t)gridDim.x * blockDim.x)
-    atomicAdd(&s_h[labels[src[e]] * B + labels[dst[e]]], w ? w[e] : 1);
+  const int64_t e0 = a.E * g / a.G, e1 = a.E * (g + 1) / a.G;
+  constexpr int kQ = 4;  // edges in flight per thread
+  for (int64_t e = e0 + t; e < e1; e += kQ * kHistThreads) {
+    int32_t u[kQ], v[kQ], w[kQ];
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      const int64_t j = e + q * kHistThreads;
+      u[q] = v[q] = -1;
+      w[q] = 1;
+      if (j < e1) {
+        u[q] = a.src[j];
+        v[q] = a.g.out_idx[j];
+        if (a.g.out_w) w[q] = a.g.out_w[j];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kQ; ++q)
+      if (u[q] >= 0) {
+        u[q] = a.labels[u[q]] - r0;
+        v[q] = a.labels[v[q]];
+      }
+#pragma unroll
+    for (int q = 0; q < kQ; ++q)
+      if (u[q] >= 0 && u[q] < nr) atomicAdd(&s_h[u[q] * B + v[q]], w[q]);
+  }
+  const int64_t n0 = (int64_t)a.g.N * g / a.G, n1 = (int64_t)a.g.N * (g + 1) / a.G;
+  if (half == 0)
+    for (int64_t n = n0 + t; n < n1; n += kHistThreads) atomicAdd(&s_size[a.labels[n]], 1);
   __syncthreads();
-  for (int i = threadIdx.x; i < B * B; i += blockDim.x) {
-    const int32_t v = s_h[i];
-    if (!v) continue;
-    const int32_t a = i / B, b = i - a * B;
-    atomicAdd(&M.cnt[M.off[a] + b].o, v);
-    atomicAdd(&M.cnt[M.off[b] + a].i, v);
+  int32_t* out = a.part + (int64_t)g * B * B + (int64_t)r0 * B;
+  for (int32_t i = t; i < cells; i += kHistThreads) out[i] = s_h[i];
+  int32_t* d = a.part_d + ((int64_t)half * a.G + g) * 3 * kHistB;
+  if (t < kHistB) {  // row sums (each row from a column of its own: no bank conflicts)
+    int32_t sum = 0;
+    if (t >= r0 && t < r0 + nr)
+      for (int32_t j = 0, c = t % B; j < B; ++j, c = c + 1 == B ? 0 : c + 1)
+        sum += s_h[(t - r0) * B + c];
+    d[t] = sum;
+  } else if (t < 2 * kHistB) {  // column sums
+    int32_t sum = 0;
+    if (t - kHistB < B)
+      for (int32_t j = 0; j < nr; ++j) sum += s_h[j * B + (t - kHistB)];
+    d[t] = sum;
+  } else if (t < 3 * kHistB) {
+    d[t] = s_size[t - 2 * kHistB];
   }
 }
 
-// M build for kSmallB < B <= kPairSortB (rows mostly direct, few distinct
+// M, the row headers, degrees and sizes from k_hist's counts: block row a by
+// workgroup a, degrees and sizes by the last one.
+struct HistSum {
+  MView M;
+  int64_t* off;
+  int32_t* cap;
+  int32_t *d_out, *d_in, *bsize;
+  const int32_t* part;
+  const int32_t* part_d;
+  int32_t G, parts_d;
+};
+
+__global__ __launch_bounds__(kHistB) void k_hist_sum(HistSum a) {
+  const int32_t B = a.M.B, t = threadIdx.x, r = blockIdx.x;
+  constexpr int kQ = 8;
+  if (r < B) {
+    const int64_t n = (int64_t)B * B;
+    if (t < B) {
+      const int32_t* p = a.part + (int64_t)r * B + t;
+      int32_t v = 0;
+      for (int32_t g = 0; g < a.G; g += kQ) {
+        int32_t x[kQ];
+#pragma unroll
+        for (int q = 0; q < kQ; ++q) x[q] = g + q < a.G ? p[(g + q) * n] : 0;
+#pragma unroll
+        for (int q = 0; q < kQ; ++q) v += x[q];
+      }
+      a.M.cnt[(int64_t)r * B + t].o = v;
+      a.M.cnt[(int64_t)t * B + r].i = v;
+    }
+    if (t == 0) {
+      a.off[r] = (int64_t)r * B;
+      a.cap[r] = B;
+    }
+    return;
+  }
+  int32_t sum[3] = {0, 0, 0};
+  for (int32_t g = 0; g < a.parts_d; ++g)
+    for (int k = 0; k < 3; ++k) sum[k] += a.part_d[((int64_t)g * 3 + k) * kHistB + t];
+  if (t < B) {
+    a.d_out[t] = sum[0];
+    a.d_in[t] = sum[1];
+    a.bsize[t] = sum[2];
+  }
+  for (int i = t; i < kGrowBlocks; i += kHistB) a.M.gst->chunk[i].pos = a.M.gst->chunk[i].end = 0;
+  if (t == 0) {
+    a.off[B] = (int64_t)B * B;
+    a.M.gst->nospace = 0;
+    a.M.gst->ovf_n = 0;
+    a.M.gst->used = (unsigned long long)B * (unsigned long long)B;
+  }
+}
+
+// M build for kHistB < B <= kPairSortB (rows mostly direct, few distinct
 // block pairs, so per-edge atomics would pile onto the same counts): the
 // edges' block pairs a*B + b are sorted and summed per pair, then each pair
 // is added once.
@@ -3764,6 +3871,8 @@ struct usap_engine {
   uint64_t epoch = 0;  // bumped by every device allocation (pointers may change)
   int64_t graph_captures = 0;
   int32_t* build_flags = nullptr;  // [0] build overflow flags, [1] blocks holding != 1 node, [2] distinct block pairs
+  int32_t* hist = nullptr;  // counts of the build by histograms
+  int64_t hist_cap = 0;
   uint32_t* pair_key[2] = {nullptr, nullptr};  // block-pair builds [E]
   int32_t* pair_val[2] = {nullptr, nullptr};
   int64_t pair_cap = 0;  // edges the pair buffers hold
@@ -4034,10 +4143,87 @@ int build_rows(usap_engine* e) {
   return USAP_OK;
 }
 
+// Slots for a rebuild that needs `total`: two thirds of the pool is headroom for
+// rows that grow.
+int reserve_pool(usap_engine* e, int64_t total) {
+  DevSpM& m = e->M;
+  m.total = total;
+  m.slack = e->p.slab_slack;
+  if (3 * total <= m.P) return USAP_OK;
+  dfree(e, m.key);
+  dfree(e, m.cnt);
+  const int64_t P = 3 * total + (int64_t)4 * e->B + 4096;
+  m.P = 0;
+  if (int rc = dalloc(e, &m.key, (size_t)P)) return rc;
+  if (int rc = dalloc(e, &m.cnt, (size_t)P)) return rc;
+  m.P = P;
+  return USAP_OK;
+}
+
+// The build for B <= kHistB.  About 4096 edges a workgroup at least: fewer make
+// the counts' way through memory longer than the edges'.
+int build_hist(usap_engine* e) {
+  const int32_t B = e->B;
+  hipStream_t st = e->stream;
+  const bool one = B <= kHistOne;
+  const int32_t halves = one ? 1 : 2;
+  const int32_t G = (int32_t)std::max<int64_t>(1, std::min<int64_t>(e->E / 4096, 256 / halves));
+  const int64_t need = (int64_t)G * B * B + (int64_t)G * halves * 3 * kHistB;
+  if (need > e->hist_cap) {
+    dfree(e, e->hist);
+    e->hist_cap = 0;
+    if (int rc = dalloc(e, &e->hist, (size_t)need)) return rc;
+    e->hist_cap = need;
+  }
+  if (int rc = reserve_pool(e, (int64_t)B * B)) return rc;
+  e->all_direct = true;
+  HistArgs a;
+  a.g = gview(e);
+  a.src = e->out_src;
+  a.labels = e->labels;
+  a.E = e->E;
+  a.B = B;
+  a.G = G;
+  a.rows = one ? B : (B + 1) / 2;
+  a.part = e->hist;
+  a.part_d = e->hist + (int64_t)G * B * B;
+  const dim3 grid((unsigned)G, (unsigned)halves);
+  if (B * a.rows <= 4096)
+    k_hist<4096><<<grid, kHistThreads, 0, st>>>(a);
+  else if (B * a.rows <= 16384)
+    k_hist<16384><<<grid, kHistThreads, 0, st>>>(a);
+  else
+    k_hist<kHistOne * kHistOne><<<grid, kHistThreads, 0, st>>>(a);
+  HistSum b;
+  b.M = view(e->M, B);
+  b.off = e->M.off;
+  b.cap = e->M.cap;
+  b.d_out = e->d_out;
+  b.d_in = e->d_in;
+  b.bsize = e->bsize;
+  b.part = a.part;
+  b.part_d = a.part_d;
+  b.G = G;
+  b.parts_d = G * halves;
+  k_hist_sum<<<(unsigned)B + 1, kHistB, 0, st>>>(b);
+  HIPCHK(hipGetLastError());
+  return USAP_OK;
+}
+
 int rebuild_M(usap_engine* e) {
   const int32_t B = e->B;
   hipStream_t st = e->stream;
   ev_rec(e, 0);
+  if (B <= kHistB) {
+    if (int rc = build_hist(e)) return rc;
+    ev_rec(e, 1);
+    if (e->prof) {
+      HIPCHK(hipStreamSynchronize(st));
+      prof_add(e, USAP_K_BUILD, ev_ms(e, 0, 1), 1, 0.0);
+    }
+    e->rebuilds++;
+    return USAP_OK;
+  }
   {
     ClearArgs c;
     int32_t* arr[kClearArrays] = {e->d_out, e->d_in, e->ecnt_out, e->ecnt_in,
@@ -4078,21 +4264,11 @@ int rebuild_M(usap_engine* e) {
   HIPCHK(hipMemcpyAsync(&tot, e->M.off + B, sizeof(int64_t), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
   DevSpM& m = e->M;
-  m.total = tot;
-  m.slack = e->p.slab_slack;
+  if (int rc = reserve_pool(e, tot)) return rc;
   // every row direct-mapped (cap B each; a hashed row's cap is below B/8):
   // no insert probes, so no row ever needs growth or an increment parked until
   // the next rebuild, and k_grow only has the batch's error flags to fold
   e->all_direct = tot == (int64_t)B * B;
-  if (3 * m.total > m.P) {  // two thirds of the pool is headroom for rows that grow
-    dfree(e, m.key);
-    dfree(e, m.cnt);
-    const int64_t P = 3 * m.total + (int64_t)4 * B + 4096;
-    m.P = 0;
-    if (int rc = dalloc(e, &m.key, (size_t)P)) return rc;
-    if (int rc = dalloc(e, &m.cnt, (size_t)P)) return rc;
-    m.P = P;
-  }
   if (m.total > 0) k_fill<<<std::min<int64_t>(blocks_for(m.total, 256), 8192), 256, 0, st>>>(
       e->all_direct ? nullptr : m.key, m.cnt, m.total);
   k_reset_grow<<<blocks_for(kGrowBlocks, 256), 256, 0, st>>>(m.gst, (unsigned long long)m.total);
@@ -4105,9 +4281,6 @@ int rebuild_M(usap_engine* e) {
     if (maybe_single && nonsingle == 0)
       k_build_single<<<blocks_for(e->N, kNodalWaves), kWave * kNodalWaves, 0, st>>>(
           gview(e), e->labels, view(e->M, B), e->big_off, e->big_tab, e->build_flags);
-    else if (B <= kSmallB)
-      k_insert_small<<<256, 256, 0, st>>>(e->E, e->out_src, e->out_idx, e->out_w, e->labels,
-                                          view(e->M, B));
     else if (B <= kPairSortB) {
       if (int rc = build_by_pairs(e)) return rc;
     } else if (B < kRowBuildB) {
@@ -4242,6 +4415,7 @@ int usap_destroy(usap_engine* e) {
     dfree(e, e->pair_val[i]);
   }
   dfree(e, e->pair_tmp);
+  dfree(e, e->hist);
   dfree(e, e->lam);
   dfree(e, e->labels);
   dfree(e, e->d_out);
@@ -4907,7 +5081,9 @@ int usap_set_labels(usap_engine* e, const int32_t* labels, int32_t B) {
   e->B = B;
   e->has_labels = true;
   e->merge_B = -1;
-  return rebuild_M(e);
+  if (int rc = rebuild_M(e)) return rc;
+  HIPCHK(hipStreamSynchronize(e->stream));  // the labels are the caller's
+  return USAP_OK;
 }
 
 int usap_get_labels(usap_engine* e, int32_t* out) {
@@ -5242,7 +5418,9 @@ int usap_merge_apply(usap_engine* e, int32_t B_to_merge, int32_t* B_new) {
   e->B = B - B_to_merge;
   e->merge_B = -1;
   if (B_new) *B_new = e->B;
-  return rebuild_M(e);
+  if (int rc = rebuild_M(e)) return rc;
+  HIPCHK(hipStreamSynchronize(st));  // `map` is released on return
+  return USAP_OK;
 }
 
 }  // extern "C"
