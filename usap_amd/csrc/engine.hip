@@ -1390,9 +1390,11 @@ __global__ void k_reset_grow(GrowState* g, unsigned long long used) {
   }
 }
 
-__global__ void k_relabel(int32_t N, int32_t* labels, const int32_t* __restrict__ map) {
+// short_of: the carry-out ran out of candidates, the labels stay.
+__global__ void k_relabel(int32_t N, int32_t* labels, const int32_t* __restrict__ map,
+                          const int32_t* short_of) {
   const int32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-  if (x < N) labels[x] = map[labels[x]];
+  if (x < N && *short_of == 0) labels[x] = map[labels[x]];
 }
 
 // ---------------------------------------------------------------------------
@@ -1524,6 +1526,252 @@ __global__ void k_sort_hi(int32_t B, const long* __restrict__ hi, const int32_t*
                           unsigned long long* key) {
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < B) key[i] = (unsigned long long)hi[perm[i]] ^ (1ull << 63);
+}
+
+// Carry-out (graph_parallel.hpp:1225-1279) on the device.  The reference goes
+// through the blocks in order and links block i to the current block of its
+// target best[i], unless that is i itself, until B_to_merge links are made.
+// Only i's own turn links i, so a link fails exactly when it would close a
+// cycle of i -> best[i]: each component of that functional graph has one cycle,
+// and its member that comes last in the order stays.  So:
+//   f^(2^K) maps every block onto a cycle (2^K >= B), and onto all of them;
+//   the largest order among i, f(i), ..., by the same doubling, is i's own on
+//   a cycle exactly at its last member;
+//   the links made are the first B_to_merge successes in the order (a scan);
+//   the roots by pointer jumping over them, then the surviving labels ranked
+//   ascending.
+// The host's loop with its copies took 4 ms at B = 200000 and 60 us and a host
+// wait more at B = 50.
+struct CarryArgs {
+  int32_t B, B_to_merge;
+  const int32_t* best;
+  const long* hi;            // dS words (k_carry_one up to kCarryRank blocks)
+  const unsigned long* lo;
+  const int32_t* order;      // blocks by (dS, id), above that
+  const int32_t* bsize;
+  int32_t* map;
+  int32_t* short_of;         // 1: fewer than B_to_merge links can be made
+  int32_t* host_short;       // the same, in the host's memory
+};
+
+constexpr int kCarryThreads = 1024;
+constexpr int kCarryRank = 1024;  // blocks ranked by comparing all pairs
+constexpr int kCarryOne = 8192;   // blocks one workgroup carries out in its LDS
+
+// Inclusive scan over the workgroup of each thread's own value; the total in
+// *total for every thread.
+__device__ __forceinline__ int32_t block_scan(int32_t v, int32_t* s_w, int32_t* total) {
+  const int w = threadIdx.x / kWave, nw = blockDim.x / kWave;
+  const int32_t inc = (int32_t)wave_incl_scan32((uint32_t)v);
+  __syncthreads();
+  if (lane_id() == kWave - 1) s_w[w] = inc;
+  __syncthreads();
+  int32_t before = 0, all = 0;
+  for (int i = 0; i < nw; ++i) {
+    if (i < w) before += s_w[i];
+    all += s_w[i];
+  }
+  *total = all;
+  return before + inc;
+}
+
+template <int kMax>
+__global__ __launch_bounds__(kCarryThreads) void k_carry_one(CarryArgs a) {
+  constexpr int kI = kMax / kCarryThreads;  // blocks per thread: t + k * kCarryThreads
+  __shared__ int32_t s_p[kMax], s_m[kMax], s_a[kMax];
+  __shared__ int32_t s_w[kCarryThreads / kWave];
+  const int32_t B = a.B, t = threadIdx.x;
+  int32_t rank[kI], f[kI], p[kI], m[kI];
+  if (kMax <= kCarryRank) {
+    __shared__ long s_hi[kCarryRank];
+    __shared__ unsigned long s_lo[kCarryRank];
+    if (t < B) {
+      s_hi[t] = a.hi[t];
+      s_lo[t] = a.lo[t];
+    }
+    __syncthreads();
+    rank[0] = 0;
+    if (t < B) {
+      const long h = s_hi[t];
+      const unsigned long l = s_lo[t];
+      for (int32_t j = 0; j < B; ++j) {
+        const bool before = s_hi[j] < h || (s_hi[j] == h && (s_lo[j] < l || (s_lo[j] == l && j < t)));
+        rank[0] += before;
+      }
+    }
+  } else {
+    for (int32_t j = t; j < B; j += kCarryThreads) s_a[a.order[j]] = j;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kI; ++k)
+      rank[k] = t + k * kCarryThreads < B ? s_a[t + k * kCarryThreads] : 0;
+    __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < kI; ++k) {
+    const int32_t i = t + k * kCarryThreads;
+    if (i < B) {
+      f[k] = p[k] = s_p[i] = a.best[i];
+      m[k] = s_m[i] = rank[k];
+      s_a[i] = 0;
+    }
+  }
+  for (int32_t w = 1; w < B; w <<= 1) {
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kI; ++k)
+      if (t + k * kCarryThreads < B) {
+        m[k] = max(m[k], s_m[p[k]]);
+        p[k] = s_p[p[k]];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kI; ++k)
+      if (t + k * kCarryThreads < B) {
+        s_p[t + k * kCarryThreads] = p[k];
+        s_m[t + k * kCarryThreads] = m[k];
+      }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kI; ++k)
+    if (t + k * kCarryThreads < B) s_a[p[k]] = 1;
+  __syncthreads();
+  bool link[kI];
+#pragma unroll
+  for (int k = 0; k < kI; ++k) {
+    const int32_t i = t + k * kCarryThreads;
+    link[k] = false;
+    if (i < B) {
+      link[k] = !(s_a[i] && m[k] == rank[k]);
+      s_p[rank[k]] = link[k];
+    }
+  }
+  __syncthreads();
+  // successes up to each rank: thread t scans ranks [t * kI, (t + 1) * kI)
+  int32_t mine = 0, total;
+#pragma unroll
+  for (int k = 0; k < kI; ++k)
+    if (t * kI + k < B) mine += s_p[t * kI + k];
+  int32_t run = block_scan(mine, s_w, &total) - mine;
+#pragma unroll
+  for (int k = 0; k < kI; ++k)
+    if (t * kI + k < B) {
+      run += s_p[t * kI + k];
+      s_m[t * kI + k] = run;
+    }
+  __syncthreads();
+  const bool fails = total < a.B_to_merge;
+  if (t == 0) {
+    *a.short_of = fails;
+    *a.host_short = fails;
+  }
+  if (fails) return;  // the same for every thread
+#pragma unroll
+  for (int k = 0; k < kI; ++k) {
+    const int32_t i = t + k * kCarryThreads;
+    if (i < B) {
+      s_p[i] = link[k] && s_m[rank[k]] <= a.B_to_merge ? f[k] : i;
+      s_a[i] = 0;
+    }
+  }
+  for (int32_t w = 1; w < B; w <<= 1) {
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kI; ++k)  // in place: what is read is an ancestor at least as far
+      if (t + k * kCarryThreads < B)
+        s_p[t + k * kCarryThreads] = s_p[s_p[t + k * kCarryThreads]];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kI; ++k) {
+    const int32_t i = t + k * kCarryThreads;
+    if (i < B && a.bsize[i] > 0) s_a[s_p[i]] = 1;
+  }
+  __syncthreads();
+  mine = 0;
+#pragma unroll
+  for (int k = 0; k < kI; ++k)
+    if (t * kI + k < B) mine += s_a[t * kI + k];
+  run = block_scan(mine, s_w, &total) - mine;
+#pragma unroll
+  for (int k = 0; k < kI; ++k)
+    if (t * kI + k < B) {
+      s_m[t * kI + k] = run;
+      run += s_a[t * kI + k];
+    }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kI; ++k) {
+    const int32_t i = t + k * kCarryThreads;
+    if (i < B) a.map[i] = s_a[s_p[i]] ? s_m[s_p[i]] : 0;
+  }
+}
+
+// The same steps over the whole GPU (more than kCarryOne blocks).
+__global__ void k_carry_init(int32_t B, const int32_t* __restrict__ order,
+                             const int32_t* __restrict__ best, int32_t* rank, int2* pm,
+                             int32_t* cyc) {
+  const int32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= B) return;
+  const int32_t i = order[j];
+  rank[i] = j;
+  pm[i] = make_int2(best[i], j);
+  cyc[i] = 0;
+}
+
+__global__ void k_carry_jump(int32_t B, const int2* __restrict__ in, int2* __restrict__ out) {
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= B) return;
+  const int2 x = in[i];
+  const int2 y = in[x.x];
+  out[i] = make_int2(y.x, max(x.y, y.y));
+}
+
+__global__ void k_carry_cycle(int32_t B, const int2* __restrict__ pm, int32_t* cyc) {
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < B) cyc[pm[i].x] = 1;
+}
+
+__global__ void k_carry_success(int32_t B, const int2* __restrict__ pm,
+                                const int32_t* __restrict__ cyc, const int32_t* __restrict__ rank,
+                                int32_t* succ) {
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < B) succ[rank[i]] = !(cyc[i] && pm[i].y == rank[i]);
+}
+
+__global__ void k_carry_link(int32_t B, int32_t B_to_merge, const int32_t* __restrict__ best,
+                             const int32_t* __restrict__ rank, const int32_t* __restrict__ succ,
+                             const int32_t* __restrict__ scan, int32_t* par, int32_t* alive,
+                             int32_t* short_of, int32_t* host_short) {
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= B) return;
+  const int32_t r = rank[i];
+  par[i] = succ[r] && scan[r] <= B_to_merge ? best[i] : i;
+  alive[i] = 0;
+  if (i == 0) {
+    const int32_t fails = scan[B - 1] < B_to_merge;
+    *short_of = fails;
+    *host_short = fails;
+  }
+}
+
+__global__ void k_carry_root(int32_t B, int32_t* par) {
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < B) par[i] = par[par[i]];  // in place: an ancestor at least as far
+}
+
+__global__ void k_carry_alive(int32_t B, const int32_t* __restrict__ bsize,
+                              const int32_t* __restrict__ par, int32_t* alive) {
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < B && bsize[i] > 0) alive[par[i]] = 1;
+}
+
+__global__ void k_carry_map(int32_t B, const int32_t* __restrict__ par,
+                            const int32_t* __restrict__ alive, const int32_t* __restrict__ before,
+                            int32_t* map) {
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < B) map[i] = alive[par[i]] ? before[par[i]] : 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -3870,7 +4118,10 @@ struct usap_engine {
   uint64_t g_epoch = 0;
   uint64_t epoch = 0;  // bumped by every device allocation (pointers may change)
   int64_t graph_captures = 0;
-  int32_t* build_flags = nullptr;  // [0] build overflow flags, [1] blocks holding != 1 node, [2] distinct block pairs
+  int32_t* build_flags = nullptr;  // [0] build overflow flags, [1] blocks holding != 1 node,
+                                   // [2] distinct block pairs, [3] carry-out out of candidates
+  int32_t* h_short = nullptr;      // the last in pinned host memory, and its device address
+  int32_t* d_short = nullptr;
   int32_t* hist = nullptr;  // counts of the build by histograms
   int64_t hist_cap = 0;
   uint32_t* pair_key[2] = {nullptr, nullptr};  // block-pair builds [E]
@@ -4466,6 +4717,7 @@ int usap_destroy(usap_engine* e) {
   dfree(e, e->tstamp);
   pin_put(e->h_sweep, sizeof(Sweep));
   for (int i = 0; i < 2; ++i) pin_put(e->h_chunk[i], sizeof(Sweep));
+  pin_put(e->h_short, 64);
   dfree(e, e->big_off);
   dfree(e, e->big_tab);
   dfree(e, e->ent_part);
@@ -4822,6 +5074,8 @@ int append_edges(usap_engine* e, int64_t n, const int32_t* src, const int32_t* d
   return USAP_OK;
 }
 
+constexpr size_t kShortBytes = 64;  // usap_engine::h_short
+
 // Device arrays sized by N only (labels, degrees, row tables, batch buffers).
 int alloc_state(usap_engine* e) {
   const int32_t N = e->N;
@@ -4854,13 +5108,15 @@ int alloc_state(usap_engine* e) {
   TRY(dalloc(e, &e->status, 1));
   TRY(dalloc(e, &e->part, blocks_for(N, kNodalWaves)));
   TRY(dalloc(e, &e->sweep, 1));
-  TRY(dalloc(e, &e->build_flags, 3));
+  TRY(dalloc(e, &e->build_flags, 4));
   TRY(dalloc(e, &e->ent_part, 2 * kEntropyBlocks));
   e->h_sweep = (Sweep*)pin_get(sizeof(Sweep));
   e->h_ent_part = (long*)pin_get(sizeof(long) * 2 * kEntropyBlocks);
   for (int i = 0; i < 2; ++i) e->h_chunk[i] = (Sweep*)pin_get(sizeof(Sweep));
-  if (!e->h_sweep || !e->h_ent_part || !e->h_chunk[0] || !e->h_chunk[1])
+  e->h_short = (int32_t*)pin_get(kShortBytes);
+  if (!e->h_sweep || !e->h_ent_part || !e->h_chunk[0] || !e->h_chunk[1] || !e->h_short)
     return set_err(e, USAP_ENOMEM, "hipHostMalloc");
+  HIPCHK(hipHostGetDevicePointer((void**)&e->d_short, e->h_short, 0));
   hipStream_t st = e->stream;
   HIPCHK(hipMemsetAsync(e->status, 0, sizeof(Status), st));
   HIPCHK(hipMemsetAsync(e->sweep, 0, sizeof(Sweep), st));
@@ -5342,85 +5598,112 @@ int usap_merge_result_fx(usap_engine* e, int32_t* best_s, int64_t* hi, uint64_t*
   return USAP_OK;
 }
 
-int usap_merge_apply(usap_engine* e, int32_t B_to_merge, int32_t* B_new) {
-  if (int rc = check_engine(e)) return rc;
+}  // extern "C"
+
+namespace {
+
+// e->map and build_flags[3] (and *h_short) for B_to_merge merges of the last
+// proposal round.  The arrays of the next rebuild serve as scratch.
+int carry_out(usap_engine* e, int32_t B_to_merge) {
   const int32_t B = e->B;
-  if (e->merge_B != B) return set_err(e, USAP_ESTATE, "merge_apply without merge_propose");
-  if (B_to_merge < 0 || B_to_merge >= B) return set_err(e, USAP_EINVAL, "B_to_merge out of range");
-  std::vector<int32_t> best((size_t)B), bsize((size_t)B), order((size_t)B);
   hipStream_t st = e->stream;
-  // order by (dS, block id) on the device: the reference sorts by dS with an
-  // unstable sort (graph_parallel.hpp:1230)
+  CarryArgs a;
+  a.B = B;
+  a.B_to_merge = B_to_merge;
+  a.best = e->best_s;
+  a.hi = e->best_hi;
+  a.lo = e->best_lo;
+  a.order = nullptr;
+  a.bsize = e->bsize;
+  a.map = e->map;
+  a.short_of = e->build_flags + 3;
+  a.host_short = e->d_short;
+  if (B <= kCarryRank) {
+    k_carry_one<kCarryRank><<<1, kCarryThreads, 0, st>>>(a);
+    HIPCHK(hipGetLastError());
+    return USAP_OK;
+  }
+  // order by (dS, block id): the reference sorts by dS with an unstable sort
+  // (graph_parallel.hpp:1230)
   if (!e->sort_idx[0]) {
     for (int i = 0; i < 2; ++i) {
       if (int rc = dalloc(e, &e->sort_key[i], e->N)) return rc;
       if (int rc = dalloc(e, &e->sort_idx[i], e->N)) return rc;
     }
   }
-  size_t bytes = 0;
+  size_t bytes = 0, scan_bytes = 0;
   HIPCHK(rocprim::radix_sort_pairs(nullptr, bytes, e->sort_key[0], e->sort_key[1], e->sort_idx[0],
                                    e->sort_idx[1], (size_t)B, 0, 64, st));
+  int32_t *cyc = e->ecnt_out, *succ = e->ecnt_in, *scan = e->bl_off, *alive = e->bl_cur,
+          *par = e->bl_nodes;
+  HIPCHK(rocprim::inclusive_scan(nullptr, scan_bytes, succ, scan, (size_t)B,
+                                 rocprim::plus<int32_t>(), st));
+  bytes = std::max(bytes, scan_bytes);
+  HIPCHK(rocprim::exclusive_scan(nullptr, scan_bytes, alive, scan, (int32_t)0, (size_t)B,
+                                 rocprim::plus<int32_t>(), st));
+  bytes = std::max(bytes, scan_bytes);
   if (bytes > e->sort_tmp_bytes) {
     dfree(e, e->sort_tmp);
     if (int rc = dalloc_raw(e, &e->sort_tmp, bytes)) return rc;
     e->sort_tmp_bytes = bytes;
   }
-  k_sort_init<<<blocks_for(B, 256), 256, 0, st>>>(B, e->best_lo, e->sort_key[0], e->sort_idx[0]);
+  const unsigned g = blocks_for(B, 256);
+  k_sort_init<<<g, 256, 0, st>>>(B, e->best_lo, e->sort_key[0], e->sort_idx[0]);
   bytes = e->sort_tmp_bytes;
   HIPCHK(rocprim::radix_sort_pairs(e->sort_tmp, bytes, e->sort_key[0], e->sort_key[1],
                                    e->sort_idx[0], e->sort_idx[1], (size_t)B, 0, 64, st));
-  k_sort_hi<<<blocks_for(B, 256), 256, 0, st>>>(B, e->best_hi, e->sort_idx[1], e->sort_key[0]);
+  k_sort_hi<<<g, 256, 0, st>>>(B, e->best_hi, e->sort_idx[1], e->sort_key[0]);
   bytes = e->sort_tmp_bytes;
   HIPCHK(rocprim::radix_sort_pairs(e->sort_tmp, bytes, e->sort_key[0], e->sort_key[1],
                                    e->sort_idx[1], e->sort_idx[0], (size_t)B, 0, 64, st));
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(order.data(), e->sort_idx[0], sizeof(int32_t) * B, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipMemcpyAsync(best.data(), e->best_s, sizeof(int32_t) * B, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipMemcpyAsync(bsize.data(), e->bsize, sizeof(int32_t) * B, hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
-  // greedy merges: block_map of graph_parallel.hpp:1236-1257 as a union-find
-  // whose root is the representative (the merge target's current block)
-  std::vector<int32_t> parent((size_t)B);
-  std::iota(parent.begin(), parent.end(), 0);
-  auto find = [&](int32_t x) {
-    int32_t r = x;
-    while (parent[r] != r) r = parent[r];
-    while (parent[x] != r) {
-      const int32_t n = parent[x];
-      parent[x] = r;
-      x = n;
-    }
-    return r;
-  };
-  int32_t num = 0, counter = 0;
-  while (num < B_to_merge) {
-    if (counter >= B) return set_err(e, USAP_EINFEASIBLE, "carry-out ran out of candidate merges");
-    const int32_t from = order[counter++];
-    const int32_t to = find(best[from]);
-    if (to != from) {
-      parent[from] = to;
-      ++num;
-    }
+  a.order = e->sort_idx[0];
+  if (B <= kCarryOne) {
+    k_carry_one<kCarryOne><<<1, kCarryThreads, 0, st>>>(a);
+    HIPCHK(hipGetLastError());
+    return USAP_OK;
   }
-  // compaction: surviving labels ranked ascending (graph_parallel.hpp:1260-1277)
-  std::vector<char> alive((size_t)B, 0);
-  for (int32_t b = 0; b < B; ++b)
-    if (bsize[b] > 0) alive[find(b)] = 1;
-  std::vector<int32_t> rank((size_t)B, -1);
-  int32_t next = 0;
-  for (int32_t b = 0; b < B; ++b)
-    if (alive[b]) rank[b] = next++;
-  std::vector<int32_t> map((size_t)B);
-  for (int32_t b = 0; b < B; ++b) map[b] = rank[find(b)] < 0 ? 0 : rank[find(b)];
-  HIPCHK(hipMemcpyAsync(e->map, map.data(), sizeof(int32_t) * B, hipMemcpyHostToDevice, st));
-  k_relabel<<<blocks_for(e->N, 256), 256, 0, st>>>(e->N, e->labels, e->map);
+  int32_t* rank = e->sort_idx[1];
+  int2* pm[2] = {reinterpret_cast<int2*>(e->sort_key[0]), reinterpret_cast<int2*>(e->sort_key[1])};
+  k_carry_init<<<g, 256, 0, st>>>(B, a.order, a.best, rank, pm[0], cyc);
+  int cur = 0;
+  for (int64_t w = 1; w < B; w <<= 1, cur ^= 1)
+    k_carry_jump<<<g, 256, 0, st>>>(B, pm[cur], pm[cur ^ 1]);
+  k_carry_cycle<<<g, 256, 0, st>>>(B, pm[cur], cyc);
+  k_carry_success<<<g, 256, 0, st>>>(B, pm[cur], cyc, rank, succ);
+  bytes = e->sort_tmp_bytes;
+  HIPCHK(rocprim::inclusive_scan(e->sort_tmp, bytes, succ, scan, (size_t)B,
+                                 rocprim::plus<int32_t>(), st));
+  k_carry_link<<<g, 256, 0, st>>>(B, B_to_merge, a.best, rank, succ, scan, par, alive, a.short_of,
+                                  a.host_short);
+  for (int64_t w = 1; w < B; w <<= 1) k_carry_root<<<g, 256, 0, st>>>(B, par);
+  k_carry_alive<<<g, 256, 0, st>>>(B, a.bsize, par, alive);
+  bytes = e->sort_tmp_bytes;
+  HIPCHK(rocprim::exclusive_scan(e->sort_tmp, bytes, alive, scan, (int32_t)0, (size_t)B,
+                                 rocprim::plus<int32_t>(), st));
+  k_carry_map<<<g, 256, 0, st>>>(B, par, alive, scan, a.map);
   HIPCHK(hipGetLastError());
+  return USAP_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int usap_merge_apply(usap_engine* e, int32_t B_to_merge, int32_t* B_new) {
+  if (int rc = check_engine(e)) return rc;
+  const int32_t B = e->B;
+  if (e->merge_B != B) return set_err(e, USAP_ESTATE, "merge_apply without merge_propose");
+  if (B_to_merge < 0 || B_to_merge >= B) return set_err(e, USAP_EINVAL, "B_to_merge out of range");
+  hipStream_t st = e->stream;
+  if (int rc = carry_out(e, B_to_merge)) return rc;
+  k_relabel<<<blocks_for(e->N, 256), 256, 0, st>>>(e->N, e->labels, e->map, e->build_flags + 3);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(st));
+  if (*e->h_short) return set_err(e, USAP_EINFEASIBLE, "carry-out ran out of candidate merges");
   e->B = B - B_to_merge;
   e->merge_B = -1;
   if (B_new) *B_new = e->B;
-  if (int rc = rebuild_M(e)) return rc;
-  HIPCHK(hipStreamSynchronize(st));  // `map` is released on return
-  return USAP_OK;
+  return rebuild_M(e);
 }
 
 }  // extern "C"
