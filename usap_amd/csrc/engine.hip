@@ -1467,7 +1467,8 @@ __global__ void k_iota(int64_t n, int32_t* v) {
 // data_S = -(sum_ab L(M_ab) - sum_a L(d_out[a]) - sum_b L(d_in[b]))
 // ---------------------------------------------------------------------------
 
-__device__ void block_store(Acc v, long* out) {
+// Sum over the workgroup's threads (every thread calls); thread 0 returns it.
+__device__ __forceinline__ i128 block_sum(Acc v) {
   __shared__ long s_h[16], s_l[16];
   v.h = wave_sum(v.h);
   v.l = wave_sum(v.l);
@@ -1477,16 +1478,82 @@ __device__ void block_store(Acc v, long* out) {
     s_l[w] = v.l;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    Acc t{0, 0};
+  Acc t{0, 0};
+  if (threadIdx.x == 0)
     for (int i = 0; i < (int)(blockDim.x / kWave); ++i) {
       t.h += s_h[i];
       t.l += s_l[i];
     }
-    const i128 x = acc_value(t);
+  return acc_value(t);
+}
+
+__device__ void block_store(Acc v, long* out) {
+  const i128 x = block_sum(v);
+  if (threadIdx.x == 0) {
     out[0] = (long)(x >> 64);
     out[1] = (long)(unsigned long)(u128)x;
   }
+}
+
+// The same for int128 partials.
+__device__ __forceinline__ i128 block_sum128(i128 t) {
+  __shared__ long s_hi[16];
+  __shared__ unsigned long s_lo[16];
+  t = wave_sum128(t);
+  const int w = threadIdx.x / kWave;
+  if (lane_id() == 0) {
+    s_hi[w] = (long)(t >> 64);
+    s_lo[w] = (unsigned long)(u128)t;
+  }
+  __syncthreads();
+  i128 tot = 0;
+  if (threadIdx.x == 0)
+    for (int i = 0; i < (int)(blockDim.x / kWave); ++i)
+      tot += (i128)(((u128)(unsigned long)s_hi[i] << 64) | (u128)s_lo[i]);
+  return tot;
+}
+
+// minus data_S of a state, for one workgroup: from k_entropy's nparts
+// partials, or, M all direct with at most kEntropyOne slots, from M itself
+// (one launch and one pass over the partials less).
+constexpr int32_t kEntropyOne = 16384;
+struct EntropyIn {
+  const long* part;
+  int32_t nparts;  // 0: from M
+  const Cnt* cnt;
+  const int32_t *d_out, *d_in;
+  int32_t B;
+  const int64_t* lam;
+};
+
+__device__ __forceinline__ i128 block_entropy(const EntropyIn& a) {
+  if (a.nparts > 0) {
+    i128 t = 0;
+    for (int32_t i = threadIdx.x; i < a.nparts; i += blockDim.x)
+      t += (i128)(((u128)(unsigned long)a.part[2 * i] << 64) | (u128)(unsigned long)a.part[2 * i + 1]);
+    return block_sum128(t);
+  }
+  Acc acc{0, 0};
+  const int32_t n = a.B * a.B;
+  constexpr int kQ = 8;
+  for (int32_t i0 = threadIdx.x; i0 < n; i0 += kQ * blockDim.x) {
+    int32_t v[kQ];
+    int64_t L[kQ];
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      const int32_t i = i0 + q * (int32_t)blockDim.x;
+      v[q] = i < n ? a.cnt[i].o : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) L[q] = a.lam[v[q]];
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) acc_add(acc, v[q], L[q]);
+  }
+  for (int32_t b = threadIdx.x; b < a.B; b += blockDim.x) {
+    sub_L(acc, a.lam, a.d_out[b]);
+    sub_L(acc, a.lam, a.d_in[b]);
+  }
+  return block_sum(acc);
 }
 
 __global__ __launch_bounds__(256) void k_entropy(const Cnt* __restrict__ cnt,
@@ -2270,22 +2337,6 @@ __device__ __forceinline__ void list_entry(const GraphView& g, int64_t o0, int64
 __device__ __forceinline__ void lds_order() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
-}
-
-// The Philox words of nodes [beg, end), 4 per node, batch i = [beg + i * batch,
-// ...) from stream sweep->stream0 + i: one thread per node, where every lane of
-// a node's k_nodal wavefront would compute the same 80 multiplies.
-__global__ void k_draw(int32_t beg, int32_t end, int32_t batch, uint64_t seed, const Sweep* sweep,
-                       uint64_t* __restrict__ draws) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (beg + i >= end) return;
-  const int64_t n = beg + i;
-  uint64_t x[4];
-  usap::philox4x64((uint64_t)n, 0, sweep->stream0 + (uint64_t)(i / batch), usap::kTagNodal, seed, 0,
-                   x);
-  ulonglong2* q = reinterpret_cast<ulonglong2*>(draws + 4 * n);
-  q[0] = make_ulonglong2(x[0], x[1]);
-  q[1] = make_ulonglong2(x[2], x[3]);
 }
 
 // What moving node n from r to s changes outside the neighbour blocks: the
@@ -3103,28 +3154,83 @@ __device__ double fx_to_double_dev(i128 v) {
   return neg ? -d : d;
 }
 
-// A sweep's starting S from k_entropy's per-workgroup partials, stored in
-// the device sweep state: the exact int128 sum, then model + data in the same
-// IEEE double operations as usap_entropy on the host.
-__global__ __launch_bounds__(256) void k_entropy_to_sweep(const long* __restrict__ part,
-                                                          int32_t nparts, double model, Sweep* sw) {
-  __shared__ long s_hi[4];
-  __shared__ unsigned long s_lo[4];
-  i128 t = 0;
-  for (int32_t i = threadIdx.x; i < nparts; i += blockDim.x)
-    t += (i128)(((u128)(unsigned long)part[2 * i] << 64) | (u128)(unsigned long)part[2 * i + 1]);
-  t = wave_sum128(t);
-  const int w = threadIdx.x / kWave;
-  if (lane_id() == 0) {
-    s_hi[w] = (long)(t >> 64);
-    s_lo[w] = (unsigned long)(u128)t;
+// A sweep's beginning.  Workgroup 0 stores its state: `init`, and in S, when
+// from_state is set, the MDL of the current state, model + data in the same
+// IEEE double operations as usap_entropy on the host.  The others make the
+// Philox words of nodes [beg, end), 4 per node, batch i = [beg + i * batch, ...)
+// from stream init.stream0 + i: one thread per node, where every lane of a
+// node's k_nodal wavefront would compute the same 80 multiplies.
+constexpr int kBeginThreads = 1024;
+struct BeginArgs {
+  Sweep init;
+  Sweep* sweep;
+  int32_t from_state;
+  double model;
+  EntropyIn ent;
+  int32_t beg, end, batch;
+  uint64_t seed;
+  uint64_t* draws;
+};
+
+__device__ __forceinline__ void draw_node(int64_t n, uint64_t stream, uint64_t seed,
+                                          uint64_t* draws) {
+  uint64_t x[4];
+  usap::philox4x64((uint64_t)n, 0, stream, usap::kTagNodal, seed, 0, x);
+  ulonglong2* q = reinterpret_cast<ulonglong2*>(draws + 4 * n);
+  q[0] = make_ulonglong2(x[0], x[1]);
+  q[1] = make_ulonglong2(x[2], x[3]);
+}
+
+__global__ __launch_bounds__(kBeginThreads) void k_begin(BeginArgs a) {
+  if (blockIdx.x == 0) {
+    double S = a.init.S;
+    if (a.from_state) S = a.model + fx_to_double_dev(-block_entropy(a.ent));
+    if (threadIdx.x == 0) {
+      *a.sweep = a.init;
+      a.sweep->S = S;
+    }
+    return;
+  }
+  const int64_t i = (int64_t)(blockIdx.x - 1) * kBeginThreads + threadIdx.x;
+  if (a.beg + i < a.end)
+    draw_node(a.beg + i, a.init.stream0 + (uint64_t)(i / a.batch), a.seed, a.draws);
+}
+
+// The words alone, from the state's stream (captured sweeps).
+__global__ void k_draw(int32_t beg, int32_t end, int32_t batch, uint64_t seed, const Sweep* sweep,
+                       uint64_t* __restrict__ draws) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (beg + i < end) draw_node(beg + i, sweep->stream0 + (uint64_t)(i / batch), seed, draws);
+}
+
+// The batches' error and rebuild flags folded into the sweep's state: errors
+// override convergence, which overrides a rebuild request, as the decision
+// comes after the batch.
+__device__ __forceinline__ void fold_flags(Status* status, Sweep* sweep) {
+  const int32_t f = status->flags;
+  if (f) {
+    atomicOr(&sweep->flags, f);
+    if (f & (kFlagMissing | kFlagNegative))
+      atomicExch(&sweep->stop, 3);
+    else if (f & kFlagFull)
+      atomicCAS(&sweep->stop, 0, 2);
+    status->flags = 0;
+  }
+}
+
+// The state after a sweep, or after a chunk of its batches, in the host's
+// pinned memory (a copy would be a launch of the runtime's own kernel).
+__global__ __launch_bounds__(kWave) void k_finish(Status* status, Sweep* sweep, Sweep* host) {
+  if (threadIdx.x == 0) {
+    fold_flags(status, sweep);
+    __threadfence();
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    i128 tot = 0;
-    for (int i = 0; i < (int)(blockDim.x / kWave); ++i)
-      tot += (i128)(((u128)(unsigned long)s_hi[i] << 64) | (u128)s_lo[i]);
-    sw->S = model + fx_to_double_dev(-tot);
+  static_assert(sizeof(Sweep) % 8 == 0 && sizeof(Sweep) / 8 <= kWave, "one word per thread");
+  if (threadIdx.x < sizeof(Sweep) / 8) {
+    unsigned long long* w = reinterpret_cast<unsigned long long*>(sweep) + threadIdx.x;
+    reinterpret_cast<unsigned long long*>(host)[threadIdx.x] =
+        __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -3942,19 +4048,9 @@ __global__ __launch_bounds__(256) void k_grow(GrowArgs ga) {
   const int w = threadIdx.x / kWave;
   bool any = false;  // thread 0: s_al is loaded
   if (ga.tstamp && threadIdx.x == 0) ga.tstamp[blockIdx.x] = wall_clock64();
-  // the batch's flags (raised by its k_nodal and k_apply, both complete):
-  // errors override convergence, which overrides a rebuild request, as the
-  // decision comes after the batch
+  // the batch's flags (raised by its k_nodal and k_apply, both complete)
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    const int32_t f = ga.status->flags;
-    if (f) {
-      atomicOr(&ga.sweep->flags, f);
-      if (f & (kFlagMissing | kFlagNegative))
-        atomicExch(&ga.sweep->stop, 3);
-      else if (f & kFlagFull)
-        atomicCAS(&ga.sweep->stop, 0, 2);
-      ga.status->flags = 0;
-    }
+    fold_flags(ga.status, ga.sweep);
     g.gst->full += (unsigned long long)g.gst->ovf_n;
   }
   const int32_t per = (B + (int32_t)gridDim.x - 1) / (int32_t)gridDim.x;
@@ -4101,6 +4197,8 @@ struct usap_engine {
   Sweep* sweep = nullptr;     // device sweep state
   Sweep* h_sweep = nullptr;   // pinned host copy
   Sweep* h_chunk[2] = {nullptr, nullptr};  // sweep state after alternate launch chunks
+  Sweep* d_hsweep = nullptr;               // device addresses of the two
+  Sweep* d_hchunk[2] = {nullptr, nullptr};
   hipEvent_t chunk_ev[2] = {nullptr, nullptr};
   // reference-algorithm byte counts (profiling): drawn neighbour's block per
   // batch node, per-block batch stamps, device totals [nodal per-node,
@@ -4134,7 +4232,8 @@ struct usap_engine {
   int64_t max_list = 0;  // list entries of the largest node
   // entropy
   long* ent_part = nullptr;
-  long* h_ent_part = nullptr;
+  int64_t* h_fx = nullptr;  // usap_entropy's result in pinned host memory, and its device address
+  int64_t* d_fx = nullptr;
   // snapshots
   int32_t* snap_labels[kNumSnap] = {};
   int32_t snap_B[kNumSnap] = {};
@@ -4721,7 +4820,7 @@ int usap_destroy(usap_engine* e) {
   dfree(e, e->big_off);
   dfree(e, e->big_tab);
   dfree(e, e->ent_part);
-  pin_put(e->h_ent_part, sizeof(long) * 2 * kEntropyBlocks);
+  pin_put(e->h_fx, 64);
   for (int i = 0; i < kNumSnap; ++i) dfree(e, e->snap_labels[i]);
   if (e->stream) (void)hipStreamSynchronize(e->stream);
   {
@@ -5074,7 +5173,7 @@ int append_edges(usap_engine* e, int64_t n, const int32_t* src, const int32_t* d
   return USAP_OK;
 }
 
-constexpr size_t kShortBytes = 64;  // usap_engine::h_short
+constexpr size_t kShortBytes = 64;  // usap_engine::h_short, h_fx
 
 // Device arrays sized by N only (labels, degrees, row tables, batch buffers).
 int alloc_state(usap_engine* e) {
@@ -5111,12 +5210,16 @@ int alloc_state(usap_engine* e) {
   TRY(dalloc(e, &e->build_flags, 4));
   TRY(dalloc(e, &e->ent_part, 2 * kEntropyBlocks));
   e->h_sweep = (Sweep*)pin_get(sizeof(Sweep));
-  e->h_ent_part = (long*)pin_get(sizeof(long) * 2 * kEntropyBlocks);
+  e->h_fx = (int64_t*)pin_get(kShortBytes);
   for (int i = 0; i < 2; ++i) e->h_chunk[i] = (Sweep*)pin_get(sizeof(Sweep));
   e->h_short = (int32_t*)pin_get(kShortBytes);
-  if (!e->h_sweep || !e->h_ent_part || !e->h_chunk[0] || !e->h_chunk[1] || !e->h_short)
+  if (!e->h_sweep || !e->h_fx || !e->h_chunk[0] || !e->h_chunk[1] || !e->h_short)
     return set_err(e, USAP_ENOMEM, "hipHostMalloc");
   HIPCHK(hipHostGetDevicePointer((void**)&e->d_short, e->h_short, 0));
+  HIPCHK(hipHostGetDevicePointer((void**)&e->d_fx, e->h_fx, 0));
+  HIPCHK(hipHostGetDevicePointer((void**)&e->d_hsweep, e->h_sweep, 0));
+  for (int i = 0; i < 2; ++i)
+    HIPCHK(hipHostGetDevicePointer((void**)&e->d_hchunk[i], e->h_chunk[i], 0));
   hipStream_t st = e->stream;
   HIPCHK(hipMemsetAsync(e->status, 0, sizeof(Status), st));
   HIPCHK(hipMemsetAsync(e->sweep, 0, sizeof(Sweep), st));
@@ -5416,13 +5519,17 @@ int usap_get_M_coo(usap_engine* e, int64_t cap, int32_t* rows, int32_t* cols, in
 namespace {
 // k_entropy over the pool in use: about four slots per thread, at most
 // kEntropyBlocks workgroups (a scan of 1 GB pools at B = 250k is bound by the
-// loads in flight).  Returns the grid (the number of partials).
-int launch_entropy(usap_engine* e, long* part = nullptr) {
+// loads in flight).
+// No launch when one workgroup takes M itself (k_begin, k_entropy_out).
+EntropyIn launch_entropy(usap_engine* e, long* part) {
+  EntropyIn in{part, 0, e->M.cnt, e->d_out, e->d_in, e->B, e->lam};
+  if (e->all_direct && (int64_t)e->B * e->B <= kEntropyOne) return in;
   const int64_t work = std::max<int64_t>(e->M.P, e->B);
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(kEntropyBlocks, blocks_for(work, 1024)));
   k_entropy<<<grid, 256, 0, e->stream>>>(e->M.cnt, e->M.gst, e->d_out, e->d_in, e->B, e->lam,
-                                         e->M.P, part ? part : e->ent_part);
-  return grid;
+                                         e->M.P, part);
+  in.nparts = grid;
+  return in;
 }
 
 // ---- allocation-free MDL -----------------------------------------------------
@@ -5437,28 +5544,13 @@ constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 long* g_scratch_ptr[kMaxDevices] = {};
 
-// The MDL from k_entropy's nparts partials, into the caller's device memory
-// (S: model + data term; fx: the data term's int128 words, hi then lo): the
-// same integer sum and IEEE operations as usap_entropy on the host.
-__global__ __launch_bounds__(256) void k_entropy_out(const long* __restrict__ part, int32_t nparts,
-                                                     double model, double* S, int64_t* fx) {
-  __shared__ long s_hi[4];
-  __shared__ unsigned long s_lo[4];
-  i128 t = 0;
-  for (int32_t i = threadIdx.x; i < nparts; i += blockDim.x)
-    t += (i128)(((u128)(unsigned long)part[2 * i] << 64) | (u128)(unsigned long)part[2 * i + 1]);
-  t = wave_sum128(t);
-  const int w = threadIdx.x / kWave;
-  if (lane_id() == 0) {
-    s_hi[w] = (long)(t >> 64);
-    s_lo[w] = (unsigned long)(u128)t;
-  }
-  __syncthreads();
+// The MDL into the caller's device memory (S: model + data term; fx: the data
+// term's int128 words, hi then lo): the same integer sum and IEEE operations as
+// usap_entropy on the host.
+__global__ __launch_bounds__(kBeginThreads) void k_entropy_out(EntropyIn in, double model, double* S,
+                                                               int64_t* fx) {
+  const i128 data = -block_entropy(in);
   if (threadIdx.x == 0) {
-    i128 tot = 0;
-    for (int i = 0; i < (int)(blockDim.x / kWave); ++i)
-      tot += (i128)(((u128)(unsigned long)s_hi[i] << 64) | (u128)s_lo[i]);
-    const i128 data = -tot;
     if (S) *S = model + fx_to_double_dev(data);
     if (fx) {
       fx[0] = (int64_t)(data >> 64);
@@ -5496,17 +5588,13 @@ int usap_entropy(usap_engine* e, double* S, int64_t* hi, uint64_t* lo) {
   if (int rc = check_engine(e)) return rc;
   hipStream_t st = e->stream;
   ev_rec(e, 0);
-  const int grid = launch_entropy(e);
-  HIPCHK(hipGetLastError());
+  const EntropyIn in = launch_entropy(e, e->ent_part);
   ev_rec(e, 1);
-  HIPCHK(hipMemcpyAsync(e->h_ent_part, e->ent_part, sizeof(long) * 2 * grid, hipMemcpyDeviceToHost,
-                        st));
+  k_entropy_out<<<1, kBeginThreads, 0, st>>>(in, 0.0, nullptr, e->d_fx);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(st));
-  prof_add(e, USAP_K_ENTROPY, ev_ms(e, 0, 1), 1, 8.0 * e->B + 16.0 * grid);
-  i128 t = 0;
-  for (int i = 0; i < grid; ++i)
-    t += mk128(e->h_ent_part[2 * i], (unsigned long)e->h_ent_part[2 * i + 1]);
-  const i128 data = -t;
+  prof_add(e, USAP_K_ENTROPY, ev_ms(e, 0, 1), 1, 8.0 * e->B + 16.0 * in.nparts);
+  const i128 data = mk128((long)e->h_fx[0], (unsigned long)e->h_fx[1]);
   if (hi) *hi = (int64_t)(data >> 64);
   if (lo) *lo = (uint64_t)(u128)data;
   if (S) *S = usap_model_S(e->N, e->E, e->B) + fx_to_double(data);
@@ -5523,8 +5611,8 @@ int usap_entropy_noalloc(usap_engine* e, double* S_dev, int64_t* fx_dev) {
   const int64_t need = std::min<int64_t>(kEntropyBlocks, blocks_for(std::max<int64_t>(e->M.P, e->B), 1024));
   if (need > kScratchParts)
     return set_err(e, USAP_EINVAL, "usap_entropy_noalloc: more partials than the 64 KiB scratch holds");
-  const int grid = launch_entropy(e, part);
-  k_entropy_out<<<1, 256, 0, e->stream>>>(part, grid, usap_model_S(e->N, e->E, e->B), S_dev, fx_dev);
+  const EntropyIn in = launch_entropy(e, part);
+  k_entropy_out<<<1, kBeginThreads, 0, e->stream>>>(in, usap_model_S(e->N, e->E, e->B), S_dev, fx_dev);
   HIPCHK(hipGetLastError());
   return USAP_OK;
 }
@@ -5773,12 +5861,32 @@ ApplyKernel apply_kernel(bool dense, bool weighted, bool hubs) {
   return k[4 * dense + 2 * weighted + hubs];
 }
 
-// The Philox words of nodes [beg, end) in batches of `batch` (batch i: stream
-// sweep->stream0 + i), before their first batch (pre-drawn mode has its own).
-int launch_draws(usap_engine* e, int32_t beg, int32_t end, int32_t batch) {
-  if (e->uni) return USAP_OK;
-  k_draw<<<blocks_for((int64_t)end - beg, 256), 256, 0, e->stream>>>(beg, end, batch, e->p.seed,
-                                                                     e->sweep, e->draws);
+// The device state *h_sweep, and the Philox words of nodes [beg, end) in batches
+// of `batch` (pre-drawn mode has its own, a captured sweep makes them in the
+// graph).  from_state: the starting S is the MDL of the current state, computed
+// on the device (no host wait for it).
+int launch_begin(usap_engine* e, int32_t beg, int32_t end, int32_t batch, bool from_state,
+                 bool draws) {
+  BeginArgs a;
+  a.init = *e->h_sweep;
+  a.sweep = e->sweep;
+  a.from_state = from_state;
+  a.model = from_state ? usap_model_S(e->N, e->E, e->B) : 0.0;
+  a.ent = EntropyIn{};
+  if (from_state) a.ent = launch_entropy(e, e->ent_part);
+  a.beg = beg;
+  a.end = end;
+  a.batch = batch;
+  a.seed = e->p.seed;
+  a.draws = e->draws;
+  const unsigned n = draws && !e->uni ? blocks_for((int64_t)end - beg, kBeginThreads) : 0;
+  k_begin<<<1 + n, kBeginThreads, 0, e->stream>>>(a);
+  HIPCHK(hipGetLastError());
+  return USAP_OK;
+}
+
+int launch_finish(usap_engine* e, Sweep* host) {
+  k_finish<<<1, kWave, 0, e->stream>>>(e->status, e->sweep, host);
   HIPCHK(hipGetLastError());
   return USAP_OK;
 }
@@ -5898,7 +6006,9 @@ int sweep_graph(usap_engine* e, int32_t batch, int32_t nb) {
       e->gexec = nullptr;
     }
     HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    int rc = launch_draws(e, 0, e->N, batch);
+    int rc = USAP_OK;
+    if (!e->uni)
+      k_draw<<<blocks_for(e->N, 256), 256, 0, st>>>(0, e->N, batch, e->p.seed, e->sweep, e->draws);
     for (int32_t i = 0; i < nb && rc == USAP_OK; ++i) {
       const int32_t beg = i * batch;
       const int32_t end = std::min<int64_t>((int64_t)beg + batch, e->N);
@@ -5945,8 +6055,6 @@ int run_sweep(usap_engine* e, int32_t batch, int32_t first, int32_t last, int32_
     } else {
       if (e->prof)
         if (int rc = prof_begin(e, (size_t)(last - next), batch)) return rc;
-      if (next == 0)  // a resumed round still has the sweep's draws
-        if (int rc = launch_draws(e, 0, e->N, batch)) return rc;
       // A sweep whose convergence test is active stops at a batch nobody
       // knows in advance, and the batches launched after it exit at once
       // (a few us each).  Such a sweep goes out in chunks of kChunk batches,
@@ -5961,14 +6069,14 @@ int run_sweep(usap_engine* e, int32_t batch, int32_t first, int32_t last, int32_
         for (int32_t i = i0; i < upto; ++i, ++slot) {
           const int32_t beg = i * batch;
           const int32_t end = std::min<int64_t>((int64_t)beg + batch, e->N);
-          // with every row direct, the chunk's last k_grow folds the error
-          // flags of all its batches (they only report inconsistent M)
-          const bool grow = !e->all_direct || e->prof || i == upto - 1;
+          // with every row direct nothing grows, and the flags of the chunk's
+          // batches (they only report inconsistent M) are folded at its end
+          const bool grow = !e->all_direct || e->prof;
           if (int rc = launch_batch(e, beg, end, slot, grow)) return rc;
         }
         i0 = upto;
         if (!chunked) break;
-        HIPCHK(hipMemcpyAsync(e->h_chunk[c & 1], e->sweep, sizeof(Sweep), hipMemcpyDeviceToHost, st));
+        if (int rc = launch_finish(e, e->d_hchunk[c & 1])) return rc;
         HIPCHK(hipEventRecord(e->chunk_ev[c & 1], st));
         if (c > 0) {
           HIPCHK(hipEventSynchronize(e->chunk_ev[(c - 1) & 1]));
@@ -5976,7 +6084,7 @@ int run_sweep(usap_engine* e, int32_t batch, int32_t first, int32_t last, int32_
         }
       }
     }
-    HIPCHK(hipMemcpyAsync(&hs, e->sweep, sizeof(Sweep), hipMemcpyDeviceToHost, st));
+    if (int rc = launch_finish(e, e->d_hsweep)) return rc;
     HIPCHK(hipStreamSynchronize(st));
     const int32_t executed = first + hs.done - next;  // batches run in this launch round
     if (e->prof)
@@ -6030,15 +6138,14 @@ int usap_nodal_batch(usap_engine* e, int32_t begin, int32_t end, uint64_t stream
   e->last_end = end;
   init_sweep(e, stream, 0.0, 0.0, 0.0, 0);
   if (begin < end) {
-    HIPCHK(hipMemcpyAsync(e->sweep, e->h_sweep, sizeof(Sweep), hipMemcpyHostToDevice, e->stream));
     // one batch of size end-begin starting at begin: index 0 of a sweep whose
     // "batch" starts at begin
+    if (int rc = launch_begin(e, begin, end, end - begin, false, true)) return rc;
     if (e->prof)
       if (int rc = prof_begin(e, 1, end - begin)) return rc;
-    if (int rc = launch_draws(e, begin, end, end - begin)) return rc;
     if (int rc = launch_batch(e, begin, end, 0)) return rc;
     Sweep& hs = *e->h_sweep;
-    HIPCHK(hipMemcpyAsync(&hs, e->sweep, sizeof(Sweep), hipMemcpyDeviceToHost, e->stream));
+    if (int rc = launch_finish(e, e->d_hsweep)) return rc;
     HIPCHK(hipStreamSynchronize(e->stream));
     if (e->prof) {
       if (int rc = prof_end(e, 1)) return rc;
@@ -6115,13 +6222,7 @@ int nodal_sweep(usap_engine* e, int32_t batch, uint64_t stream0, const double* S
     stream0 = (uint64_t)e->uni_pos;
   }
   init_sweep(e, stream0, S ? *S : 0.0, mean, thr, check);
-  HIPCHK(hipMemcpyAsync(e->sweep, e->h_sweep, sizeof(Sweep), hipMemcpyHostToDevice, e->stream));
-  if (!S) {
-    const int grid = launch_entropy(e);
-    k_entropy_to_sweep<<<1, 256, 0, e->stream>>>(e->ent_part, grid,
-                                                 usap_model_S(e->N, e->E, e->B), e->sweep);
-    HIPCHK(hipGetLastError());
-  }
+  if (int rc = launch_begin(e, 0, e->N, batch, !S, !(e->p.graphs && !e->prof))) return rc;
   int32_t rebuilds = 0;
   if (int rc = run_sweep(e, batch, 0, nb, &rebuilds)) return rc;
   const Sweep& hs = *e->h_sweep;
