@@ -302,6 +302,46 @@ __device__ __forceinline__ int32_t m_window(const MView& m, Row R, int32_t b, ui
   return kk;
 }
 
+// A window of row R for key b in flight (direct: only h).
+struct Window {
+  Key4 lo, hi;
+  uint32_t w0, home;
+};
+
+__device__ __forceinline__ Window win_issue(const MView& m, Row R, int32_t b, bool direct) {
+  Window w;
+  if (direct) {
+    w.w0 = w.home = (uint32_t)b;
+    w.lo = w.hi = Key4{b, b, b, b};
+    return w;
+  }
+  w.home = hash32(b) & ((uint32_t)R.c - 1);
+  w.w0 = min(w.home, (uint32_t)R.c - kWin);
+  const Key4* k = reinterpret_cast<const Key4*>(m.key + R.o + w.w0);
+  w.lo = k[0];
+  w.hi = k[1];
+  return w;
+}
+
+// The slot within the row that ends key b's probe chain (found: it holds b), or
+// the window's last one, whose other key k is then returned >= 0.
+__device__ __forceinline__ uint32_t win_end(const Window& w, int32_t b, bool direct, int32_t& k) {
+  if (direct) {
+    k = b;
+    return w.home;
+  }
+  const int32_t kk[kWin] = {w.lo[0], w.lo[1], w.lo[2], w.lo[3], w.hi[0], w.hi[1], w.hi[2], w.hi[3]};
+  k = kk[kWin - 1];
+  uint32_t pos = w.w0 + kWin - 1;
+#pragma unroll
+  for (int q = kWin - 2; q >= 0; --q)
+    if (w.w0 + q >= w.home && (kk[q] == b || kk[q] < 0)) {
+      k = kk[q];
+      pos = w.w0 + q;
+    }
+  return pos;
+}
+
 // Where m_add_at starts for key b in row R: the end of its probe chain, or as
 // far along it as one window reaches.
 template <bool kD = false>
@@ -2205,6 +2245,7 @@ struct NodalArgs {
   const int32_t* d_out;
   const int32_t* d_in;
   const int64_t* lam;
+  int32_t lam_last;  // its last entry, at most kLamLds - 1
   int32_t B;
   int32_t beg, end;
   int32_t exact;
@@ -2349,6 +2390,13 @@ struct Corner {
   int32_t wself;               // n's self-loops
 };
 
+// lambda(m) from the first kLamLds entries in LDS, or, big, from the table.
+constexpr int kLamLds = 256;
+__device__ __forceinline__ int64_t lam_at(const int64_t* lam, const int64_t* s_lam, bool big,
+                                          int32_t m) {
+  return big ? lam[max(m, 0)] : s_lam[max(m, 0)];
+}
+
 // Adds the move's 16 corner and degree terms to acc, one per lane (in every
 // lane they were a quarter of the kernel's arithmetic); inf: the moved state
 // has an infinite term.  Lane bits: col (0: column r, 1: s), row (0: row r, 1:
@@ -2357,8 +2405,9 @@ struct Corner {
 //   deg = 1: the row's other out-edges X (col = 0) or the column's other
 //            in-edges Y (col = 1) of block `row`, m * lambda(degree)
 // each + before and - after, the degree terms the other way round.
-__device__ __forceinline__ void corner_terms(const NodalArgs& a, const Corner& c, Acc& acc,
-                                             bool& inf) {
+// s_lam: LDS copy of lambda's first kLamLds entries, or null.
+__device__ __forceinline__ void corner_terms(const NodalArgs& a, const Corner& c,
+                                             const int64_t* s_lam, Acc& acc, bool& inf) {
   const int lane = lane_id();
   int32_t rr2, rs2, sr2, ss2;
   if (!a.exact) {  // graph_parallel.hpp:1117-1145: only out-edges update the rows
@@ -2389,7 +2438,12 @@ __device__ __forceinline__ void corner_terms(const NodalArgs& a, const Corner& c
   const int32_t m = deg ? mp : mt;
   const int32_t d1 = deg && !col ? dout : din, d2 = deg ? 1 : dout;  // lambda(1) = 0
   const bool bad = d1 <= 0 || d2 <= 0;
-  const int64_t L = lam_of(a.lam, deg ? 0 : m) - lam_of(a.lam, d1) - lam_of(a.lam, d2);
+  int64_t L;
+  if (!s_lam || __ballot(lane < 16 && max(max(deg ? 0 : m, d1), d2) >= kLamLds))
+    L = lam_of(a.lam, deg ? 0 : m) - lam_of(a.lam, d1) - lam_of(a.lam, d2);
+  else  // lanes past 15 read in range too
+    L = s_lam[min(max(deg ? 0 : m, 0), kLamLds - 1)] - s_lam[min(max(d1, 0), kLamLds - 1)] -
+        s_lam[min(max(d2, 0), kLamLds - 1)];
   if (lane < 16) {
     const int32_t mm = bad ? 0 : max(m, 0);
     acc_add(acc, now ? -mm : mm, L);
@@ -2433,20 +2487,28 @@ __device__ __forceinline__ uint32_t unit_key(int32_t b, bool in) {
 // The kernel is bound by its chain of dependent loads, so each step's are in
 // flight together: the list, with r's row header and degrees and those of the
 // uniform draw's block; the entries' labels (the drawn neighbour's among
-// them); then row r's counts of every entry's block, the drawn block's
-// degrees and, M hashed (B is then at least 16 times a row's degree, so the
-// uniform draw is nearly always the proposal), the uniform block's keys, or, M
-// dense (the drawn block's row decides most often), that row's bucket sums;
-// then s's counts unless they are there; then the lambda table.
-// Launch averages against one path through an LDS table with row headers
-// always read (90 VGPRs, 40 KB of LDS a workgroup, Philox in every lane): N =
-// 1000 12.1 -> 5.8 us, N = 20000 (5000-node batches) 28.8 -> 9.8, N = 50000
-// (12500-node batches) 42.5 -> 15.8, 4096-node batches at B = 100000 28.8 ->
-// 20.1.
+// them); then
+//   M dense: row r's counts of every entry's block, the drawn block's degrees
+//     and its row's weights (it decides the proposal most often); then s's
+//     counts and degrees;
+//   M hashed (B is then at least 16 times a row's degree, so the uniform draw
+//     is nearly always the proposal): 8-key windows of row r and of the uniform
+//     block's row for every entry's block -- the keys alone of a block that
+//     most often has none of them, and one round of loads for nearly every
+//     probe chain, where slot by slot the longest of 64 lanes' chains took
+//     three or four; then the counts found there;
+// then the lambda table (hashed rows' counts are small: its first entries are
+// in LDS).  Launch averages against one path through an LDS table with row
+// headers always read (90 VGPRs, 40 KB of LDS a workgroup, Philox in every
+// lane): N = 1000 12.1 -> 5.8 us, N = 20000 (5000-node batches) 28.8 -> 9.8, N =
+// 50000 (12500-node batches) 42.5 -> 15.8, 4096-node batches at B = 100000 28.8
+// -> 17.5 and at B = 250000 29.2 -> 21.9 (20.1 and 27.3 with single slots and
+// the whole lambda table).
 template <bool kD, bool kW, int U>
 __device__ __forceinline__ void nodal_regs(const NodalArgs& a, int32_t n, int32_t r, int64_t o0,
                                            int64_t i0, int32_t kco, int32_t kc,
-                                           const uint64_t x[4], int32_t* lds, Nodal& out) {
+                                           const uint64_t x[4], int32_t* lds,
+                                           const int64_t* s_lam, Nodal& out) {
   const int lane = lane_id();
   const GraphView& g = a.g;
   const MView& M = a.M;
@@ -2521,52 +2583,75 @@ __device__ __forceinline__ void nodal_regs(const NodalArgs& a, int32_t n, int32_
   const uint32_t da = (uint32_t)a.d_out[u] + (uint32_t)a.d_in[u];
   Sums bk;
   if (kD) bk = load_sums(M, u, m_row<kD>(M, u));
-  Probe p0[U];
-  int32_t ks[U];  // row s's key at the block's home slot
-  const bool pdir = kD || pM.c == B;
+  // row r's and row s's counts of the unit's block, in its direction: o, or i
+  // for an in-edge
+  int32_t m0[U], m1[U];
+  auto count = [&](Row R, int32_t h, int q) {
+    return reinterpret_cast<const int32_t*>(M.cnt + R.o + h)[q * kWave + lane >= kco];
+  };
 #pragma unroll
-  for (int q = 0; q < U; ++q) {
-    p0[q] = Probe{0, -1, {0, 0}};
-    ks[q] = lb[q];
-    if (v[q] >= 0) {
-      p0[q] = m_probe<kD>(M, rM, lb[q]);
-      if (!pdir) ks[q] = M.key[pM.o + m_home(M, pM, lb[q])];
+  for (int q = 0; q < U; ++q) m0[q] = m1[q] = 0;
+  Cnt cRR{0, 0}, cRS{0, 0}, cSS{0, 0};
+  // hashed: the windows of kG units a lane at a time, and, with the first
+  // ones, the corner's in lanes 0 (row r, key r), 1 (r, s), 2 (s, s)
+  constexpr int kG = U == 2 ? 2 : 1;
+  const bool rdir = kD || __builtin_amdgcn_readfirstlane(rM.c) == B;
+  Window wr[kG], ws[kG], wc;
+  auto corner_row = [&](Row sM) { return lane < 2 ? rM : sM; };
+  auto corner_key = [&](int32_t s) { return lane == 0 ? r : s; };
+  auto issue = [&](int q0, Row sM, bool sdir, bool with_r) {
+#pragma unroll
+    for (int i = 0; i < kG; ++i) {
+      const int32_t b = max(lb[q0 + i], 0);  // an absent entry reads block 0's
+      if (with_r) wr[i] = win_issue(M, rM, b, rdir);
+      ws[i] = win_issue(M, sM, b, sdir);
     }
+  };
+  if (kD) {
+#pragma unroll
+    for (int q = 0; q < U; ++q)
+      if (v[q] >= 0) m0[q] = count(rM, lb[q], q);
+    cRR = M.cnt[rM.o + r];
   }
-  const Probe pRR = m_probe<kD>(M, rM, r);
-  Probe pRS, pSS;
+  const bool pdir = kD || __builtin_amdgcn_readfirstlane(pM.c) == B;
   if (!kD) {
-    pRS = m_probe(M, rM, s_pre);
-    pSS = m_probe(M, pM, s_pre);
+    issue(0, pM, pdir, true);
+    const Row cM = corner_row(pM);
+    wc = win_issue(M, cM, corner_key(s_pre), cM.c == B);
   }
-  // units: the owner of each (block, direction), its summed weight
-  uint32_t hs[U];
+  // units: the owner of each (block, direction), its summed weight; every
+  // entry's first claim before any is resolved
+  uint32_t hs[U], old[U];
   bool own[U];
 #pragma unroll
   for (int q = 0; q < U; ++q) {
+    const uint32_t key = unit_key(lb[q], q * kWave + lane >= kco);
+    hs[q] = hash32((int32_t)key) & (kCap - 1);
+    old[q] = key;
+    if (v[q] >= 0) old[q] = atomicCAS(&tk[hs[q]], kNoUnit, key);
+  }
+#pragma unroll
+  for (int q = 0; q < U; ++q) {
     own[q] = false;
-    hs[q] = 0;
     if (v[q] >= 0) {
       const uint32_t key = unit_key(lb[q], q * kWave + lane >= kco);
-      uint32_t h = hash32((int32_t)key) & (kCap - 1);
-      for (;;) {
-        const uint32_t old = atomicCAS(&tk[h], kNoUnit, key);
-        own[q] = old == kNoUnit;
-        if (own[q] || old == key) break;
-        h = (h + 1) & (kCap - 1);
+      own[q] = old[q] == kNoUnit;
+      while (!own[q] && old[q] != key) {
+        hs[q] = (hs[q] + 1) & (kCap - 1);
+        old[q] = atomicCAS(&tk[hs[q]], kNoUnit, key);
+        own[q] = old[q] == kNoUnit;
       }
-      hs[q] = h;
-      atomicAdd(&tw[h], w[q]);
+      atomicAdd(&tw[hs[q]], w[q]);
     }
   }
   lds_order();
   int32_t wself = 0;
   if (a.exact) {
-    uint32_t ws = 0;
+    uint32_t sum = 0;
 #pragma unroll
     for (int q = 0; q < U; ++q)
-      if (q * kWave + lane < kco && v[q] == n) ws += (uint32_t)w[q];
-    if (__ballot(ws != 0)) wself = (int32_t)wave_sum32(ws);  // self-loops are rare
+      if (q * kWave + lane < kco && v[q] == n) sum += (uint32_t)w[q];
+    if (__ballot(sum != 0)) wself = (int32_t)wave_sum32(sum);  // self-loops are rare
   }
 #pragma unroll
   for (int q = 0; q < U; ++q) w[q] = own[q] ? tw[hs[q]] : 0;
@@ -2591,41 +2676,84 @@ __device__ __forceinline__ void nodal_regs(const NodalArgs& a, int32_t n, int32_
   const bool pre = s == s_pre;
   const Row sM = pre ? pM : m_row<kD>(M, s);
   const int32_t dos = pre ? dos_pre : a.d_out[s], dis = pre ? dis_pre : a.d_in[s];
-  const bool sdir = kD || sM.c == B;
-  if (kD || !pre) {
-    pRS = m_probe<kD>(M, rM, s);
-    pSS = m_probe<kD>(M, sM, s);
-  }
-  Cnt cs[U];
+  const bool sdir = kD || __builtin_amdgcn_readfirstlane(sM.c) == B;
+  // blocks r and s own one unit each per direction at most
   int32_t wor = 0, wir = 0, wos = 0, wis = 0, units = 0;
 #pragma unroll
   for (int q = 0; q < U; ++q) {
     const bool in = q * kWave + lane >= kco;
     const bool isr = own[q] && lb[q] == r, iss = own[q] && lb[q] == s;
-    const unsigned long long mr = __ballot(isr), ms = __ballot(iss);
-    if (mr) {  // at most one owner per direction
+    if (__ballot(isr)) {
       const unsigned long long o = __ballot(isr && !in), i = __ballot(isr && in);
       if (o) wor = __builtin_amdgcn_readlane(w[q], __ffsll(o) - 1);
       if (i) wir = __builtin_amdgcn_readlane(w[q], __ffsll(i) - 1);
     }
-    if (ms) {
+    if (__ballot(iss)) {
       const unsigned long long o = __ballot(iss && !in), i = __ballot(iss && in);
       if (o) wos = __builtin_amdgcn_readlane(w[q], __ffsll(o) - 1);
       if (i) wis = __builtin_amdgcn_readlane(w[q], __ffsll(i) - 1);
     }
     own[q] = own[q] && !isr && !iss;
     units += __popcll(__ballot(own[q]));
-    cs[q] = Cnt{0, 0};
-    if (own[q]) {
-      if (sdir) {
-        cs[q] = M.cnt[sM.o + lb[q]];
-      } else {
-        const uint32_t h = m_home(M, sM, lb[q]);
-        if (!pre) ks[q] = M.key[sM.o + h];
-        if (ks[q] == lb[q])
-          cs[q] = M.cnt[sM.o + h];
-        else if (ks[q] >= 0)
-          cs[q] = m_value_more(M, sM, lb[q], h);
+  }
+  if (kD) {
+#pragma unroll
+    for (int q = 0; q < U; ++q) {
+      if (own[q])
+        m1[q] = count(sM, lb[q], q);
+      else
+        m0[q] = 0;
+    }
+    cRS = M.cnt[rM.o + s];
+    cSS = M.cnt[sM.o + s];
+  } else {
+    if (!pre) {
+      issue(0, sM, sdir, false);
+      const Row cM = corner_row(sM);
+      wc = win_issue(M, cM, corner_key(s), cM.c == B);
+    }
+#pragma unroll
+    for (int q0 = 0; q0 < U; q0 += kG) {
+      if (q0 > 0) issue(q0, sM, sdir, true);
+      uint32_t hr[kG], hq[kG];
+      int32_t kr[kG], kq[kG];
+#pragma unroll
+      for (int i = 0; i < kG; ++i) {
+        const int32_t b = max(lb[q0 + i], 0);
+        hr[i] = win_end(wr[i], b, rdir, kr[i]);
+        hq[i] = win_end(ws[i], b, sdir, kq[i]);
+        if (!own[q0 + i]) kr[i] = kq[i] = -1;
+        if (own[q0 + i] && kr[i] == b) m0[q0 + i] = count(rM, (int32_t)hr[i], q0 + i);
+        if (own[q0 + i] && kq[i] == b) m1[q0 + i] = count(sM, (int32_t)hq[i], q0 + i);
+      }
+      if (q0 == 0) {  // the corner
+        const Row cM = corner_row(sM);
+        const int32_t ck = corner_key(s);
+        int32_t kk;
+        const uint32_t h = win_end(wc, ck, cM.c == B, kk);
+        Cnt c{0, 0};
+        if (lane < 3) {
+          if (kk == ck)
+            c = M.cnt[cM.o + h];
+          else if (kk >= 0)
+            c = m_value_more(M, cM, ck, h);
+        }
+        cRR = Cnt{__builtin_amdgcn_readlane(c.o, 0), __builtin_amdgcn_readlane(c.i, 0)};
+        cRS = Cnt{__builtin_amdgcn_readlane(c.o, 1), __builtin_amdgcn_readlane(c.i, 1)};
+        cSS = Cnt{__builtin_amdgcn_readlane(c.o, 2), __builtin_amdgcn_readlane(c.i, 2)};
+      }
+#pragma unroll
+      for (int i = 0; i < kG; ++i) {  // chains past a window
+        const int32_t b = lb[q0 + i];
+        const bool in = (q0 + i) * kWave + lane >= kco;
+        if (kr[i] >= 0 && kr[i] != b) {
+          const Cnt y = m_value_more(M, rM, b, hr[i]);
+          m0[q0 + i] = in ? y.i : y.o;
+        }
+        if (kq[i] >= 0 && kq[i] != b) {
+          const Cnt y = m_value_more(M, sM, b, hq[i]);
+          m1[q0 + i] = in ? y.i : y.o;
+        }
       }
     }
   }
@@ -2635,28 +2763,24 @@ __device__ __forceinline__ void nodal_regs(const NodalArgs& a, int32_t n, int32_
   out.bytes = bytes;
   Acc acc{0, 0};
   int64_t L[U][4];
-  int32_t m0[U], m1[U];
-  bool neg = false;
+  bool neg = false, big = kD;
 #pragma unroll
   for (int q = 0; q < U; ++q) {
-    const bool in = q * kWave + lane >= kco;
-    Cnt cr{0, 0};
-    if (own[q])
-      cr = m_value<kD>(M, rM, lb[q], p0[q]);
-    else
-      w[q] = 0;
-    m0[q] = in ? cr.i : cr.o;
-    m1[q] = in ? cs[q].i : cs[q].o;
+    if (!own[q]) w[q] = 0;
     neg |= m0[q] < w[q];
-    L[q][0] = lam_of(a.lam, m0[q]);
-    L[q][1] = lam_of(a.lam, m1[q]);
-    L[q][2] = lam_of(a.lam, m0[q] - w[q]);
-    L[q][3] = lam_of(a.lam, m1[q] + w[q]);
+    big |= max(m0[q], m1[q] + w[q]) >= kLamLds;
   }
-  const Cnt crs = m_value<kD>(M, rM, s, pRS);
-  const Corner c{m_value<kD>(M, rM, r, pRR).o, crs.o, crs.i, m_value<kD>(M, sM, s, pSS).o,
-                 dor, dir, dos, dis, k_out, k_in, wor, wir, wos, wis, wself};
-  corner_terms(a, c, acc, out.inf);
+  if (!kD) big = __ballot(big) != 0;
+#pragma unroll
+  for (int q = 0; q < U; ++q) {
+    L[q][0] = lam_at(a.lam, s_lam, big, m0[q]);
+    L[q][1] = lam_at(a.lam, s_lam, big, m1[q]);
+    L[q][2] = lam_at(a.lam, s_lam, big, m0[q] - w[q]);
+    L[q][3] = lam_at(a.lam, s_lam, big, m1[q] + w[q]);
+  }
+  const Corner c{cRR.o, cRS.o, cRS.i, cSS.o, dor, dir, dos, dis,
+                 k_out, k_in, wor, wir, wos, wis, wself};
+  corner_terms(a, c, kD ? nullptr : s_lam, acc, out.inf);
 #pragma unroll
   for (int q = 0; q < U; ++q) unit_terms(acc, L[q], m0[q], m1[q], w[q]);
   if (neg) atomicOr(&a.status->flags, kFlagNegative);
@@ -2876,7 +3000,7 @@ __device__ __forceinline__ void nodal_hub(const NodalArgs& a, int32_t n, int32_t
                    a.d_out[r], a.d_in[r], a.d_out[s], a.d_in[s], k_out, k_in,
                    hub.w[0], hub.w[1], hub.w[2], hub.w[3], hub.wself};
     Acc t{0, 0};
-    corner_terms(a, c, t, out.inf);
+    corner_terms(a, c, nullptr, t, out.inf);
     t.h = wave_sum(t.h);
     t.l = wave_sum(t.l);
     for (int i = 0; i < kNodalWaves; ++i) {
@@ -2893,10 +3017,11 @@ __device__ __forceinline__ void nodal_hub(const NodalArgs& a, int32_t n, int32_t
 // large for a wavefront are left to the whole workgroup afterwards (kHub: the
 // graph has such nodes; their code costs registers).
 template <bool kD, bool kW, bool kHub>
-__global__ __launch_bounds__(kWave* kNodalWaves, 4) void k_nodal(NodalArgs a) {
+__global__ __launch_bounds__(kWave* kNodalWaves, kD ? 5 : 4) void k_nodal(NodalArgs a) {
   __shared__ __align__(16) int32_t s_lds[kNodalWaves][kLdsWave];
   __shared__ unsigned long long s_p[kNodalWaves][6];
   __shared__ int32_t s_large[kNodalWaves];
+  __shared__ int64_t s_lam[kD ? 1 : kLamLds];
   const int w = threadIdx.x / kWave;
   if (a.tstamp && threadIdx.x == 0) a.tstamp[blockIdx.x] = wall_clock64();
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -2925,28 +3050,35 @@ __global__ __launch_bounds__(kWave* kNodalWaves, 4) void k_nodal(NodalArgs a) {
   bool large = false;
   if (lane_id() == 0)
     for (int i = 0; i < 6; ++i) s_p[w][i] = 0;
-  if (n64 < a.end) {
-    // the sweep's stop flag is read together with the node's first loads
-    const int32_t n = (int32_t)n64;
-    const int32_t stop = a.sweep->stop;
-    uint64_t x[4];
-    predrawn(a.draws, (a.predrawn ? a.sweep->stream0 : 0) + (uint64_t)n, x);
-    const int32_t r = a.labels[n];
-    const int64_t o0 = a.g.out_ptr[n], i0 = a.g.in_ptr[n];
-    const int64_t kco = a.g.out_ptr[n + 1] - o0, kc = kco + (a.g.in_ptr[n + 1] - i0);
-    if (!stop) {
-      large = kHub && kc > kRegUnits * kWave;
-      if (!large) {
-        Nodal p;
-        const int32_t ko = (int32_t)kco, kk = (int32_t)kc;
-        if (kk <= kWave)
-          nodal_regs<kD, kW, 1>(a, n, r, o0, i0, ko, kk, x, s_lds[w], p);
-        else if (kk <= 2 * kWave)
-          nodal_regs<kD, kW, 2>(a, n, r, o0, i0, ko, kk, x, s_lds[w], p);
-        else
-          nodal_regs<kD, kW, kRegUnits>(a, n, r, o0, i0, ko, kk, x, s_lds[w], p);
-        if (lane_id() == 0) store(item, w, r, kk, p);
-      }
+  // the sweep's stop flag and lambda's first entries are read together with the
+  // node's first loads
+  static_assert(kLamLds == kWave * kNodalWaves, "one entry per thread");
+  int64_t lam = 0;
+  if (!kD) lam = a.lam[min((int32_t)threadIdx.x, a.lam_last)];
+  const bool in = n64 < a.end;
+  const int32_t n = in ? (int32_t)n64 : a.beg;
+  const int32_t stop = a.sweep->stop;
+  uint64_t x[4];
+  predrawn(a.draws, (a.predrawn ? a.sweep->stream0 : 0) + (uint64_t)n, x);
+  const int32_t r = a.labels[n];
+  const int64_t o0 = a.g.out_ptr[n], i0 = a.g.in_ptr[n];
+  const int64_t kco = a.g.out_ptr[n + 1] - o0, kc = kco + (a.g.in_ptr[n + 1] - i0);
+  if (!kD) {
+    s_lam[threadIdx.x] = lam;
+    __syncthreads();
+  }
+  if (in && !stop) {
+    large = kHub && kc > kRegUnits * kWave;
+    if (!large) {
+      Nodal p;
+      const int32_t ko = (int32_t)kco, kk = (int32_t)kc;
+      if (kk <= kWave)
+        nodal_regs<kD, kW, 1>(a, n, r, o0, i0, ko, kk, x, s_lds[w], s_lam, p);
+      else if (kk <= 2 * kWave)
+        nodal_regs<kD, kW, 2>(a, n, r, o0, i0, ko, kk, x, s_lds[w], s_lam, p);
+      else
+        nodal_regs<kD, kW, kRegUnits>(a, n, r, o0, i0, ko, kk, x, s_lds[w], s_lam, p);
+      if (lane_id() == 0) store(item, w, r, kk, p);
     }
   }
   if (kHub && lane_id() == 0) s_large[w] = large;
@@ -5902,6 +6034,7 @@ int launch_batch(usap_engine* e, int32_t beg, int32_t end, size_t ev_slot, bool 
   a.d_out = e->d_out;
   a.d_in = e->d_in;
   a.lam = e->lam;
+  a.lam_last = (int32_t)std::min<int64_t>(e->Wtot, kLamLds - 1);
   a.B = B;
   a.beg = beg;
   a.end = end;
