@@ -79,7 +79,9 @@ constexpr int kTabMaxDeg = kTab * 3 / 4; // larger nodes use a global-memory tab
 constexpr int kMergeWaves = 4;           // wavefronts per workgroup in k_merge
 constexpr int kNBK = 512;                // bucket sums per block row
 constexpr int kLookupRatio = 8;          // a hashed slab this many times a bucket is looked up per key
-constexpr int kScr = 3 * kTab;           // per-wavefront LDS scratch (ints) for one bucket
+constexpr int kScr = 1024;               // per-wavefront LDS scratch (ints) for one bucket
+constexpr int kMergeMany = 16;           // and for few blocks
+constexpr int32_t kMergeFew = 1024;
 constexpr int kDegLds = 1024;            // k_degrees privatises its counters for B <= this
 constexpr int kHistB = 256;              // M is built by histograms in LDS up to here
 constexpr int kEntropyBlocks = 4096;  // k_entropy grid at most
@@ -1890,6 +1892,7 @@ struct MergeArgs {
   const int32_t* d_out;
   const int32_t* d_in;
   const int64_t* lam;
+  int32_t lam_last;  // its last entry, at most kLamMerge - 1
   int32_t B;
   int32_t K;
   uint64_t seed, stream;  // pre-drawn mode: stream = the round's first draw
@@ -1899,82 +1902,102 @@ struct MergeArgs {
   unsigned long* best_lo;
 };
 
-// + L(m1) + L(m2) - L(m1+m2) when both counts are non-zero (no branch: a
-// wavefront's pairs are rarely all zero, and the loads of two pairs overlap).
-__device__ __forceinline__ void overlap_pair(Acc& acc, const int64_t* lam, int32_t m1,
-                                             int32_t m2) {
-  const bool both = m1 > 0 && m2 > 0;
-  const int32_t a = both ? m1 : 0, b = both ? m2 : 0;
-  const int64_t La = lam[a], Lb = lam[b], Lab = lam[a + b];
-  acc_add(acc, a, La);
-  acc_add(acc, b, Lb);
-  acc_add(acc, -(a + b), Lab);
+// L(m1) + L(m2) - L(m1 + m2) over the two counts of a key in two rows, where
+// both are non-zero (no branch per pair: a wavefront's pairs are rarely all
+// zero).  lambda from LDS while the counts are small.
+constexpr int kLamMerge = 512;
+__device__ __forceinline__ void overlap_pair(Acc& acc, const int64_t* lam, const int64_t* s_lam,
+                                             Cnt x, Cnt y) {
+  const bool bo = x.o > 0 && y.o > 0, bi = x.i > 0 && y.i > 0;
+  if (!__ballot(bo || bi)) return;
+  const int32_t a = bo ? x.o : 0, b = bo ? y.o : 0, c = bi ? x.i : 0, d = bi ? y.i : 0;
+  int64_t L[6];
+  if (__ballot(max(a + b, c + d) >= kLamMerge)) {
+    L[0] = lam[a];
+    L[1] = lam[b];
+    L[2] = lam[a + b];
+    L[3] = lam[c];
+    L[4] = lam[d];
+    L[5] = lam[c + d];
+  } else {
+    L[0] = s_lam[a];
+    L[1] = s_lam[b];
+    L[2] = s_lam[a + b];
+    L[3] = s_lam[c];
+    L[4] = s_lam[d];
+    L[5] = s_lam[c + d];
+  }
+  acc_add(acc, a, L[0]);
+  acc_add(acc, b, L[1]);
+  acc_add(acc, -(a + b), L[2]);
+  acc_add(acc, c, L[3]);
+  acc_add(acc, d, L[4]);
+  acc_add(acc, -(c + d), L[5]);
 }
 
 // per-lane part of sum_{i not in {r,s}} [L(m1) + L(m2) - L(m1+m2)] over the
 // keys where rows r and s of M are both non-zero, and the same over the
 // columns (the only terms that survive the factorised merge dS): one pass
-// over the shorter block row, probing the other for each of its keys.
-__device__ Acc merge_overlap_lane(const MView& m, const int64_t* lam, int32_t r, int32_t s) {
+// over the shorter block row, four of its slots per lane at a time, probing
+// the other for each of its keys.
+__device__ Acc merge_overlap_lane(const MView& m, const int64_t* lam, const int64_t* s_lam,
+                                  int32_t r, int32_t s) {
   const int lane = lane_id();
   const bool r_short = m.cap[r] <= m.cap[s];
   const int32_t a1 = r_short ? r : s, a2 = r_short ? s : r;
   const Row R1 = m_row(m, a1), R2 = m_row(m, a2);
-  const bool direct = R1.c == m.B;
+  const bool direct = R1.c == m.B;  // then so is the longer row: key j sits at slot j of both
   Acc acc{0, 0};
-  if (direct) {  // then so is the longer row: key j sits at slot j of both
-    for (int32_t j = lane; j < R1.c; j += kWave) {
-      const Cnt c1 = m.cnt[R1.o + j], c2 = m.cnt[R2.o + j];
-      if (j == r || j == s) continue;
-      overlap_pair(acc, lam, c1.o, c2.o);
-      overlap_pair(acc, lam, c1.i, c2.i);
-    }
-    return acc;
-  }
-  // hashed shorter row: kOvl of its slots per lane, all their probes of
-  // the other row issued before any is resolved
-  constexpr int kOvl = 4;
+  constexpr int kOvl = 2;
   for (int32_t base = 0; base < R1.c; base += kOvl * kWave) {
     int32_t k[kOvl];
-    Cnt q[kOvl];
+    Cnt x[kOvl], y[kOvl];
 #pragma unroll
     for (int u = 0; u < kOvl; ++u) {
       const int32_t j = base + u * kWave + lane;
-      k[u] = j < R1.c ? m.key[R1.o + j] : -1;
-      q[u] = j < R1.c ? m.cnt[R1.o + j] : Cnt{0, 0};
+      k[u] = -1;
+      x[u] = y[u] = Cnt{0, 0};
+      if (j < R1.c) {
+        k[u] = direct ? j : m.key[R1.o + j];
+        x[u] = m.cnt[R1.o + j];
+        if (direct) y[u] = m.cnt[R2.o + j];
+      }
     }
-    Probe p[kOvl];
+    if (!direct) {
+      Probe p[kOvl];
+#pragma unroll
+      for (int u = 0; u < kOvl; ++u) {
+        if (x[u].o <= 0 && x[u].i <= 0) k[u] = -1;
+        if (k[u] >= 0) p[u] = m_probe(m, R2, k[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < kOvl; ++u)
+        if (k[u] >= 0) y[u] = m_value(m, R2, k[u], p[u]);
+    }
 #pragma unroll
     for (int u = 0; u < kOvl; ++u) {
-      if ((q[u].o <= 0 && q[u].i <= 0) || k[u] == r || k[u] == s) k[u] = -1;
-      if (k[u] >= 0) p[u] = m_probe(m, R2, k[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < kOvl; ++u) {
-      if (k[u] < 0) continue;
-      const Cnt c2 = m_value(m, R2, k[u], p[u]);
-      overlap_pair(acc, lam, q[u].o, c2.o);
-      overlap_pair(acc, lam, q[u].i, c2.i);
+      if (k[u] == r || k[u] == s) x[u] = Cnt{0, 0};
+      overlap_pair(acc, lam, s_lam, x[u], y[u]);
     }
   }
   return acc;
 }
 
-// Row r of a k_merge workgroup in LDS, shared by its K proposals: its
-// non-zero keys in ascending order with both counts and the running sum of
-// o + i (n = -1: the row has more than kRowLds non-zero keys and the
-// proposals read it from M).
+// A block's row in LDS, shared by its K proposals: its non-zero keys in
+// ascending order with both counts and the running sum of o + i (n = -1: the
+// row has more than kRowLds of them and the proposals read it from M).
 constexpr int kRowLds = 256;
 struct RowLds {
   const int32_t* k;
   const int32_t* o;
   const int32_t* i;
-  const long* cum;
+  const uint32_t* cum;
   int32_t n;
 };
 
-// Index of the first entry whose running sum exceeds t (t < the row's total).
-__device__ __forceinline__ int32_t rowlds_pick(const RowLds& L, int64_t t) {
+// Position of the first entry whose running sum exceeds t (t < the row's
+// total).
+__device__ __forceinline__ int32_t rowlds_pick(const RowLds& L, uint32_t t) {
   int32_t lo = 0, hi = L.n - 1;
   while (lo < hi) {
     const int32_t mid = (lo + hi) >> 1;
@@ -1983,11 +2006,11 @@ __device__ __forceinline__ int32_t rowlds_pick(const RowLds& L, int64_t t) {
     else
       lo = mid + 1;
   }
-  return L.k[lo];
+  return lo;
 }
 
-// Position of key b among the row's keys, or -1.
-__device__ __forceinline__ int32_t rowlds_find(const RowLds& L, int32_t b) {
+// The counts of key b in the row.
+__device__ __forceinline__ Cnt rowlds_find(const RowLds& L, int32_t b) {
   int32_t lo = 0, hi = L.n;
   while (lo < hi) {
     const int32_t mid = (lo + hi) >> 1;
@@ -1996,80 +2019,39 @@ __device__ __forceinline__ int32_t rowlds_find(const RowLds& L, int32_t b) {
     else
       hi = mid;
   }
-  return lo < L.n && L.k[lo] == b ? lo : -1;
+  return lo < L.n && L.k[lo] == b ? Cnt{L.o[lo], L.i[lo]} : Cnt{0, 0};
 }
 
-// merge_overlap_lane with row r from LDS: r's entries probe row s, or, when
-// s's slab is at most four times r's key count, s's slab is scanned and its
-// keys are looked up in r.
-__device__ Acc merge_overlap_lds(const MView& m, const int64_t* lam, int32_t r, int32_t s,
-                                  const RowLds& L) {
+// merge_overlap_lane with row r from LDS: r's entries look themselves up in
+// row s.
+__device__ Acc merge_overlap_lds(const MView& m, const int64_t* lam, const int64_t* s_lam,
+                                 int32_t r, int32_t s, Row RS, const RowLds& L) {
   const int lane = lane_id();
-  const Row RS = m_row(m, s);
+  const bool direct = RS.c == m.B;
   Acc acc{0, 0};
-  if (RS.c <= 4 * L.n) {
-    const bool direct = RS.c == m.B;
-    for (int32_t j = lane; j < RS.c; j += kWave) {
-      const Cnt q = m.cnt[RS.o + j];
-      const int32_t i = direct ? j : m.key[RS.o + j];
-      if (i < 0 || (q.o <= 0 && q.i <= 0) || i == r || i == s) continue;
-      const int32_t p = rowlds_find(L, i);
-      if (p < 0) continue;
-      overlap_pair(acc, lam, L.o[p], q.o);
-      overlap_pair(acc, lam, L.i[p], q.i);
-    }
-  } else {
-    for (int32_t e = lane; e < L.n; e += kWave) {
-      const int32_t i = L.k[e];
-      if (i == r || i == s) continue;
-      const Cnt c2 = m_value(m, RS, i, m_probe(m, RS, i));
-      overlap_pair(acc, lam, L.o[e], c2.o);
-      overlap_pair(acc, lam, L.i[e], c2.i);
-    }
+  for (int32_t e0 = 0; e0 < L.n; e0 += kWave) {
+    const int32_t e = min(e0 + lane, L.n - 1);
+    const int32_t b = L.k[e];
+    int32_t kk;
+    const Window w = win_issue(m, RS, b, direct);
+    const uint32_t h = win_end(w, b, direct, kk);
+    const bool in = e0 + lane < L.n && b != r && b != s;
+    Cnt x{0, 0}, y{0, 0};
+    if (in && kk == b)
+      y = m.cnt[RS.o + h];
+    else if (in && kk >= 0)
+      y = m_value_more(m, RS, b, h);
+    if (in) x = Cnt{L.o[e], L.i[e]};
+    overlap_pair(acc, lam, s_lam, x, y);
   }
   return acc;
 }
 
-__device__ void merge_one(const MergeArgs& a, int32_t r, int32_t idx, int32_t* scr,
-                          const RowLds& L, int32_t& s_out, i128& dS_out) {
-  const int32_t B = a.B;
-  const int32_t dor = a.d_out[r], dir = a.d_in[r];
-  const int64_t k = (int64_t)dor + dir;
-  uint64_t x[4];
-  if (a.uni)
-    predrawn(a.uni, a.stream + (uint64_t)r * (uint64_t)a.K + (uint64_t)idx, x);
-  else
-    usap::philox4x64((uint64_t)r, (uint64_t)idx, a.stream, usap::kTagMerge, a.seed, 0, x);
-  int32_t s;
-  if (k == 0) {
-    s = (int32_t)usap::idx_of(x[2], B);
-  } else {
-    long bytes = 0;
-    const int64_t t0 = (int64_t)usap::idx_of(x[0], k);
-    const int32_t u = L.n >= 0 ? rowlds_pick(L, t0) : select_combined<false>(a.M, r, (uint32_t)t0, -1, nullptr, scr, kScr, bytes);
-    const int64_t da = (int64_t)a.d_out[u] + a.d_in[u];
-    if (usap::uniform_branch(x[1], da, B)) {
-      s = usap::uniform_not_r(x[2], r, B);
-    } else {
-      const Cnt ur = m_get(a.M, u, r);  // M[u][r], M[r][u]
-      const int64_t W2 = da - ur.o - ur.i;
-      s = W2 == 0 ? usap::uniform_not_r(x[2], r, B)
-                  : select_combined<false>(a.M, u, idx32(x[3], (uint32_t)W2), r, nullptr, scr, kScr, bytes);
-    }
-  }
-  s_out = s;
-  if (s == r) {
-    dS_out = 0;
-    return;
-  }
-  const int64_t* lam = a.lam;
-  const Cnt crs = m_get(a.M, r, s);  // M[r][s], M[s][r]
-  const int32_t Mrr = m_get(a.M, r, r).o, Mrs = crs.o;
-  const int32_t Msr = crs.i, Mss = m_get(a.M, s, s).o;
-  const int32_t dos = a.d_out[s], dis = a.d_in[s];
+// The terms of merging r into s outside the overlap: corner and degrees.
+__device__ __forceinline__ void merge_terms(Acc& acc, const int64_t* lam, int32_t dor, int32_t dir,
+                                            int32_t dos, int32_t dis, int32_t Mrr, int32_t Mrs,
+                                            int32_t Msr, int32_t Mss) {
   const int32_t dos2 = dos + dor, dis2 = dis + dir;
-  const Acc ov = L.n >= 0 ? merge_overlap_lds(a.M, lam, r, s, L) : merge_overlap_lane(a.M, lam, r, s);
-  Acc acc{wave_sum(ov.h), wave_sum(ov.l)};
   bool inf = false;
   add_T(acc, lam, 1, Mrr, dir, dor, inf);
   add_T(acc, lam, 1, Mrs, dis, dor, inf);
@@ -2084,113 +2066,423 @@ __device__ void merge_one(const MergeArgs& a, int32_t r, int32_t idx, int32_t* s
   add_P(acc, lam, -1, Yr, dir, inf);
   add_P(acc, lam, -1, Ys, dis, inf);
   add_P(acc, lam, 1, Yr + Ys, dis2, inf);
+}
+
+__device__ __forceinline__ void merge_draw(const MergeArgs& a, int32_t r, int32_t idx,
+                                           uint64_t x[4]) {
+  if (a.uni)
+    predrawn(a.uni, a.stream + (uint64_t)r * (uint64_t)a.K + (uint64_t)idx, x);
+  else
+    usap::philox4x64((uint64_t)r, (uint64_t)idx, a.stream, usap::kTagMerge, a.seed, 0, x);
+}
+
+// One proposal by one wavefront (kD: every row is direct).
+template <bool kD>
+__device__ void merge_one(const MergeArgs& a, int32_t r, int32_t idx, int32_t* scr,
+                          const RowLds& L, const int64_t* s_lam, int32_t& s_out, i128& dS_out) {
+  const int32_t B = a.B;
+  const int32_t dor = a.d_out[r], dir = a.d_in[r];
+  const uint32_t k = (uint32_t)dor + (uint32_t)dir;
+  uint64_t x[4];
+  merge_draw(a, r, idx, x);
+  int32_t s;
+  if (k == 0) {
+    s = (int32_t)usap::idx_of(x[2], B);
+  } else {
+    long bytes = 0;
+    const uint32_t t0 = idx32(x[0], k);
+    const int32_t u = L.n >= 0 ? L.k[rowlds_pick(L, t0)]
+                               : select_combined<kD>(a.M, r, t0, -1, nullptr, scr, kScr, bytes);
+    const uint32_t da = (uint32_t)a.d_out[u] + (uint32_t)a.d_in[u];
+    if (usap::uniform_branch(x[1], da, B)) {
+      s = usap::uniform_not_r(x[2], r, B);
+    } else {
+      const Cnt ur = L.n >= 0 ? rowlds_find(L, u) : m_get(a.M, r, u);  // M[r][u], M[u][r]
+      const uint32_t W2 = da - (uint32_t)ur.o - (uint32_t)ur.i;
+      s = W2 == 0 ? usap::uniform_not_r(x[2], r, B)
+                  : select_combined<kD>(a.M, u, idx32(x[3], W2), r, nullptr, scr, kScr, bytes);
+    }
+  }
+  s_out = s;
+  if (s == r) {
+    dS_out = 0;
+    return;
+  }
+  const Row RS = m_row(a.M, s);
+  const Cnt crs = L.n >= 0 ? rowlds_find(L, s) : m_get(a.M, r, s);  // M[r][s], M[s][r]
+  const int32_t Mrr = L.n >= 0 ? rowlds_find(L, r).o : m_get(a.M, r, r).o;
+  const int32_t Mss = m_value(a.M, RS, s, m_probe(a.M, RS, s)).o;
+  const int32_t dos = a.d_out[s], dis = a.d_in[s];
+  const Acc ov = L.n >= 0 ? merge_overlap_lds(a.M, a.lam, s_lam, r, s, RS, L)
+                          : merge_overlap_lane(a.M, a.lam, s_lam, r, s);
+  Acc acc{wave_sum(ov.h), wave_sum(ov.l)};
+  merge_terms(acc, a.lam, dor, dir, dos, dis, Mrr, crs.o, crs.i, Mss);
   dS_out = acc_value(acc);
 }
 
-__global__ __launch_bounds__(kWave* kMergeWaves, 5) void k_merge(MergeArgs a) {
-  __shared__ long s_hi[kMergeWaves];
-  __shared__ unsigned long s_lo[kMergeWaves];
-  __shared__ int32_t s_idx[kMergeWaves];
-  __shared__ int32_t s_s[kMergeWaves];
-  __shared__ int32_t s_scr[kMergeWaves][kScr];
-  __shared__ int32_t s_rk[kRowLds], s_ro[kRowLds], s_ri[kRowLds];
-  __shared__ long s_cum[kRowLds];
+// The K proposals of a block by one workgroup, a wavefront each in turn: every
+// block (list null), or those k_merge_rows left to it.  kWaves: 4, or, where
+// the blocks are too few to fill the GPU, up to 16, so that all of a block's
+// proposals run at once (B = 42: 26 -> 13 us a round).
+template <int kWaves, bool kD>
+__global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(
+    MergeArgs a, const int32_t* list, const int32_t* list_n) {
+  __shared__ long s_hi[kWaves];
+  __shared__ unsigned long s_lo[kWaves];
+  __shared__ int32_t s_idx[kWaves];
+  __shared__ int32_t s_s[kWaves];
+  __shared__ __align__(16) int32_t s_scr[kWaves][kD ? 4 : kScr];  // direct rows need none
+  __shared__ __align__(16) int32_t s_rk[kRowLds], s_ro[kRowLds], s_ri[kRowLds];
+  __shared__ uint32_t s_cum[kRowLds];
+  __shared__ int64_t s_lam[kLamMerge];
   __shared__ int32_t s_rn;
-  const int32_t r = blockIdx.x;
-  const int w = threadIdx.x / kWave;
+  const int w = threadIdx.x / kWave, lane = lane_id();
   const int nw = blockDim.x / kWave;
-  // row r's non-zero keys into LDS once for the K proposals (unordered), then
-  // ordered by key (ranks: keys are distinct), then the running sums
-  const Row R = m_row(a.M, r);
-  const bool fits = R.c <= 8 * kRowLds;  // the same for every thread
-  if (threadIdx.x == 0) s_rn = 0;
-  __syncthreads();
-  if (fits) {
-    const bool direct = R.c == a.B;
-    for (int32_t j = threadIdx.x; j < R.c; j += blockDim.x) {
-      const Cnt q = a.M.cnt[R.o + j];
-      const int32_t key = direct ? j : a.M.key[R.o + j];
-      if (key >= 0 && (q.o > 0 || q.i > 0)) {
-        const int32_t p = atomicAdd(&s_rn, 1);
-        if (p < kRowLds) {
-          s_rk[p] = key;
-          s_ro[p] = q.o;
-          s_ri[p] = q.i;
+  for (int i = threadIdx.x; i < kLamMerge; i += blockDim.x) s_lam[i] = a.lam[min(i, a.lam_last)];
+  const int32_t count = list ? *list_n : a.B;
+  for (int32_t item = blockIdx.x; item < count; item += gridDim.x) {
+    const int32_t r = list ? list[item] : item;
+    // row r's non-zero keys into LDS once for the K proposals (unordered), then
+    // ordered by key (ranks: keys are distinct), then the running sums
+    const Row R = m_row(a.M, r);
+    const bool fits = R.c <= 8 * kRowLds;  // the same for every thread
+    __syncthreads();
+    if (threadIdx.x == 0) s_rn = 0;
+    __syncthreads();
+    if (fits) {
+      const bool direct = R.c == a.B;
+      for (int32_t j = threadIdx.x; j < R.c; j += blockDim.x) {
+        const Cnt q = a.M.cnt[R.o + j];
+        const int32_t key = direct ? j : a.M.key[R.o + j];
+        if (key >= 0 && (q.o > 0 || q.i > 0)) {
+          const int32_t p = atomicAdd(&s_rn, 1);
+          if (p < kRowLds) {
+            s_rk[p] = key;
+            s_ro[p] = q.o;
+            s_ri[p] = q.i;
+          }
         }
       }
     }
-  }
-  __syncthreads();
-  const int32_t rn = fits ? s_rn : kRowLds + 1;
-  RowLds L{s_rk, s_ro, s_ri, s_cum, rn <= kRowLds ? rn : -1};
-  if (L.n > 0) {
-    constexpr int kPer = kRowLds / kWave;  // entries per thread (blockDim >= one wavefront)
-    int32_t mk[kPer], mo[kPer], mi[kPer], rank[kPer];
+    __syncthreads();
+    const int32_t rn = fits ? s_rn : kRowLds + 1;
+    RowLds L{s_rk, s_ro, s_ri, s_cum, rn <= kRowLds ? rn : -1};
+    if (L.n > 0) {
+      constexpr int kPer = kRowLds / kWave;  // entries per thread (blockDim >= one wavefront)
+      int32_t mk[kPer], mo[kPer], mi[kPer], rank[kPer];
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      const int32_t e = threadIdx.x + q * blockDim.x;
-      rank[q] = -1;
-      if (e < L.n) {
-        mk[q] = s_rk[e];
-        mo[q] = s_ro[e];
-        mi[q] = s_ri[e];
-        rank[q] = 0;
-        for (int32_t j = 0; j < L.n; ++j) rank[q] += s_rk[j] < mk[q];
+      for (int q = 0; q < kPer; ++q) {
+        const int32_t e = threadIdx.x + q * blockDim.x;
+        rank[q] = -1;
+        if (e < L.n) {
+          mk[q] = s_rk[e];
+          mo[q] = s_ro[e];
+          mi[q] = s_ri[e];
+          rank[q] = 0;
+          for (int32_t j = 0; j < L.n; ++j) rank[q] += s_rk[j] < mk[q];
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < kPer; ++q) {
+        if (rank[q] < 0) continue;
+        s_rk[rank[q]] = mk[q];
+        s_ro[rank[q]] = mo[q];
+        s_ri[rank[q]] = mi[q];
+      }
+      __syncthreads();
+      if (w == 0) {
+        uint32_t v[kPer], own = 0;
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+          const int32_t e = lane * kPer + q;
+          own += e < L.n ? (uint32_t)s_ro[e] + (uint32_t)s_ri[e] : 0u;
+          v[q] = own;
+        }
+        const uint32_t before = wave_incl_scan32(own) - own;
+#pragma unroll
+        for (int q = 0; q < kPer; ++q)
+          if (lane * kPer + q < L.n) s_cum[lane * kPer + q] = before + v[q];
+      }
+      __syncthreads();
+    }
+    int32_t bidx = -1, bs = -1;
+    i128 bd = 0;
+    for (int32_t idx = w; idx < a.K; idx += nw) {
+      int32_t s;
+      i128 d;
+      merge_one<kD>(a, r, idx, s_scr[w], L, s_lam, s, d);
+      if (bidx < 0 || d < bd) {  // strict less: the earliest proposal wins ties
+        bidx = idx;
+        bs = s;
+        bd = d;
       }
     }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      if (rank[q] < 0) continue;
-      s_rk[rank[q]] = mk[q];
-      s_ro[rank[q]] = mo[q];
-      s_ri[rank[q]] = mi[q];
+    if (lane == 0) {
+      s_hi[w] = (long)(bd >> 64);
+      s_lo[w] = (unsigned long)(u128)bd;
+      s_idx[w] = bidx;
+      s_s[w] = bs;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-      long c = 0;
-      for (int32_t j = 0; j < L.n; ++j) {
-        c += (long)s_ro[j] + s_ri[j];
-        s_cum[j] = c;
+      int best = -1;
+      i128 bv = 0;
+      for (int i = 0; i < nw; ++i) {
+        if (s_idx[i] < 0) continue;
+        const i128 v = (i128)(((u128)(unsigned long)s_hi[i] << 64) | (u128)s_lo[i]);
+        if (best < 0 || v < bv || (v == bv && s_idx[i] < s_idx[best])) {
+          best = i;
+          bv = v;
+        }
+      }
+      a.best_s[r] = s_s[best];
+      a.best_hi[r] = s_hi[best];
+      a.best_lo[r] = s_lo[best];
+    }
+  }
+}
+
+// The K proposals of a block by one wavefront, for hashed rows of at most
+// kRowSlots slots with at most kRowLds non-zero keys (the others go to `list`
+// for k_merge).  Proposal j's draws, picks, decision, corner and degree terms
+// are lane j's; only a multinomial pick and the overlap are the whole
+// wavefront's, proposal by proposal, the overlap two proposals at a time: r's
+// entries look themselves up in row s, whose eight-key windows nearly always
+// answer in one round of loads, mostly that there is nothing (s is a uniform
+// draw most often).  A workgroup per block with a wavefront per proposal spent
+// its time in the same chain K times over, three proposals one after another
+// per wavefront, Philox and terms in every lane: B = 200000 4890 -> 1150 us a
+// round.
+constexpr int kRowSlots = 1024;
+__global__ __launch_bounds__(kWave* kMergeWaves, 4) void k_merge_rows(MergeArgs a, int32_t* list,
+                                                                    int32_t* list_n) {
+  __shared__ __align__(16) int32_t s_k[kMergeWaves][kRowLds], s_o[kMergeWaves][kRowLds],
+      s_i[kMergeWaves][kRowLds];
+  __shared__ uint32_t s_cum[kMergeWaves][kRowLds];
+  __shared__ __align__(16) int32_t s_scr[kMergeWaves][kScr];
+  __shared__ int64_t s_lam[kLamMerge];
+  const int w = threadIdx.x / kWave, lane = lane_id();
+  for (int i = threadIdx.x; i < kLamMerge; i += blockDim.x) s_lam[i] = a.lam[min(i, a.lam_last)];
+  const int32_t B = a.B;
+  const int32_t r = blockIdx.x * kMergeWaves + w;
+  const bool in = r < B;
+  const Row R = m_row(a.M, in ? r : 0);
+  const int32_t dor = in ? a.d_out[r] : 0, dir = in ? a.d_in[r] : 0;
+  __syncthreads();
+  if (!in) return;
+  if (R.c == B || R.c > kRowSlots) {
+    if (lane == 0) list[atomicAdd(list_n, 1)] = r;
+    return;
+  }
+  // the row's non-zero entries, unordered
+  int32_t n = 0;
+  constexpr int kQ = 4;
+  for (int32_t base = 0; base < R.c; base += kQ * kWave) {
+    int32_t key[kQ];
+    Cnt x[kQ];
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      const int32_t j = base + q * kWave + lane;
+      key[q] = -1;
+      x[q] = Cnt{0, 0};
+      if (j < R.c) {
+        key[q] = a.M.key[R.o + j];
+        x[q] = a.M.cnt[R.o + j];
       }
     }
-    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) {
+      const bool live = key[q] >= 0 && (x[q].o > 0 || x[q].i > 0);
+      const unsigned long long m = __ballot(live);
+      const int32_t p = n + __popcll(m & ((1ull << lane) - 1ull));
+      if (live && p < kRowLds) {
+        s_k[w][p] = key[q];
+        s_o[w][p] = x[q].o;
+        s_i[w][p] = x[q].i;
+      }
+      n += __popcll(m);
+    }
   }
-  int32_t bidx = -1, bs = -1;
+  if (n > kRowLds) {
+    if (lane == 0) list[atomicAdd(list_n, 1)] = r;
+    return;
+  }
+  wave_fence();
+  // ordered by key
+  constexpr int kPer = kRowLds / kWave;
+  {
+    int32_t mk[kPer], mo[kPer], mi[kPer], rank[kPer];
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      const int32_t e = lane + q * kWave;
+      rank[q] = 0;
+      mk[q] = e < n ? s_k[w][e] : 0;
+      mo[q] = e < n ? s_o[w][e] : 0;
+      mi[q] = e < n ? s_i[w][e] : 0;
+    }
+    for (int32_t j = 0; j < n; ++j) {
+      const int32_t k = s_k[w][j];
+#pragma unroll
+      for (int q = 0; q < kPer; ++q) rank[q] += k < mk[q];
+    }
+    wave_fence();
+#pragma unroll
+    for (int q = 0; q < kPer; ++q)
+      if (lane + q * kWave < n) {
+        s_k[w][rank[q]] = mk[q];
+        s_o[w][rank[q]] = mo[q];
+        s_i[w][rank[q]] = mi[q];
+      }
+    wave_fence();
+    uint32_t v[kPer], own = 0;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      const int32_t e = lane * kPer + q;
+      own += e < n ? (uint32_t)s_o[w][e] + (uint32_t)s_i[w][e] : 0u;
+      v[q] = own;
+    }
+    const uint32_t before = wave_incl_scan32(own) - own;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q)
+      if (lane * kPer + q < n) s_cum[w][lane * kPer + q] = before + v[q];
+    wave_fence();
+  }
+  const RowLds L{s_k[w], s_o[w], s_i[w], s_cum[w], n};
+  const int32_t Mrr = rowlds_find(L, r).o;
+  const uint32_t k = (uint32_t)dor + (uint32_t)dir;
+  int32_t bidx = -1, bs = -1;  // the best so far, in every lane
   i128 bd = 0;
-  for (int32_t idx = w; idx < a.K; idx += nw) {
-    int32_t s;
-    i128 d;
-    merge_one(a, r, idx, s_scr[w], L, s, d);
-    if (bidx < 0 || d < bd) {  // strict less: the earliest proposal wins ties
+  for (int32_t j0 = 0; j0 < a.K; j0 += kWave) {
+    const int32_t m = min(a.K - j0, kWave);
+    const bool act = lane < m;
+    uint64_t x[4];
+    merge_draw(a, r, j0 + (act ? lane : 0), x);
+    int32_t s, u = 0;
+    uint32_t t = 0;
+    bool pend = false;
+    if (k == 0) {
+      s = (int32_t)usap::idx_of(x[2], B);
+    } else {
+      const int32_t e = rowlds_pick(L, idx32(x[0], k));
+      u = L.k[e];
+      const uint32_t da = (uint32_t)a.d_out[u] + (uint32_t)a.d_in[u];
+      s = usap::uniform_not_r(x[2], r, B);
+      if (!usap::uniform_branch(x[1], da, B)) {
+        const uint32_t W2 = da - (uint32_t)L.o[e] - (uint32_t)L.i[e];
+        pend = W2 != 0;
+        t = pend ? idx32(x[3], W2) : 0;
+      }
+    }
+    for (unsigned long long todo = __ballot(act && pend); todo; todo &= todo - 1ull) {
+      const int l = __ffsll(todo) - 1;
+      long bytes = 0;
+      const int32_t sel = select_combined<false>(a.M, __builtin_amdgcn_readlane(u, l),
+                                                 read_lane32(t, l), r, nullptr, s_scr[w], kScr,
+                                                 bytes);
+      if (lane == l) s = sel;
+    }
+    const bool move = act && s != r;
+    const Row RS = m_row(a.M, move ? s : r);
+    const int32_t dos = a.d_out[move ? s : r], dis = a.d_in[move ? s : r];
+    const bool sdir = RS.c == B;
+    int32_t Mss = 0;
+    if (move) {
+      int32_t kk;
+      const Window win = win_issue(a.M, RS, s, sdir);
+      const uint32_t h = win_end(win, s, sdir, kk);
+      if (kk == s)
+        Mss = a.M.cnt[RS.o + h].o;
+      else if (kk >= 0)
+        Mss = m_value_more(a.M, RS, s, h).o;
+    }
+    const Cnt crs = rowlds_find(L, s);  // M[r][s], M[s][r]
+    Acc acc{0, 0};
+    if (move) merge_terms(acc, a.lam, dor, dir, dos, dis, Mrr, crs.o, crs.i, Mss);
+    // overlaps, two proposals at a time
+    unsigned long long todo = __ballot(move);
+    while (todo) {
+      int l[2];
+      l[0] = __ffsll(todo) - 1;
+      todo &= todo - 1ull;
+      l[1] = todo ? __ffsll(todo) - 1 : -1;
+      todo &= todo - 1ull;
+      int32_t ss[2];
+      Row S[2];
+      bool dirct[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int from = l[i] < 0 ? l[0] : l[i];
+        ss[i] = __builtin_amdgcn_readlane(s, from);
+        S[i] = Row{read_lane((long)RS.o, from), __builtin_amdgcn_readlane(RS.c, from)};
+        dirct[i] = S[i].c == B;
+      }
+      Acc ov[2] = {{0, 0}, {0, 0}};
+      bool any[2] = {false, false};
+      for (int32_t e0 = 0; e0 < n; e0 += kWave) {
+        const int32_t e = min(e0 + lane, n - 1);
+        const int32_t b = L.k[e];
+        Window win[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) win[i] = win_issue(a.M, S[i], b, dirct[i]);
+        Cnt y[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          int32_t kk;
+          const uint32_t h = win_end(win[i], b, dirct[i], kk);
+          const bool ok = l[i] >= 0 && e0 + lane < n && b != r && b != ss[i];
+          y[i] = Cnt{0, 0};
+          if (ok && kk == b)
+            y[i] = a.M.cnt[S[i].o + h];
+          else if (ok && kk >= 0)
+            y[i] = m_value_more(a.M, S[i], b, h);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          if (!__ballot(y[i].o != 0 || y[i].i != 0)) continue;
+          any[i] = true;
+          overlap_pair(ov[i], a.lam, s_lam, Cnt{L.o[e], L.i[e]}, y[i]);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if (!any[i]) continue;
+        const long h = wave_sum(ov[i].h), lo = wave_sum(ov[i].l);
+        if (lane == l[i]) {
+          acc.h += h;
+          acc.l += lo;
+        }
+      }
+    }
+    // the least dS; the earliest proposal wins ties
+    i128 d = act ? acc_value(acc) : (i128)0;
+    int32_t idx = act ? j0 + lane : -1, sv = s;
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+      const long h2 = __shfl_xor((long)(d >> 64), off);
+      const unsigned long l2 = __shfl_xor((unsigned long)(u128)d, off);
+      const int32_t i2 = __shfl_xor(idx, off), s2 = __shfl_xor(sv, off);
+      const i128 d2 = (i128)(((u128)(unsigned long)h2 << 64) | (u128)l2);
+      if (i2 >= 0 && (idx < 0 || d2 < d || (d2 == d && i2 < idx))) {
+        d = d2;
+        idx = i2;
+        sv = s2;
+      }
+    }
+    if (bidx < 0 || d < bd) {
       bidx = idx;
-      bs = s;
+      bs = sv;
       bd = d;
     }
   }
-  if (lane_id() == 0) {
-    s_hi[w] = (long)(bd >> 64);
-    s_lo[w] = (unsigned long)(u128)bd;
-    s_idx[w] = bidx;
-    s_s[w] = bs;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int best = -1;
-    i128 bv = 0;
-    for (int i = 0; i < nw; ++i) {
-      if (s_idx[i] < 0) continue;
-      const i128 v = (i128)(((u128)(unsigned long)s_hi[i] << 64) | (u128)s_lo[i]);
-      if (best < 0 || v < bv || (v == bv && s_idx[i] < s_idx[best])) {
-        best = i;
-        bv = v;
-      }
-    }
-    a.best_s[r] = s_s[best];
-    a.best_hi[r] = s_hi[best];
-    a.best_lo[r] = s_lo[best];
+  if (lane == 0) {
+    a.best_s[r] = bs;
+    a.best_hi[r] = (long)(bd >> 64);
+    a.best_lo[r] = (unsigned long)(u128)bd;
   }
 }
+
+__global__ void k_zero1(int32_t* p) { *p = 0; }
 
 // ---------------------------------------------------------------------------
 // Nodal proposal, graph_parallel.hpp:990-1222
@@ -5759,6 +6051,7 @@ int usap_merge_propose(usap_engine* e, int32_t K, uint64_t stream, int32_t* best
   a.d_out = e->d_out;
   a.d_in = e->d_in;
   a.lam = e->lam;
+  a.lam_last = (int32_t)std::min<int64_t>(e->Wtot, kLamMerge - 1);
   a.B = B;
   a.K = K;
   a.seed = e->p.seed;
@@ -5775,9 +6068,20 @@ int usap_merge_propose(usap_engine* e, int32_t K, uint64_t stream, int32_t* best
   a.best_s = e->best_s;
   a.best_hi = e->best_hi;
   a.best_lo = e->best_lo;
-  const int nw = std::min(K, kMergeWaves);
   ev_rec(e, 0);
-  k_merge<<<B, nw * kWave, 0, e->stream>>>(a);
+  if (!e->all_direct) {
+    // hashed rows by wavefronts; what they leave (direct or large rows) by the
+    // workgroups of a grid that fills the GPU (the rebuild's arrays are scratch)
+    int32_t *list = e->ecnt_out, *list_n = e->build_flags + 2;
+    k_zero1<<<1, 1, 0, e->stream>>>(list_n);
+    k_merge_rows<<<blocks_for(B, kMergeWaves), kMergeWaves * kWave, 0, e->stream>>>(a, list, list_n);
+    k_merge<kMergeWaves, false><<<(unsigned)std::min<int32_t>(B, 1280), std::min(K, kMergeWaves) * kWave, 0,
+                           e->stream>>>(a, list, list_n);
+  } else if (B <= kMergeFew && K > kMergeWaves) {
+    k_merge<kMergeMany, true><<<B, std::min(K, kMergeMany) * kWave, 0, e->stream>>>(a, nullptr, nullptr);
+  } else {
+    k_merge<kMergeWaves, true><<<B, std::min(K, kMergeWaves) * kWave, 0, e->stream>>>(a, nullptr, nullptr);
+  }
   HIPCHK(hipGetLastError());
   if (e->uni) e->uni_pos += (int64_t)B * K;
   ev_rec(e, 1);
