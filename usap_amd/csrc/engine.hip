@@ -916,45 +916,77 @@ __device__ int32_t pick_neighbor(const GraphView& g, int64_t o0, int64_t kco, in
 // M build
 // ---------------------------------------------------------------------------
 
-// Block degrees, edge counts and node counts from the labels; counters are
-// privatised in LDS when B is small (many nodes share a block).
-__global__ __launch_bounds__(256) void k_degrees(GraphView g, const int32_t* __restrict__ labels,
-                                                 int32_t B, int32_t* d_out, int32_t* d_in,
-                                                 int32_t* ecnt_out, int32_t* ecnt_in,
-                                                 int32_t* bsize) {
-  __shared__ int32_t s_c[5][kDegLds];
-  const bool lds = B <= kDegLds;
-  if (lds) {
-    for (int i = threadIdx.x; i < 5 * kDegLds; i += blockDim.x) (&s_c[0][0])[i] = 0;
-    __syncthreads();
+// A workgroup's nodes by block: slot of block a in the LDS hash `key` of kSlots
+// slots (-1: empty) with room for every node of the workgroup.
+template <int kSlots>
+__device__ __forceinline__ uint32_t block_slot(int32_t* key, int32_t a) {
+  uint32_t h = hash32(a) & (kSlots - 1);
+  for (;;) {
+    const int32_t old = atomicCAS(&key[h], -1, a);
+    if (old == -1 || old == a) return h;
+    h = (h + 1) & (kSlots - 1);
   }
-  int32_t* dst[5] = {d_out, d_in, ecnt_out, ecnt_in, bsize};
-  for (int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; x < g.N;
-       x += (int64_t)gridDim.x * blockDim.x) {
+}
+
+// Block degrees, list entries (weighted graphs; else they are the degrees) and
+// node counts from the labels, `per` nodes to a workgroup, summed in LDS first:
+// for B <= kDegLds by block, above in a hash of the workgroup's blocks.  A block
+// that absorbed 7000 nodes in one merge phase (B = 100000) would take as many
+// atomics on one address, ~30 ns each: 363 -> 24 us.  kW: 16 lanes sum a node's
+// weights (one lane a node waited for each weight in turn: N = 3000 with hubs
+// of 1000 edges 86 -> 13 us).
+constexpr int kNodesWg = 1024;
+constexpr int kNodesWgW = 256;
+constexpr int kWSum = 16;  // lanes per weighted node
+template <bool kW, bool kHash>
+__global__ __launch_bounds__(256) void k_degrees(GraphView g, const int32_t* __restrict__ labels,
+                                                 int32_t B, int32_t per, int32_t* d_out,
+                                                 int32_t* d_in, int32_t* ecnt_out,
+                                                 int32_t* ecnt_in, int32_t* bsize) {
+  constexpr int kC = kW ? 5 : 3;  // counters
+  constexpr int kSlots = kHash ? 2 * (kW ? kNodesWgW : kNodesWg) : kDegLds;
+  __shared__ int32_t s_c[kC][kSlots];
+  __shared__ int32_t s_key[kHash ? kSlots : 1];
+  for (int i = threadIdx.x; i < kC * kSlots; i += 256) (&s_c[0][0])[i] = 0;
+  if (kHash)
+    for (int i = threadIdx.x; i < kSlots; i += 256) s_key[i] = -1;
+  __syncthreads();
+  const int64_t beg = (int64_t)blockIdx.x * per, end = min<int64_t>(beg + per, g.N);
+  constexpr int kL = kW ? kWSum : 1;
+  for (int64_t x = beg + threadIdx.x / kL; x < end; x += 256 / kL) {
     const int32_t a = labels[x];
     const int64_t o0 = g.out_ptr[x], o1 = g.out_ptr[x + 1];
     const int64_t i0 = g.in_ptr[x], i1 = g.in_ptr[x + 1];
-    int64_t wo = o1 - o0, wi = i1 - i0;
-    if (g.out_w) {
-      wo = 0;
-      wi = 0;
-      for (int64_t e = o0; e < o1; ++e) wo += g.out_w[e];
-      for (int64_t e = i0; e < i1; ++e) wi += g.in_w[e];
+    int32_t v[5] = {(int32_t)(o1 - o0), (int32_t)(i1 - i0), 1, (int32_t)(o1 - o0),
+                    (int32_t)(i1 - i0)};
+    if (kW) {
+      const int sub = threadIdx.x % kL;
+      v[0] = v[1] = 0;
+      for (int64_t e = o0 + sub; e < o1; e += kL) v[0] += g.out_w[e];
+      for (int64_t e = i0 + sub; e < i1; e += kL) v[1] += g.in_w[e];
+#pragma unroll
+      for (int d = kL / 2; d > 0; d >>= 1) {  // a node's lanes loop alike
+        v[0] += __shfl_xor(v[0], d);
+        v[1] += __shfl_xor(v[1], d);
+      }
+      if (sub != 0) continue;
     }
-    const int32_t v[5] = {(int32_t)wo, (int32_t)wi, (int32_t)(o1 - o0), (int32_t)(i1 - i0), 1};
-    for (int k = 0; k < 5; ++k) {
-      if (!v[k]) continue;
-      if (lds)
-        atomicAdd(&s_c[k][a], v[k]);
-      else
-        atomicAdd(&dst[k][a], v[k]);
-    }
+    const uint32_t h = kHash ? block_slot<kSlots>(s_key, a) : (uint32_t)a;
+#pragma unroll
+    for (int k = 0; k < kC; ++k)
+      if (v[k]) atomicAdd(&s_c[k][h], v[k]);
   }
-  if (lds) {
-    __syncthreads();
-    for (int32_t b = threadIdx.x; b < B; b += blockDim.x)
-      for (int k = 0; k < 5; ++k)
-        if (s_c[k][b]) atomicAdd(&dst[k][b], s_c[k][b]);
+  __syncthreads();
+  int32_t* dst[5] = {d_out, d_in, bsize, ecnt_out, ecnt_in};
+  const int32_t n = kHash ? kSlots : B;
+  for (int32_t i = threadIdx.x; i < n; i += 256) {
+    const int32_t a = kHash ? s_key[i] : i;
+    if (a < 0) continue;
+#pragma unroll
+    for (int k = 0; k < kC; ++k) {
+      const int32_t v = s_c[k][i];
+      if (v) atomicAdd(&dst[k][a], v);
+    }
   }
 }
 
@@ -971,8 +1003,18 @@ __device__ __forceinline__ int32_t cap_for(int32_t B, int32_t ecnt, int32_t slac
 
 // Block row a holds the keys of its out-edges and of its in-edges: its slab
 // is sized for ecnt_out[a] + ecnt_in[a] keys.
+// items (if not null): the pieces of the rows k_build_big builds, kBigNodes
+// nodes each.
+constexpr int kBigNodes = 64;
+__device__ __forceinline__ int32_t big_pieces(int32_t nodes) {
+  return max(1, (nodes + kBigNodes - 1) / kBigNodes);
+}
+constexpr int kRowTab = 1024;
+__device__ __forceinline__ bool lds_row(int32_t cap, int32_t B) { return cap < B && cap <= kRowTab; }
+
 __global__ void k_caps(int32_t B, int32_t slack, const int32_t* ecnt_out, const int32_t* ecnt_in,
-                       int32_t* cap, int64_t* tmp) {
+                       const int32_t* bsize, int32_t* cap, int64_t* tmp, int2* items,
+                       int32_t* n_items) {
   const int32_t a = blockIdx.x * blockDim.x + threadIdx.x;
   if (a > B) return;
   if (a == B) {
@@ -983,6 +1025,11 @@ __global__ void k_caps(int32_t B, int32_t slack, const int32_t* ecnt_out, const 
   const int32_t c = cap_for(B, (int32_t)min<int64_t>(ec, (int64_t)B), slack);
   cap[a] = c;
   tmp[a] = c;
+  if (items && !lds_row(c, B)) {
+    const int32_t k = big_pieces(bsize[a]);
+    const int32_t p = atomicAdd(n_items, k);
+    for (int32_t i = 0; i < k; ++i) items[p + i] = make_int2(a, i);
+  }
 }
 
 // key null: every row is direct, no key is read.
@@ -994,58 +1041,59 @@ __global__ void k_fill(int32_t* key, Cnt* cnt, int64_t n) {
   }
 }
 
-// Edge u -> v between blocks a -> b: o of row a at key b and i of row b at
-// key a (one update when a == b).
-// A row that k_build_rows lays out in LDS: hashed, at most kRowTab slots.
-constexpr int kRowTab = 1024;
-__device__ __forceinline__ bool lds_row(int32_t cap, int32_t B) { return cap < B && cap <= kRowTab; }
-
-// kSkipLds: only the rows k_build_rows does not build (direct, or hashed
-// above kRowTab slots), which may hold many nodes: edge by edge keeps them
-// load-balanced.
-template <bool kSkipLds>
-__global__ void k_insert_edges(int64_t E, const int32_t* __restrict__ src,
-                               const int32_t* __restrict__ dst, const int32_t* __restrict__ w,
-                               const int32_t* __restrict__ labels, MView M, int32_t* flags) {
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < E;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    const int32_t a = labels[src[e]];
-    const int32_t b = labels[dst[e]];
-    const int32_t ww = w ? w[e] : 1;
-    const bool ia = !kSkipLds || !lds_row(M.cap[a], M.B);
-    const bool ib = !kSkipLds || !lds_row(M.cap[b], M.B);
-    if (a == b) {
-      if (ia) m_add(M, a, a, ww, ww, flags);
-    } else {
-      if (ia) m_add(M, a, b, ww, 0, flags);
-      if (ib) m_add(M, b, a, 0, ww, flags);
+// Nodes grouped by block (for the per-row build): node x goes to
+// nodes[off[labels[x]] + k], k an arrival order in its block, counted by
+// workgroup in LDS first (as k_degrees: 292 -> 11 us).
+__global__ __launch_bounds__(256) void k_node_lists(int32_t N, const int32_t* __restrict__ labels,
+                                                    const int32_t* __restrict__ off, int32_t* cur,
+                                                    int32_t* nodes) {
+  __shared__ int32_t s_key[2 * kNodesWg], s_n[2 * kNodesWg];
+  for (int i = threadIdx.x; i < 2 * kNodesWg; i += 256) {
+    s_key[i] = -1;
+    s_n[i] = 0;
+  }
+  __syncthreads();
+  constexpr int kQ = kNodesWg / 256;
+  uint32_t h[kQ];
+  int32_t rank[kQ];
+#pragma unroll
+  for (int q = 0; q < kQ; ++q) {
+    const int64_t x = (int64_t)blockIdx.x * kNodesWg + q * 256 + threadIdx.x;
+    rank[q] = -1;
+    if (x < N) {
+      h[q] = block_slot<2 * kNodesWg>(s_key, labels[x]);
+      rank[q] = atomicAdd(&s_n[h[q]], 1);
     }
   }
-}
-
-// Nodes grouped by block (for the per-row build): node x goes to
-// nodes[off[labels[x]] + k], k its arrival order in its block.
-__global__ void k_node_lists(int32_t N, const int32_t* __restrict__ labels,
-                             const int32_t* __restrict__ off, int32_t* cur, int32_t* nodes) {
-  for (int32_t x = blockIdx.x * blockDim.x + threadIdx.x; x < N; x += gridDim.x * blockDim.x) {
-    const int32_t a = labels[x];
-    nodes[off[a] + atomicAdd(&cur[a], 1)] = x;
+  __syncthreads();
+#pragma unroll
+  for (int i = threadIdx.x; i < 2 * kNodesWg; i += 256) {
+    const int32_t a = s_key[i];
+    if (a >= 0) s_n[i] = off[a] + atomicAdd(&cur[a], s_n[i]);
   }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kQ; ++q)
+    if (rank[q] >= 0)
+      nodes[s_n[h[q]] + rank[q]] =
+          (int32_t)((int64_t)blockIdx.x * kNodesWg + q * 256 + threadIdx.x);
 }
 
-// M build for large B: each hashed row of at most kRowTab slots by one
-// wavefront, from the lists of the row's own nodes alone -- an out-edge
+// M build for large B: each hashed row of more than kMin and at most kSlots
+// slots by one wavefront, from the lists of the row's own nodes alone -- an out-edge
 // x -> v adds to M[a][label v] (o), an in-edge u -> x to M[label u][a] (i) --
 // laid out in LDS and written out whole (a slab that size holds at most
-// (kRowTab - 16) / 2 list entries, so no wavefront has a long row).  The
-// per-edge build sends every edge to two rows' slabs at random instead; it
-// still builds the other rows (k_insert_edges<true>).
+// (kRowTab - 16) / slack list entries, so no wavefront has a long row).  Sending
+// every edge to two rows' slabs at random instead took three times as long.
+// Two launches, up to 256 slots and above: the LDS of 1024 a row would leave
+// a CU 12 wavefronts, and each is one chain of loads (B = 200000: 393 -> 174 + 35 us).
+template <int kSlots, int kMin>
 __global__ __launch_bounds__(kWave* kNodalWaves) void k_build_rows(
     GraphView g, const int32_t* __restrict__ labels, const int32_t* __restrict__ bl_off,
     const int32_t* __restrict__ bl_nodes, MView M, int32_t* flags) {
-  __shared__ int32_t s_k[kNodalWaves][kRowTab];
-  __shared__ int32_t s_o[kNodalWaves][kRowTab];
-  __shared__ int32_t s_i[kNodalWaves][kRowTab];
+  __shared__ int32_t s_k[kNodalWaves][kSlots];
+  __shared__ int32_t s_o[kNodalWaves][kSlots];
+  __shared__ int32_t s_i[kNodalWaves][kSlots];
   __shared__ int32_t s_pre[kNodalWaves][kWave + 1];
   const int w = threadIdx.x / kWave;
   const int lane = lane_id();
@@ -1053,7 +1101,7 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_build_rows(
   if (a >= M.B) return;  // no workgroup barrier below
   const int64_t o = M.off[a];
   const int32_t c = M.cap[a];
-  if (!lds_row(c, M.B)) return;
+  if (!lds_row(c, M.B) || c <= kMin || c > kSlots) return;
   int32_t* tk = s_k[w];
   int32_t* to = s_o[w];
   int32_t* ti = s_i[w];
@@ -1131,6 +1179,122 @@ __global__ __launch_bounds__(kWave* kNodalWaves) void k_build_rows(
   }
   if (__ballot(full)) {
     if (lane == 0) atomicOr(flags, kFlagFull);
+  }
+}
+
+// Fills the slabs of the rows of `items`, an item's share by gridDim.y
+// workgroups: empty keys (null: no row has any), zero counts.
+__global__ __launch_bounds__(256) void k_fill_big(MView M, int32_t* key, const int32_t* bsize,
+                                                  const int2* items, const int32_t* n_items) {
+  const int32_t n = *n_items;
+  for (int32_t it = blockIdx.x; it < n; it += gridDim.x) {
+    const int2 q = items[it];
+    const Row R = m_row(M, q.x);
+    const int64_t shares = (int64_t)big_pieces(bsize[q.x]) * gridDim.y;
+    const int64_t at = (int64_t)q.y * gridDim.y + blockIdx.y;
+    const int32_t j1 = (int32_t)(R.c * (at + 1) / shares);
+    for (int32_t j = (int32_t)(R.c * at / shares) + threadIdx.x; j < j1; j += 256) {
+      if (key) key[R.o + j] = -1;
+      M.cnt[R.o + j] = Cnt{0, 0};
+    }
+  }
+}
+
+// The other rows, kBigNodes nodes of a block (an item of k_caps) to a workgroup,
+// an item of many list entries to up to gridDim.y of them: the entries are
+// summed per neighbour block in LDS, then each sum goes to M with one atomic.
+// (An atomic per edge end piled onto a large block's own count: B = 100000
+// with a block of 7000 nodes 526 -> 191 us.)  Keys beyond what the table holds near
+// their home are added to M directly.
+constexpr int kBigTab = 4096;
+constexpr int kBigWalk = 8;
+constexpr int32_t kBigPart = 8192;  // list entries from which an item is split
+constexpr int kBigParts = 4;
+constexpr unsigned kBigGrid = 768;  // three workgroups of 51 KB of LDS per CU
+__global__ __launch_bounds__(256) void k_build_big(GraphView g, const int32_t* __restrict__ labels,
+                                                   const int32_t* __restrict__ bl_off,
+                                                   const int32_t* __restrict__ bl_nodes, MView M,
+                                                   const int2* items, const int32_t* n_items,
+                                                   int32_t* flags) {
+  __shared__ int32_t s_k[kBigTab], s_o[kBigTab], s_i[kBigTab];
+  __shared__ int64_t s_o0[kBigNodes], s_i0[kBigNodes];
+  __shared__ long s_ko[kBigNodes], s_pre[kBigNodes + 1];
+  const int lane = lane_id();
+  const int32_t n = *n_items;
+  for (int32_t it = blockIdx.x; it < n; it += gridDim.x) {
+    const int2 q = items[it];
+    const int32_t a = q.x;
+    const int32_t n0 = bl_off[a] + q.y * kBigNodes;
+    const int32_t n1 = min(n0 + kBigNodes, a + 1 < M.B ? bl_off[a + 1] : g.N);
+    __syncthreads();  // the previous item's table is written out
+    if (threadIdx.x < kWave) {
+      const int32_t j = n0 + lane;
+      int64_t o0 = 0, i0 = 0;
+      long ko = 0, kn = 0;
+      if (j < n1) {
+        const int32_t x = bl_nodes[j];
+        o0 = g.out_ptr[x];
+        i0 = g.in_ptr[x];
+        ko = g.out_ptr[x + 1] - o0;
+        kn = ko + (g.in_ptr[x + 1] - i0);
+      }
+      const long inc = wave_incl_scan(kn);
+      if (lane < kBigNodes) {
+        s_o0[lane] = o0;
+        s_i0[lane] = i0;
+        s_ko[lane] = ko;
+        s_pre[lane + 1] = inc;
+        if (lane == 0) s_pre[0] = 0;
+      }
+    }
+    __syncthreads();
+    const long tot = s_pre[kBigNodes];
+    const long parts = tot > kBigPart ? (long)gridDim.y : 1;
+    if ((long)blockIdx.y >= parts) continue;  // the same for every thread
+    const long e0 = tot * (long)blockIdx.y / parts, e1 = tot * ((long)blockIdx.y + 1) / parts;
+    int32_t tab = 256;  // a power of two >= twice the entries, at most kBigTab
+    while (tab < kBigTab && tab < 2 * (e1 - e0)) tab <<= 1;
+    for (int i = threadIdx.x; i < tab; i += 256) {
+      s_k[i] = -1;
+      s_o[i] = 0;
+      s_i[i] = 0;
+    }
+    __syncthreads();
+    for (long ei = e0 + threadIdx.x; ei < e1; ei += 256) {
+      int lo = 0, hi = kBigNodes - 1;  // the node of entry ei
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (s_pre[mid] <= ei)
+          lo = mid;
+        else
+          hi = mid - 1;
+      }
+      const long r = ei - s_pre[lo], ko = s_ko[lo];
+      const bool out = r < ko;
+      int32_t v, wt = 1;
+      if (out) {
+        v = g.out_idx[s_o0[lo] + r];
+        if (g.out_w) wt = g.out_w[s_o0[lo] + r];
+      } else {
+        v = g.in_idx[s_i0[lo] + (r - ko)];
+        if (g.in_w) wt = g.in_w[s_i0[lo] + (r - ko)];
+      }
+      const int32_t b = labels[v];
+      uint32_t h = hash32(b) & (uint32_t)(tab - 1);
+      bool done = false;
+      for (int p = 0; p < kBigWalk && !done; ++p) {
+        const int32_t old = atomicCAS(&s_k[h], -1, b);
+        if (old == -1 || old == b) {
+          atomicAdd(out ? &s_o[h] : &s_i[h], wt);
+          done = true;
+        }
+        h = (h + 1) & (uint32_t)(tab - 1);
+      }
+      if (!done) m_add(M, a, b, out ? wt : 0, out ? 0 : wt, flags);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < tab; i += 256)
+      if (s_k[i] >= 0) m_add(M, a, s_k[i], s_o[i], s_i[i], flags);
   }
 }
 
@@ -1270,7 +1434,7 @@ __global__ __launch_bounds__(kHistB) void k_hist_sum(HistSum a) {
 // edges' block pairs a*B + b are sorted and summed per pair, then each pair
 // is added once.
 constexpr int32_t kPairSortB = 4096;
-constexpr int32_t kRowBuildB = 16384;  // from here up the build goes by rows (k_build_rows)
+// Above, rows are mostly hashed and the build goes by rows (k_build_rows).
 
 __global__ void k_pair_keys(int64_t E, const int32_t* __restrict__ src,
                             const int32_t* __restrict__ dst, const int32_t* __restrict__ w,
@@ -1300,24 +1464,19 @@ __global__ void k_insert_pairs(int64_t E, const uint32_t* __restrict__ key,
   }
 }
 
-// Blocks holding other than one node (0 means every block is a single node).
-__global__ void k_count_nonsingle(int32_t B, const int32_t* __restrict__ bsize, int32_t* out) {
-  for (int32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < B; i += gridDim.x * blockDim.x)
-    if (bsize[i] != 1) atomicAdd(out, 1);
-}
-
-// Bucket sums (o + i) of the block rows that keep them: kSumRows rows to a
-// workgroup, which handles those of them one by one (a block that absorbed
-// thousands of nodes has a slab of 16384 slots or more: 4 wavefronts with 8
-// slots a thread in flight, where one with one slot a lane took 0.8 ms).  Sets
+// Bucket sums (o + i) of the block rows that keep them: up to kSumRows rows to a
+// workgroup (fewer while that leaves the GPU short of workgroups: B = 2500, 64
+// a workgroup 194 us, now 19), which handles those of them one by one (a block
+// that absorbed thousands of nodes has a slab of 16384 slots or more: 16
+// wavefronts with 8 slots a thread in flight take 92 us, 4 took 124).  Sets
 // the hashed ones' marks too (room_mark).
 constexpr int kSumRows = 64;
-__global__ __launch_bounds__(256) void k_bucket_sums(MView m) {
+__global__ __launch_bounds__(1024) void k_bucket_sums(MView m, int32_t rows) {
   __shared__ int32_t s_b[kNBK];
   __shared__ int32_t s_keys;
   const int lane = lane_id();
-  const int64_t a0 = (int64_t)blockIdx.x * kSumRows;
-  const int32_t cl = a0 + lane < m.B ? m.cap[a0 + lane] : 0;
+  const int64_t a0 = (int64_t)blockIdx.x * rows;
+  const int32_t cl = lane < rows && a0 + lane < m.B ? m.cap[a0 + lane] : 0;
   unsigned long long todo = __ballot(cl > 0 && row_sums(m, cl));  // the same in every wavefront
   while (todo) {
     const int l = __ffsll(todo) - 1;
@@ -2574,80 +2733,6 @@ __device__ __forceinline__ void tab_add(int32_t* tk, int32_t* tv, uint32_t mask,
   }
 }
 
-// The neighbour-block table of node n: slots [0, cap) of tk (block), two
-// (weight of n's out-edges into it) and twi (in-edges), in LDS for nodes with
-// at most kTabMaxDeg list entries, else in the node's global-memory table.
-struct Table {
-  int32_t *tk, *two, *twi;
-  int32_t cap;
-};
-
-// kBig selects the node's global table (more than kTabMaxDeg list entries)
-// or the wavefront's LDS table at compile time, so the LDS form compiles to
-// LDS instructions (a pointer that may be either would make every table
-// access a flat access that also waits for the wavefront's global loads).
-template <bool kBig>
-__device__ __forceinline__ Table tab_open(int32_t* lds, const int64_t* big_off, int32_t* big_tab,
-                                          int32_t n, int64_t kc) {
-  const int lane = lane_id();
-  Table T;
-  if (kBig) {
-    int32_t cap = 1;
-    while (cap < 2 * kc) cap <<= 1;
-    T.cap = cap;
-    T.tk = big_tab + big_off[n];
-    T.two = T.tk + cap;
-    T.twi = T.tk + 2 * cap;
-  } else {
-    int32_t cap = kWave;  // >= 4/3 of the distinct neighbour blocks, <= kTab
-    while (cap < 2 * kc && cap < kTab) cap <<= 1;
-    T.cap = cap;
-    T.tk = lds;
-    T.two = lds + kTab;
-    T.twi = lds + 2 * kTab;
-  }
-  for (int32_t i = lane; i < T.cap; i += kWave) {
-    T.tk[i] = -1;
-    T.two[i] = 0;
-    T.twi[i] = 0;
-  }
-  wave_fence();
-  return T;
-}
-
-// Moves the table's entries, except those of blocks r and s (whose weights
-// are returned in wor/wir/wos/wis), to its front in place; returns their
-// number.  Chunk by chunk: every lane reads its slot before any write, and a
-// write never lands after the chunk being read.
-__device__ __forceinline__ int32_t tab_compact(const Table& T, int32_t r, int32_t s, long& wor,
-                                               long& wir, long& wos, long& wis) {
-  const int lane = lane_id();
-  const unsigned long long below = (1ull << lane) - 1ull;
-  int32_t nent = 0;
-  for (int32_t base = 0; base < T.cap; base += kWave) {  // cap is a multiple of kWave
-    const int32_t i = base + lane;
-    int32_t b = T.tk[i];
-    const int32_t wo = T.two[i], wi = T.twi[i];
-    const bool isr = b >= 0 && b == r, iss = b >= 0 && b == s;
-    wor += isr ? wo : 0;
-    wir += isr ? wi : 0;
-    wos += iss ? wo : 0;
-    wis += iss ? wi : 0;
-    if (isr || iss) b = -1;
-    const unsigned long long live = __ballot(b >= 0);
-    const int32_t pos = nent + __popcll(live & below);
-    wave_fence();
-    if (b >= 0) {
-      T.tk[pos] = b;
-      T.two[pos] = wo;
-      T.twi[pos] = wi;
-    }
-    nent += __popcll(live);
-    wave_fence();
-  }
-  return nent;
-}
-
 // List entry j of node n (out-edges then in-edges): neighbour id (-1 past the
 // end) and weight.
 __device__ __forceinline__ void list_entry(const GraphView& g, int64_t o0, int64_t kco,
@@ -3503,49 +3588,6 @@ __global__ __launch_bounds__(256) void k_nnz_bytes(const Cnt* __restrict__ cnt, 
   if (lane_id() == 0 && c)
     atomicAdd(&acc[(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave) % kAqSlots],
               16ull * (unsigned long long)c);
-}
-
-// M build when every block holds one node (the identity start, B == N): block
-// row labels[n] is node n's own list -- out-edges as o, in-edges as i -- so
-// one wavefront builds it alone from its neighbour-block table, with no
-// contention from other wavefronts (graph_parallel.hpp:703-759).
-template <bool kBig>
-__device__ __forceinline__ void build_single_one(const GraphView& g, const int32_t* labels,
-                                                 const MView& M, const int64_t* big_off,
-                                                 int32_t* big_tab, int32_t n, int32_t* tab,
-                                                 int32_t* flags) {
-  const int lane = lane_id();
-  const int64_t o0 = g.out_ptr[n], i0 = g.in_ptr[n];
-  const int64_t kco = g.out_ptr[n + 1] - o0, kci = g.in_ptr[n + 1] - i0;
-  const int64_t kc = kco + kci;
-  const int32_t a = labels[n];
-  const Table T = tab_open<kBig>(tab, big_off, big_tab, n, kc);
-  const uint32_t mask = (uint32_t)T.cap - 1;
-  for (int64_t j = lane; j < kc; j += kWave) {
-    int32_t v, w;
-    list_entry(g, o0, kco, i0, kc, j, v, w);
-    tab_add(T.tk, j < kco ? T.two : T.twi, mask, labels[v], w);
-  }
-  wave_fence();
-  long x0 = 0, x1 = 0, x2 = 0, x3 = 0;
-  const int32_t nent = tab_compact(T, -2, -2, x0, x1, x2, x3);
-  for (int32_t j = lane; j < nent; j += kWave) m_add(M, a, T.tk[j], T.two[j], T.twi[j], flags);
-}
-
-__global__ __launch_bounds__(kWave* kNodalWaves) void k_build_single(GraphView g,
-                                                                    const int32_t* labels, MView M,
-                                                                    const int64_t* big_off,
-                                                                    int32_t* big_tab,
-                                                                    int32_t* flags) {
-  __shared__ int32_t s_tab[kNodalWaves][3 * kTab];
-  const int w = threadIdx.x / kWave;
-  const int64_t n = (int64_t)blockIdx.x * kNodalWaves + w;
-  if (n >= g.N) return;
-  const int64_t kc = (g.out_ptr[n + 1] - g.out_ptr[n]) + (g.in_ptr[n + 1] - g.in_ptr[n]);
-  if (kc > kTabMaxDeg)
-    build_single_one<true>(g, labels, M, big_off, big_tab, (int32_t)n, s_tab[w], flags);
-  else
-    build_single_one<false>(g, labels, M, big_off, big_tab, (int32_t)n, s_tab[w], flags);
 }
 
 // ---------------------------------------------------------------------------
@@ -4601,6 +4643,7 @@ struct usap_engine {
           *bsize = nullptr;
   // nodes grouped by block for the per-row build: offsets, arrival cursors, nodes
   int32_t *bl_off = nullptr, *bl_cur = nullptr, *bl_nodes = nullptr;
+  int2* big_items = nullptr;
   DevSpM M;  // block rows (both orientations of M)
   int64_t* tmpM = nullptr;
   void* scan_tmp = nullptr;
@@ -4898,7 +4941,7 @@ int build_by_pairs(usap_engine* e) {
 }
 
 // Full M build from the labels (graph_parallel.hpp:703-759).
-// The M build for B >= kRowBuildB: nodes grouped by block (offsets by an
+// The M build for B > kPairSortB: nodes grouped by block (offsets by an
 // exclusive scan of the block sizes, then a scatter), k_build_rows for the
 // rows it lays out in LDS, per-edge inserts for the others.
 int build_rows(usap_engine* e) {
@@ -4915,12 +4958,18 @@ int build_rows(usap_engine* e) {
   bytes = e->scan_tmp_bytes;
   HIPCHK(rocprim::exclusive_scan(e->scan_tmp, bytes, e->bsize, e->bl_off, (int32_t)0, (size_t)B,
                                  rocprim::plus<int32_t>(), st));
-  k_node_lists<<<std::min<unsigned>(blocks_for(e->N, 256), 4096u), 256, 0, st>>>(
-      e->N, e->labels, e->bl_off, e->bl_cur, e->bl_nodes);
-  k_build_rows<<<blocks_for(B, kNodalWaves), kWave * kNodalWaves, 0, st>>>(
-      gview(e), e->labels, e->bl_off, e->bl_nodes, view(e->M, B), e->build_flags);
-  k_insert_edges<true><<<std::min<int64_t>(blocks_for(e->E, 256), 16384), 256, 0, st>>>(
-      e->E, e->out_src, e->out_idx, e->out_w, e->labels, view(e->M, B), e->build_flags);
+  k_node_lists<<<blocks_for(e->N, kNodesWg), 256, 0, st>>>(e->N, e->labels, e->bl_off, e->bl_cur,
+                                                           e->bl_nodes);
+  const MView M = view(e->M, B);
+  const int32_t* n_items = e->build_flags + 1;
+  k_fill_big<<<dim3(kBigGrid, kBigParts), 256, 0, st>>>(M, e->all_direct ? nullptr : e->M.key,
+                                                        e->bsize, e->big_items, n_items);
+  k_build_rows<256, 0><<<blocks_for(B, kNodalWaves), kWave * kNodalWaves, 0, st>>>(
+      gview(e), e->labels, e->bl_off, e->bl_nodes, M, e->build_flags);
+  k_build_rows<kRowTab, 256><<<blocks_for(B, kNodalWaves), kWave * kNodalWaves, 0, st>>>(
+      gview(e), e->labels, e->bl_off, e->bl_nodes, M, e->build_flags);
+  k_build_big<<<dim3(kBigGrid, kBigParts), 256, 0, st>>>(gview(e), e->labels, e->bl_off, e->bl_nodes,
+                                                         M, e->big_items, n_items, e->build_flags);
   HIPCHK(hipGetLastError());
   return USAP_OK;
 }
@@ -5016,12 +5065,18 @@ int rebuild_M(usap_engine* e) {
     k_clear_build<<<std::max(1u, std::min(blocks_for(B, 256), 1024u)), 256, 0, st>>>(c);
   }
   if (e->N > 0) {
-    const unsigned g = std::min<unsigned>(blocks_for(e->N, 256), B <= kDegLds ? 256u : 4096u);
-    k_degrees<<<g, 256, 0, st>>>(gview(e), e->labels, B, e->d_out, e->d_in, e->ecnt_out,
-                                 e->ecnt_in, e->bsize);
+    const auto k = e->out_w ? (B <= kDegLds ? k_degrees<true, false> : k_degrees<true, true>)
+                            : (B <= kDegLds ? k_degrees<false, false> : k_degrees<false, true>);
+    const int32_t per = e->out_w ? (e->N < 65536 ? 64 : kNodesWgW) : (e->N < 65536 ? 256 : kNodesWg);
+    k<<<blocks_for(e->N, per), 256, 0, st>>>(gview(e), e->labels, B, per, e->d_out, e->d_in,
+                                             e->ecnt_out, e->ecnt_in, e->bsize);
   }
-  k_caps<<<blocks_for((int64_t)B + 1, 256), 256, 0, st>>>(B, e->p.slab_slack, e->ecnt_out,
-                                                          e->ecnt_in, e->M.cap, e->tmpM);
+  const bool by_rows = B > kPairSortB;
+  int2* items = by_rows ? e->big_items : nullptr;
+  int32_t* n_items = e->build_flags + 1;
+  k_caps<<<blocks_for((int64_t)B + 1, 256), 256, 0, st>>>(
+      B, e->p.slab_slack, e->out_w ? e->ecnt_out : e->d_out, e->out_w ? e->ecnt_in : e->d_in,
+      e->bsize, e->M.cap, e->tmpM, items, n_items);
   HIPCHK(hipGetLastError());
   size_t bytes = 0;
   HIPCHK(rocprim::exclusive_scan(nullptr, bytes, e->tmpM, e->M.off, (int64_t)0, (size_t)B + 1,
@@ -5034,14 +5089,6 @@ int rebuild_M(usap_engine* e) {
   bytes = e->scan_tmp_bytes;
   HIPCHK(rocprim::exclusive_scan(e->scan_tmp, bytes, e->tmpM, e->M.off, (int64_t)0, (size_t)B + 1,
                                  rocprim::plus<int64_t>(), st));
-  // B == N: is every block a single node (rows built per node)?
-  const bool maybe_single = B == e->N && e->E > 0;
-  int32_t nonsingle = 1;
-  if (maybe_single) {
-    k_count_nonsingle<<<std::min<unsigned>(blocks_for(B, 256), 1024u), 256, 0, st>>>(
-        B, e->bsize, e->build_flags + 1);
-    HIPCHK(hipMemcpyAsync(&nonsingle, e->build_flags + 1, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-  }
   int64_t tot = 0;
   HIPCHK(hipMemcpyAsync(&tot, e->M.off + B, sizeof(int64_t), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
@@ -5051,7 +5098,7 @@ int rebuild_M(usap_engine* e) {
   // no insert probes, so no row ever needs growth or an increment parked until
   // the next rebuild, and k_grow only has the batch's error flags to fold
   e->all_direct = tot == (int64_t)B * B;
-  if (m.total > 0) k_fill<<<std::min<int64_t>(blocks_for(m.total, 256), 8192), 256, 0, st>>>(
+  if (m.total > 0 && !by_rows) k_fill<<<std::min<int64_t>(blocks_for(m.total, 256), 8192), 256, 0, st>>>(
       e->all_direct ? nullptr : m.key, m.cnt, m.total);
   k_reset_grow<<<blocks_for(kGrowBlocks, 256), 256, 0, st>>>(m.gst, (unsigned long long)m.total);
   if (B > kNBK && m.bs_rows < B) {
@@ -5059,20 +5106,15 @@ int rebuild_M(usap_engine* e) {
     if (int rc = dalloc(e, &m.bs, (size_t)B * kNBK)) return rc;
     m.bs_rows = B;
   }
-  if (e->E > 0) {
-    if (maybe_single && nonsingle == 0)
-      k_build_single<<<blocks_for(e->N, kNodalWaves), kWave * kNodalWaves, 0, st>>>(
-          gview(e), e->labels, view(e->M, B), e->big_off, e->big_tab, e->build_flags);
-    else if (B <= kPairSortB) {
-      if (int rc = build_by_pairs(e)) return rc;
-    } else if (B < kRowBuildB) {
-      k_insert_edges<false><<<std::min<int64_t>(blocks_for(e->E, 256), 16384), 256, 0, st>>>(
-          e->E, e->out_src, e->out_idx, e->out_w, e->labels, view(e->M, B), e->build_flags);
-    } else {
-      if (int rc = build_rows(e)) return rc;
-    }
+  if (by_rows) {
+    if (int rc = build_rows(e)) return rc;
+  } else if (e->E > 0) {
+    if (int rc = build_by_pairs(e)) return rc;
   }
-  if (B > kNBK) k_bucket_sums<<<blocks_for(B, kSumRows), 256, 0, st>>>(view(e->M, B));
+  if (B > kNBK) {
+    const int32_t rows = std::min(kSumRows, 1 + B / 2048);
+    k_bucket_sums<<<blocks_for(B, rows), 1024, 0, st>>>(view(e->M, B), rows);
+  }
   HIPCHK(hipGetLastError());
   ev_rec(e, 1);
   int32_t flags = 0;
@@ -5208,6 +5250,7 @@ int usap_destroy(usap_engine* e) {
   dfree(e, e->bl_off);
   dfree(e, e->bl_cur);
   dfree(e, e->bl_nodes);
+  dfree(e, e->big_items);
   for (DevSpM* m : {&e->M}) {
     dfree(e, m->off);
     dfree(e, m->cap);
@@ -5619,6 +5662,7 @@ int alloc_state(usap_engine* e) {
   TRY(dalloc(e, &e->bl_off, N));
   TRY(dalloc(e, &e->bl_cur, N));
   TRY(dalloc(e, &e->bl_nodes, N));
+  TRY(dalloc(e, &e->big_items, (size_t)N + N / kBigNodes + 1));
   for (DevSpM* m : {&e->M}) {
     TRY(dalloc(e, &m->off, (size_t)N + 1));
     TRY(dalloc(e, &m->cap, N));
