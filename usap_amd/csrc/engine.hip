@@ -55,6 +55,8 @@
 
 #include <algorithm>
 #include <cmath>
+#include <chrono>
+#include <climits>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -119,6 +121,19 @@ struct Sweep {
   int32_t flags;    // OR of the batches' flags
   int32_t stop_n;   // stop as the running batch's k_nodal saw it (0: the batch runs)
 };
+
+// A word in the host's memory that a call's last kernel sets once its results
+// are there (p null: none).
+struct HostWord {
+  int32_t* p;
+  int32_t value;
+};
+__device__ __forceinline__ void host_done(const HostWord& w) {
+  if (w.p) {
+    __threadfence_system();
+    __hip_atomic_store(w.p, w.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
 
 struct GraphView {
   int32_t N;
@@ -1857,6 +1872,7 @@ struct CarryArgs {
   int32_t* map;
   int32_t* short_of;         // 1: fewer than B_to_merge links can be made
   int32_t* host_short;       // the same, in the host's memory
+  HostWord done;             // told after it
 };
 
 constexpr int kCarryThreads = 1024;
@@ -1970,6 +1986,7 @@ __global__ __launch_bounds__(kCarryThreads) void k_carry_one(CarryArgs a) {
   if (t == 0) {
     *a.short_of = fails;
     *a.host_short = fails;
+    host_done(a.done);
   }
   if (fails) return;  // the same for every thread
 #pragma unroll
@@ -2048,7 +2065,7 @@ __global__ void k_carry_success(int32_t B, const int2* __restrict__ pm,
 __global__ void k_carry_link(int32_t B, int32_t B_to_merge, const int32_t* __restrict__ best,
                              const int32_t* __restrict__ rank, const int32_t* __restrict__ succ,
                              const int32_t* __restrict__ scan, int32_t* par, int32_t* alive,
-                             int32_t* short_of, int32_t* host_short) {
+                             int32_t* short_of, int32_t* host_short, HostWord done) {
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= B) return;
   const int32_t r = rank[i];
@@ -2058,6 +2075,7 @@ __global__ void k_carry_link(int32_t B, int32_t B_to_merge, const int32_t* __res
     const int32_t fails = scan[B - 1] < B_to_merge;
     *short_of = fails;
     *host_short = fails;
+    host_done(done);
   }
 }
 
@@ -3722,7 +3740,8 @@ __device__ __forceinline__ void fold_flags(Status* status, Sweep* sweep, int32_t
 
 // The state after a sweep, or after a chunk of its batches, in the host's
 // pinned memory (a copy would be a launch of the runtime's own kernel).
-__global__ __launch_bounds__(kWave) void k_finish(Status* status, Sweep* sweep, Sweep* host) {
+__global__ __launch_bounds__(kWave) void k_finish(Status* status, Sweep* sweep, Sweep* host,
+                                                  HostWord done) {
   if (threadIdx.x == 0) {
     fold_flags(status, sweep, status->flags);
     __threadfence();
@@ -3734,6 +3753,7 @@ __global__ __launch_bounds__(kWave) void k_finish(Status* status, Sweep* sweep, 
     reinterpret_cast<unsigned long long*>(host)[threadIdx.x] =
         __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+  if (threadIdx.x == 0) host_done(done);  // the stores above are this wavefront's
 }
 
 // graph_parallel.hpp:433-458 after the moves of one batch (sum: exact sum of
@@ -4732,6 +4752,8 @@ struct usap_engine {
                                    // [2] distinct block pairs, [3] carry-out out of candidates
   int32_t* h_short = nullptr;      // the last in pinned host memory, and its device address
   int32_t* d_short = nullptr;
+  int32_t word_want[3] = {0, 0, 0};
+  int32_t word_seq = 0;  // the last value given to a host word (h_short[4 + slot])
   int32_t* hist = nullptr;  // counts of the build by histograms
   int64_t hist_cap = 0;
   uint32_t* pair_key[2] = {nullptr, nullptr};  // block-pair builds [E]
@@ -5728,6 +5750,7 @@ int alloc_state(usap_engine* e) {
   e->h_short = (int32_t*)pin_get(kShortBytes);
   if (!e->h_sweep || !e->h_fx || !e->h_chunk[0] || !e->h_chunk[1] || !e->h_short)
     return set_err(e, USAP_ENOMEM, "hipHostMalloc");
+  std::memset(e->h_short, 0, kShortBytes);  // a pooled buffer holds another engine's words
   HIPCHK(hipHostGetDevicePointer((void**)&e->d_short, e->h_short, 0));
   HIPCHK(hipHostGetDevicePointer((void**)&e->d_fx, e->h_fx, 0));
   HIPCHK(hipHostGetDevicePointer((void**)&e->d_hsweep, e->h_sweep, 0));
@@ -6030,6 +6053,37 @@ int usap_get_M_coo(usap_engine* e, int64_t cap, int32_t* rows, int32_t* cols, in
 }  // extern "C"
 
 namespace {
+// The host's wait for a word its last launch sets (kWord*): a few microseconds
+// after the kernel's store, where a stream synchronisation queues a marker and
+// sleeps on its interrupt (N = 20000, 106 sweeps: 21.6 us from a sweep's last
+// kernel to the next one's first, now 15).  A sweep that takes longer than
+// kSpinUs, or an error, is left to the synchronisation.  Profiled calls read
+// events and always synchronise.
+enum { kWordShort = 0, kWordSweep = 1, kWordFx = 2 };
+constexpr int kSpinUs = 1000;
+
+HostWord host_word(usap_engine* e, int slot) {
+  e->word_seq = e->word_seq == INT32_MAX ? 1 : e->word_seq + 1;
+  e->word_want[slot] = e->word_seq;
+  return HostWord{e->d_short + 4 + slot, e->word_seq};
+}
+
+int wait_word(usap_engine* e, int slot) {
+  if (!e->prof) {
+    const int32_t* p = e->h_short + 4 + slot;
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int i = 0;; ++i) {
+      if (__atomic_load_n(p, __ATOMIC_ACQUIRE) == e->word_want[slot]) return USAP_OK;
+      __builtin_ia32_pause();
+      if (i % 64 == 63 &&
+          std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(kSpinUs))
+        break;
+    }
+  }
+  HIPCHK(hipStreamSynchronize(e->stream));
+  return USAP_OK;
+}
+
 // k_entropy over the pool in use: about four slots per thread, at most
 // kEntropyBlocks workgroups (a scan of 1 GB pools at B = 250k is bound by the
 // loads in flight).
@@ -6061,7 +6115,7 @@ long* g_scratch_ptr[kMaxDevices] = {};
 // term's int128 words, hi then lo): the same integer sum and IEEE operations as
 // usap_entropy on the host.
 __global__ __launch_bounds__(kBeginThreads) void k_entropy_out(EntropyIn in, double model, double* S,
-                                                               int64_t* fx) {
+                                                               int64_t* fx, HostWord done) {
   const i128 data = -block_entropy(in);
   if (threadIdx.x == 0) {
     if (S) *S = model + fx_to_double_dev(data);
@@ -6069,6 +6123,7 @@ __global__ __launch_bounds__(kBeginThreads) void k_entropy_out(EntropyIn in, dou
       fx[0] = (int64_t)(data >> 64);
       fx[1] = (int64_t)(uint64_t)(u128)data;
     }
+    host_done(done);
   }
 }
 
@@ -6103,9 +6158,9 @@ int usap_entropy(usap_engine* e, double* S, int64_t* hi, uint64_t* lo) {
   ev_rec(e, 0);
   const EntropyIn in = launch_entropy(e, e->ent_part);
   ev_rec(e, 1);
-  k_entropy_out<<<1, kBeginThreads, 0, st>>>(in, 0.0, nullptr, e->d_fx);
+  k_entropy_out<<<1, kBeginThreads, 0, st>>>(in, 0.0, nullptr, e->d_fx, host_word(e, kWordFx));
   HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(st));
+  if (int rc = wait_word(e, kWordFx)) return rc;
   prof_add(e, USAP_K_ENTROPY, ev_ms(e, 0, 1), 1, 8.0 * e->B + 16.0 * in.nparts);
   const i128 data = mk128((long)e->h_fx[0], (unsigned long)e->h_fx[1]);
   if (hi) *hi = (int64_t)(data >> 64);
@@ -6125,7 +6180,8 @@ int usap_entropy_noalloc(usap_engine* e, double* S_dev, int64_t* fx_dev) {
   if (need > kScratchParts)
     return set_err(e, USAP_EINVAL, "usap_entropy_noalloc: more partials than the 64 KiB scratch holds");
   const EntropyIn in = launch_entropy(e, part);
-  k_entropy_out<<<1, kBeginThreads, 0, e->stream>>>(in, usap_model_S(e->N, e->E, e->B), S_dev, fx_dev);
+  k_entropy_out<<<1, kBeginThreads, 0, e->stream>>>(in, usap_model_S(e->N, e->E, e->B), S_dev, fx_dev,
+                                                    HostWord{nullptr, 0});
   HIPCHK(hipGetLastError());
   return USAP_OK;
 }
@@ -6231,6 +6287,7 @@ int carry_out(usap_engine* e, int32_t B_to_merge) {
   a.map = e->map;
   a.short_of = e->build_flags + 3;
   a.host_short = e->d_short;
+  a.done = host_word(e, kWordShort);
   if (B <= kCarryRank) {
     k_carry_one<kCarryRank><<<1, kCarryThreads, 0, st>>>(a);
     HIPCHK(hipGetLastError());
@@ -6287,7 +6344,7 @@ int carry_out(usap_engine* e, int32_t B_to_merge) {
   HIPCHK(rocprim::inclusive_scan(e->sort_tmp, bytes, succ, scan, (size_t)B,
                                  rocprim::plus<int32_t>(), st));
   k_carry_link<<<g, 256, 0, st>>>(B, B_to_merge, a.best, rank, succ, scan, par, alive, a.short_of,
-                                  a.host_short);
+                                  a.host_short, a.done);
   for (int64_t w = 1; w < B; w <<= 1) k_carry_root<<<g, 256, 0, st>>>(B, par);
   k_carry_alive<<<g, 256, 0, st>>>(B, a.bsize, par, alive);
   bytes = e->sort_tmp_bytes;
@@ -6311,7 +6368,7 @@ int usap_merge_apply(usap_engine* e, int32_t B_to_merge, int32_t* B_new) {
   if (int rc = carry_out(e, B_to_merge)) return rc;
   k_relabel<<<blocks_for(e->N, 256), 256, 0, st>>>(e->N, e->labels, e->map, e->build_flags + 3);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(st));
+  if (int rc = wait_word(e, kWordShort)) return rc;
   if (*e->h_short) return set_err(e, USAP_EINFEASIBLE, "carry-out ran out of candidate merges");
   e->B = B - B_to_merge;
   e->merge_B = -1;
@@ -6411,7 +6468,7 @@ int launch_begin(usap_engine* e, int32_t beg, int32_t end, int32_t batch, bool f
 }
 
 int launch_finish(usap_engine* e, Sweep* host) {
-  k_finish<<<1, kWave, 0, e->stream>>>(e->status, e->sweep, host);
+  k_finish<<<1, kWave, 0, e->stream>>>(e->status, e->sweep, host, host_word(e, kWordSweep));
   HIPCHK(hipGetLastError());
   return USAP_OK;
 }
@@ -6611,7 +6668,7 @@ int run_sweep(usap_engine* e, int32_t batch, int32_t first, int32_t last, int32_
       }
     }
     if (int rc = launch_finish(e, e->d_hsweep)) return rc;
-    HIPCHK(hipStreamSynchronize(st));
+    if (int rc = wait_word(e, kWordSweep)) return rc;
     const int32_t executed = first + hs.done - next;  // batches run in this launch round
     if (e->prof)
       if (int rc = prof_end(e, (size_t)executed)) return rc;
@@ -6672,7 +6729,7 @@ int usap_nodal_batch(usap_engine* e, int32_t begin, int32_t end, uint64_t stream
     if (int rc = launch_batch(e, begin, end, 0)) return rc;
     Sweep& hs = *e->h_sweep;
     if (int rc = launch_finish(e, e->d_hsweep)) return rc;
-    HIPCHK(hipStreamSynchronize(e->stream));
+    if (int rc = wait_word(e, kWordSweep)) return rc;
     if (e->prof) {
       if (int rc = prof_end(e, 1)) return rc;
       e->kp[USAP_K_NODAL].bytes += (double)hs.nodal_bytes;
