@@ -2698,6 +2698,9 @@ __global__ __launch_bounds__(kWave* kMergeWaves, 4) void k_merge_rows(MergeArgs 
 
 __global__ void k_zero1(int32_t* p) { *p = 0; }
 
+// Ends a call whose last kernel tells the host nothing.
+__global__ void k_word(HostWord done) { host_done(done); }
+
 // ---------------------------------------------------------------------------
 // Nodal proposal, graph_parallel.hpp:990-1222
 // ---------------------------------------------------------------------------
@@ -3663,6 +3666,8 @@ struct ApplyArgs {
   uint32_t nparts;
   Status* status;
   Sweep* sweep;
+  Sweep* host;    // set: this launch is the sweep's last and ends it
+  HostWord done;
   unsigned long long* tstamp;  // as NodalArgs::tstamp, for this kernel
   int32_t tstride;
 };
@@ -3738,10 +3743,11 @@ __device__ __forceinline__ void fold_flags(Status* status, Sweep* sweep, int32_t
   }
 }
 
-// The state after a sweep, or after a chunk of its batches, in the host's
-// pinned memory (a copy would be a launch of the runtime's own kernel).
-__global__ __launch_bounds__(kWave) void k_finish(Status* status, Sweep* sweep, Sweep* host,
-                                                  HostWord done) {
+// The batches' flags folded into the sweep's state, and the state copied to the
+// host's pinned memory (a copy would be a launch of the runtime's own kernel),
+// by one workgroup.
+__device__ __forceinline__ void finish_sweep(Status* status, Sweep* sweep, Sweep* host,
+                                             const HostWord& done) {
   if (threadIdx.x == 0) {
     fold_flags(status, sweep, status->flags);
     __threadfence();
@@ -3754,6 +3760,12 @@ __global__ __launch_bounds__(kWave) void k_finish(Status* status, Sweep* sweep, 
         __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (threadIdx.x == 0) host_done(done);  // the stores above are this wavefront's
+}
+
+// After a sweep, or after a chunk of its batches, where the last k_apply did not.
+__global__ __launch_bounds__(kWave) void k_finish(Status* status, Sweep* sweep, Sweep* host,
+                                                  HostWord done) {
+  finish_sweep(status, sweep, host, done);
 }
 
 // graph_parallel.hpp:433-458 after the moves of one batch (sum: exact sum of
@@ -4023,7 +4035,10 @@ __device__ __forceinline__ void batch_tail(const BlockPart* part, uint32_t npart
   __syncthreads();
 }
 
-// Block 0 runs the batch's update step; every other block applies the moves
+// Block 0 runs the batch's update step and, where it is the sweep's last and
+// every row is direct, ends the sweep: on direct rows the applying blocks raise
+// no flags, so there is nothing to wait for (k_finish is one launch more, 6 us
+// of a sweep of 4 batches).  Every other block applies the moves
 // of its four batch nodes: each moving node's wavefront writes its records,
 // then all the block's records are spread over all its threads (a block holds
 // 0-4 moving nodes, most often 0 or 1, so a node's records do not wait for its
@@ -4039,6 +4054,7 @@ __global__ __launch_bounds__(kWave* kNodalWaves, 4) void k_apply(ApplyArgs a) {
   if (blockIdx.x == 0) {
     if (a.tstamp && threadIdx.x == 0) a.tstamp[0] = wall_clock64();
     if (a.sweep->stop_n == 0) batch_tail(a.part, a.nparts, a.sweep);
+    if (kD && a.host) finish_sweep(a.status, a.sweep, a.host, a.done);
     if (a.tstamp) {
       __syncthreads();
       if (threadIdx.x == 0) a.tstamp[a.tstride] = wall_clock64();
@@ -6263,6 +6279,11 @@ int usap_merge_result_fx(usap_engine* e, int32_t* best_s, int64_t* hi, uint64_t*
   if (best_s) HIPCHK(hipMemcpyAsync(best_s, e->best_s, sizeof(int32_t) * B, hipMemcpyDeviceToHost, e->stream));
   if (hi) HIPCHK(hipMemcpyAsync(hi, e->best_hi, sizeof(int64_t) * B, hipMemcpyDeviceToHost, e->stream));
   if (lo) HIPCHK(hipMemcpyAsync(lo, e->best_lo, sizeof(uint64_t) * B, hipMemcpyDeviceToHost, e->stream));
+  if (!best_s && !hi && !lo) {  // only the wait
+    k_word<<<1, 1, 0, e->stream>>>(host_word(e, kWordShort));
+    HIPCHK(hipGetLastError());
+    return wait_word(e, kWordShort);
+  }
   HIPCHK(hipStreamSynchronize(e->stream));
   return USAP_OK;
 }
@@ -6474,7 +6495,8 @@ int launch_finish(usap_engine* e, Sweep* host) {
 }
 
 // Launches k_nodal + k_apply + k_grow for nodes [beg, end).
-int launch_batch(usap_engine* e, int32_t beg, int32_t end, size_t ev_slot, bool grow = true) {
+int launch_batch(usap_engine* e, int32_t beg, int32_t end, size_t ev_slot, bool grow = true,
+                 bool finish = false) {
   const int32_t B = e->B;
   hipStream_t st = e->stream;
   NodalArgs a;
@@ -6521,6 +6543,8 @@ int launch_batch(usap_engine* e, int32_t beg, int32_t end, size_t ev_slot, bool 
   b.nparts = grid;
   b.status = e->status;
   b.sweep = e->sweep;
+  b.host = finish ? e->d_hsweep : nullptr;
+  b.done = finish ? host_word(e, kWordSweep) : HostWord{nullptr, 0};
   b.tstamp = ts ? ts + 2 * (size_t)G : nullptr;
   b.tstride = G + 1;
   GrowArgs ga;
@@ -6633,6 +6657,7 @@ int run_sweep(usap_engine* e, int32_t batch, int32_t first, int32_t last, int32_
   Sweep& hs = *e->h_sweep;
   int32_t next = first;
   for (;;) {
+    bool finished = false;  // by the last batch's k_apply
     if (e->p.graphs && !e->prof && next == 0) {
       if (int rc = sweep_graph(e, batch, last)) return rc;
     } else {
@@ -6655,7 +6680,8 @@ int run_sweep(usap_engine* e, int32_t batch, int32_t first, int32_t last, int32_
           // with every row direct nothing grows, and the flags of the chunk's
           // batches (they only report inconsistent M) are folded at its end
           const bool grow = !e->all_direct || e->prof;
-          if (int rc = launch_batch(e, beg, end, slot, grow)) return rc;
+          finished = !grow && !chunked && i + 1 == last;
+          if (int rc = launch_batch(e, beg, end, slot, grow, finished)) return rc;
         }
         i0 = upto;
         if (!chunked) break;
@@ -6667,7 +6693,8 @@ int run_sweep(usap_engine* e, int32_t batch, int32_t first, int32_t last, int32_
         }
       }
     }
-    if (int rc = launch_finish(e, e->d_hsweep)) return rc;
+    if (!finished)
+      if (int rc = launch_finish(e, e->d_hsweep)) return rc;
     if (int rc = wait_word(e, kWordSweep)) return rc;
     const int32_t executed = first + hs.done - next;  // batches run in this launch round
     if (e->prof)
