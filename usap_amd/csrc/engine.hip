@@ -11,25 +11,29 @@
 //   cap[a] == B  -> direct-mapped row (slot = key), used when a hashed row
 //                   would need >= B slots (dense regime, small B);
 //   cap[a] <  B  -> open-addressing hash (power of two, linear probing);
-//                   a slot is 16 bytes (key, -, o, i; key -1 = empty), so a
-//                   probe and the count update after it share a cache line
-//                   and one 64-bit atomic updates both counts.
-// Keys are never deleted inside a sweep (counts may drop to 0).  Each row
-// also keeps kNBK bucket sums (sum of o + i per key range) for the two-level
-// inverse-CDF pick over the combined weights M[a][b] + M[b][a].  An
+//                   keys (-1 = empty) and counts (o, i) are arrays of their
+//                   own, so eight keys of a chain are two loads, and one 64-bit
+//                   atomic updates both counts.
+// Keys are never deleted inside a sweep (counts may drop to 0).  Rows too long
+// to read whole keep kNBK bucket sums (sum of o + i per key range) for the
+// two-level inverse-CDF pick over the combined weights M[a][b] + M[b][a].  An
 // increment that finds no free slot near its key during nodal batches is
-// parked in an overflow buffer; between two batches k_grow finds the rows
-// whose key count passed 1/slack of the slab or that have parked increments,
-// compacts them in place or moves them to a larger slab at the pool's tail,
-// and replays the parked increments.
+// parked in an overflow buffer; between two batches k_grow takes the rows that
+// have parked increments, and every few batches those marked as past 1/slack of
+// their slab, compacts them in place or moves them to a larger slab at the
+// pool's tail, and replays the parked increments.
 // The host rebuilds M from the labels only when the pool runs out.
 //
 // Kernels (one wavefront of 64 lanes per proposal item):
-//   k_degrees / k_caps / k_fill / k_insert_* / k_build_rows : M build from
-//        labels (graph_parallel.hpp:703-759)
-//   k_merge   : K merge proposals per block + best per block
-//        (graph_parallel.hpp:349-368, :761-988), one workgroup per block,
-//        one wavefront per proposal
+//   k_hist / k_hist_sum : M build from labels (graph_parallel.hpp:703-759) for
+//        few blocks, by LDS histograms
+//   k_degrees / k_caps / k_fill / k_insert_pairs / k_node_lists / k_build_* /
+//        k_bucket_sums : for more, by sorted block pairs or row by row
+//   k_merge_rows / k_merge : K merge proposals per block + best per block
+//        (graph_parallel.hpp:349-368, :761-988), one wavefront per block, or
+//        one workgroup with a wavefront per proposal
+//   k_carry_* : the greedy carry-out (graph_parallel.hpp:1225-1279)
+//   k_begin / k_draw / k_finish : a sweep's state, random words and result
 //   k_nodal   : one nodal proposal per node against the frozen M
 //        (graph_parallel.hpp:990-1222), one wavefront per node
 //   k_apply   : accepted moves -> M, degrees (atomics) and labels; equals
@@ -54,9 +58,9 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cmath>
 #include <chrono>
 #include <climits>
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -2199,8 +2203,12 @@ __device__ Acc merge_overlap_lane(const MView& m, const int64_t* lam, const int6
 
 // A block's row in LDS, shared by its K proposals: its non-zero keys in
 // ascending order with both counts and the running sum of o + i (n = -1: the
-// row has more than kRowLds of them and the proposals read it from M).
-constexpr int kRowLds = 256;
+// row has more than kRowLds of them and the proposals read it from M).  512 of at
+// most 4096 slots: a direct row of 2500 slots with 360 of them non-zero is then
+// read once, not scanned beside row s for each proposal (B = 2500 283 -> 229 us a
+// round, with 256 of 2048 slots before).
+constexpr int kRowLds = 512;
+constexpr int kRowMax = 4096;  // slots of a row looked through for them
 struct RowLds {
   const int32_t* k;
   const int32_t* o;
@@ -2346,7 +2354,8 @@ __global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(
   __shared__ int32_t s_idx[kWaves];
   __shared__ int32_t s_s[kWaves];
   __shared__ __align__(16) int32_t s_scr[kWaves][kD ? 4 : kScr];  // direct rows need none
-  __shared__ __align__(16) int32_t s_rk[kRowLds], s_ro[kRowLds], s_ri[kRowLds];
+  __shared__ int32_t s_uk[kRowLds], s_uo[kRowLds], s_ui[kRowLds];  // as found
+  __shared__ int32_t s_rk[kRowLds], s_ro[kRowLds], s_ri[kRowLds];  // by key
   __shared__ uint32_t s_cum[kRowLds];
   __shared__ int64_t s_lam[kLamMerge];
   __shared__ int32_t s_rn;
@@ -2359,7 +2368,7 @@ __global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(
     // row r's non-zero keys into LDS once for the K proposals (unordered), then
     // ordered by key (ranks: keys are distinct), then the running sums
     const Row R = m_row(a.M, r);
-    const bool fits = R.c <= 8 * kRowLds;  // the same for every thread
+    const bool fits = R.c <= kRowMax;  // the same for every thread
     __syncthreads();
     if (threadIdx.x == 0) s_rn = 0;
     __syncthreads();
@@ -2371,9 +2380,9 @@ __global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(
         if (key >= 0 && (q.o > 0 || q.i > 0)) {
           const int32_t p = atomicAdd(&s_rn, 1);
           if (p < kRowLds) {
-            s_rk[p] = key;
-            s_ro[p] = q.o;
-            s_ri[p] = q.i;
+            s_uk[p] = key;
+            s_uo[p] = q.o;
+            s_ui[p] = q.i;
           }
         }
       }
@@ -2382,41 +2391,30 @@ __global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(
     const int32_t rn = fits ? s_rn : kRowLds + 1;
     RowLds L{s_rk, s_ro, s_ri, s_cum, rn <= kRowLds ? rn : -1};
     if (L.n > 0) {
-      constexpr int kPer = kRowLds / kWave;  // entries per thread (blockDim >= one wavefront)
-      int32_t mk[kPer], mo[kPer], mi[kPer], rank[kPer];
-#pragma unroll
-      for (int q = 0; q < kPer; ++q) {
-        const int32_t e = threadIdx.x + q * blockDim.x;
-        rank[q] = -1;
-        if (e < L.n) {
-          mk[q] = s_rk[e];
-          mo[q] = s_ro[e];
-          mi[q] = s_ri[e];
-          rank[q] = 0;
-          for (int32_t j = 0; j < L.n; ++j) rank[q] += s_rk[j] < mk[q];
-        }
-      }
-      __syncthreads();
-#pragma unroll
-      for (int q = 0; q < kPer; ++q) {
-        if (rank[q] < 0) continue;
-        s_rk[rank[q]] = mk[q];
-        s_ro[rank[q]] = mo[q];
-        s_ri[rank[q]] = mi[q];
+      for (int32_t e = threadIdx.x; e < L.n; e += blockDim.x) {
+        const int32_t key = s_uk[e];
+        int32_t rank = 0;
+#pragma unroll 4
+        for (int32_t j = 0; j < L.n; ++j) rank += s_uk[j] < key;
+        s_rk[rank] = key;
+        s_ro[rank] = s_uo[e];
+        s_ri[rank] = s_ui[e];
       }
       __syncthreads();
       if (w == 0) {
-        uint32_t v[kPer], own = 0;
-#pragma unroll
+        constexpr int kPer = kRowLds / kWave;
+        uint32_t own = 0;
         for (int q = 0; q < kPer; ++q) {
           const int32_t e = lane * kPer + q;
           own += e < L.n ? (uint32_t)s_ro[e] + (uint32_t)s_ri[e] : 0u;
-          v[q] = own;
         }
-        const uint32_t before = wave_incl_scan32(own) - own;
-#pragma unroll
-        for (int q = 0; q < kPer; ++q)
-          if (lane * kPer + q < L.n) s_cum[lane * kPer + q] = before + v[q];
+        uint32_t run = wave_incl_scan32(own) - own;
+        for (int q = 0; q < kPer; ++q) {
+          const int32_t e = lane * kPer + q;
+          if (e >= L.n) break;
+          run += (uint32_t)s_ro[e] + (uint32_t)s_ri[e];
+          s_cum[e] = run;
+        }
       }
       __syncthreads();
     }
@@ -2469,11 +2467,12 @@ __global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(
 // per wavefront, Philox and terms in every lane: B = 200000 4890 -> 1150 us a
 // round.
 constexpr int kRowSlots = 1024;
+constexpr int kRowWave = 256;
 __global__ __launch_bounds__(kWave* kMergeWaves, 4) void k_merge_rows(MergeArgs a, int32_t* list,
                                                                     int32_t* list_n) {
-  __shared__ __align__(16) int32_t s_k[kMergeWaves][kRowLds], s_o[kMergeWaves][kRowLds],
-      s_i[kMergeWaves][kRowLds];
-  __shared__ uint32_t s_cum[kMergeWaves][kRowLds];
+  __shared__ __align__(16) int32_t s_k[kMergeWaves][kRowWave], s_o[kMergeWaves][kRowWave],
+      s_i[kMergeWaves][kRowWave];
+  __shared__ uint32_t s_cum[kMergeWaves][kRowWave];
   __shared__ __align__(16) int32_t s_scr[kMergeWaves][kScr];
   __shared__ int64_t s_lam[kLamMerge];
   const int w = threadIdx.x / kWave, lane = lane_id();
@@ -2510,7 +2509,7 @@ __global__ __launch_bounds__(kWave* kMergeWaves, 4) void k_merge_rows(MergeArgs 
       const bool live = key[q] >= 0 && (x[q].o > 0 || x[q].i > 0);
       const unsigned long long m = __ballot(live);
       const int32_t p = n + __popcll(m & ((1ull << lane) - 1ull));
-      if (live && p < kRowLds) {
+      if (live && p < kRowWave) {
         s_k[w][p] = key[q];
         s_o[w][p] = x[q].o;
         s_i[w][p] = x[q].i;
@@ -2518,13 +2517,13 @@ __global__ __launch_bounds__(kWave* kMergeWaves, 4) void k_merge_rows(MergeArgs 
       n += __popcll(m);
     }
   }
-  if (n > kRowLds) {
+  if (n > kRowWave) {
     if (lane == 0) list[atomicAdd(list_n, 1)] = r;
     return;
   }
   wave_fence();
   // ordered by key
-  constexpr int kPer = kRowLds / kWave;
+  constexpr int kPer = kRowWave / kWave;
   {
     int32_t mk[kPer], mo[kPer], mi[kPer], rank[kPer];
 #pragma unroll
@@ -4146,7 +4145,7 @@ constexpr int32_t kOvfCap = 1 << 22;  // parked increments
 // past 1/slack load) can wait: k_grow looks at marks after a call's first batch
 // and every kGrowEvery-th from there, and else ends after its flags, 5.0 us
 // instead of 9.6 (its launch and first loads), for chains no longer than the
-// walk before parking (E = 10 M, N = 500000, 13600 such batches: 1010 -> 916 ms
+// walk before parking (E = 11 M, N = 500000, 13600 such batches: 1010 -> 916 ms
 // in all; every 4th batch 934).
 constexpr int kGrowEvery = 8;
 static_assert(kNodalWaves * 3 * kWaveSlab == 6 * kGrowLds, "one LDS pool for both paths");
