@@ -2046,12 +2046,20 @@ __global__ void k_carry_init(int32_t B, const int32_t* __restrict__ order,
   cyc[i] = 0;
 }
 
+// kCarryHops of in's windows joined to one: its end and the last rank in it.
+// Two a launch (doubling) took 18 launches at B = 100000, each little more than
+// its own launch and gap (6.5 us); eight a launch take 6 of 6 us.
+constexpr int kCarryHops = 8;
 __global__ void k_carry_jump(int32_t B, const int2* __restrict__ in, int2* __restrict__ out) {
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= B) return;
-  const int2 x = in[i];
-  const int2 y = in[x.x];
-  out[i] = make_int2(y.x, max(x.y, y.y));
+  int2 x = in[i];
+#pragma unroll
+  for (int q = 1; q < kCarryHops; ++q) {
+    const int2 y = in[x.x];
+    x = make_int2(y.x, max(x.y, y.y));
+  }
+  out[i] = x;
 }
 
 __global__ void k_carry_cycle(int32_t B, const int2* __restrict__ pm, int32_t* cyc) {
@@ -2083,9 +2091,22 @@ __global__ void k_carry_link(int32_t B, int32_t B_to_merge, const int32_t* __res
   }
 }
 
+// par[i] to the ancestor kRootHops links of par up, or the root: in place, as
+// another thread's new value is an ancestor too and at least as far.  So the
+// reach is multiplied by kRootHops a launch, whatever the chains (doubling: 18
+// launches, now 4).
+constexpr int kRootHops = 32;
 __global__ void k_carry_root(int32_t B, int32_t* par) {
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < B) par[i] = par[par[i]];  // in place: an ancestor at least as far
+  if (i >= B) return;
+  const int32_t first = par[i];
+  int32_t x = first;
+  for (int q = 1; q < kRootHops; ++q) {
+    const int32_t y = par[x];
+    if (y == x) break;
+    x = y;
+  }
+  if (x != first) par[i] = x;
 }
 
 __global__ void k_carry_alive(int32_t B, const int32_t* __restrict__ bsize,
@@ -6356,7 +6377,7 @@ int carry_out(usap_engine* e, int32_t B_to_merge) {
   int2* pm[2] = {reinterpret_cast<int2*>(e->sort_key[0]), reinterpret_cast<int2*>(e->sort_key[1])};
   k_carry_init<<<g, 256, 0, st>>>(B, a.order, a.best, rank, pm[0], cyc);
   int cur = 0;
-  for (int64_t w = 1; w < B; w <<= 1, cur ^= 1)
+  for (int64_t w = 1; w < B; w *= kCarryHops, cur ^= 1)
     k_carry_jump<<<g, 256, 0, st>>>(B, pm[cur], pm[cur ^ 1]);
   k_carry_cycle<<<g, 256, 0, st>>>(B, pm[cur], cyc);
   k_carry_success<<<g, 256, 0, st>>>(B, pm[cur], cyc, rank, succ);
@@ -6365,7 +6386,7 @@ int carry_out(usap_engine* e, int32_t B_to_merge) {
                                  rocprim::plus<int32_t>(), st));
   k_carry_link<<<g, 256, 0, st>>>(B, B_to_merge, a.best, rank, succ, scan, par, alive, a.short_of,
                                   a.host_short, a.done);
-  for (int64_t w = 1; w < B; w <<= 1) k_carry_root<<<g, 256, 0, st>>>(B, par);
+  for (int64_t w = 1; w < B; w *= kRootHops) k_carry_root<<<g, 256, 0, st>>>(B, par);
   k_carry_alive<<<g, 256, 0, st>>>(B, a.bsize, par, alive);
   bytes = e->sort_tmp_bytes;
   HIPCHK(rocprim::exclusive_scan(e->sort_tmp, bytes, alive, scan, (int32_t)0, (size_t)B,
