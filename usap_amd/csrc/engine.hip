@@ -4781,6 +4781,7 @@ struct usap_engine {
   // captured sweep (usap_params.graphs): replayed while its key matches
   hipGraphExec_t gexec = nullptr;
   int32_t g_B = -1, g_batch = -1, g_nb = -1;
+  bool g_direct = false;  // all_direct at its capture
   uint64_t g_epoch = 0;
   uint64_t epoch = 0;  // bumped by every device allocation (pointers may change)
   int64_t graph_captures = 0;
@@ -6619,14 +6620,19 @@ int launch_batch(usap_engine* e, int32_t beg, int32_t end, size_t ev_slot, bool 
 }
 
 // The batches [0, nb) of a sweep as one HIP graph, captured on first use
-// and replayed while B, the batch size and every device pointer the batch
-// kernels take (epoch) stay the same; the sweep's state (random stream,
-// convergence inputs) lives in device memory, so the kernels' arguments do
-// not change between sweeps.  The graph holds kernel nodes only.
+// and replayed while B, the batch size, every device pointer the batch
+// kernels take (epoch) and whether every row of M is direct stay the same; the
+// sweep's state (random stream, convergence inputs) lives in device memory, so
+// the kernels' arguments do not change between sweeps.  all_direct picks the
+// kernels and what k_grow looks at, and follows the labels, not B alone (a
+// block with few edges has a hashed row at B > 256), so a rebuild at the same B
+// that allocates nothing may change it.  GrowSide::chunk follows the rebuild's
+// total too, but any chunk is right; within one pool it differs by half at
+// most.  The graph holds kernel nodes only.
 int sweep_graph(usap_engine* e, int32_t batch, int32_t nb) {
   hipStream_t st = e->stream;
   if (!e->gexec || e->g_B != e->B || e->g_batch != batch || e->g_nb != nb ||
-      e->g_epoch != e->epoch) {
+      e->g_direct != e->all_direct || e->g_epoch != e->epoch) {
     if (e->gexec) {
       std::lock_guard<std::mutex> lk(g_hip_mu);
       (void)hipGraphExecDestroy(e->gexec);
@@ -6659,6 +6665,7 @@ int sweep_graph(usap_engine* e, int32_t batch, int32_t nb) {
     e->g_B = e->B;
     e->g_batch = batch;
     e->g_nb = nb;
+    e->g_direct = e->all_direct;
     e->g_epoch = e->epoch;
     e->graph_captures++;
   }
