@@ -87,6 +87,7 @@ constexpr int kNBK = 512;                // bucket sums per block row
 constexpr int kLookupRatio = 8;          // a hashed slab this many times a bucket is looked up per key
 constexpr int kScr = 1024;               // per-wavefront LDS scratch (ints) for one bucket
 constexpr int kMergeMany = 16;           // and for few blocks
+constexpr int32_t kMergeGrid = 8192;     // workgroups of k_merge over a list
 constexpr int32_t kMergeFew = 1024;
 constexpr int kDegLds = 1024;            // k_degrees privatises its counters for B <= this
 constexpr int kHistB = 256;              // M is built by histograms in LDS up to here
@@ -2363,13 +2364,25 @@ __device__ void merge_one(const MergeArgs& a, int32_t r, int32_t idx, int32_t* s
   dS_out = acc_value(acc);
 }
 
+// Blocks: the long rows from r[0] on, n[0] of them, the others from r[B - 1]
+// down, n[1] of them (r null: every block).
+struct MergeList {
+  int32_t* r;
+  int32_t* n;
+};
+
 // The K proposals of a block by one workgroup, a wavefront each in turn: every
-// block (list null), or those k_merge_rows left to it.  kWaves: 4, or, where
+// block, or those k_merge_rows left to it.  kWaves: 4, or, where
 // the blocks are too few to fill the GPU, up to 16, so that all of a block's
 // proposals run at once (B = 42: 26 -> 13 us a round).
+// The list's long rows come first: one of 20000 slots
+// is the length of the launch, and started last it adds to it.  A workgroup
+// takes every gridDim.x-th item; kMergeGrid of them are handed out as others end,
+// where one per place on the GPU left some with 7 rows and most with 6 (B =
+// 8000, K = 10, nearly all rows direct: 1280 workgroups 2270 us, 8192 1705; a list
+// of few rows loses nothing to the rest, B = 200000 1345 either way).
 template <int kWaves, bool kD>
-__global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(
-    MergeArgs a, const int32_t* list, const int32_t* list_n) {
+__global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(MergeArgs a, MergeList list) {
   __shared__ long s_hi[kWaves];
   __shared__ unsigned long s_lo[kWaves];
   __shared__ int32_t s_idx[kWaves];
@@ -2383,9 +2396,11 @@ __global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(
   const int w = threadIdx.x / kWave, lane = lane_id();
   const int nw = blockDim.x / kWave;
   for (int i = threadIdx.x; i < kLamMerge; i += blockDim.x) s_lam[i] = a.lam[min(i, a.lam_last)];
-  const int32_t count = list ? *list_n : a.B;
+  const int32_t nlong = list.r ? list.n[0] : 0;
+  const int32_t count = list.r ? nlong + list.n[1] : a.B;
   for (int32_t item = blockIdx.x; item < count; item += gridDim.x) {
-    const int32_t r = list ? list[item] : item;
+    const int32_t r =
+        !list.r ? item : item < nlong ? list.r[item] : list.r[a.B - 1 - (item - nlong)];
     // row r's non-zero keys into LDS once for the K proposals (unordered), then
     // ordered by key (ranks: keys are distinct), then the running sums
     const Row R = m_row(a.M, r);
@@ -2409,7 +2424,7 @@ __global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(
       }
     }
     __syncthreads();
-    const int32_t rn = fits ? s_rn : kRowLds + 1;
+    const int32_t rn = fits ? s_rn : INT32_MAX;
     RowLds L{s_rk, s_ro, s_ri, s_cum, rn <= kRowLds ? rn : -1};
     if (L.n > 0) {
       for (int32_t e = threadIdx.x; e < L.n; e += blockDim.x) {
@@ -2477,8 +2492,8 @@ __global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(
 }
 
 // The K proposals of a block by one wavefront, for hashed rows of at most
-// kRowSlots slots with at most kRowLds non-zero keys (the others go to `list`
-// for k_merge).  Proposal j's draws, picks, decision, corner and degree terms
+// kRowSlots slots with at most kRowWave non-zero keys (the others are marked in
+// best_s for k_merge).  Proposal j's draws, picks, decision, corner and degree terms
 // are lane j's; only a multinomial pick and the overlap are the whole
 // wavefront's, proposal by proposal, the overlap two proposals at a time: r's
 // entries look themselves up in row s, whose eight-key windows nearly always
@@ -2489,8 +2504,9 @@ __global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(
 // round.
 constexpr int kRowSlots = 1024;
 constexpr int kRowWave = 256;
-__global__ __launch_bounds__(kWave* kMergeWaves, 4) void k_merge_rows(MergeArgs a, int32_t* list,
-                                                                    int32_t* list_n) {
+enum : int32_t { kLeft = -1, kLeftLong = -2 };  // in best_s: a block left to k_merge
+__global__ __launch_bounds__(kWave* kMergeWaves, 4) void k_merge_rows(MergeArgs a,
+                                                                    MergeList list) {
   __shared__ __align__(16) int32_t s_k[kMergeWaves][kRowWave], s_o[kMergeWaves][kRowWave],
       s_i[kMergeWaves][kRowWave];
   __shared__ uint32_t s_cum[kMergeWaves][kRowWave];
@@ -2498,6 +2514,7 @@ __global__ __launch_bounds__(kWave* kMergeWaves, 4) void k_merge_rows(MergeArgs 
   __shared__ int64_t s_lam[kLamMerge];
   const int w = threadIdx.x / kWave, lane = lane_id();
   for (int i = threadIdx.x; i < kLamMerge; i += blockDim.x) s_lam[i] = a.lam[min(i, a.lam_last)];
+  if (blockIdx.x == 0 && threadIdx.x < 2) list.n[threadIdx.x] = 0;  // for k_merge_list
   const int32_t B = a.B;
   const int32_t r = blockIdx.x * kMergeWaves + w;
   const bool in = r < B;
@@ -2506,7 +2523,7 @@ __global__ __launch_bounds__(kWave* kMergeWaves, 4) void k_merge_rows(MergeArgs 
   __syncthreads();
   if (!in) return;
   if (R.c == B || R.c > kRowSlots) {
-    if (lane == 0) list[atomicAdd(list_n, 1)] = r;
+    if (lane == 0) a.best_s[r] = R.c > kRowMax ? kLeftLong : kLeft;
     return;
   }
   // the row's non-zero entries, unordered
@@ -2537,9 +2554,10 @@ __global__ __launch_bounds__(kWave* kMergeWaves, 4) void k_merge_rows(MergeArgs 
       }
       n += __popcll(m);
     }
+    if (n > kRowWave) break;
   }
   if (n > kRowWave) {
-    if (lane == 0) list[atomicAdd(list_n, 1)] = r;
+    if (lane == 0) a.best_s[r] = kLeft;
     return;
   }
   wave_fence();
@@ -2716,7 +2734,28 @@ __global__ __launch_bounds__(kWave* kMergeWaves, 4) void k_merge_rows(MergeArgs 
   }
 }
 
-__global__ void k_zero1(int32_t* p) { *p = 0; }
+// The blocks k_merge_rows left.  Two atomics a workgroup: one a block, on one
+// counter, took 1.1 ms of the round where 15000 rows were left (~70 ns each, one
+// after another).
+constexpr int kMergeListThreads = 1024;
+__global__ __launch_bounds__(kMergeListThreads) void k_merge_list(
+    int32_t B, const int32_t* __restrict__ best_s, MergeList list) {
+  __shared__ int32_t s_w[kMergeListThreads / kWave];
+  __shared__ int32_t s_base[2];
+  const int32_t r = blockIdx.x * kMergeListThreads + threadIdx.x;
+  const int32_t left = r < B ? best_s[r] : 0;
+  // both ranks in one scan: long rows in the high half (a workgroup has 1024)
+  int32_t total;
+  const int32_t at =
+      block_scan(left == kLeftLong ? 1 << 16 : left == kLeft ? 1 : 0, s_w, &total);
+  if (total == 0) return;
+  if (threadIdx.x < 2)
+    s_base[threadIdx.x] =
+        atomicAdd(&list.n[threadIdx.x], threadIdx.x == 0 ? total >> 16 : total & 0xffff);
+  __syncthreads();
+  if (left == kLeftLong) list.r[s_base[0] + (at >> 16) - 1] = r;
+  if (left == kLeft) list.r[B - 1 - (s_base[1] + (at & 0xffff) - 1)] = r;
+}
 
 // Ends a call whose last kernel tells the host nothing.
 __global__ void k_word(HostWord done) { host_done(done); }
@@ -6252,17 +6291,18 @@ int usap_merge_propose(usap_engine* e, int32_t K, uint64_t stream, int32_t* best
   a.best_lo = e->best_lo;
   ev_rec(e, 0);
   if (!e->all_direct) {
-    // hashed rows by wavefronts; what they leave (direct or large rows) by the
-    // workgroups of a grid that fills the GPU (the rebuild's arrays are scratch)
-    int32_t *list = e->ecnt_out, *list_n = e->build_flags + 2;
-    k_zero1<<<1, 1, 0, e->stream>>>(list_n);
-    k_merge_rows<<<blocks_for(B, kMergeWaves), kMergeWaves * kWave, 0, e->stream>>>(a, list, list_n);
-    k_merge<kMergeWaves, false><<<(unsigned)std::min<int32_t>(B, 1280), std::min(K, kMergeWaves) * kWave, 0,
-                           e->stream>>>(a, list, list_n);
+    // hashed rows by wavefronts; what they leave (direct or large rows) by
+    // workgroups (the rebuild's arrays are scratch)
+    const MergeList list{e->ecnt_out, e->build_flags + 1};
+    k_merge_rows<<<blocks_for(B, kMergeWaves), kMergeWaves * kWave, 0, e->stream>>>(a, list);
+    k_merge_list<<<blocks_for(B, kMergeListThreads), kMergeListThreads, 0, e->stream>>>(B, a.best_s,
+                                                                                     list);
+    k_merge<kMergeWaves, false><<<(unsigned)std::min<int32_t>(B, kMergeGrid), std::min(K, kMergeWaves) * kWave,
+                                  0, e->stream>>>(a, list);
   } else if (B <= kMergeFew && K > kMergeWaves) {
-    k_merge<kMergeMany, true><<<B, std::min(K, kMergeMany) * kWave, 0, e->stream>>>(a, nullptr, nullptr);
+    k_merge<kMergeMany, true><<<B, std::min(K, kMergeMany) * kWave, 0, e->stream>>>(a, MergeList{});
   } else {
-    k_merge<kMergeWaves, true><<<B, std::min(K, kMergeWaves) * kWave, 0, e->stream>>>(a, nullptr, nullptr);
+    k_merge<kMergeWaves, true><<<B, std::min(K, kMergeWaves) * kWave, 0, e->stream>>>(a, MergeList{});
   }
   HIPCHK(hipGetLastError());
   if (e->uni) e->uni_pos += (int64_t)B * K;
