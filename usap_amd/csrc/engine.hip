@@ -2225,12 +2225,15 @@ __device__ Acc merge_overlap_lane(const MView& m, const int64_t* lam, const int6
 
 // A block's row in LDS, shared by its K proposals: its non-zero keys in
 // ascending order with both counts and the running sum of o + i (n = -1: the
-// row has more than kRowLds of them and the proposals read it from M).  512 of at
-// most 4096 slots: a direct row of 2500 slots with 360 of them non-zero is then
-// read once, not scanned beside row s for each proposal (B = 2500 283 -> 229 us a
-// round, with 256 of 2048 slots before).
-constexpr int kRowLds = 512;
-constexpr int kRowMax = 4096;  // slots of a row looked through for them
+// row has too many of them and the proposals read it from M).  512 of at most 4096
+// slots where K exceeds the workgroup's kMergeWaves: a direct row of 2500 slots
+// with 360 of them non-zero is then read once, not scanned beside row s for each
+// proposal (B = 2500, K = 10 283 -> 229 us a round, with 256 of 2048 slots).  With
+// fewer proposals, all of which run at once, ordering more than 256 keys costs
+// more than it saves (B = 500, all non-zero: K = 1 45 us without and 113 with, K = 4
+// 45 and 65, K = 5 66 and 67).
+constexpr int kRowLds = 512, kRowLdsFew = 256;
+constexpr int kRowSlotsPerKey = 8;  // slots of a row looked through for them, per key
 struct RowLds {
   const int32_t* k;
   const int32_t* o;
@@ -2375,22 +2378,22 @@ struct MergeList {
 // block, or those k_merge_rows left to it.  kWaves: 4, or, where
 // the blocks are too few to fill the GPU, up to 16, so that all of a block's
 // proposals run at once (B = 42: 26 -> 13 us a round).
-// The list's long rows come first: one of 20000 slots
+// kKeys: kRowLds or kRowLdsFew.  The list's long rows come first: one of 20000 slots
 // is the length of the launch, and started last it adds to it.  A workgroup
 // takes every gridDim.x-th item; kMergeGrid of them are handed out as others end,
 // where one per place on the GPU left some with 7 rows and most with 6 (B =
 // 8000, K = 10, nearly all rows direct: 1280 workgroups 2270 us, 8192 1705; a list
 // of few rows loses nothing to the rest, B = 200000 1345 either way).
-template <int kWaves, bool kD>
+template <int kWaves, bool kD, int kKeys>
 __global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(MergeArgs a, MergeList list) {
   __shared__ long s_hi[kWaves];
   __shared__ unsigned long s_lo[kWaves];
   __shared__ int32_t s_idx[kWaves];
   __shared__ int32_t s_s[kWaves];
   __shared__ __align__(16) int32_t s_scr[kWaves][kD ? 4 : kScr];  // direct rows need none
-  __shared__ int32_t s_uk[kRowLds], s_uo[kRowLds], s_ui[kRowLds];  // as found
-  __shared__ int32_t s_rk[kRowLds], s_ro[kRowLds], s_ri[kRowLds];  // by key
-  __shared__ uint32_t s_cum[kRowLds];
+  __shared__ int32_t s_uk[kKeys], s_uo[kKeys], s_ui[kKeys];  // as found
+  __shared__ int32_t s_rk[kKeys], s_ro[kKeys], s_ri[kKeys];  // by key
+  __shared__ uint32_t s_cum[kKeys];
   __shared__ int64_t s_lam[kLamMerge];
   __shared__ int32_t s_rn;
   const int w = threadIdx.x / kWave, lane = lane_id();
@@ -2404,7 +2407,7 @@ __global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(MergeArgs a, MergeLi
     // row r's non-zero keys into LDS once for the K proposals (unordered), then
     // ordered by key (ranks: keys are distinct), then the running sums
     const Row R = m_row(a.M, r);
-    const bool fits = R.c <= kRowMax;  // the same for every thread
+    const bool fits = R.c <= kRowSlotsPerKey * kKeys;  // the same for every thread
     __syncthreads();
     if (threadIdx.x == 0) s_rn = 0;
     __syncthreads();
@@ -2415,7 +2418,7 @@ __global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(MergeArgs a, MergeLi
         const int32_t key = direct ? j : a.M.key[R.o + j];
         if (key >= 0 && (q.o > 0 || q.i > 0)) {
           const int32_t p = atomicAdd(&s_rn, 1);
-          if (p < kRowLds) {
+          if (p < kKeys) {
             s_uk[p] = key;
             s_uo[p] = q.o;
             s_ui[p] = q.i;
@@ -2425,7 +2428,7 @@ __global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(MergeArgs a, MergeLi
     }
     __syncthreads();
     const int32_t rn = fits ? s_rn : INT32_MAX;
-    RowLds L{s_rk, s_ro, s_ri, s_cum, rn <= kRowLds ? rn : -1};
+    RowLds L{s_rk, s_ro, s_ri, s_cum, rn <= kKeys ? rn : -1};
     if (L.n > 0) {
       for (int32_t e = threadIdx.x; e < L.n; e += blockDim.x) {
         const int32_t key = s_uk[e];
@@ -2438,7 +2441,7 @@ __global__ __launch_bounds__(kWave* kWaves, 4) void k_merge(MergeArgs a, MergeLi
       }
       __syncthreads();
       if (w == 0) {
-        constexpr int kPer = kRowLds / kWave;
+        constexpr int kPer = kKeys / kWave;
         uint32_t own = 0;
         for (int q = 0; q < kPer; ++q) {
           const int32_t e = lane * kPer + q;
@@ -2523,7 +2526,7 @@ __global__ __launch_bounds__(kWave* kMergeWaves, 4) void k_merge_rows(MergeArgs 
   __syncthreads();
   if (!in) return;
   if (R.c == B || R.c > kRowSlots) {
-    if (lane == 0) a.best_s[r] = R.c > kRowMax ? kLeftLong : kLeft;
+    if (lane == 0) a.best_s[r] = R.c > kRowSlotsPerKey * kRowLds ? kLeftLong : kLeft;
     return;
   }
   // the row's non-zero entries, unordered
@@ -6297,12 +6300,17 @@ int usap_merge_propose(usap_engine* e, int32_t K, uint64_t stream, int32_t* best
     k_merge_rows<<<blocks_for(B, kMergeWaves), kMergeWaves * kWave, 0, e->stream>>>(a, list);
     k_merge_list<<<blocks_for(B, kMergeListThreads), kMergeListThreads, 0, e->stream>>>(B, a.best_s,
                                                                                      list);
-    k_merge<kMergeWaves, false><<<(unsigned)std::min<int32_t>(B, kMergeGrid), std::min(K, kMergeWaves) * kWave,
-                                  0, e->stream>>>(a, list);
-  } else if (B <= kMergeFew && K > kMergeWaves) {
-    k_merge<kMergeMany, true><<<B, std::min(K, kMergeMany) * kWave, 0, e->stream>>>(a, MergeList{});
+    const auto k = K > kMergeWaves ? k_merge<kMergeWaves, false, kRowLds>
+                                   : k_merge<kMergeWaves, false, kRowLdsFew>;
+    k<<<(unsigned)std::min<int32_t>(B, kMergeGrid), std::min(K, kMergeWaves) * kWave, 0, e->stream>>>(a,
+                                                                                                   list);
+  } else if (K <= kMergeWaves) {
+    k_merge<kMergeWaves, true, kRowLdsFew><<<B, K * kWave, 0, e->stream>>>(a, MergeList{});
+  } else if (B <= kMergeFew) {
+    k_merge<kMergeMany, true, kRowLds><<<B, std::min(K, kMergeMany) * kWave, 0, e->stream>>>(a,
+                                                                                            MergeList{});
   } else {
-    k_merge<kMergeWaves, true><<<B, std::min(K, kMergeWaves) * kWave, 0, e->stream>>>(a, MergeList{});
+    k_merge<kMergeWaves, true, kRowLds><<<B, kMergeWaves * kWave, 0, e->stream>>>(a, MergeList{});
   }
   HIPCHK(hipGetLastError());
   if (e->uni) e->uni_pos += (int64_t)B * K;
