@@ -1881,7 +1881,10 @@ struct CarryArgs {
 };
 
 constexpr int kCarryThreads = 1024;
-constexpr int kCarryRank = 1024;  // blocks ranked by comparing all pairs
+// Blocks ranked by comparing all pairs, above that by the two sorts: a
+// carry-out with its build takes 49 us so and 58 sorted at B = 300, 60 and 58 at
+// 400, 71 and 58 at 512, 355 and 294 at 1024.
+constexpr int kCarryRank = 384;
 constexpr int kCarryOne = 8192;   // blocks one workgroup carries out in its LDS
 
 // Inclusive scan over the workgroup of each thread's own value; the total in
@@ -1903,7 +1906,8 @@ __device__ __forceinline__ int32_t block_scan(int32_t v, int32_t* s_w, int32_t* 
 
 template <int kMax>
 __global__ __launch_bounds__(kCarryThreads) void k_carry_one(CarryArgs a) {
-  constexpr int kI = kMax / kCarryThreads;  // blocks per thread: t + k * kCarryThreads
+  // blocks per thread: t + k * kCarryThreads
+  constexpr int kI = (kMax + kCarryThreads - 1) / kCarryThreads;
   __shared__ int32_t s_p[kMax], s_m[kMax], s_a[kMax];
   __shared__ int32_t s_w[kCarryThreads / kWave];
   const int32_t B = a.B, t = threadIdx.x;
