@@ -1458,12 +1458,14 @@ __global__ __launch_bounds__(kHistB* kSumGroups) void k_hist_sum(HistSum a) {
   }
 }
 
-// M build for kHistB < B <= kPairSortB (rows mostly direct, few distinct
+// M build for kHistB < B <= kPairSortB, B < N (rows mostly direct, few distinct
 // block pairs, so per-edge atomics would pile onto the same counts): the
 // edges' block pairs a*B + b are sorted and summed per pair, then each pair
-// is added once.
+// is added once.  Above, rows are mostly hashed and the build goes by rows
+// (k_build_rows), as it does for B = N, a search's start from one block per node:
+// its pairs are as many as its edges, and sorting them takes longer (set_labels at
+// B = N = 500 128 us by pairs and 107 by rows, 2000 164 and 123, 4096 177 and 120).
 constexpr int32_t kPairSortB = 4096;
-// Above, rows are mostly hashed and the build goes by rows (k_build_rows).
 
 __global__ void k_pair_keys(int64_t E, const int32_t* __restrict__ src,
                             const int32_t* __restrict__ dst, const int32_t* __restrict__ w,
@@ -5213,7 +5215,7 @@ int rebuild_M(usap_engine* e) {
     k<<<blocks_for(e->N, per), 256, 0, st>>>(gview(e), e->labels, B, per, e->d_out, e->d_in,
                                              e->ecnt_out, e->ecnt_in, e->bsize);
   }
-  const bool by_rows = B > kPairSortB;
+  const bool by_rows = B > kPairSortB || B == e->N;
   int2* items = by_rows ? e->big_items : nullptr;
   int32_t* n_items = e->build_flags + 1;
   k_caps<<<blocks_for((int64_t)B + 1, 256), 256, 0, st>>>(
