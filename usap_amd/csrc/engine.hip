@@ -1496,13 +1496,15 @@ __global__ void k_insert_pairs(int64_t E, const uint32_t* __restrict__ key,
 }
 
 // Bucket sums (o + i) of the block rows that keep them: up to kSumRows rows to a
-// workgroup (fewer while that leaves the GPU short of workgroups: B = 2500, 64
-// a workgroup 194 us, now 19), which handles those of them one by one (a block
-// that absorbed thousands of nodes has a slab of 16384 slots or more: 16
-// wavefronts with 8 slots a thread in flight take 92 us, 4 took 124).  Sets
-// the hashed ones' marks too (room_mark).
+// workgroup (fewer while that leaves the GPU short of workgroups), which handles
+// those of them one by one, eight slots a thread in flight.  Most rows that keep
+// sums have up to a few thousand slots: workgroups of 4 wavefronts take 6.1 us at
+// B = 513, 12.3 at 2000, 26 at 4000 and 38 at 5000, of 16 11.8, 31, 62 and 75; a block
+// that absorbed thousands of nodes (slabs of 16384 slots and more at B = 20000) takes
+// 93 with 4 and 96 with 16.  Sets the hashed ones' marks too (room_mark).
 constexpr int kSumRows = 64;
-__global__ __launch_bounds__(1024) void k_bucket_sums(MView m, int32_t rows) {
+constexpr int kSumThreads = 256;
+__global__ __launch_bounds__(kSumThreads) void k_bucket_sums(MView m, int32_t rows) {
   __shared__ int32_t s_b[kNBK];
   __shared__ int32_t s_keys;
   const int lane = lane_id();
@@ -5256,8 +5258,8 @@ int rebuild_M(usap_engine* e) {
     if (int rc = build_by_pairs(e)) return rc;
   }
   if (B > kNBK) {
-    const int32_t rows = std::min(kSumRows, 1 + B / 2048);
-    k_bucket_sums<<<blocks_for(B, rows), 1024, 0, st>>>(view(e->M, B), rows);
+    const int32_t rows = std::min(kSumRows, 1 + B / 4096);
+    k_bucket_sums<<<blocks_for(B, rows), kSumThreads, 0, st>>>(view(e->M, B), rows);
   }
   HIPCHK(hipGetLastError());
   ev_rec(e, 1);
