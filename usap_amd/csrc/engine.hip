@@ -80,8 +80,6 @@ namespace {
 
 constexpr int kWave = 64;
 constexpr int kNodalWaves = 4;           // wavefronts per workgroup in k_nodal / k_apply
-constexpr int kTab = 512;                // per-wavefront LDS table slots
-constexpr int kTabMaxDeg = kTab * 3 / 4; // larger nodes use a global-memory table
 constexpr int kMergeWaves = 4;           // wavefronts per workgroup in k_merge
 constexpr int kNBK = 512;                // bucket sums per block row
 constexpr int kLookupRatio = 8;          // a hashed slab this many times a bucket is looked up per key
@@ -215,11 +213,6 @@ struct Row {
 template <bool kD = false>
 __device__ __forceinline__ Row m_row(const MView& m, int32_t a) {
   return kD ? Row{(int64_t)a * m.B, m.B} : Row{m.off[a], m.cap[a]};
-}
-
-// First slot of key b in row R (the column itself in a direct row).
-__device__ __forceinline__ int64_t m_slot(const MView& m, Row R, int32_t b) {
-  return R.c == m.B ? R.o + b : R.o + (int64_t)(hash32(b) & (uint32_t)(R.c - 1));
 }
 
 // A lookup's first probe: the slot with the key and counts found there.  The
@@ -593,10 +586,7 @@ __device__ __forceinline__ int64_t lam_of(const int64_t* lam, int32_t m) {
   return lam[max(m, 0)];
 }
 
-// + or - m * lambda(m): one L term (0 for m <= 0)
-__device__ __forceinline__ void add_L(Acc& a, const int64_t* lam, int32_t m) {
-  acc_add(a, max(m, 0), lam_of(lam, m));
-}
+// - m * lambda(m): one L term (0 for m <= 0)
 __device__ __forceinline__ void sub_L(Acc& a, const int64_t* lam, int32_t m) {
   acc_add(a, -max(m, 0), lam_of(lam, m));
 }
@@ -2843,23 +2833,6 @@ struct NodalArgs {
   unsigned long long* tstamp;  // workgroup stamps (start [b], end [tstride + b]) or null
   int32_t tstride;
 };
-
-__device__ __forceinline__ void tab_add(int32_t* tk, int32_t* tv, uint32_t mask, int32_t b,
-                                        int32_t w) {
-  uint32_t h = hash32(b) & mask;
-  for (;;) {
-    int32_t k = __hip_atomic_load(&tk[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-    if (k < 0) {
-      k = atomicCAS(&tk[h], -1, b);
-      if (k == -1) k = b;
-    }
-    if (k == b) {
-      atomicAdd(&tv[h], w);
-      return;
-    }
-    h = (h + 1) & mask;
-  }
-}
 
 // List entry j of node n (out-edges then in-edges): neighbour id (-1 past the
 // end) and weight.
@@ -5509,8 +5482,35 @@ void lambda_prefix(int64_t maxv, int64_t* out) { lambda_range(0, maxv, out); }
     if (_rc) return _rc; \
   } while (0)
 
+// Global-memory unit tables of the nodes that may have more units than the
+// workgroup's LDS table holds (hub_terms<.., true>), and the largest list, from
+// the host copy of the offsets.
+int build_big_tables(usap_engine* e) {
+  const int32_t N = e->N;
+  std::vector<int64_t> big((size_t)N, -1);
+  int64_t big_total = 0;
+  e->max_list = 0;
+  for (int32_t x = 0; x < N; ++x) {
+    const int64_t k = (e->h_out_ptr[x + 1] - e->h_out_ptr[x]) + (e->h_in_ptr[x + 1] - e->h_in_ptr[x]);
+    e->max_list = std::max(e->max_list, k);
+    if (k > kHubUnits) {
+      int64_t cap = 1;
+      while (cap < 2 * k) cap <<= 1;
+      big[x] = big_total;
+      big_total += 2 * cap;
+    }
+  }
+  dfree(e, e->big_off);
+  dfree(e, e->big_tab);
+  TRY(dalloc(e, &e->big_off, N));
+  TRY(dalloc(e, &e->big_tab, big_total));
+  HIPCHK(hipMemcpyAsync(e->big_off, big.data(), sizeof(int64_t) * N, hipMemcpyHostToDevice, e->stream));
+  HIPCHK(hipStreamSynchronize(e->stream));  // `big` is released on return
+  return USAP_OK;
+}
+
 // The graph's edges on the device: host copy, CSR/CSC, edge sources, the
-// lambda table over [0, wtot] and the global tables of large nodes.  Frees
+// lambda table over [0, wtot] and the tables of large nodes.  Frees
 // the previous graph's arrays first (same N).
 int load_graph(usap_engine* e, const usap_graph* g, int64_t wtot) {
   const int32_t N = g->N;
@@ -5537,9 +5537,8 @@ int load_graph(usap_engine* e, const usap_graph* g, int64_t wtot) {
   e->hg.in_idx = e->h_in_idx.data();
   e->hg.out_w = e->weighted ? e->h_out_w.data() : nullptr;
   e->hg.in_w = e->weighted ? e->h_in_w.data() : nullptr;
-  for (int32_t** q : {&e->out_idx, &e->in_idx, &e->out_src, &e->out_w, &e->in_w, &e->big_tab})
-    dfree(e, *q);
-  for (int64_t** q : {&e->out_ptr, &e->in_ptr, &e->lam, &e->big_off}) dfree(e, *q);
+  for (int32_t** q : {&e->out_idx, &e->in_idx, &e->out_src, &e->out_w, &e->in_w}) dfree(e, *q);
+  for (int64_t** q : {&e->out_ptr, &e->in_ptr, &e->lam}) dfree(e, *q);
   TRY(dalloc(e, &e->out_ptr, N + 1));
   TRY(dalloc(e, &e->in_ptr, N + 1));
   TRY(dalloc(e, &e->out_idx, E));
@@ -5557,22 +5556,6 @@ int load_graph(usap_engine* e, const usap_graph* g, int64_t wtot) {
   std::vector<int32_t> src((size_t)E);
   for (int32_t x = 0; x < N; ++x)
     for (int64_t j = g->out_ptr[x]; j < g->out_ptr[x + 1]; ++j) src[j] = x;
-  // global-memory neighbour tables of the nodes too large for LDS
-  std::vector<int64_t> big((size_t)N, -1);
-  int64_t big_total = 0;
-  e->max_list = 0;
-  for (int32_t x = 0; x < N; ++x) {
-    const int64_t k = (g->out_ptr[x + 1] - g->out_ptr[x]) + (g->in_ptr[x + 1] - g->in_ptr[x]);
-    e->max_list = std::max(e->max_list, k);
-    if (k > kTabMaxDeg) {
-      int64_t cap = 1;
-      while (cap < 2 * k) cap <<= 1;
-      big[x] = big_total;
-      big_total += 3 * cap;
-    }
-  }
-  TRY(dalloc(e, &e->big_off, N));
-  TRY(dalloc(e, &e->big_tab, big_total));
   hipStream_t st = e->stream;
   HIPCHK(hipMemcpyAsync(e->out_ptr, g->out_ptr, sizeof(int64_t) * (N + 1), hipMemcpyHostToDevice, st));
   HIPCHK(hipMemcpyAsync(e->in_ptr, g->in_ptr, sizeof(int64_t) * (N + 1), hipMemcpyHostToDevice, st));
@@ -5586,35 +5569,9 @@ int load_graph(usap_engine* e, const usap_graph* g, int64_t wtot) {
     }
   }
   HIPCHK(hipMemcpyAsync(e->lam, lam.data(), sizeof(int64_t) * (wtot + 1), hipMemcpyHostToDevice, st));
-  HIPCHK(hipMemcpyAsync(e->big_off, big.data(), sizeof(int64_t) * N, hipMemcpyHostToDevice, st));
+  TRY(build_big_tables(e));
   // the host vectors above are released when this returns: wait for the copies
   HIPCHK(hipStreamSynchronize(st));
-  return USAP_OK;
-}
-
-// Global-memory neighbour tables of the nodes whose lists exceed the LDS
-// table (kTabMaxDeg), from the host copy of the offsets.
-int build_big_tables(usap_engine* e) {
-  const int32_t N = e->N;
-  std::vector<int64_t> big((size_t)N, -1);
-  int64_t big_total = 0;
-  e->max_list = 0;
-  for (int32_t x = 0; x < N; ++x) {
-    const int64_t k = (e->h_out_ptr[x + 1] - e->h_out_ptr[x]) + (e->h_in_ptr[x + 1] - e->h_in_ptr[x]);
-    e->max_list = std::max(e->max_list, k);
-    if (k > kTabMaxDeg) {
-      int64_t cap = 1;
-      while (cap < 2 * k) cap <<= 1;
-      big[x] = big_total;
-      big_total += 3 * cap;
-    }
-  }
-  dfree(e, e->big_off);
-  dfree(e, e->big_tab);
-  TRY(dalloc(e, &e->big_off, N));
-  TRY(dalloc(e, &e->big_tab, big_total));
-  HIPCHK(hipMemcpyAsync(e->big_off, big.data(), sizeof(int64_t) * N, hipMemcpyHostToDevice, e->stream));
-  HIPCHK(hipStreamSynchronize(e->stream));  // `big` is released on return
   return USAP_OK;
 }
 
