@@ -37,12 +37,10 @@ class Engine:
         self.params = default_params(**params)
         h = C.c_void_p()
         if edges is not None:
-            src, dst, w = edges
-            check(lib().usap_create_from_edges(
-                graph.N, len(src), ptr(np.ascontiguousarray(src, np.int32)),
-                ptr(np.ascontiguousarray(dst, np.int32)),
-                None if w is None else ptr(np.ascontiguousarray(w, np.int32)),
-                C.byref(self.params), C.byref(h)))
+            # held by these names until the call is over: ptr() is an address only
+            src, dst, w = (None if x is None else np.ascontiguousarray(x, np.int32) for x in edges)
+            check(lib().usap_create_from_edges(graph.N, len(src), ptr(src), ptr(dst), ptr(w),
+                                               C.byref(self.params), C.byref(h)))
         else:
             self._gs = graph.as_struct()
             check(lib().usap_create(C.byref(self._gs), C.byref(self.params), C.byref(h)))
@@ -52,8 +50,8 @@ class Engine:
         """Append edges after the current ones (usap_append_edges)."""
         src = np.ascontiguousarray(src, np.int32)
         dst = np.ascontiguousarray(dst, np.int32)
-        wp = None if w is None else ptr(np.ascontiguousarray(w, np.int32))
-        self._ck(lib().usap_append_edges(self.h, len(src), ptr(src), ptr(dst), wp))
+        w = None if w is None else np.ascontiguousarray(w, np.int32)
+        self._ck(lib().usap_append_edges(self.h, len(src), ptr(src), ptr(dst), ptr(w)))
 
     def close(self):
         if getattr(self, "h", None):
