@@ -1489,12 +1489,14 @@ __global__ void k_insert_pairs(int64_t E, const uint32_t* __restrict__ key,
 // workgroup (fewer while that leaves the GPU short of workgroups), which handles
 // those of them one by one, eight slots a thread in flight.  Most rows that keep
 // sums have up to a few thousand slots: workgroups of 4 wavefronts take 6.1 us at
-// B = 513, 12.3 at 2000, 26 at 4000 and 38 at 5000, of 16 11.8, 31, 62 and 75; a block
-// that absorbed thousands of nodes (slabs of 16384 slots and more at B = 20000) takes
-// 93 with 4 and 96 with 16.  Sets the hashed ones' marks too (room_mark).
+// B = 513, 12.3 at 2000, 26 at 4000 and 38 at 5000, of 16 11.8, 31, 62 and 75.  Above
+// B = 16384 few rows keep sums and one may be longer than 4 wavefronts take in a
+// few rounds: a direct row of 100000 slots costs 33 us more with 4, blocks of
+// thousands of nodes at B = 20000 take 93 with 4 and 96 with 16.  Sets the hashed
+// ones' marks too (room_mark).
 constexpr int kSumRows = 64;
-constexpr int kSumThreads = 256;
-__global__ __launch_bounds__(kSumThreads) void k_bucket_sums(MView m, int32_t rows) {
+constexpr int32_t kSumLongB = 16384;
+__global__ __launch_bounds__(1024) void k_bucket_sums(MView m, int32_t rows) {
   __shared__ int32_t s_b[kNBK];
   __shared__ int32_t s_keys;
   const int lane = lane_id();
@@ -5232,7 +5234,7 @@ int rebuild_M(usap_engine* e) {
   }
   if (B > kNBK) {
     const int32_t rows = std::min(kSumRows, 1 + B / 4096);
-    k_bucket_sums<<<blocks_for(B, rows), kSumThreads, 0, st>>>(view(e->M, B), rows);
+    k_bucket_sums<<<blocks_for(B, rows), B > kSumLongB ? 1024 : 256, 0, st>>>(view(e->M, B), rows);
   }
   HIPCHK(hipGetLastError());
   ev_rec(e, 1);
