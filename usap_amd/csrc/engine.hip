@@ -1215,38 +1215,47 @@ __global__ __launch_bounds__(256) void k_fill_big(MView M, int32_t* key, const i
 // summed per neighbour block in LDS, then each sum goes to M with one atomic.
 // (An atomic per edge end piled onto a large block's own count: B = 100000
 // with a block of 7000 nodes 526 -> 191 us.)  Keys beyond what the table holds near
-// their home are added to M directly.
+// their home are added to M directly.  kHuge: nodes of more than kBigPart entries
+// are left out of the items and come kHugePart entries a workgroup (`items`: node
+// and part, n_huge of them), where one node in its item's kBigParts workgroups set
+// the length of the build (set_labels at N = 100000, B = 20000 with one node of
+// 2 M entries 4179 us, now 356, of 200000 648 and 261, of 9000 241 and 233; by parts
+// of 2048 entries 376, 273 and 246).  Their rows are always among these: they have
+// more than kBigPart entries, or are direct.
 constexpr int kBigTab = 4096;
 constexpr int kBigWalk = 8;
 constexpr int32_t kBigPart = 8192;  // list entries from which an item is split
 constexpr int kBigParts = 4;
+constexpr int32_t kHugePart = 1024;  // list entries of a huge node to a workgroup
 constexpr unsigned kBigGrid = 768;  // three workgroups of 51 KB of LDS per CU
+template <bool kHuge>
 __global__ __launch_bounds__(256) void k_build_big(GraphView g, const int32_t* __restrict__ labels,
                                                    const int32_t* __restrict__ bl_off,
                                                    const int32_t* __restrict__ bl_nodes, MView M,
                                                    const int2* items, const int32_t* n_items,
-                                                   int32_t* flags) {
+                                                   int32_t n_huge, int32_t* flags) {
   __shared__ int32_t s_k[kBigTab], s_o[kBigTab], s_i[kBigTab];
   __shared__ int64_t s_o0[kBigNodes], s_i0[kBigNodes];
   __shared__ long s_ko[kBigNodes], s_pre[kBigNodes + 1];
   const int lane = lane_id();
-  const int32_t n = *n_items;
+  const int32_t n = kHuge ? n_huge : *n_items;
   for (int32_t it = blockIdx.x; it < n; it += gridDim.x) {
     const int2 q = items[it];
-    const int32_t a = q.x;
-    const int32_t n0 = bl_off[a] + q.y * kBigNodes;
-    const int32_t n1 = min(n0 + kBigNodes, a + 1 < M.B ? bl_off[a + 1] : g.N);
+    const int32_t a = kHuge ? labels[q.x] : q.x;
+    const int32_t n0 = kHuge ? 0 : bl_off[a] + q.y * kBigNodes;
+    const int32_t n1 = kHuge ? 1 : min(n0 + kBigNodes, a + 1 < M.B ? bl_off[a + 1] : g.N);
     __syncthreads();  // the previous item's table is written out
     if (threadIdx.x < kWave) {
       const int32_t j = n0 + lane;
       int64_t o0 = 0, i0 = 0;
       long ko = 0, kn = 0;
       if (j < n1) {
-        const int32_t x = bl_nodes[j];
+        const int32_t x = kHuge ? q.x : bl_nodes[j];
         o0 = g.out_ptr[x];
         i0 = g.in_ptr[x];
         ko = g.out_ptr[x + 1] - o0;
         kn = ko + (g.in_ptr[x + 1] - i0);
+        if (!kHuge && kn > kBigPart) kn = 0;
       }
       const long inc = wave_incl_scan(kn);
       if (lane < kBigNodes) {
@@ -1260,8 +1269,9 @@ __global__ __launch_bounds__(256) void k_build_big(GraphView g, const int32_t* _
     __syncthreads();
     const long tot = s_pre[kBigNodes];
     const long parts = tot > kBigPart ? (long)gridDim.y : 1;
-    if ((long)blockIdx.y >= parts) continue;  // the same for every thread
-    const long e0 = tot * (long)blockIdx.y / parts, e1 = tot * ((long)blockIdx.y + 1) / parts;
+    if (!kHuge && (long)blockIdx.y >= parts) continue;  // the same for every thread
+    const long e0 = kHuge ? (long)q.y * kHugePart : tot * (long)blockIdx.y / parts;
+    const long e1 = kHuge ? min(tot, e0 + kHugePart) : tot * ((long)blockIdx.y + 1) / parts;
     int32_t tab = 256;  // a power of two >= twice the entries, at most kBigTab
     while (tab < kBigTab && tab < 2 * (e1 - e0)) tab <<= 1;
     for (int i = threadIdx.x; i < tab; i += 256) {
@@ -4825,6 +4835,8 @@ struct usap_engine {
   size_t pair_tmp_bytes = 0;
   int64_t* big_off = nullptr;
   int32_t* big_tab = nullptr;
+  int2* huge_parts = nullptr;  // (node, part of kHugePart list entries) of nodes of more than kBigPart
+  int32_t n_huge = 0;
   int64_t max_list = 0;  // list entries of the largest node
   // entropy
   long* ent_part = nullptr;
@@ -5089,8 +5101,12 @@ int build_rows(usap_engine* e) {
       gview(e), e->labels, e->bl_off, e->bl_nodes, M, e->build_flags);
   k_build_rows<kRowTab, 256><<<blocks_for(B, kNodalWaves), kWave * kNodalWaves, 0, st>>>(
       gview(e), e->labels, e->bl_off, e->bl_nodes, M, e->build_flags);
-  k_build_big<<<dim3(kBigGrid, kBigParts), 256, 0, st>>>(gview(e), e->labels, e->bl_off, e->bl_nodes,
-                                                         M, e->big_items, n_items, e->build_flags);
+  k_build_big<false><<<dim3(kBigGrid, kBigParts), 256, 0, st>>>(
+      gview(e), e->labels, e->bl_off, e->bl_nodes, M, e->big_items, n_items, 0, e->build_flags);
+  if (e->n_huge > 0)
+    k_build_big<true><<<std::min<unsigned>((unsigned)e->n_huge, kBigGrid * kBigParts), 256, 0, st>>>(
+        gview(e), e->labels, e->bl_off, e->bl_nodes, M, e->huge_parts, nullptr, e->n_huge,
+        e->build_flags);
   HIPCHK(hipGetLastError());
   return USAP_OK;
 }
@@ -5415,6 +5431,7 @@ int usap_destroy(usap_engine* e) {
   pin_put(e->h_short, 64);
   dfree(e, e->big_off);
   dfree(e, e->big_tab);
+  dfree(e, e->huge_parts);
   dfree(e, e->ent_part);
   pin_put(e->h_fx, 64);
   for (int i = 0; i < kNumSnap; ++i) dfree(e, e->snap_labels[i]);
@@ -5485,11 +5502,13 @@ void lambda_prefix(int64_t maxv, int64_t* out) { lambda_range(0, maxv, out); }
   } while (0)
 
 // Global-memory unit tables of the nodes that may have more units than the
-// workgroup's LDS table holds (hub_terms<.., true>), and the largest list, from
-// the host copy of the offsets.
+// workgroup's LDS table holds (hub_terms<.., true>), the parts of the nodes that
+// builds split (k_build_big<true>), and the largest list, from the host copy of
+// the offsets.
 int build_big_tables(usap_engine* e) {
   const int32_t N = e->N;
   std::vector<int64_t> big((size_t)N, -1);
+  std::vector<int2> huge;
   int64_t big_total = 0;
   e->max_list = 0;
   for (int32_t x = 0; x < N; ++x) {
@@ -5501,13 +5520,23 @@ int build_big_tables(usap_engine* e) {
       big[x] = big_total;
       big_total += 2 * cap;
     }
+    if (k > kBigPart)
+      for (int64_t i = 0; i * kHugePart < k; ++i) huge.push_back(make_int2(x, (int32_t)i));
   }
   dfree(e, e->big_off);
   dfree(e, e->big_tab);
+  dfree(e, e->huge_parts);
+  e->n_huge = 0;
   TRY(dalloc(e, &e->big_off, N));
   TRY(dalloc(e, &e->big_tab, big_total));
   HIPCHK(hipMemcpyAsync(e->big_off, big.data(), sizeof(int64_t) * N, hipMemcpyHostToDevice, e->stream));
-  HIPCHK(hipStreamSynchronize(e->stream));  // `big` is released on return
+  if (!huge.empty()) {
+    TRY(dalloc(e, &e->huge_parts, huge.size()));
+    HIPCHK(hipMemcpyAsync(e->huge_parts, huge.data(), sizeof(int2) * huge.size(),
+                          hipMemcpyHostToDevice, e->stream));
+    e->n_huge = (int32_t)huge.size();
+  }
+  HIPCHK(hipStreamSynchronize(e->stream));  // the vectors are released on return
   return USAP_OK;
 }
 
