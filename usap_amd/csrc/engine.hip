@@ -168,6 +168,7 @@ struct MView {
   struct GrowState* gst;
   int32_t B;
   int32_t bshift;  // bucket of key k = k >> bshift
+  int32_t stride;  // slots from a row to the next while all are direct (direct_stride)
   int32_t slack;   // slab_slack: a hashed row grows past 1/slack load
 };
 
@@ -208,11 +209,11 @@ struct Row {
 };
 
 // kD: every row of M is direct (the host knows it from the rebuild), so row a
-// is the a-th B slots of the pool: no row header to load before a lookup, no
-// key, no probing.
+// is the first B of the a-th `stride` slots of the pool: no row header to load
+// before a lookup, no key, no probing.
 template <bool kD = false>
 __device__ __forceinline__ Row m_row(const MView& m, int32_t a) {
-  return kD ? Row{(int64_t)a * m.B, m.B} : Row{m.off[a], m.cap[a]};
+  return kD ? Row{(int64_t)a * m.stride, m.B} : Row{m.off[a], m.cap[a]};
 }
 
 // A lookup's first probe: the slot with the key and counts found there.  The
@@ -1413,7 +1414,8 @@ struct HistSum {
 constexpr int kSumGroups = 4;
 __global__ __launch_bounds__(kHistB* kSumGroups) void k_hist_sum(HistSum a) {
   __shared__ int32_t s_v[kSumGroups][kHistB];
-  const int32_t B = a.M.B, t = threadIdx.x % kHistB, w = threadIdx.x / kHistB, r = blockIdx.x;
+  const int32_t B = a.M.B, stride = a.M.stride;
+  const int32_t t = threadIdx.x % kHistB, w = threadIdx.x / kHistB, r = blockIdx.x;
   const bool row = r < B;
   const int32_t k = r - B;  // which of d_out, d_in, sizes
   const int64_t n = row ? (int64_t)B * B : 3 * kHistB;
@@ -1435,25 +1437,28 @@ __global__ __launch_bounds__(kHistB* kSumGroups) void k_hist_sum(HistSum a) {
 #pragma unroll
     for (int q = 1; q < kSumGroups; ++q) v += s_v[q][t];
     if (row) {
-      a.M.cnt[(int64_t)r * B + t].o = v;
-      a.M.cnt[(int64_t)t * B + r].i = v;
+      a.M.cnt[(int64_t)r * stride + t].o = v;
+      a.M.cnt[(int64_t)t * stride + r].i = v;
     } else {
       (k == 0 ? a.d_out : k == 1 ? a.d_in : a.bsize)[t] = v;
     }
   }
+  if (row)
+    for (int32_t i = B + threadIdx.x; i < stride; i += kHistB * kSumGroups)
+      a.M.cnt[(int64_t)r * stride + i] = Cnt{0, 0};
   if (row) {
     if (threadIdx.x == 0) {
-      a.off[r] = (int64_t)r * B;
+      a.off[r] = (int64_t)r * stride;
       a.cap[r] = B;
     }
   } else if (k == 0) {
     for (int i = threadIdx.x; i < kGrowBlocks; i += kHistB * kSumGroups)
       a.M.gst->chunk[i].pos = a.M.gst->chunk[i].end = 0;
     if (threadIdx.x == 0) {
-      a.off[B] = (int64_t)B * B;
+      a.off[B] = (int64_t)B * stride;
       a.M.gst->nospace = 0;
       a.M.gst->ovf_n = 0;
-      a.M.gst->used = (unsigned long long)B * (unsigned long long)B;
+      a.M.gst->used = (unsigned long long)B * (unsigned long long)stride;
     }
   }
 }
@@ -1757,6 +1762,7 @@ struct EntropyIn {
   const long* part;
   int32_t nparts;  // 0: from M
   const Cnt* cnt;
+  int64_t slots;
   const int32_t *d_out, *d_in;
   int32_t B;
   const int64_t* lam;
@@ -1770,7 +1776,7 @@ __device__ __forceinline__ i128 block_entropy(const EntropyIn& a) {
     return block_sum128(t);
   }
   Acc acc{0, 0};
-  const int32_t n = a.B * a.B;
+  const int32_t n = (int32_t)a.slots;
   constexpr int kQ = 8;
   for (int32_t i0 = threadIdx.x; i0 < n; i0 += kQ * blockDim.x) {
     int32_t v[kQ];
@@ -4739,6 +4745,7 @@ struct DevSpM {
   GrowState* gst = nullptr;
   int64_t P = 0;      // allocated slots
   int64_t total = 0;  // slots in use after the last rebuild
+  int32_t stride = 0;  // MView::stride
   int32_t slack = 2;  // usap_params.slab_slack
 };
 
@@ -4969,6 +4976,13 @@ int32_t bucket_shift(int32_t B) {
   return sh;
 }
 
+// Slots from a row to the next after a histogram build: for few blocks each row
+// begins a 256-byte piece of its own, as k_apply's atomics from all XCDs on a few
+// neighbouring lines hold each other up.  N = 100000, 25000-node batches from random
+// labels (10000 moves), k_apply packed and so: B = 4 603 and 383 us, 7 696 and 324, 10
+// 468 and 270, 20 268 and 200, 30 192 and 185, 50 142 and 140.
+int32_t direct_stride(int32_t B) { return B <= 64 ? (B + 31) / 32 * 32 : B; }
+
 MView view(const DevSpM& m, int32_t B) {
   MView v;
   v.off = m.off;
@@ -4983,6 +4997,7 @@ MView view(const DevSpM& m, int32_t B) {
   v.gst = m.gst;
   v.B = B;
   v.bshift = bucket_shift(B);
+  v.stride = m.stride;
   v.slack = m.slack;
   return v;
 }
@@ -5136,6 +5151,7 @@ int build_hist(usap_engine* e) {
   const bool one = B <= kHistOne;
   const int32_t halves = one ? 1 : 2;
   const int32_t G = (int32_t)std::max<int64_t>(1, std::min<int64_t>(e->E / 4096, 256 / halves));
+  e->M.stride = direct_stride(B);
   const int64_t need = (int64_t)G * B * B + (int64_t)G * halves * 3 * kHistB;
   if (need > e->hist_cap) {
     dfree(e, e->hist);
@@ -5143,7 +5159,7 @@ int build_hist(usap_engine* e) {
     if (int rc = dalloc(e, &e->hist, (size_t)need)) return rc;
     e->hist_cap = need;
   }
-  if (int rc = reserve_pool(e, (int64_t)B * B)) return rc;
+  if (int rc = reserve_pool(e, (int64_t)B * e->M.stride)) return rc;
   e->all_direct = true;
   HistArgs a;
   a.g = gview(e);
@@ -5235,6 +5251,7 @@ int rebuild_M(usap_engine* e) {
   // no insert probes, so no row ever needs growth or an increment parked until
   // the next rebuild, and k_grow only has the batch's error flags to fold
   e->all_direct = tot == (int64_t)B * B;
+  m.stride = B;
   if (m.total > 0 && !by_rows) k_fill<<<std::min<int64_t>(blocks_for(m.total, 256), 8192), 256, 0, st>>>(
       e->all_direct ? nullptr : m.key, m.cnt, m.total);
   k_reset_grow<<<blocks_for(kGrowBlocks, 256), 256, 0, st>>>(m.gst, (unsigned long long)m.total);
@@ -6164,8 +6181,8 @@ int wait_word(usap_engine* e, int slot) {
 // loads in flight).
 // No launch when one workgroup takes M itself (k_begin, k_entropy_out).
 EntropyIn launch_entropy(usap_engine* e, long* part) {
-  EntropyIn in{part, 0, e->M.cnt, e->d_out, e->d_in, e->B, e->lam};
-  if (e->all_direct && (int64_t)e->B * e->B <= kEntropyOne) return in;
+  EntropyIn in{part, 0, e->M.cnt, e->M.total, e->d_out, e->d_in, e->B, e->lam};
+  if (e->all_direct && in.slots <= kEntropyOne) return in;
   const int64_t work = std::max<int64_t>(e->M.P, e->B);
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(kEntropyBlocks, blocks_for(work, 1024)));
   k_entropy<<<grid, 256, 0, e->stream>>>(e->M.cnt, e->M.gst, e->d_out, e->d_in, e->B, e->lam,
