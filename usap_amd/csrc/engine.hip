@@ -2932,8 +2932,9 @@ __device__ __forceinline__ void corner_terms(const NodalArgs& a, const Corner& c
   const int32_t dW = now ? (col ? Wi : Wo) : 0;
   const int32_t mp = (col ? (row ? Ys : Yr) : (row ? Xs : Xr)) + (row ? dW : -dW);
   const int32_t m = deg ? mp : mt;
-  const int32_t d1 = deg && !col ? dout : din, d2 = deg ? 1 : dout;  // lambda(1) = 0
-  const bool bad = d1 <= 0 || d2 <= 0;
+  // lambda(0) = 0 stands for what a degree term lacks (the table may end there)
+  const int32_t d1 = deg && !col ? dout : din, d2 = deg ? 0 : dout;
+  const bool bad = d1 <= 0 || (!deg && d2 <= 0);
   int64_t L;
   if (!s_lam || __ballot(lane < 16 && max(max(deg ? 0 : m, d1), d2) >= kLamLds))
     L = lam_of(a.lam, deg ? 0 : m) - lam_of(a.lam, d1) - lam_of(a.lam, d2);
