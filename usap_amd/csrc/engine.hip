@@ -1784,7 +1784,7 @@ __device__ __forceinline__ i128 block_entropy(const EntropyIn& a) {
 #pragma unroll
     for (int q = 0; q < kQ; ++q) {
       const int32_t i = i0 + q * (int32_t)blockDim.x;
-      v[q] = i < n ? a.cnt[i].o : 0;
+      v[q] = i < n ? max(a.cnt[i].o, 0) : 0;
     }
 #pragma unroll
     for (int q = 0; q < kQ; ++q) L[q] = a.lam[v[q]];
