@@ -67,6 +67,7 @@
 #include <numeric>
 #include <rocprim/rocprim.hpp>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "engine_internal.hpp"
@@ -6149,9 +6150,12 @@ namespace {
 // The host's wait for a word its last launch sets (kWord*): a few microseconds
 // after the kernel's store, where a stream synchronisation queues a marker and
 // sleeps on its interrupt (N = 20000, 106 sweeps: 21.6 us from a sweep's last
-// kernel to the next one's first, now 15).  A sweep that takes longer than
-// kSpinUs, or an error, is left to the synchronisation.  Profiled calls read
-// events and always synchronise.
+// kernel to the next one's first, now 15).  It yields between reads, so that with
+// more workers than CPUs the others run meanwhile (32 graphs of N = 4000, 8 workers
+// on 2 CPUs: 127 graphs/s synchronised, 221 without and 334 with the yield; on 16
+// CPUs, and for one engine, the same with it as without).  A sweep that takes
+// longer than kSpinUs, or an error, is left to the synchronisation.  Profiled
+// calls read events and always synchronise.
 enum { kWordShort = 0, kWordSweep = 1, kWordFx = 2 };
 constexpr int kSpinUs = 1000;
 
@@ -6168,9 +6172,10 @@ int wait_word(usap_engine* e, int slot) {
     for (int i = 0;; ++i) {
       if (__atomic_load_n(p, __ATOMIC_ACQUIRE) == e->word_want[slot]) return USAP_OK;
       __builtin_ia32_pause();
-      if (i % 64 == 63 &&
-          std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(kSpinUs))
-        break;
+      if (i % 64 == 63) {
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(kSpinUs)) break;
+        std::this_thread::yield();
+      }
     }
   }
   HIPCHK(hipStreamSynchronize(e->stream));
