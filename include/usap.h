@@ -367,9 +367,10 @@ typedef struct usap_serve_stats {
   int64_t max_bytes;    /* their summed footprint at the peak */
 } usap_serve_stats;
 
-/* Estimated device bytes of an engine for a graph of N nodes and E edges
- * (graph arrays, state, bucket sums and M slabs at B = N), used for
- * admission. */
+/* Device bytes that an engine for an unweighted graph of N nodes and E edges
+ * takes at most with the default slab_slack (graph arrays, state, bucket sums,
+ * build scratch, and M's slabs at the block count where they are largest),
+ * used for admission. */
 int64_t usap_footprint(int32_t N, int64_t E);
 
 /* Serves n graphs: graph g arrives at graphs[g].arrival_s and its stage k

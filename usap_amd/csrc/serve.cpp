@@ -226,14 +226,24 @@ extern "C" {
 int64_t usap_footprint(int32_t N, int64_t E) {
   if (N < 1 || E < 0) return 0;
   const int64_t n = N, m = E;
-  const int64_t graph = 16 * (n + 1) + 20 * m + 8 * (m + 1) + 8 * n + 96 * m;  // + lambda, large-node tables
-  const int64_t state = 160 * n + 24 * std::min<int64_t>(1 << 22, 2 * m + 4096) + 65536;
+  // lists with sources and weights, lambda (of an unweighted graph), tables of
+  // large nodes (at most 32 bytes a list entry), and what an append holds
+  // beside the new lists
+  const int64_t graph = 24 * n + 28 * m + 64 * m + 28 * m;
+  // per node: labels, block arrays, proposals, random words, carry-out's sort,
+  // four snapshots; parked increments; the growth state and MDL partials
+  const int64_t state = 252 * n + 16 * std::min<int64_t>(1 << 22, 2 * m + 4096) + 131072;
   const int64_t buckets = n * 512 * 4;  // bucket sums at B = N
-  // block-row slabs: 16-byte slots, three times the rows' capacities (each a
-  // power of two below 2 * (2 * (out + in edges) + 16), slab_slack 2) plus
-  // headroom
-  const int64_t pools = 16 * (3 * (8 * m + 32 * n) + 4 * n + 4096);
-  return graph + state + buckets + pools;
+  // counts of the histogram builds (256 parts of 256 x 256 at most), pairs of the sorted ones
+  const int64_t few = std::min<int64_t>(n, 256);
+  const int64_t builds = 4 * std::min<int64_t>(256, m / 4096 + 1) * (few * few + 1536) + 24 * m;
+  // block-row slabs, 12 bytes a slot, three times the largest M's.  A hashed row
+  // of ec entries has fewer than 2 * (2 * ec + 16) slots (slab_slack 2), a direct
+  // one has B, at most 8 times as many: with both ends of each edge fewer than
+  // 64 E + 32 B in all (reached where B * B is near that: B = 12500 at E = 4 M).
+  const int64_t slots = std::min<int64_t>(64 * m + 32 * n + 65536, n * n);
+  const int64_t pools = 12 * (3 * slots + 4 * n + 4096);
+  return graph + state + buckets + builds + pools;
 }
 
 int usap_serve(int32_t n, const usap_serve_graph* graphs, const usap_serve_opts* opt,
