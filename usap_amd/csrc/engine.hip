@@ -85,9 +85,9 @@ constexpr int kMergeWaves = 4;           // wavefronts per workgroup in k_merge
 constexpr int kNBK = 512;                // bucket sums per block row
 constexpr int kLookupRatio = 8;          // a hashed slab this many times a bucket is looked up per key
 constexpr int kScr = 1024;               // per-wavefront LDS scratch (ints) for one bucket
-constexpr int kMergeMany = 16;           // and for few blocks
+constexpr int kMergeMany = 16;           // and for at most kMergeFew blocks
+constexpr int32_t kMergeFew = 512;
 constexpr int32_t kMergeGrid = 8192;     // workgroups of k_merge over a list
-constexpr int32_t kMergeFew = 1024;
 constexpr int kDegLds = 1024;            // k_degrees privatises its counters for B <= this
 constexpr int kHistB = 256;              // M is built by histograms in LDS up to here
 constexpr int kEntropyBlocks = 4096;  // k_entropy grid at most
@@ -2392,9 +2392,10 @@ struct MergeList {
 };
 
 // The K proposals of a block by one workgroup, a wavefront each in turn: every
-// block, or those k_merge_rows left to it.  kWaves: 4, or, where
-// the blocks are too few to fill the GPU, up to 16, so that all of a block's
-// proposals run at once (B = 42: 26 -> 13 us a round).
+// block, or those k_merge_rows left to it.  kWaves: 4, or, where the blocks are
+// too few to fill the GPU, up to 16, so that all of a block's proposals run at
+// once (K = 10, us a round with 4 and 16: B = 20 19 and 14, 100 24 and 17, 300 41 and
+// 41, 500 54 and 53, 800 58 and 77, 1000 68 and 97).
 // kKeys: kRowLds or kRowLdsFew.  The list's long rows come first: one of 20000 slots
 // is the length of the launch, and started last it adds to it.  A workgroup
 // takes every gridDim.x-th item; kMergeGrid of them are handed out as others end,
