@@ -5175,9 +5175,9 @@ int build_hist(usap_engine* e) {
   a.part = e->hist;
   a.part_d = e->hist + (int64_t)G * B * B;
   const dim3 grid((unsigned)G, (unsigned)halves);
-  if (B * a.rows <= 4096)
-    k_hist<4096><<<grid, kHistThreads, 0, st>>>(a);
-  else if (B * a.rows <= 16384)
+  // LDS for 128 blocks leaves room for two workgroups a CU, for all 200 for one
+  // (B = 128, E = 4 M 26 and 28 us)
+  if (B * a.rows <= 16384)
     k_hist<16384><<<grid, kHistThreads, 0, st>>>(a);
   else
     k_hist<kHistOne * kHistOne><<<grid, kHistThreads, 0, st>>>(a);
@@ -5223,6 +5223,10 @@ int rebuild_M(usap_engine* e) {
   if (e->N > 0) {
     const auto k = e->out_w ? (B <= kDegLds ? k_degrees<true, false> : k_degrees<true, true>)
                             : (B <= kDegLds ? k_degrees<false, false> : k_degrees<false, true>);
+    // fewer nodes a workgroup while full ones would leave CUs without any (N =
+    // 20000, B = 1000: 256 nodes 4.1 us and 1024 5.6, weighted 64 16 and 256 26), more
+    // where the workgroups' sums meet on the blocks' counters (N = 500000, B = 1000:
+    // 256 47 and 1024 17, weighted 64 126 and 256 120)
     const int32_t per = e->out_w ? (e->N < 65536 ? 64 : kNodesWgW) : (e->N < 65536 ? 256 : kNodesWg);
     k<<<blocks_for(e->N, per), 256, 0, st>>>(gview(e), e->labels, B, per, e->d_out, e->d_in,
                                              e->ecnt_out, e->ecnt_in, e->bsize);
