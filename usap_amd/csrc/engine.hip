@@ -1508,8 +1508,10 @@ __global__ void k_insert_pairs(int64_t E, const uint32_t* __restrict__ key,
 // B = 513, 12.3 at 2000, 26 at 4000 and 38 at 5000, of 16 11.8, 31, 62 and 75.  Above
 // B = 16384 few rows keep sums and one may be longer than 4 wavefronts take in a
 // few rounds: a direct row of 100000 slots costs 33 us more with 4, blocks of
-// thousands of nodes at B = 20000 take 93 with 4 and 96 with 16.  Sets the hashed
-// ones' marks too (room_mark).
+// thousands of nodes at B = 20000 take 93 with 4 and 96 with 16; fewer rows a
+// workgroup do not help there (two launches at B = 200000 and 100000 89 us with up
+// to 64 and 49 rows, 103 with 49 and 25).  Sets the hashed ones' marks too
+// (room_mark).
 constexpr int kSumRows = 64;
 constexpr int32_t kSumLongB = 16384;
 __global__ __launch_bounds__(1024) void k_bucket_sums(MView m, int32_t rows) {
@@ -5273,8 +5275,9 @@ int rebuild_M(usap_engine* e) {
     if (int rc = build_by_pairs(e)) return rc;
   }
   if (B > kNBK) {
-    const int32_t rows = std::min(kSumRows, 1 + B / 4096);
-    k_bucket_sums<<<blocks_for(B, rows), B > kSumLongB ? 1024 : 256, 0, st>>>(view(e->M, B), rows);
+    const bool lng = B > kSumLongB;
+    const int32_t rows = std::min(kSumRows, 1 + B / (lng ? 2048 : 4096));
+    k_bucket_sums<<<blocks_for(B, rows), lng ? 1024 : 256, 0, st>>>(view(e->M, B), rows);
   }
   HIPCHK(hipGetLastError());
   ev_rec(e, 1);
