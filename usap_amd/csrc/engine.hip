@@ -29,7 +29,7 @@
 //        few blocks, by LDS histograms
 //   k_degrees / k_caps / k_fill / k_insert_pairs / k_node_lists / k_build_* /
 //        k_bucket_sums : for more, by sorted block pairs or row by row
-//   k_merge_rows / k_merge : K merge proposals per block + best per block
+//   k_merge_rows / k_merge_list / k_merge : K merge proposals per block + best per block
 //        (graph_parallel.hpp:349-368, :761-988), one wavefront per block, or
 //        one workgroup with a wavefront per proposal
 //   k_carry_* : the greedy carry-out (graph_parallel.hpp:1225-1279)
@@ -555,17 +555,20 @@ __device__ __forceinline__ uint32_t idx32(uint64_t x, uint32_t W) {
   return (uint32_t)((hi + (lo >> 32)) >> 32);
 }
 
-// A sum of terms m * lambda, |m| < 2^31 (a count, degree or sum of them),
-// |lambda| < 2^54: each lambda is split at bit 24 and the two products are
-// summed apart, value = h * 2^24 + l, so a term is two 32-bit multiply-adds
-// (an int128 product of 64-bit operands is about ten, at a quarter of the
-// ALU's rate).  Exact: the terms of one dS or MDL change or hold disjoint
-// edges' counts, so the |m| of each kind of term sum to at most the total
-// weight (< 2^31), at most four kinds of term do so, and |lambda| <= ln(2^31)
-// * 2^48 < 2^52.5 puts |h| below 2^62 and |l| below 2^58.  With the wavefront
-// sums by DPP and a dS's 16 uniform terms spread over 16 lanes it took
-// k_nodal from 126 to 90 VGPRs, a resumed chain at N = 50000 from 2.60 to
-// 2.19 ms and the N = 20000 partition from 25.5 to 22.5 ms.
+// A sum of terms m * L, |m| < 2^31 (a count, degree or sum of them), L a lambda
+// or lambda(m) - lambda(x) - lambda(y), |L| < 2^54: each L is split at bit 24 and
+// the two products are summed apart, value = h * 2^24 + l, so a term is two 32-bit
+// multiply-adds (an int128 product of 64-bit operands is about ten, at a quarter
+// of the ALU's rate).  Exact, with W < 2^31 the total weight and lambda <= A =
+// ln(2^31) * 2^48 < 2^52.43: out-edges of two blocks weigh at most W together, and
+// so do their in-edges.  With C in the corner of the two, a dS has on each side,
+// before and after, at most 2 (W - C) in its rows' other counts at A each, C in the
+// corner at up to 2 A each, and 2 (W - C) in degree terms at A each (a merge: the
+// same, its counts in the overlap).  That is below 4 W A a side, 8 W A in all, and
+// an MDL's three sums are below 3 W A: |h| < 2^62.5, and |l| < 8 W 2^24 = 2^58.  With the
+// wavefront sums by DPP and a dS's 16 uniform terms spread over 16 lanes it took
+// k_nodal from 126 to 90 VGPRs, a resumed chain at N = 50000 from 2.60 to 2.19 ms
+// and the N = 20000 partition from 25.5 to 22.5 ms.
 constexpr int kAccSplit = 24;
 struct Acc {
   long h, l;
@@ -1561,12 +1564,6 @@ __global__ __launch_bounds__(1024) void k_bucket_sums(MView m, int32_t rows) {
   }
 }
 
-// Workgroup stamps of profiled batch launches (100 MHz wall clock; 0 = the
-// workgroup did not run).  Each workgroup of a profiled k_nodal, k_apply or
-// k_grow writes its start at t[b] and its end at t[stride + b] with plain
-// stores: one atomic per workgroup on a shared word costs more than the
-// kernel's own tail.  Per batch slot: k_nodal's starts and ends (G each),
-// k_apply's (G + 1 each), k_grow's (kGrowBlocks each).
 // The per-block counters and flags a rebuild starts from, zeroed in one
 // launch (degrees, edge counts, sizes, growth marks, parked
 // counts: B entries each; build_flags[0..2]).
@@ -1585,6 +1582,12 @@ __global__ void k_clear_build(ClearArgs c) {
   if (blockIdx.x == 0 && threadIdx.x < 3) c.flags[threadIdx.x] = 0;
 }
 
+// Workgroup stamps of profiled batch launches (100 MHz wall clock; 0 = the
+// workgroup did not run).  Each workgroup of a profiled k_nodal, k_apply or
+// k_grow writes its start at t[b] and its end at t[stride + b] with plain
+// stores: one atomic per workgroup on a shared word costs more than the
+// kernel's own tail.  Per batch slot: k_nodal's starts and ends (G each),
+// k_apply's (G + 1 each), k_grow's (kGrowBlocks each).
 __global__ void k_stamp_init(unsigned long long* t, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
@@ -3004,7 +3007,12 @@ __device__ __forceinline__ uint32_t unit_key(int32_t b, bool in) {
 // lane): N = 1000 12.1 -> 5.8 us, N = 20000 (5000-node batches) 28.8 -> 9.8, N =
 // 50000 (12500-node batches) 42.5 -> 15.8, 4096-node batches at B = 100000 28.8
 // -> 17.5 and at B = 250000 29.2 -> 21.9 (20.1 and 27.3 with single slots and
-// the whole lambda table).
+// the whole lambda table).  Registers: dense 96 VGPRs, none spilled but one with
+// hub code; hashed all 128 that four wavefronts a SIMD leave, where U = 4 with its
+// windows spills 2 with hub code, 19 weighted and 24 both (60 bytes a lane; hub
+// code also spills 99 to 145 scalar registers to vector ones).  A weighted sweep
+// on hashed rows takes 4-7% longer than an unweighted one all the same (N = 50000,
+// B = 25000, 4096-node batches 623 and 596 us).
 template <bool kD, bool kW, int U>
 __device__ __forceinline__ void nodal_regs(const NodalArgs& a, int32_t n, int32_t r, int64_t o0,
                                            int64_t i0, int32_t kco, int32_t kc,
@@ -4832,8 +4840,9 @@ struct usap_engine {
   uint64_t g_epoch = 0;
   uint64_t epoch = 0;  // bumped by every device allocation (pointers may change)
   int64_t graph_captures = 0;
-  int32_t* build_flags = nullptr;  // [0] build overflow flags, [1] blocks holding != 1 node,
-                                   // [2] distinct block pairs, [3] carry-out out of candidates
+  int32_t* build_flags = nullptr;  // [0] build overflow flags; [1] pieces of large rows (a build's),
+                                   // [2] distinct block pairs (a build's); both: rows left to
+                                   // k_merge (MergeList::n); [3] carry-out out of candidates
   int32_t* h_short = nullptr;      // the last in pinned host memory, and its device address
   int32_t* d_short = nullptr;
   int32_t word_want[3] = {0, 0, 0};
@@ -5093,10 +5102,9 @@ int build_by_pairs(usap_engine* e) {
   return USAP_OK;
 }
 
-// Full M build from the labels (graph_parallel.hpp:703-759).
-// The M build for B > kPairSortB: nodes grouped by block (offsets by an
-// exclusive scan of the block sizes, then a scatter), k_build_rows for the
-// rows it lays out in LDS, per-edge inserts for the others.
+// The M build by rows: nodes grouped by block (offsets by an exclusive scan of
+// the block sizes, then a scatter), k_build_rows for the rows it lays out in LDS,
+// k_fill_big and k_build_big for the others.
 int build_rows(usap_engine* e) {
   const int32_t B = e->B;
   hipStream_t st = e->stream;
@@ -5199,6 +5207,7 @@ int build_hist(usap_engine* e) {
   return USAP_OK;
 }
 
+// Full M build from the labels (graph_parallel.hpp:703-759).
 int rebuild_M(usap_engine* e) {
   const int32_t B = e->B;
   hipStream_t st = e->stream;
@@ -5556,13 +5565,12 @@ int build_big_tables(usap_engine* e) {
   e->n_huge = 0;
   TRY(dalloc(e, &e->big_off, N));
   TRY(dalloc(e, &e->big_tab, big_total));
+  TRY(dalloc(e, &e->huge_parts, huge.size()));
   HIPCHK(hipMemcpyAsync(e->big_off, big.data(), sizeof(int64_t) * N, hipMemcpyHostToDevice, e->stream));
-  if (!huge.empty()) {
-    TRY(dalloc(e, &e->huge_parts, huge.size()));
+  if (!huge.empty())
     HIPCHK(hipMemcpyAsync(e->huge_parts, huge.data(), sizeof(int2) * huge.size(),
                           hipMemcpyHostToDevice, e->stream));
-    e->n_huge = (int32_t)huge.size();
-  }
+  e->n_huge = (int32_t)huge.size();
   HIPCHK(hipStreamSynchronize(e->stream));  // the vectors are released on return
   return USAP_OK;
 }
